@@ -45,6 +45,11 @@ struct HeavyRow {
   uint64_t r;
 };
 
+// A work queue of the persistent kernels: WQ counters a cache line apart.
+constexpr uint32_t WQ = 8, WQ_STRIDE = 16, WQ_WORDS = WQ * WQ_STRIDE;
+// Counters of one task group of a streamed launch: 5 queues, 2 heavy-row counts.
+constexpr uint32_t GROUP_WORDS = 5 * WQ_WORDS + WQ_STRIDE;
+
 struct VQueryState {
   const QueryDev *qd = nullptr;
   // A relaxed query sharing its parent's candidates and tables: planned on its

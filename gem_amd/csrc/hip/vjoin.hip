@@ -45,7 +45,7 @@ namespace gemd {
 constexpr uint32_t VB = 256;  // rows per task block
 constexpr uint32_t VW = VB / 64;
 // survivors a wave stages in LDS before it reserves output rows for them (a
-// step adds at most 128)
+// step of k_vext adds at most 256, one of k_vext_heavy 128)
 constexpr uint32_t VSTAGE = 512;
 
 __device__ __forceinline__ uint32_t vposition_in(const uint64_t *bm, const uint32_t *rank, uint32_t v) {
@@ -74,19 +74,17 @@ __device__ __forceinline__ uint32_t find_item(const uint64_t *blk_prefix, uint32
 // ------------------------------------------------------------ length pass
 // Per 64-row unit (wave w of 256-row block g -> unit_u[4g + w]): the sum over
 // its rows of the shortest backward list, an upper bound on its output rows.
+// Rows cost nearly the same (one offset pair per list), so blocks take the
+// 256-row tasks in turn: a work queue is one device-wide atomic per task, about
+// 11.5 ns each on one address, which bounded this kernel (4.5 ms for the
+// 400,000 tasks of a 10^8-row level, whose reads take a tenth of that).
 __global__ void __launch_bounds__(VB) k_vlen(const VItem *__restrict__ items, uint32_t nitems,
-                                            const uint64_t *__restrict__ blk_prefix,
-                                            unsigned int *__restrict__ queue, uint64_t *__restrict__ unit_u) {
-  __shared__ uint32_t task;
+                                            const uint64_t *__restrict__ blk_prefix, uint64_t *__restrict__ unit_u) {
   const uint64_t total = blk_prefix[nitems];
-  for (;;) {
-    if (threadIdx.x == 0) task = atomicAdd(queue, 1u);
-    __syncthreads();
-    const uint64_t g = task;
-    __syncthreads();
-    if (g >= total) break;
-    const uint32_t t = find_item(blk_prefix, nitems, g);
-    const VItem it = items[t];
+  uint32_t t = 0;
+  for (uint64_t g = blockIdx.x; g < total; g += gridDim.x) {
+    while (blk_prefix[t + 1] <= g) ++t;
+    const VItem &it = items[t];
     GLevel &L = *(GLevel *)it.lv;
     const uint64_t r = it.row_begin + (g - blk_prefix[t]) * VB + threadIdx.x;
     uint64_t u = 0;
@@ -105,6 +103,47 @@ __global__ void __launch_bounds__(VB) k_vlen(const VItem *__restrict__ items, ui
   }
 }
 
+// Runs of consecutive tasks handed to the waves of a persistent grid.  Wave
+// w starts on run w without asking; later runs come from nq = min(WQ, waves)
+// counters (wave w asks counter w % nq, which hands out the runs that are w
+// modulo nq, so every counter has a wave that empties it).  One
+// counter is an atomic on one address, which the device serves one per 11.5
+// ns whatever asks: 8,192 waves finding an empty queue took 95 us, and a queue
+// of 64-row tasks bounded every large launch.  Runs are as long as leaves a
+// wave about CLAIMS of them, so uneven tasks still even out.
+constexpr uint32_t CLAIMS = 8, MAX_RUN = 32;
+struct Runs {
+  uint64_t ntask, nrun, run;
+  uint32_t per, nq, sub, given;
+  unsigned int *q;
+  // w, nw: this wave and the waves of the grid
+  __device__ __forceinline__ Runs(uint64_t n, uint32_t w, uint32_t nw, uint32_t max_run, unsigned int *queue)
+      : ntask(n), run(w) {
+    const uint64_t p = n / ((uint64_t)nw * CLAIMS);
+    per = p < 1 ? 1 : p > max_run ? max_run : (uint32_t)p;
+    nrun = (n + per - 1) / per;
+    nq = nw < WQ ? nw : WQ;
+    sub = w % nq;
+    given = (nw - sub + nq - 1) / nq;
+    q = queue + sub * WQ_STRIDE;
+  }
+  __device__ __forceinline__ bool valid() const { return run < nrun; }
+  __device__ __forceinline__ uint64_t begin() const { return run * per; }
+  __device__ __forceinline__ uint64_t end() const {
+    const uint64_t e = run * per + per;
+    return e < ntask ? e : ntask;
+  }
+  __device__ __forceinline__ void next() {
+    if ((uint64_t)given * nq + sub >= nrun) {  // every run was given at the start
+      run = nrun;
+      return;
+    }
+    uint32_t c = 0;
+    if (lane_id() == 0) c = atomicAdd(q, 1u);
+    run = ((uint64_t)given + readlane_u32(c, 0)) * nq + sub;
+  }
+};
+
 // Device address of the list of key p in backward table j (b = its first
 // offset): in HBM, or through the streamed tables' block map.
 template <bool OOC>
@@ -114,8 +153,7 @@ __device__ __forceinline__ uint64_t list_addr(GLevel &L, uint32_t j, uint32_t p,
 }
 
 // ------------------------------------------------------ extend (walk) pass
-// Each wave pulls 64-row tasks from the launch's queue on its own (no block
-// barrier).  For each of its rows the shortest backward list drives; a row
+// Each wave takes runs of 64-row tasks on its own (no block barrier).  For each of its rows the shortest backward list drives; a row
 // whose driving list is longer than heavy_t is not walked here but appended to
 // the heavy-row list (when it has room), which k_vext_heavy then walks in
 // fixed-size chunks spread over all waves: a hub row no longer holds one wave
@@ -124,8 +162,9 @@ __device__ __forceinline__ uint64_t list_addr(GLevel &L, uint32_t j, uint32_t p,
 // dup positions ndup x 64 u32 (blocks of one wave when four waves' share
 // would not fit a block's LDS).
 // Survivors are written as whole rows: their (parent row, new value) pairs are
-// staged in LDS, then the wave writes the step's new rows as one run of
-// consecutive words.
+// staged in LDS, over all tasks of the item that the wave has in hand, then
+// the wave reserves output rows for all of them at once (one atomic on the
+// item's counter) and writes them as one run of consecutive words.
 // The item count is read from device memory so that one captured graph can
 // replay the launch for any number of items.  Tasks [g_begin, g_end) of the
 // launch (256-row units) are processed (streamed tables run a launch in task
@@ -138,31 +177,65 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
        uint64_t g_end, HeavyRow *__restrict__ heavy, unsigned int *__restrict__ heavy_n, uint32_t heavy_cap,
        uint32_t heavy_t) {
   const uint32_t nitems = *nitems_p;
+  const uint64_t total = blk_prefix[nitems] < g_end ? blk_prefix[nitems] : g_end;
+  if (g_begin >= total) return;
   __shared__ uint32_t st[VW][65];
   __shared__ uint64_t drv[VW][64];  // address of each row's driving list
-  __shared__ uint8_t sv_row[VW][VSTAGE];    // staged survivors of the task: row in the task
+  __shared__ uint32_t sv_row[VW][VSTAGE];  // staged survivors: row in the item's range
   __shared__ uint32_t sv_val[VW][VSTAGE];  // and new value
   extern __shared__ unsigned char vlds[];
-  const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
+  const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64;
   const uint32_t per_wave = 64 * ((max_nb > 0 ? max_nb - 1 : 0) * 12 + max_ndup * 4);
   unsigned char *mine = vlds + (size_t)w * per_wave;
   uint64_t *obase = reinterpret_cast<uint64_t *>(mine);                                  // [nb-1][64]
   uint32_t *olen = reinterpret_cast<uint32_t *>(mine + (size_t)64 * 8 * (max_nb - 1));   // [nb-1][64]
   uint32_t *dpos = reinterpret_cast<uint32_t *>(mine + (size_t)64 * 12 * (max_nb - 1));  // [ndup][64]
-  const uint64_t total = blk_prefix[nitems] < g_end ? blk_prefix[nitems] : g_end;
   uint64_t walked = 0, written = 0;
-  for (;;) {
-    uint32_t wt = 0;
-    if (l == 0) wt = atomicAdd(queue, 1u);
-    wt = readlane_u32(wt, 0);
-    const uint64_t q = g_begin * VW + wt;  // 64-row task
-    if (q >= total * VW) break;
+  uint32_t t = NOT_FOUND;  // item in hand
+  VItem it{};
+  uint64_t survivors = 0;  // final level: survivors of the item in hand
+  uint32_t pend = 0;       // survivors staged in LDS, not yet written
+  // write the staged survivors: one reservation for all of them, then
+  // their rows as one run of consecutive words (word q is column q % (k+1)
+  // of survivor q / (k+1): k parent columns, then the value).  q / (k+1) by
+  // the reciprocal rounded up: exact while q * (k+1) < 2^32.
+  auto flush = [&]() {
+    if (FINAL) {
+      if (l == 0 && survivors) atomicAdd(it.counter, (unsigned long long)survivors);
+      survivors = 0;
+      return;
+    }
+    if (!pend) return;
+    uint64_t base = 0;
+    if (l == 0) base = atomicAdd(it.counter, (unsigned long long)pend);
+    base = readlane_u64(base, 0);
+    const uint32_t k = it.k, rl = k + 1, inv = 0xFFFFFFFFu / rl + 1;
+    written += (uint64_t)pend * 4 * rl;
+    for (uint32_t q = l; q < pend * rl; q += 64) {
+      const uint32_t i = __umulhi(q, inv), c = q - i * rl;
+      if (base + i < it.out_cap)
+        stg(it.out + (base + i) * rl + c,
+            c < k ? ldg(it.rows + (it.row_begin + sv_row[w][i]) * k + c) : sv_val[w][i]);
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    pend = 0;
+  };
+  const uint32_t bw = blockDim.x / 64;
+  Runs runs((total - g_begin) * VW, blockIdx.x * bw + w, gridDim.x * bw, MAX_RUN, queue);
+  for (; runs.valid(); runs.next())
+  for (uint64_t q = g_begin * VW + runs.begin(), qe = g_begin * VW + runs.end(); q < qe; ++q) {  // 64-row task
     const uint64_t g = q / VW;
-    const uint32_t t = find_item(blk_prefix, nitems, g);
-    const VItem it = items[t];
+    if (t == NOT_FOUND || g < blk_prefix[t] || g >= blk_prefix[t + 1]) {
+      if (t != NOT_FOUND) flush();
+      t = find_item(blk_prefix, nitems, g);
+      it = items[t];
+    }
     GLevel &L = *(GLevel *)it.lv;
     const uint32_t nb = L.nb, ndup = L.ndup, k = it.k;
     const uint64_t rbase = it.row_begin + (g - blk_prefix[t]) * VB + (q % VW) * 64;
+    if (rbase >= it.row_end) continue;
+    const uint32_t roff = (uint32_t)(rbase - it.row_begin);
     const uint64_t r = rbase + l;
     const bool valid = r < it.row_end;
     const uint32_t *row = it.rows + r * k;
@@ -183,12 +256,15 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
           dp = p;
         }
       }
-      if (heavy && dlen > heavy_t) {
-        const uint32_t h = atomicAdd(heavy_n, 1u);
-        if (h < heavy_cap) {
-          heavy[h] = HeavyRow{t, dlen, r};
-          dlen = 0;  // walked by k_vext_heavy
-        }
+    }
+    const uint64_t hv = heavy ? __ballot(dlen > heavy_t) : 0;
+    if (hv) {
+      uint32_t h = 0;
+      if (l == 0) h = atomicAdd(heavy_n, (uint32_t)__popcll(hv));
+      h = readlane_u32(h, 0) + rank_below(hv);
+      if (((hv >> l) & 1ull) && h < heavy_cap) {
+        heavy[h] = HeavyRow{t, dlen, r};
+        dlen = 0;  // walked by k_vext_heavy
       }
     }
     // a row with nothing to walk here (empty driving list, or set aside as a
@@ -219,26 +295,6 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     walked += wtotal;
-    uint64_t survivors = 0;
-    uint32_t pend = 0;  // survivors staged in LDS, not yet written
-    // write the staged survivors: one reservation for all of them, then
-    // their rows as one run of consecutive words (word q is column q % (k+1)
-    // of survivor q / (k+1): k parent columns, then the value)
-    auto flush = [&]() {
-      uint64_t base = 0;
-      if (l == 0) base = atomicAdd(it.counter, (unsigned long long)pend);
-      base = readlane_u64(base, 0);
-      written += (uint64_t)pend * 4 * (k + 1);
-      const uint32_t rl = k + 1;
-      for (uint32_t q = l; q < pend * rl; q += 64) {
-        const uint32_t i = q / rl, c = q - i * rl;
-        if (base + i < it.out_cap)
-          stg(it.out + (base + i) * rl + c, c < k ? ldg(it.rows + (rbase + sv_row[w][i]) * k + c) : sv_val[w][i]);
-      }
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      pend = 0;
-    };
     // 256 items per step, four per lane (items s + 64 g + l), so that each
     // lane has four loads in flight at every stage of the probes
     for (uint32_t s = 0; s < wtotal; s += 256) {
@@ -283,7 +339,7 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
         for (int g = 0; g < 4; ++g)
           if (keep[g]) {
             const uint32_t i = pend + before[g] + rank_below(m[g]);
-            sv_row[w][i] = rw[g];
+            sv_row[w][i] = roff + rw[g];
             sv_val[w][i] = val[g];
           }
         __builtin_amdgcn_wave_barrier();
@@ -292,12 +348,11 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
         if (pend > VSTAGE - 256) flush();
       }
     }
-    if (!FINAL && pend) flush();
-    if (FINAL && l == 0 && survivors) atomicAdd(it.counter, (unsigned long long)survivors);
     // st / drv / LDS lists of this wave are rewritten by its next task
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   }
+  if (t != NOT_FOUND) flush();
   if (prof_items && l == 0 && walked) atomicAdd(prof_items, (unsigned long long)walked);
   if (prof_out && l == 0 && written) atomicAdd(prof_out, (unsigned long long)written);
 }
@@ -338,16 +393,16 @@ k_vext_heavy(const VItem *__restrict__ items, const HeavyRow *__restrict__ heavy
   __shared__ uint32_t olen[VW][GEM_MAX_QV], dpos[VW][GEM_MAX_QV];
   __shared__ uint32_t wend[VW][64];   // window ends in the first other list
   __shared__ uint32_t win[VW][HWIN];  // staged window
-  __shared__ uint32_t prow[VW][GEM_MAX_QV], hsv[VW][128];  // parent row, this step's surviving values
-  const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
+  __shared__ uint32_t prow[VW][GEM_MAX_QV], hsv[VW][VSTAGE];  // parent row, staged surviving values
+  const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64;
   const uint32_t n = *heavy_n < heavy_cap ? *heavy_n : heavy_cap;
   const uint64_t total = pre[n];
+  if (!total) return;
   uint64_t walked = 0, written = 0;
-  for (;;) {
-    uint32_t wt = 0;
-    if (l == 0) wt = atomicAdd(queue, 1u);
-    wt = readlane_u32(wt, 0);
-    if (wt >= total) break;
+  const uint32_t bw = blockDim.x / 64;
+  Runs runs(total, blockIdx.x * bw + w, gridDim.x * bw, 1, queue);  // a piece is long enough to ask for one at a time
+  for (; runs.valid(); runs.next()) {
+    const uint64_t wt = runs.begin();
     const uint32_t h = find_item(pre, n, wt);
     const HeavyRow e = heavy[h];
     const VItem it = items[e.t];
@@ -388,6 +443,23 @@ k_vext_heavy(const VItem *__restrict__ items, const HeavyRow *__restrict__ heavy
     const uint64_t s1 = s0 + chunk < dlen ? s0 + chunk : dlen;
     walked += s1 - s0;
     uint64_t survivors = 0;
+    uint32_t pend = 0;  // surviving values staged, not yet written
+    // the staged rows share the parent row: pend * (k + 1) consecutive words
+    // of the output, reserved by one atomic, written by consecutive lanes
+    auto flush = [&]() {
+      uint64_t base = 0;
+      if (l == 0) base = atomicAdd(it.counter, (unsigned long long)pend);
+      base = readlane_u64(base, 0);
+      const uint32_t rl = k + 1, inv = 0xFFFFFFFFu / rl + 1;
+      written += (uint64_t)pend * 4 * rl;
+      for (uint32_t q = l; q < pend * rl; q += 64) {
+        const uint32_t i = __umulhi(q, inv), c = q - i * rl;
+        if (base + i < it.out_cap) stg(it.out + (base + i) * rl + c, c < k ? prow[w][c] : hsv[w][i]);
+      }
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      pend = 0;
+    };
     // Two items per lane per step, as in k_vext.  The first other list is
     // probed through windows: for each 128-entry step of the chunk, the range
     // of that list that can hold the step's values (both lists are sorted and
@@ -443,29 +515,19 @@ k_vext_heavy(const VItem *__restrict__ items, const HeavyRow *__restrict__ heavy
         if (FINAL) {
           survivors += nk;
         } else if (nk) {
-          uint64_t base = 0;
-          if (l == 0) base = atomicAdd(it.counter, (unsigned long long)nk);
-          base = readlane_u64(base, 0);
-          written += (uint64_t)nk * 4 * (k + 1);
-          // the nk new rows share the parent row: they are nk * (k + 1)
-          // consecutive words of the output, written by consecutive lanes
-          if (keep0) hsv[w][rank_below(m0)] = val0;
-          if (keep1) hsv[w][nk0 + rank_below(m1)] = val1;
+          if (keep0) hsv[w][pend + rank_below(m0)] = val0;
+          if (keep1) hsv[w][pend + nk0 + rank_below(m1)] = val1;
           __builtin_amdgcn_wave_barrier();
           __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-          const uint32_t rl = k + 1;
-          for (uint32_t q = l; q < nk * rl; q += 64) {
-            const uint32_t r = q / rl, c = q - r * rl;
-            if (base + r < it.out_cap) stg(it.out + (base + r) * rl + c, c < k ? prow[w][c] : hsv[w][r]);
-          }
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+          pend += nk;
+          if (pend > VSTAGE - 128) flush();
         }
       }
       // wend of this wave is rewritten by the next group of steps
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
+    if (!FINAL && pend) flush();
     if (FINAL && l == 0 && survivors) atomicAdd(it.counter, (unsigned long long)survivors);
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -474,31 +536,48 @@ k_vext_heavy(const VItem *__restrict__ items, const HeavyRow *__restrict__ heavy
   if (prof_out && l == 0 && written) atomicAdd(prof_out, (unsigned long long)written);
 }
 
-// Last level, one backward list: |list| - equal-label columns present.
+// Last level, one backward list: |list| - equal-label columns present.  A
+// block takes runs of 256-row tasks and keeps its count while they belong to
+// one item, so an item's counter sees one atomic per block and item change
+// (with one per 256 rows, and one for the work queue, two atomics bounded the
+// kernel: 6.4 ms for the 280,000 tasks of a 7 * 10^7-row level).
 template <bool OOC>
 __global__ void __launch_bounds__(VB) k_vcount1(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p,
                                                const uint64_t *__restrict__ blk_prefix,
                                                unsigned int *__restrict__ queue, uint64_t g_begin, uint64_t g_end) {
   const uint32_t nitems = *nitems_p;
-  __shared__ uint32_t task;
-  __shared__ uint64_t sm[VW];
   const uint64_t total = blk_prefix[nitems] < g_end ? blk_prefix[nitems] : g_end;
-  for (;;) {
-    if (threadIdx.x == 0) task = atomicAdd(queue, 1u);
+  if (g_begin >= total) return;
+  __shared__ uint64_t sm[VW], next_run;
+  uint32_t t = NOT_FOUND;  // item in hand
+  VItem it{};
+  uint64_t cnt = 0;  // this thread's part of the item's count
+  auto flush = [&]() {
+    const uint64_t c = wave_sum_u64(cnt);
+    cnt = 0;
+    if (threadIdx.x % 64 == 0) sm[threadIdx.x / 64] = c;
     __syncthreads();
-    const uint64_t g = g_begin + task;
+    if (threadIdx.x == 0) {
+      const uint64_t s = sm[0] + sm[1] + sm[2] + sm[3];
+      if (s) atomicAdd(it.counter, (unsigned long long)s);
+    }
     __syncthreads();
-    if (g >= total) break;
-    const uint32_t t = find_item(blk_prefix, nitems, g);
-    const VItem it = items[t];
-    GLevel &L = *(GLevel *)it.lv;
-    const uint64_t r = it.row_begin + (g - blk_prefix[t]) * VB + threadIdx.x;
-    uint64_t cnt = 0;
-    if (r < it.row_end) {
+  };
+  Runs runs(total - g_begin, blockIdx.x, gridDim.x, MAX_RUN, queue);
+  while (runs.valid()) {
+    for (uint64_t g = g_begin + runs.begin(), ge = g_begin + runs.end(); g < ge; ++g) {
+      if (t == NOT_FOUND || g < blk_prefix[t] || g >= blk_prefix[t + 1]) {
+        if (t != NOT_FOUND) flush();
+        t = find_item(blk_prefix, nitems, g);
+        it = items[t];
+      }
+      GLevel &L = *(GLevel *)it.lv;
+      const uint64_t r = it.row_begin + (g - blk_prefix[t]) * VB + threadIdx.x;
+      if (r >= it.row_end) continue;
       const uint32_t *row = it.rows + r * it.k;
       const uint32_t p = ldg(row + L.key_col[0]);
       const uint64_t b = ldg(L.toff[0] + p), e = ldg(L.toff[0] + p + 1);
-      cnt = e - b;
+      cnt += e - b;
       const uint32_t *lst = nullptr;
       if (L.ndup) lst = reinterpret_cast<const uint32_t *>(list_addr<OOC>(L, 0, p, b));
       for (uint32_t c = 0; c < L.ndup; ++c) {
@@ -506,15 +585,16 @@ __global__ void __launch_bounds__(VB) k_vcount1(const VItem *__restrict__ items,
         if (pos != NOT_FOUND && sorted_contains(lst, e - b, pos)) --cnt;
       }
     }
-    cnt = wave_sum_u64(cnt);
-    if (threadIdx.x % 64 == 0) sm[threadIdx.x / 64] = cnt;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const uint64_t s = sm[0] + sm[1] + sm[2] + sm[3];
-      if (s) atomicAdd(it.counter, (unsigned long long)s);
+    // the block's first wave asks for the next run
+    if (threadIdx.x < 64) {
+      runs.next();
+      if (threadIdx.x == 0) next_run = runs.run;
     }
     __syncthreads();
+    runs.run = next_run;
+    __syncthreads();
   }
+  if (t != NOT_FOUND) flush();
 }
 
 // Streamed tables: for every table block a row of the launch will read, the
@@ -659,17 +739,15 @@ struct Launch {
 
 // Upload an item table + block prefix, return device pointers (kept alive by bufs).
 struct DevLaunch {
-  DevBuf items, blk, queue;
+  DevBuf items, blk;
 };
 
 void upload(gem_ctx *c, const Launch &L, DevLaunch &D) {
   hipStream_t s = c->stream;
   D.items.alloc(sizeof(VItem) * L.items.size(), s);
   D.blk.alloc(8 * L.blk.size(), s);
-  D.queue.alloc(4, s);
   GEM_HIP_CHECK(hipMemcpyAsync(D.items.p, L.items.data(), sizeof(VItem) * L.items.size(), hipMemcpyHostToDevice, s));
   GEM_HIP_CHECK(hipMemcpyAsync(D.blk.p, L.blk.data(), 8 * L.blk.size(), hipMemcpyHostToDevice, s));
-  GEM_HIP_CHECK(hipMemsetAsync(D.queue.p, 0, 4, s));
 }
 
 // persistent grid: enough blocks to fill the chip (tunable cap), never more
@@ -696,11 +774,13 @@ constexpr uint32_t HEAVY_CAP = 1u << 20;
 // is captured once as a hipGraph and replayed each iteration (no memset node:
 // the zeroed counters travel in the header copy).
 struct ExtSlot {
-  // header: item counts [3], queues [3 main + 2 heavy], heavy-row counts [2],
-  // profile counters [6] (u64: entries walked by the write / final / heavy
-  // write / heavy final kernels, bytes written by the write / heavy write
-  // kernels), result counters [cap] (u64)
-  static constexpr size_t HDR_NITEMS = 0, HDR_QUEUE = 16, HDR_HEAVYN = 40, HDR_PITEMS = 48, HDR_CTR = 96;
+  // header: item counts [3], heavy-row counts [2], profile counters [6] (u64:
+  // entries walked by the write / final / heavy write / heavy final kernels,
+  // bytes written by the write / heavy write kernels), queues [3 main + 2
+  // heavy] of WQ_WORDS words, result counters [cap] (u64, a cache line each:
+  // the waves of one launch add to several of them at once)
+  static constexpr size_t HDR_NITEMS = 0, HDR_HEAVYN = 16, HDR_PITEMS = 32, HDR_QUEUE = 128,
+                          HDR_CTR = HDR_QUEUE + 5 * 4 * WQ_WORDS, CTR_STRIDE = 8;
   uint32_t cap = 0;  // items per launch = counters
   DevBuf items[3], blk[3], hdr;
   DevBuf heavy[2], hpre[2];  // heavy rows and their chunk prefix, per walking launch
@@ -730,7 +810,7 @@ struct ExtSlot {
     grid = g_persistent_blocks;
     heavy_t = c->heavy_t;
     heavy_chunk = c->heavy_chunk;
-    hdr_bytes = HDR_CTR + 8ull * cap;
+    hdr_bytes = HDR_CTR + 8ull * CTR_STRIDE * cap;
     hdr.alloc(hdr_bytes, s);
     for (int i = 0; i < 2; ++i) {
       heavy[i].alloc(sizeof(HeavyRow) * HEAVY_CAP, s);
@@ -757,14 +837,14 @@ struct ExtSlot {
     }
   }
   uint32_t *nitems(int i) { return reinterpret_cast<uint32_t *>(h_hdr + HDR_NITEMS) + i; }
-  uint64_t *counters() { return reinterpret_cast<uint64_t *>(h_hdr + HDR_CTR); }
+  uint64_t counter(size_t i) { return reinterpret_cast<uint64_t *>(h_hdr + HDR_CTR)[i * CTR_STRIDE]; }
   uint64_t *pitems() { return reinterpret_cast<uint64_t *>(h_hdr + HDR_PITEMS); }
   unsigned long long *dev_counter(size_t i) {
-    return reinterpret_cast<unsigned long long *>(hdr.as<unsigned char>() + HDR_CTR) + i;
+    return reinterpret_cast<unsigned long long *>(hdr.as<unsigned char>() + HDR_CTR) + i * CTR_STRIDE;
   }
 
   // The step's work, enqueued on the stream (eagerly or under capture).
-  void enqueue(gem_ctx *c, bool prof_kernels, bool count_items) {
+  void enqueue(gem_ctx *c, bool captured, bool prof_kernels, bool count_items) {
     hipStream_t s = c->stream;
     unsigned char *d = hdr.as<unsigned char>();
     GEM_HIP_CHECK(hipMemcpyAsync(d, h_hdr, hdr_bytes, hipMemcpyHostToDevice, s));
@@ -775,13 +855,17 @@ struct ExtSlot {
     const uint32_t *dn = reinterpret_cast<const uint32_t *>(d + HDR_NITEMS);
     unsigned int *dq = reinterpret_cast<unsigned int *>(d + HDR_QUEUE);
     unsigned int *hn = reinterpret_cast<unsigned int *>(d + HDR_HEAVYN);
-    launch_kernels<false>(c, grid, dn, dq, dq + 3, hn, prof_kernels, count_items, 0, ~0ull, 0, ~0ull, 0, ~0ull);
+    // a captured step holds every kernel (one without items ends at once);
+    // an eager one launches those that have items
+    uint64_t e[3];
+    for (int i = 0; i < 3; ++i) e[i] = captured || *nitems(i) ? ~0ull : 0;
+    launch_kernels<false>(c, grid, dn, dq, dq + 3 * WQ_WORDS, hn, prof_kernels, count_items, 0, e[0], 0, e[1], 0, e[2]);
     GEM_HIP_CHECK(hipMemcpyAsync(h_hdr, d, hdr_bytes, hipMemcpyDeviceToHost, s));
   }
 
   // The three kernels over task ranges [b_i, e_i) of launch i (queues
-  // dq[0..2]), then the heavy rows the two walking launches set aside (queues
-  // hq[0..1], row counts hn[0..1], all starting at zero).
+  // dq, WQ_WORDS words each), then the heavy rows the two walking launches set
+  // aside (queues hq, row counts hn[0..1]; everything starts at zero).
   template <bool OOC>
   void launch_kernels(gem_ctx *c, uint32_t grd, const uint32_t *dn, unsigned int *dq, unsigned int *hq,
                       unsigned int *hn, bool prof_kernels, bool count_items, uint64_t b0, uint64_t e0, uint64_t b1,
@@ -797,14 +881,14 @@ struct ExtSlot {
     }
     if (b1 < e1) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_FINAL : -1);
-      k_vext<true, OOC><<<grd * (VB / vthreads), vthreads, lds, s>>>(items[1].as<VItem>(), dn + 1, blk[1].as<uint64_t>(), dq + 1, max_nb,
+      k_vext<true, OOC><<<grd * (VB / vthreads), vthreads, lds, s>>>(items[1].as<VItem>(), dn + 1, blk[1].as<uint64_t>(), dq + WQ_WORDS, max_nb,
                                               max_ndup, count_items ? dp + 1 : nullptr, nullptr, b1, e1,
                                               heavy[1].as<HeavyRow>(), hn + 1, HEAVY_CAP, heavy_t);
       GEM_LAUNCH_CHECK("k_vext<final>");
     }
     if (b2 < e2) {
       ProfLaunch pl(c, prof_kernels ? K_VCOUNT1 : -1);
-      k_vcount1<OOC><<<grd, VB, 0, s>>>(items[2].as<VItem>(), dn + 2, blk[2].as<uint64_t>(), dq + 2, b2, e2);
+      k_vcount1<OOC><<<grd, VB, 0, s>>>(items[2].as<VItem>(), dn + 2, blk[2].as<uint64_t>(), dq + 2 * WQ_WORDS, b2, e2);
       GEM_LAUNCH_CHECK("k_vcount1");
     }
     if (b0 < e0) {
@@ -821,7 +905,7 @@ struct ExtSlot {
       k_heavy_scan<<<1, 1024, 0, s>>>(heavy[1].as<HeavyRow>(), hn + 1, HEAVY_CAP, heavy_chunk, hpre[1].as<uint64_t>());
       GEM_LAUNCH_CHECK("k_heavy_scan");
       k_vext_heavy<true, OOC><<<grd, VB, 0, s>>>(items[1].as<VItem>(), heavy[1].as<HeavyRow>(), hn + 1, HEAVY_CAP,
-                                                  hpre[1].as<uint64_t>(), hq + 1, heavy_chunk,
+                                                  hpre[1].as<uint64_t>(), hq + WQ_WORDS, heavy_chunk,
                                                   count_items ? dp + 3 : nullptr, nullptr);
       GEM_LAUNCH_CHECK("k_vext_heavy<final>");
     }
@@ -884,8 +968,8 @@ struct ExtSlot {
         const uint64_t most = std::max(hi[0] - lo[0], std::max(hi[1] - lo[1], hi[2] - lo[2]));
         const uint32_t grd = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(grid, most));
         // per group: 3 main queues, 2 heavy queues, 2 heavy-row counts
-        unsigned int *gq = q + 7 * g;
-        launch_kernels<true>(c, grd, dn, gq, gq + 3, gq + 5, prof, prof, lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]);
+        unsigned int *gq = q + (size_t)GROUP_WORDS * g;
+        launch_kernels<true>(c, grd, dn, gq, gq + 3 * WQ_WORDS, gq + 5 * WQ_WORDS, prof, prof, lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]);
         tc.done(g);
       }
       wa = wb;
@@ -896,14 +980,14 @@ struct ExtSlot {
 
   void launch(gem_ctx *c, bool use_graph) {
     if (!use_graph) {
-      enqueue(c, c->prof.on, c->prof.on);
+      enqueue(c, false, c->prof.on, c->prof.on);
       return;
     }
     if (!exec) {
       hipStream_t s = c->stream;
       GEM_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
       try {
-        enqueue(c, false, false);
+        enqueue(c, true, false, false);
       } catch (...) {
         hipGraph_t g = nullptr;
         (void)hipStreamEndCapture(s, &g);
@@ -978,7 +1062,7 @@ struct HipSchedBackend {
     {
       ProfLaunch pl(c, K_VLEN);
       k_vlen<<<grid_for(nblk), VB, 0, s>>>(D.items.as<VItem>(), (uint32_t)L.items.size(), D.blk.as<uint64_t>(),
-                                            D.queue.as<unsigned int>(), bu.as<uint64_t>());
+                                            bu.as<uint64_t>());
       GEM_LAUNCH_CHECK("k_vlen");
     }
     scan_u64(c, bu.as<uint64_t>(), bp.as<uint64_t>(), nunit);
@@ -1038,7 +1122,7 @@ struct HipSchedBackend {
       ext_tasks += L.blk.empty() ? 0 : L.blk.back();
     }
     // counters / work queues / walked-entry counts travel zeroed in the copy
-    std::memset(slot.h_hdr + ExtSlot::HDR_QUEUE, 0, slot.hdr_bytes - ExtSlot::HDR_QUEUE);
+    std::memset(slot.h_hdr + ExtSlot::HDR_HEAVYN, 0, slot.hdr_bytes - ExtSlot::HDR_HEAVYN);
     const bool prof = c->prof.on;
     if (tc)
       slot.launch_streamed(c, *tc);
@@ -1046,14 +1130,13 @@ struct HipSchedBackend {
       slot.launch(c, c->use_graph && !prof);
     GEM_HIP_CHECK(hipStreamSynchronize(s));
     if (tc) tc->finish();
-    const uint64_t *hc = slot.counters();
     got_wr->resize(wr_items.size());
     got_fin->resize(fin_items.size());
     for (size_t t = 0; t < wr_items.size(); ++t) {
-      (*got_wr)[t] = hc[t];
-      if (hc[t] > wr_items[t].out_rows) throw Error{GEM_E_STATE, "vjoin output exceeded its bound"};
+      (*got_wr)[t] = slot.counter(t);
+      if ((*got_wr)[t] > wr_items[t].out_rows) throw Error{GEM_E_STATE, "vjoin output exceeded its bound"};
     }
-    for (size_t t = 0; t < fin_items.size(); ++t) (*got_fin)[t] = hc[fin_ctr[t]];
+    for (size_t t = 0; t < fin_items.size(); ++t) (*got_fin)[t] = slot.counter(fin_ctr[t]);
     if (prof) {
       const uint64_t *pc = slot.pitems();
       // algorithmic bytes: rows read (4 B per column + an offset pair per
@@ -1273,7 +1356,7 @@ void VBatchRunner::run(std::vector<VQueryState *> &qs) {
     total_budget = std::max<uint64_t>((free_b + pool_reusable_bytes()) / 4, 1ull << 30);
   }
   total_budget = std::max<uint64_t>(total_budget, 1ull << 20);
-  // fixed launch buffers for the run (one item per query per launch at most)
+  // fixed launch buffers for the run (at most one item per running query)
   ExtSlot slot;
   {
     uint32_t mnb = 1, mnd = 0;
@@ -1288,7 +1371,8 @@ void VBatchRunner::run(std::vector<VQueryState *> &qs) {
         mnd = std::max(mnd, S->mnd_all);
       }
     }
-    slot.init(c_, (uint32_t)qs.size(), mnb, mnd);
+    const size_t running = c_->max_active ? std::min<size_t>(qs.size(), c_->max_active) : qs.size();
+    slot.init(c_, (uint32_t)running, mnb, mnd);
   }
   // streamed tables: a block cache shared by the run's queries
   std::unique_ptr<TableCache> tc;
