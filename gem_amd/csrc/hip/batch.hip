@@ -83,7 +83,7 @@ static uint64_t query_seed(const gemh::QueryInfo &Q) {
 }
 
 static void fill_result(const VQueryState &V, uint64_t cap, gem_join_result *r, uint64_t *level_rows) {
-  const gemh::SQuery<DevBuf> &S = V.s;
+  const gemh::SQuery<LevelBuf> &S = V.s;
   r->count = S.work_limited ? 0 : (S.saturated ? cap : S.count);
   r->saturated = S.saturated ? 1 : 0;
   r->num_steps = V.qd->Q.nv - 1;

@@ -9,15 +9,21 @@
 
 namespace gemd {
 
-// One level of one query: extend rows (positions of vorder[0..i-1]) by
-// vorder[i].  Device copy, one per (query, level).
+// One level of one query: extend rows by vorder[i].  A row holds the positions
+// of the earlier vertices that this level or a later one reads (as the key of
+// a list or an equal-label column), in vertex-order; column numbers are places
+// in that row.  Device copy, one per (query, level).
+constexpr uint8_t COL_NEW = 0xFF;
 struct VLevel {
   uint32_t nb, ndup;
+  uint32_t kout;             // columns of an output row:
+  uint8_t src[GEM_MAX_QV];   // the input column each is copied from, or COL_NEW for the new position
   uint32_t key_col[GEM_MAX_QV];
   const uint64_t *toff[GEM_MAX_QV];
   const uint32_t *tval[GEM_MAX_QV];  // in-HBM tables
   uint32_t dup_col[GEM_MAX_QV];
   const uint32_t *dup_can[GEM_MAX_QV];
+  const uint32_t *can_new;  // Can(vorder[i]), its bitmap and ranks
   const uint64_t *bm_new;
   const uint32_t *rank_new;
   // streamed tables: block map of table j (address of the values of key p =
@@ -32,10 +38,21 @@ struct VItem {
   const VLevel *lv;
   const uint32_t *rows;
   uint64_t row_begin, row_end;
-  uint32_t k, pad;
+  uint32_t k;
+  uint32_t nunits;        // write walks: 64-row units of the range,
+  uint32_t run_cost, pad; // the cost of a wave's run of them
+  const uint64_t *units;  // and the prefix of their output bounds (nunits + 1)
   uint32_t *out;
   uint64_t out_cap;
   unsigned long long *counter;
+};
+
+// Rows of a pending level.  Once measured they know the device prefix of
+// their units' output bounds (from entry unit0 on; one buffer holds those of
+// all levels measured together).
+struct LevelBuf : DevBuf {
+  mutable std::shared_ptr<DevBuf> units;
+  mutable uint64_t unit0 = 0;
 };
 
 // A row whose driving list is too long for one wave: walked in chunks by
@@ -61,8 +78,9 @@ struct VQueryState {
   DevBuf levels;  // VLevel[nv]
   std::vector<VLevel> hlv;  // host copy of `levels`
   std::vector<uint32_t> max_nb, max_ndup;  // per level
+  std::vector<uint32_t> cols_in;           // per level: columns of its input rows
   // depth-first stack of pending level ranges, counts and limits (host/vsched.h)
-  gemh::SQuery<DevBuf> s;
+  gemh::SQuery<LevelBuf> s;
   // Restarts (learned batched path): the vertex orders in the order they are
   // tried and their candidate indices; ranked[cur] is the one running.
   // Attempt a runs ranked[a] while a < size, then the order whose ended

@@ -11,22 +11,29 @@
 //   k_vlen    per 64-row unit: sum over rows of the shortest list length
 //             (an upper bound on the level's output, used to size and split)
 //   k_vext    waves walk the shortest ("driver") list of each of their 64
-//             rows, 128 items per step (two per lane); each item is
+//             rows, 256 items per step (four per lane); each item is
 //             binary-searched in the row's other lists and compared with the
 //             equal-label columns; survivors are counted (last level) or
-//             appended to the output (one atomic reservation per wave step;
-//             row order is free); rows with long driving lists are left to
-//             k_vext_heavy
+//             appended to the output (row order is free); rows with long
+//             driving lists are left to k_vext_heavy
 //   k_vext_heavy  walks those rows in fixed-size pieces spread over waves
 //   k_vcount1 last level with a single backward list: |list| minus the
 //             equal-label columns found in it (no walk)
 //
 // Work distribution: each launch covers many (query, level, row range) items;
-// waves pull 64-row tasks from a device counter (persistent grid), so queries
+// the waves of a persistent grid take runs of their 64-row units, so queries
 // of very different sizes share one launch.  The host scheduler
 // (host/vsched.h) keeps, per query, a depth-first stack of pending levels and
 // cuts them into 64-row-unit ranges whose output bounds fit a memory budget
 // shared by all queries; a query stops as soon as its count exceeds the cap.
+//
+// What bounds the walks is the output: rows written, and the atomics that hand
+// out their places (one address serves one per 9-11 ns).  Hence rows hold only
+// the columns that are read again (VLevel::src; 2.1x fewer bytes written on 16
+// queries of up to 24 vertices, 2^20 R-MAT), and places are reserved once per
+// run of a one-list level and once per full stage of the others.  k_vext<write>
+// of one pass: 190 -> 107 ms on those queries, 13.3 -> 2.5 ms on 24 exact
+// queries of 4-9 vertices on 2^18.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -46,7 +53,7 @@ constexpr uint32_t VB = 256;  // rows per task block
 constexpr uint32_t VW = VB / 64;
 // survivors a wave stages in LDS before it reserves output rows for them (a
 // step of k_vext adds at most 256, one of k_vext_heavy 128)
-constexpr uint32_t VSTAGE = 512;
+constexpr uint32_t VSTAGE = 384;
 
 __device__ __forceinline__ uint32_t vposition_in(const uint64_t *bm, const uint32_t *rank, uint32_t v) {
   const uint64_t word = ldg(bm + (v >> 6));
@@ -55,8 +62,17 @@ __device__ __forceinline__ uint32_t vposition_in(const uint64_t *bm, const uint3
   return ldg(rank + (v >> 6)) + (uint32_t)__popcll(word & ((1ull << b) - 1));
 }
 
-// A level descriptor read through the global address space (see ldg).
-using GLevel = const __attribute__((address_space(1))) VLevel;
+// Level descriptors and launch tables do not change while a kernel runs: read
+// through the constant address space, uniform indexes become scalar loads.
+#define GEM_CONST const __attribute__((address_space(4)))
+using CLevel = GEM_CONST VLevel;
+using CItem = GEM_CONST VItem;
+
+// Two neighbouring offsets (start and end of a list) in one 16-byte load.
+typedef uint64_t u64x2 __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ u64x2 ld_pair(const uint64_t *p) {
+  return *(const __attribute__((address_space(1))) u64x2 *)p;
+}
 
 // task g (global block index of the launch) -> item t, row block within item
 __device__ __forceinline__ uint32_t find_item(const uint64_t *blk_prefix, uint32_t nitems, uint64_t g) {
@@ -85,7 +101,7 @@ __global__ void __launch_bounds__(VB) k_vlen(const VItem *__restrict__ items, ui
   for (uint64_t g = blockIdx.x; g < total; g += gridDim.x) {
     while (blk_prefix[t + 1] <= g) ++t;
     const VItem &it = items[t];
-    GLevel &L = *(GLevel *)it.lv;
+    CLevel &L = *(CLevel *)it.lv;
     const uint64_t r = it.row_begin + (g - blk_prefix[t]) * VB + threadIdx.x;
     uint64_t u = 0;
     if (r < it.row_end) {
@@ -111,57 +127,122 @@ __global__ void __launch_bounds__(VB) k_vlen(const VItem *__restrict__ items, ui
 // ns whatever asks: 8,192 waves finding an empty queue took 95 us, and a queue
 // of 64-row tasks bounded every large launch.  Runs are as long as leaves a
 // wave about CLAIMS of them, so uneven tasks still even out.
-constexpr uint32_t CLAIMS = 8, MAX_RUN = 32;
+constexpr uint32_t CLAIMS = 4, MAX_RUN = 32;
 struct Runs {
-  uint64_t ntask, nrun, run;
+  uint32_t ntask, nrun, run;
   uint32_t per, nq, sub, given;
   unsigned int *q;
-  // w, nw: this wave and the waves of the grid
+  // n tasks (rows / 64: below 2^32); w, nw: this wave and the waves of the grid
   __device__ __forceinline__ Runs(uint64_t n, uint32_t w, uint32_t nw, uint32_t max_run, unsigned int *queue)
-      : ntask(n), run(w) {
-    const uint64_t p = n / ((uint64_t)nw * CLAIMS);
-    per = p < 1 ? 1 : p > max_run ? max_run : (uint32_t)p;
-    nrun = (n + per - 1) / per;
+      : ntask((uint32_t)n), run(w) {
+    const uint32_t p = ntask / (nw * CLAIMS);
+    per = p < 1 ? 1 : p > max_run ? max_run : p;
+    nrun = (ntask - 1) / per + 1;
     nq = nw < WQ ? nw : WQ;
     sub = w % nq;
     given = (nw - sub + nq - 1) / nq;
     q = queue + sub * WQ_STRIDE;
   }
   __device__ __forceinline__ bool valid() const { return run < nrun; }
-  __device__ __forceinline__ uint64_t begin() const { return run * per; }
-  __device__ __forceinline__ uint64_t end() const {
-    const uint64_t e = run * per + per;
-    return e < ntask ? e : ntask;
-  }
+  __device__ __forceinline__ uint32_t begin() const { return run * per; }
+  __device__ __forceinline__ uint32_t end() const { return ntask - run * per < per ? ntask : run * per + per; }
   __device__ __forceinline__ void next() {
-    if ((uint64_t)given * nq + sub >= nrun) {  // every run was given at the start
+    if (given * nq + sub >= nrun) {  // every run was given at the start
       run = nrun;
       return;
     }
     uint32_t c = 0;
     if (lane_id() == 0) c = atomicAdd(q, 1u);
-    run = ((uint64_t)given + readlane_u32(c, 0)) * nq + sub;
+    run = (given + readlane_u32(c, 0)) * nq + sub;
   }
 };
 
 // Device address of the list of key p in backward table j (b = its first
 // offset): in HBM, or through the streamed tables' block map.
 template <bool OOC>
-__device__ __forceinline__ uint64_t list_addr(GLevel &L, uint32_t j, uint32_t p, uint64_t b) {
+__device__ __forceinline__ uint64_t list_addr(CLevel &L, uint32_t j, uint32_t p, uint64_t b) {
   if (OOC) return ldg(L.vmap[j] + (p >> L.kshift[j])) + 4 * b;
   return (uint64_t)(uintptr_t)(L.tval[j] + b);
 }
 
 // ------------------------------------------------------ extend (walk) pass
-// Each wave takes runs of 64-row tasks on its own (no block barrier).  For each of its rows the shortest backward list drives; a row
-// whose driving list is longer than heavy_t is not walked here but appended to
-// the heavy-row list (when it has room), which k_vext_heavy then walks in
-// fixed-size chunks spread over all waves: a hub row no longer holds one wave
-// for the whole launch.
-// Dynamic LDS per wave: other lists (nb-1) x 64 x (u64 address + u32 len),
-// dup positions ndup x 64 u32 (blocks of one wave when four waves' share
-// would not fit a block's LDS).
-// Survivors are written as whole rows: their (parent row, new value) pairs are
+// Cost of a 64-row unit besides the entries it walks, in entries: its rows'
+// setup.  A run of a write walk has at most RUN_COST of it.
+constexpr uint32_t UNIT_COST = 256, RUN_COST = UNIT_COST * MAX_RUN;
+
+// The units [*j0, *j1) of an item of n units whose cost starts in
+// [at, at + run): cost(j) = units[j] - units[0] + UNIT_COST * j, at < cost(n),
+// run <= RUN_COST (so they are at most MAX_RUN).  The first is searched 64
+// places at a time, the end looked up in one step.
+__device__ __forceinline__ void unit_range(const uint64_t *units, uint32_t n, uint64_t at, uint32_t run, uint32_t *j0,
+                                           uint32_t *j1) {
+  const uint64_t first = ldg(units);
+  uint32_t b = 0;
+  if (at) {
+    uint32_t a = 0;  // cost(a) < at <= cost(b)
+    b = n;
+    while (b - a > 1) {
+      const uint32_t step = (b - a - 1) / 64 + 1;
+      const uint64_t x = (uint64_t)a + (uint64_t)(lane_id() + 1) * step;
+      bool reached = x >= b;
+      if (!reached) reached = ldg(units + x) - first + (uint64_t)UNIT_COST * x >= at;
+      const uint32_t f = (uint32_t)__builtin_ctzll(__ballot(reached));
+      const uint64_t hi = (uint64_t)a + (uint64_t)(f + 1) * step;
+      a += f * step;
+      b = hi < b ? (uint32_t)hi : b;
+    }
+  }
+  const uint64_t x = (uint64_t)b + lane_id();
+  bool past = x >= n;
+  if (!past) past = ldg(units + x) - first + (uint64_t)UNIT_COST * x >= at + run;
+  *j0 = b;
+  *j1 = b + (uint32_t)__builtin_ctzll(__ballot(past));
+}
+
+// Loads of N lists (N equal-label columns) of one row at a time, so that a
+// row's setup is a few rounds of independent loads and not a chain of them.
+template <int N, class F>
+__device__ __forceinline__ void row_lists(CLevel &L, const uint32_t *row, uint32_t j, F &&f) {
+  uint32_t p[N];
+  u64x2 o[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) p[i] = ldg(row + L.key_col[j + i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) o[i] = ld_pair(L.toff[j + i] + p[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) f(j + i, p[i], o[i].x, (uint32_t)(o[i].y - o[i].x));
+}
+template <int N, class F>
+__device__ __forceinline__ void row_dups(CLevel &L, const uint32_t *row, uint32_t c, F &&f) {
+  uint32_t p[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) p[i] = ldg(row + L.dup_col[c + i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) p[i] = ldg(L.dup_can[c + i] + p[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) f(c + i, p[i]);
+}
+
+// Other lists and equal-label columns of a row that k_vext keeps in LDS; what
+// a level has beyond them is read again for the items that are still wanted
+// by then.  Sized for the levels that occur (most have one or two lists): with
+// room for every list of the widest level of a batch, a launch had 11 of a
+// CU's 32 waves.
+constexpr uint32_t LDS_LISTS = 2, LDS_DUPS = 8;
+
+// Each wave takes runs of 64-row units on its own (no block barrier): of equal
+// cost by the length pass's unit prefix, so that a run's rows are reserved
+// together however many units that takes, and no wave is left with a run of
+// long lists (runs of a fixed number of units: the longest launch took 18 ms
+// instead of 5).  For each of its rows the shortest backward list drives; a row whose driving list is
+// longer than heavy_t is not walked here but appended to the heavy-row list
+// (when it has room), which k_vext_heavy then walks in fixed-size chunks spread
+// over all waves: a hub row no longer holds one wave for the whole launch.
+// Dynamic LDS per wave: lists (lcap x 64 x (u64 address + u32 length)) and
+// vertices of equal-label columns (dcap x 64 u32).
+// An item (row, value) survives when its value is in the row's other lists and
+// its vertex differs from those of the row's equal-label columns.  Survivors
+// are written as whole rows: their (parent row, new value) pairs are
 // staged in LDS, over all tasks of the item that the wave has in hand, then
 // the wave reserves output rows for all of them at once (one atomic on the
 // item's counter) and writes them as one run of consecutive words.
@@ -170,9 +251,9 @@ __device__ __forceinline__ uint64_t list_addr(GLevel &L, uint32_t j, uint32_t p,
 // launch (256-row units) are processed (streamed tables run a launch in task
 // groups).
 template <bool FINAL, bool OOC>
-__global__ void __launch_bounds__(VB) __attribute__((amdgpu_waves_per_eu(8)))
+__global__ void __launch_bounds__(VB) __attribute__((amdgpu_waves_per_eu(6)))
 k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, const uint64_t *__restrict__ blk_prefix,
-       unsigned int *__restrict__ queue, uint32_t max_nb, uint32_t max_ndup,
+       unsigned int *__restrict__ queue, uint32_t lcap, uint32_t dcap,
        unsigned long long *__restrict__ prof_items, unsigned long long *__restrict__ prof_out, uint64_t g_begin,
        uint64_t g_end, HeavyRow *__restrict__ heavy, unsigned int *__restrict__ heavy_n, uint32_t heavy_cap,
        uint32_t heavy_t) {
@@ -180,118 +261,202 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
   const uint64_t total = blk_prefix[nitems] < g_end ? blk_prefix[nitems] : g_end;
   if (g_begin >= total) return;
   __shared__ uint32_t st[VW][65];
-  __shared__ uint64_t drv[VW][64];  // address of each row's driving list
+  __shared__ uint64_t drv[VW][64];         // address of each row's driving list
+  __shared__ uint8_t drv_j[VW][64];        // which of the row's lists drives
+  __shared__ uint8_t src[VW][GEM_MAX_QV];  // the item's output columns (VLevel::src)
+  __shared__ uint64_t aside[VW][MAX_RUN];  // counted runs: rows of each task set aside as heavy
   __shared__ uint32_t sv_row[VW][VSTAGE];  // staged survivors: row in the item's range
   __shared__ uint32_t sv_val[VW][VSTAGE];  // and new value
   extern __shared__ unsigned char vlds[];
   const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64;
-  const uint32_t per_wave = 64 * ((max_nb > 0 ? max_nb - 1 : 0) * 12 + max_ndup * 4);
-  unsigned char *mine = vlds + (size_t)w * per_wave;
-  uint64_t *obase = reinterpret_cast<uint64_t *>(mine);                                  // [nb-1][64]
-  uint32_t *olen = reinterpret_cast<uint32_t *>(mine + (size_t)64 * 8 * (max_nb - 1));   // [nb-1][64]
-  uint32_t *dpos = reinterpret_cast<uint32_t *>(mine + (size_t)64 * 12 * (max_nb - 1));  // [ndup][64]
+  unsigned char *mine = vlds + (size_t)w * 64 * (lcap * 12 + dcap * 4);
+  uint64_t *obase = reinterpret_cast<uint64_t *>(mine);                            // [lcap][64]
+  uint32_t *olen = reinterpret_cast<uint32_t *>(mine + (size_t)64 * 8 * lcap);     // [lcap][64]
+  uint32_t *dvert = reinterpret_cast<uint32_t *>(mine + (size_t)64 * 12 * lcap);   // [dcap][64]
   uint64_t walked = 0, written = 0;
-  uint32_t t = NOT_FOUND;  // item in hand
-  VItem it{};
+  // item in hand: index, its task range [ta, tb), and its fields
+  uint32_t t = NOT_FOUND;
+  uint64_t ta = 0, tb = 0;
+  const VLevel *lv = nullptr;
+  const uint32_t *in = nullptr;  // first row of the item's range
+  uint64_t nrow = 0;
+  uint32_t k = 1, ko = 1, inv = 0;  // columns read and written, 2^32 / ko rounded up
   uint64_t survivors = 0;  // final level: survivors of the item in hand
   uint32_t pend = 0;       // survivors staged in LDS, not yet written
+  bool counted = false;    // output rows already reserved, from `cursor` on
+  uint64_t cursor = 0;
   // write the staged survivors: one reservation for all of them, then
-  // their rows as one run of consecutive words (word q is column q % (k+1)
-  // of survivor q / (k+1): k parent columns, then the value).  q / (k+1) by
-  // the reciprocal rounded up: exact while q * (k+1) < 2^32.
+  // their rows as one run of consecutive words (word q is column q % ko of
+  // survivor q / ko: a parent column or the value), four words per lane in
+  // flight.  q / ko by the reciprocal rounded up: exact while q * ko < 2^32.
   auto flush = [&]() {
+    CItem &I = ((CItem *)items)[t];
     if (FINAL) {
-      if (l == 0 && survivors) atomicAdd(it.counter, (unsigned long long)survivors);
+      if (l == 0 && survivors) atomicAdd(I.counter, (unsigned long long)survivors);
       survivors = 0;
       return;
     }
     if (!pend) return;
-    uint64_t base = 0;
-    if (l == 0) base = atomicAdd(it.counter, (unsigned long long)pend);
-    base = readlane_u64(base, 0);
-    const uint32_t k = it.k, rl = k + 1, inv = 0xFFFFFFFFu / rl + 1;
-    written += (uint64_t)pend * 4 * rl;
-    for (uint32_t q = l; q < pend * rl; q += 64) {
-      const uint32_t i = __umulhi(q, inv), c = q - i * rl;
-      if (base + i < it.out_cap)
-        stg(it.out + (base + i) * rl + c,
-            c < k ? ldg(it.rows + (it.row_begin + sv_row[w][i]) * k + c) : sv_val[w][i]);
+    uint64_t base = cursor;
+    cursor += pend;
+    if (!counted) {
+      if (l == 0) base = atomicAdd(I.counter, (unsigned long long)pend);
+      base = readlane_u64(base, 0);
+    }
+    const uint64_t room = I.out_cap > base ? I.out_cap - base : 0;
+    const uint32_t n = (pend < room ? pend : (uint32_t)room) * ko;
+    uint32_t *dst = I.out + base * ko;
+    written += (uint64_t)n * 4;
+    for (uint32_t b = 0; b < n; b += 256) {
+      uint32_t x[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const uint32_t q = b + 64 * g + l < n ? b + 64 * g + l : n - 1;
+        const uint32_t i = ko > 1 ? __umulhi(q, inv) : q;
+        const uint32_t c = src[w][q - i * ko];
+        x[g] = ldg(in + (uint64_t)sv_row[w][i] * k + (c == COL_NEW ? 0 : c));
+        if (c == COL_NEW) x[g] = sv_val[w][i];
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        if (b + 64 * g + l < n) stg(dst + b + 64 * g + l, x[g]);
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     pend = 0;
   };
-  const uint32_t bw = blockDim.x / 64;
-  Runs runs((total - g_begin) * VW, blockIdx.x * bw + w, gridDim.x * bw, MAX_RUN, queue);
-  for (; runs.valid(); runs.next())
-  for (uint64_t q = g_begin * VW + runs.begin(), qe = g_begin * VW + runs.end(); q < qe; ++q) {  // 64-row task
-    const uint64_t g = q / VW;
-    if (t == NOT_FOUND || g < blk_prefix[t] || g >= blk_prefix[t + 1]) {
-      if (t != NOT_FOUND) flush();
-      t = find_item(blk_prefix, nitems, g);
-      it = items[t];
+  // the item in hand becomes item x
+  auto open = [&](uint32_t x) {
+    if (t != NOT_FOUND) flush();
+    t = x;
+    counted = false;
+    CItem &I = ((CItem *)items)[t];
+    lv = I.lv;
+    k = I.k;
+    if (!FINAL) {
+      CLevel &L = *(CLevel *)lv;
+      ko = L.kout;
+      inv = 0xFFFFFFFFu / ko + 1;
+      if (l < ko) src[w][l] = L.src[l];
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
-    GLevel &L = *(GLevel *)it.lv;
-    const uint32_t nb = L.nb, ndup = L.ndup, k = it.k;
-    const uint64_t rbase = it.row_begin + (g - blk_prefix[t]) * VB + (q % VW) * 64;
-    if (rbase >= it.row_end) continue;
-    const uint32_t roff = (uint32_t)(rbase - it.row_begin);
-    const uint64_t r = rbase + l;
-    const bool valid = r < it.row_end;
-    const uint32_t *row = it.rows + r * k;
+    in = I.rows + I.row_begin * k;
+    nrow = I.row_end - I.row_begin;
+  };
+  // walk units [j0, j1) of the item in hand (at most MAX_RUN of them)
+  auto walk = [&](uint64_t j0, uint64_t j1) {
+    CLevel &L = *(CLevel *)lv;
+    const uint32_t nb = L.nb, ndup = L.ndup;
+    if (!FINAL && nb == 1) {
+      // One list: every entry survives but those of the equal-label columns,
+      // so the run's rows are counted first (the vertices' positions searched
+      // in the list) and reserved by one atomic.
+      flush();
+      counted = true;
+      uint64_t cnt = 0;
+      for (uint64_t j = j0; j < j1; ++j) {
+        const uint64_t r = j * 64 + l;
+        const uint32_t *row = in + r * k;
+        uint32_t len = 0;
+        uint64_t addr = 0;
+        if (r < nrow) {
+          const uint32_t p = ldg(row + L.key_col[0]);
+          const u64x2 o = ld_pair(L.toff[0] + p);
+          len = (uint32_t)(o.y - o.x);
+          addr = list_addr<OOC>(L, 0, p, o.x);
+        }
+        const uint64_t hv = heavy ? __ballot(len > heavy_t) : 0;
+        uint64_t taken = 0;
+        if (hv) {
+          uint32_t h = 0;
+          if (l == 0) h = atomicAdd(heavy_n, (uint32_t)__popcll(hv));
+          h = readlane_u32(h, 0) + rank_below(hv);
+          const bool mine = ((hv >> l) & 1ull) && h < heavy_cap;
+          if (mine) {
+            heavy[h] = HeavyRow{t, len, ((CItem *)items)[t].row_begin + r};
+            len = 0;  // walked by k_vext_heavy
+          }
+          taken = __ballot(mine);
+        }
+        if (l == 0) aside[w][j - j0] = taken;
+        cnt += len;
+        if (len)
+          for (uint32_t d = 0; d < ndup; ++d) {
+            const uint32_t pos = vposition_in(L.bm_new, L.rank_new, ldg(L.dup_can[d] + ldg(row + L.dup_col[d])));
+            if (pos != NOT_FOUND && sorted_contains(reinterpret_cast<const uint32_t *>(addr), (uint64_t)len, pos))
+              --cnt;
+          }
+      }
+      cnt = wave_sum_u64(cnt);
+      cursor = 0;
+      if (l == 0 && cnt) cursor = atomicAdd(((CItem *)items)[t].counter, (unsigned long long)cnt);
+      cursor = readlane_u64(cursor, 0);
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
+  for (uint64_t j = j0; j < j1; ++j) {
+    const uint64_t rbase = j * 64;  // in the item's range
+    if (rbase >= nrow) break;
+    const bool valid = rbase + l < nrow;
+    const uint32_t *row = in + (rbase + l) * k;
     // per-row lists: the shortest one drives, the others are probed
-    uint32_t dlen = 0, dj = 0, dp = 0;
-    uint64_t dbase = 0, daddr = 0;
+    uint32_t dlen = 0, dj = 0;
+    uint64_t daddr = 0;
     if (valid) {
       dlen = 0xFFFFFFFFu;
-      for (uint32_t j = 0; j < nb; ++j) {
-        const uint32_t p = ldg(row + L.key_col[j]);
-        const uint64_t *off = L.toff[j];
-        const uint64_t b = ldg(off + p);
-        const uint32_t len = (uint32_t)(ldg(off + p + 1) - b);
-        if (len < dlen) {
+      auto take = [&](uint32_t j, uint32_t p, uint64_t b, uint32_t len) {
+        const bool less = len < dlen;
+        const uint64_t a = list_addr<OOC>(L, j, p, b);
+        if (less) {
           dlen = len;
           dj = j;
-          dbase = b;
-          dp = p;
+          daddr = a;
         }
+        if (nb > 1 && j < lcap) {
+          obase[j * 64 + l] = a;
+          olen[j * 64 + l] = len;
+        }
+      };
+      uint32_t i = 0;
+      for (; i + 4 <= nb; i += 4) row_lists<4>(L, row, i, take);
+      if (i + 2 <= nb) {
+        row_lists<2>(L, row, i, take);
+        i += 2;
       }
+      if (i < nb) row_lists<1>(L, row, i, take);
     }
-    const uint64_t hv = heavy ? __ballot(dlen > heavy_t) : 0;
+    const uint64_t hv = heavy && !counted ? __ballot(dlen > heavy_t) : 0;
+    if (!FINAL && counted && ((aside[w][j - j0] >> l) & 1ull)) dlen = 0;
     if (hv) {
       uint32_t h = 0;
       if (l == 0) h = atomicAdd(heavy_n, (uint32_t)__popcll(hv));
       h = readlane_u32(h, 0) + rank_below(hv);
       if (((hv >> l) & 1ull) && h < heavy_cap) {
-        heavy[h] = HeavyRow{t, dlen, r};
+        heavy[h] = HeavyRow{t, dlen, ((CItem *)items)[t].row_begin + rbase + l};
         dlen = 0;  // walked by k_vext_heavy
       }
     }
     // a row with nothing to walk here (empty driving list, or set aside as a
-    // heavy row) owns no item of the steps below, so its probe lists and
-    // equal-label positions are never read: skip their loads
-    if (valid && dlen) {
-      daddr = list_addr<OOC>(L, dj, dp, dbase);
-      uint32_t o = 0;
-      for (uint32_t j = 0; j < nb; ++j) {
-        if (j == dj) continue;
-        const uint32_t p = ldg(row + L.key_col[j]);
-        const uint64_t *off = L.toff[j];
-        const uint64_t b = ldg(off + p);
-        obase[o * 64 + l] = list_addr<OOC>(L, j, p, b);
-        olen[o * 64 + l] = (uint32_t)(ldg(off + p + 1) - b);
-        ++o;
+    // heavy row) owns no item of the steps below, so its equal-label columns
+    // are never read: skip their loads
+    if (dlen) {
+      auto take = [&](uint32_t c, uint32_t v) { dvert[c * 64 + l] = v; };
+      const uint32_t nd = ndup < dcap ? ndup : dcap;
+      uint32_t c = 0;
+      for (; c + 4 <= nd; c += 4) row_dups<4>(L, row, c, take);
+      if (c + 2 <= nd) {
+        row_dups<2>(L, row, c, take);
+        c += 2;
       }
-      for (uint32_t c = 0; c < ndup; ++c) {
-        const uint32_t vid = ldg(L.dup_can[c] + ldg(row + L.dup_col[c]));
-        dpos[c * 64 + l] = vposition_in(L.bm_new, L.rank_new, vid);
-      }
+      if (c < nd) row_dups<1>(L, row, c, take);
     }
     const uint32_t incl = wave_incl_scan_u32(dlen);
     const uint32_t wtotal = readlane_u32(incl, 63);
     st[w][l] = incl - dlen;
     if (l == 63) st[w][64] = wtotal;
     drv[w][l] = daddr;
+    if (nb > 1) drv_j[w][l] = (uint8_t)dj;
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     walked += wtotal;
@@ -307,20 +472,43 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
         rw[g] = keep[g] ? seg_of(st[w], item) : 0;
         val[g] = keep[g] ? ldg(reinterpret_cast<const uint32_t *>(drv[w][rw[g]]) + (item - st[w][rw[g]])) : 0;
       }
-      for (uint32_t c = 0; c < ndup; ++c) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          if (dpos[c * 64 + rw[g]] == val[g]) keep[g] = false;
-      }
-      for (uint32_t o = 0; o + 1 < nb; ++o) {
+      for (uint32_t j = 0; nb > 1 && j < nb; ++j) {
         const uint32_t *lists[4];
         uint32_t lens[4];
+        bool probe[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          lists[g] = reinterpret_cast<const uint32_t *>(obase[o * 64 + rw[g]]);
-          lens[g] = olen[o * 64 + rw[g]];
+          probe[g] = keep[g] && drv_j[w][rw[g]] != j;
+          lists[g] = nullptr;
+          lens[g] = 0;
+          if (j < lcap) {
+            lists[g] = reinterpret_cast<const uint32_t *>(obase[j * 64 + rw[g]]);
+            lens[g] = olen[j * 64 + rw[g]];
+          } else if (probe[g]) {
+            const uint32_t p = ldg(in + (rbase + rw[g]) * k + L.key_col[j]);
+            const u64x2 o = ld_pair(L.toff[j] + p);
+            lists[g] = reinterpret_cast<const uint32_t *>(list_addr<OOC>(L, j, p, o.x));
+            lens[g] = (uint32_t)(o.y - o.x);
+          }
         }
-        contains_quad(lists, lens, val, keep);
+        bool hit[4] = {probe[0], probe[1], probe[2], probe[3]};
+        contains_quad(lists, lens, val, hit, in);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) keep[g] = keep[g] && (hit[g] || !probe[g]);
+      }
+      if (ndup) {
+        uint32_t vert[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) vert[g] = keep[g] ? ldg(L.can_new + val[g]) : 0;
+        for (uint32_t c = 0; c < ndup; ++c) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            if (c < dcap)
+              keep[g] = keep[g] && dvert[c * 64 + rw[g]] != vert[g];
+            else if (keep[g])
+              keep[g] = ldg(L.dup_can[c] + ldg(in + (rbase + rw[g]) * k + L.dup_col[c])) != vert[g];
+          }
+        }
       }
       uint64_t m[4];
       uint32_t nk = 0, before[4];
@@ -339,7 +527,7 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
         for (int g = 0; g < 4; ++g)
           if (keep[g]) {
             const uint32_t i = pend + before[g] + rank_below(m[g]);
-            sv_row[w][i] = roff + rw[g];
+            sv_row[w][i] = (uint32_t)rbase + rw[g];
             sv_val[w][i] = val[g];
           }
         __builtin_amdgcn_wave_barrier();
@@ -351,6 +539,37 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
     // st / drv / LDS lists of this wave are rewritten by its next task
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  }
+  };
+  const uint32_t bw = blockDim.x / 64;
+  if (FINAL || OOC) {
+    // tasks are 64-row units, numbered through the launch
+    Runs runs((total - g_begin) * VW, blockIdx.x * bw + w, gridDim.x * bw, FINAL ? 4 : 8, queue);
+    for (; runs.valid(); runs.next())
+      for (uint64_t q = g_begin * VW + runs.begin(), qe = g_begin * VW + runs.end(); q < qe;) {
+        const uint64_t g = q / VW;
+        if (t == NOT_FOUND || g < ta || g >= tb) {
+          open(find_item(blk_prefix, nitems, g));
+          ta = blk_prefix[t];
+          tb = blk_prefix[t + 1];
+        }
+        const uint64_t qn = tb * VW < qe ? tb * VW : qe;
+        walk(q - ta * VW, qn - ta * VW);
+        q = qn;
+      }
+  } else {
+    // tasks are runs of units of about equal cost: run i of an item holds the
+    // units whose cost starts in [i, i + 1) * run_cost (the item's)
+    Runs runs(total - g_begin, blockIdx.x * bw + w, gridDim.x * bw, 1, queue);
+    for (; runs.valid(); runs.next()) {
+      const uint64_t g = g_begin + runs.begin();
+      const uint32_t x = find_item(blk_prefix, nitems, g);
+      if (x != t) open(x);
+      CItem &I = ((CItem *)items)[t];
+      uint32_t j0, j1;
+      unit_range(I.units, I.nunits, (g - blk_prefix[t]) * I.run_cost, I.run_cost, &j0, &j1);
+      if (j0 < j1) walk(j0, j1);
+    }
   }
   if (t != NOT_FOUND) flush();
   if (prof_items && l == 0 && walked) atomicAdd(prof_items, (unsigned long long)walked);
@@ -406,9 +625,9 @@ k_vext_heavy(const VItem *__restrict__ items, const HeavyRow *__restrict__ heavy
     const uint32_t h = find_item(pre, n, wt);
     const HeavyRow e = heavy[h];
     const VItem it = items[e.t];
-    GLevel &L = *(GLevel *)it.lv;
-    const uint32_t nb = L.nb, ndup = L.ndup, k = it.k;
-    const uint32_t *row = it.rows + e.r * k;
+    CLevel &L = *(CLevel *)it.lv;
+    const uint32_t nb = L.nb, ndup = L.ndup;
+    const uint32_t *row = it.rows + e.r * it.k;
     // the row's lists (every lane computes the same; lane j keeps list j)
     uint32_t dlen = 0xFFFFFFFFu, dj = 0, dp = 0;
     uint64_t dbase = 0;
@@ -436,7 +655,14 @@ k_vext_heavy(const VItem *__restrict__ items, const HeavyRow *__restrict__ heavy
       }
     }
     if (l < ndup) dpos[w][l] = vposition_in(L.bm_new, L.rank_new, ldg(L.dup_can[l] + ldg(row + L.dup_col[l])));
-    if (!FINAL && l < k) prow[w][l] = ldg(row + l);
+    const uint32_t ko = FINAL ? 1 : L.kout;
+    uint32_t newc = ko;  // the output column that takes the value (ko: none does)
+    if (!FINAL) {
+      const uint32_t c = l < ko ? L.src[l] : 0;
+      const uint64_t isnew = __ballot(l < ko && c == COL_NEW);
+      if (isnew) newc = (uint32_t)__builtin_ctzll(isnew);
+      if (l < ko && c != COL_NEW) prow[w][l] = ldg(row + c);
+    }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     const uint64_t s0 = (uint64_t)(wt - pre[h]) * chunk;
@@ -444,17 +670,17 @@ k_vext_heavy(const VItem *__restrict__ items, const HeavyRow *__restrict__ heavy
     walked += s1 - s0;
     uint64_t survivors = 0;
     uint32_t pend = 0;  // surviving values staged, not yet written
-    // the staged rows share the parent row: pend * (k + 1) consecutive words
+    // the staged rows share the parent row: pend * ko consecutive words
     // of the output, reserved by one atomic, written by consecutive lanes
     auto flush = [&]() {
       uint64_t base = 0;
       if (l == 0) base = atomicAdd(it.counter, (unsigned long long)pend);
       base = readlane_u64(base, 0);
-      const uint32_t rl = k + 1, inv = 0xFFFFFFFFu / rl + 1;
-      written += (uint64_t)pend * 4 * rl;
-      for (uint32_t q = l; q < pend * rl; q += 64) {
-        const uint32_t i = __umulhi(q, inv), c = q - i * rl;
-        if (base + i < it.out_cap) stg(it.out + (base + i) * rl + c, c < k ? prow[w][c] : hsv[w][i]);
+      const uint32_t inv = 0xFFFFFFFFu / ko + 1;
+      written += (uint64_t)pend * 4 * ko;
+      for (uint32_t q = l; q < pend * ko; q += 64) {
+        const uint32_t i = ko > 1 ? __umulhi(q, inv) : q, c = q - i * ko;
+        if (base + i < it.out_cap) stg(it.out + (base + i) * ko + c, c != newc ? prow[w][c] : hsv[w][i]);
       }
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -571,7 +797,7 @@ __global__ void __launch_bounds__(VB) k_vcount1(const VItem *__restrict__ items,
         t = find_item(blk_prefix, nitems, g);
         it = items[t];
       }
-      GLevel &L = *(GLevel *)it.lv;
+      CLevel &L = *(CLevel *)it.lv;
       const uint64_t r = it.row_begin + (g - blk_prefix[t]) * VB + threadIdx.x;
       if (r >= it.row_end) continue;
       const uint32_t *row = it.rows + r * it.k;
@@ -612,7 +838,7 @@ __global__ void __launch_bounds__(VB) k_vmark(const VItem *__restrict__ items, u
   for (uint64_t g = g0 + blockIdx.x; g < g1; g += gridDim.x) {
     const uint32_t t = find_item(blk_prefix, nitems, g);
     const VItem it = items[t];
-    GLevel &L = *(GLevel *)it.lv;
+    CLevel &L = *(CLevel *)it.lv;
     const uint64_t r = it.row_begin + (g - blk_prefix[t]) * VB + threadIdx.x;
     // k_vcount1 reads list values only to remove equal-label columns
     if (r >= it.row_end || (count_only && L.ndup == 0)) continue;
@@ -638,23 +864,34 @@ void build_vlevels(gem_ctx *c, VQueryState &S) {
   const gemh::VertexPlan &P = S.plan;
   const uint32_t nv = Qd.Q.nv;
   std::vector<VLevel> lv(nv);
+  std::vector<std::vector<uint32_t>> live;
+  gemh::live_columns(P, &live);
+  S.cols_in.assign(nv, 1);
+  for (uint32_t i = 1; i < nv; ++i) S.cols_in[i] = (uint32_t)live[i].size();
   for (uint32_t i = 1; i < nv; ++i) {
     const gemh::VLevelPlan &lp = P.levels[i];
     VLevel &L = lv[i];
     L.nb = lp.nb;
     L.ndup = lp.ndup;
+    const std::vector<uint32_t> &in = live[i];
+    auto at = [&](uint32_t col) { return (uint32_t)(std::lower_bound(in.begin(), in.end(), col) - in.begin()); };
     for (uint32_t j = 0; j < lp.nb; ++j) {
       const TableDev &T = Qd.tab[lp.directed[j]];
       if (!T.present) throw Error{GEM_E_STATE, "vertex plan uses a table that was not built"};
-      L.key_col[j] = lp.key_col[j];
+      L.key_col[j] = at(lp.key_col[j]);
       L.toff[j] = T.off.as<uint64_t>();
       L.tval[j] = T.val.as<uint32_t>();
     }
     const uint32_t u = P.vorder[i];
     for (uint32_t d = 0; d < lp.ndup; ++d) {
-      L.dup_col[d] = lp.dup_col[d];
+      L.dup_col[d] = at(lp.dup_col[d]);
       L.dup_can[d] = Qd.can.as<uint32_t>() + Qd.can_off[P.vorder[lp.dup_col[d]]];
     }
+    if (i + 1 < nv) {
+      L.kout = (uint32_t)live[i + 1].size();
+      for (uint32_t x = 0; x < L.kout; ++x) L.src[x] = live[i + 1][x] == i ? COL_NEW : (uint8_t)at(live[i + 1][x]);
+    }
+    L.can_new = Qd.can.as<uint32_t>() + Qd.can_off[u];
     L.bm_new = Qd.bitmap.as<uint64_t>() + (uint64_t)u * Qd.W;
     L.rank_new = Qd.rank.as<uint32_t>() + (uint64_t)u * (Qd.W + 1);
   }
@@ -697,8 +934,9 @@ uint64_t attempt_limit(const VQueryState &S, uint32_t a) {
 // candidates, no count yet.
 static void seed_query(gem_ctx *c, VQueryState &V) {
   hipStream_t s = c->stream;
-  gemh::SQuery<DevBuf> &Q = V.s;
+  gemh::SQuery<LevelBuf> &Q = V.s;
   Q.nb = V.max_nb;
+  Q.width = V.cols_in;
   Q.count = 0;
   Q.fin_bound = Q.fin_got = 0;
   Q.stack.clear();
@@ -709,11 +947,11 @@ static void seed_query(gem_ctx *c, VQueryState &V) {
     Q.done = true;
     return;
   }
-  auto buf = std::make_shared<DevBuf>();
+  auto buf = std::make_shared<LevelBuf>();
   buf->alloc(n0 * 4, s);
   k_viota<<<(uint32_t)((n0 + 255) / 256), 256, 0, s>>>(buf->as<uint32_t>(), n0);
   GEM_LAUNCH_CHECK("k_viota");
-  gemh::SLevel<DevBuf> L;
+  gemh::SLevel<LevelBuf> L;
   L.level = 1;
   L.rows = std::move(buf);
   L.nrows = n0;
@@ -727,10 +965,11 @@ struct Launch {
   std::vector<VItem> items;
   std::vector<uint64_t> blk;  // prefix, items.size() + 1
   uint32_t max_nb = 1, max_ndup = 0;
-  void add(const VItem &it, uint32_t nb, uint32_t ndup) {
+  // tasks: 256-row blocks unless given
+  void add(const VItem &it, uint32_t nb, uint32_t ndup, uint64_t tasks = 0) {
     if (blk.empty()) blk.push_back(0);
     items.push_back(it);
-    blk.push_back(blk.back() + (it.row_end - it.row_begin + VB - 1) / VB);
+    blk.push_back(blk.back() + (tasks ? tasks : (it.row_end - it.row_begin + VB - 1) / VB));
     max_nb = std::max(max_nb, nb);
     max_ndup = std::max(max_ndup, ndup);
   }
@@ -755,6 +994,17 @@ void upload(gem_ctx *c, const Launch &L, DevLaunch &D) {
 uint32_t g_persistent_blocks = 2048;
 uint32_t grid_for(uint64_t blocks) {
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(blocks, g_persistent_blocks));
+}
+
+// Blocks of VB threads of a kernel that the device runs at once: a persistent
+// grid has no use for more (the later ones would start when the work is done,
+// and make the runs of the others shorter).
+uint32_t resident_blocks(const void *kernel, size_t lds) {
+  int per_cu = 0, dev = 0, cus = 0;
+  GEM_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, VB, lds));
+  GEM_HIP_CHECK(hipGetDevice(&dev));
+  GEM_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  return (uint32_t)std::max(1, per_cu * cus);
 }
 
 // Rows whose driving list has more entries than the context's heavy_t are
@@ -789,9 +1039,9 @@ struct ExtSlot {
   unsigned char *h_hdr = nullptr;
   size_t hdr_bytes = 0;
   uint32_t max_nb = 1, max_ndup = 0;
+  uint32_t lcap = 0, dcap = 0;  // lists and equal-label columns k_vext keeps in LDS
   size_t lds = 0;
-  uint32_t vthreads = VB;  // k_vext block size: 64 when four waves' lists do not fit one block's LDS
-  uint32_t grid = 0;
+  uint32_t grid[5] = {};  // write walk, final walk, final count, heavy write, heavy final
   uint32_t heavy_t = 1024, heavy_chunk = 1024;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -801,13 +1051,14 @@ struct ExtSlot {
     cap = std::max<uint32_t>(capacity, 1);
     max_nb = std::max<uint32_t>(mnb, 1);
     max_ndup = mnd;
-    // per wave: (nb - 1) list addresses and lengths and ndup equal-label
-    // positions for each of its 64 rows (at most 31 KB with 32 query vertices)
-    const size_t lds_wave = (size_t)64 * ((max_nb - 1) * 12 + max_ndup * 4);
-    vthreads = lds_wave * VW <= 60 * 1024 ? VB : 64;
-    lds = lds_wave * (vthreads / 64);
-    if (lds > 60 * 1024) throw Error{GEM_E_LIMIT, "a level has too many backward edges for the vjoin LDS layout"};
-    grid = g_persistent_blocks;
+    lcap = max_nb > 1 ? std::min(max_nb, LDS_LISTS) : 0;
+    dcap = std::min(max_ndup, LDS_DUPS);
+    lds = (size_t)VW * 64 * (lcap * 12 + dcap * 4);
+    const void *kernels[5] = {(const void *)&k_vext<false, false>, (const void *)&k_vext<true, false>,
+                              (const void *)&k_vcount1<false>, (const void *)&k_vext_heavy<false, false>,
+                              (const void *)&k_vext_heavy<true, false>};
+    for (int i = 0; i < 5; ++i)
+      grid[i] = std::min(g_persistent_blocks, resident_blocks(kernels[i], i < 2 ? lds : 0));
     heavy_t = c->heavy_t;
     heavy_chunk = c->heavy_chunk;
     hdr_bytes = HDR_CTR + 8ull * CTR_STRIDE * cap;
@@ -859,43 +1110,43 @@ struct ExtSlot {
     // an eager one launches those that have items
     uint64_t e[3];
     for (int i = 0; i < 3; ++i) e[i] = captured || *nitems(i) ? ~0ull : 0;
-    launch_kernels<false>(c, grid, dn, dq, dq + 3 * WQ_WORDS, hn, prof_kernels, count_items, 0, e[0], 0, e[1], 0, e[2]);
+    launch_kernels<false>(c, ~0u, dn, dq, dq + 3 * WQ_WORDS, hn, prof_kernels, count_items, 0, e[0], 0, e[1], 0, e[2]);
     GEM_HIP_CHECK(hipMemcpyAsync(h_hdr, d, hdr_bytes, hipMemcpyDeviceToHost, s));
   }
 
-  // The three kernels over task ranges [b_i, e_i) of launch i (queues
+  // (At most `most` blocks each.)  The three kernels over task ranges [b_i, e_i) of launch i (queues
   // dq, WQ_WORDS words each), then the heavy rows the two walking launches set
   // aside (queues hq, row counts hn[0..1]; everything starts at zero).
   template <bool OOC>
-  void launch_kernels(gem_ctx *c, uint32_t grd, const uint32_t *dn, unsigned int *dq, unsigned int *hq,
+  void launch_kernels(gem_ctx *c, uint32_t most, const uint32_t *dn, unsigned int *dq, unsigned int *hq,
                       unsigned int *hn, bool prof_kernels, bool count_items, uint64_t b0, uint64_t e0, uint64_t b1,
                       uint64_t e1, uint64_t b2, uint64_t e2) {
     hipStream_t s = c->stream;
     unsigned long long *dp = reinterpret_cast<unsigned long long *>(hdr.as<unsigned char>() + HDR_PITEMS);
     if (b0 < e0) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_WRITE : -1);
-      k_vext<false, OOC><<<grd * (VB / vthreads), vthreads, lds, s>>>(items[0].as<VItem>(), dn + 0, blk[0].as<uint64_t>(), dq + 0, max_nb,
-                                               max_ndup, count_items ? dp : nullptr, count_items ? dp + 4 : nullptr,
+      k_vext<false, OOC><<<std::min(most, grid[0]), VB, lds, s>>>(items[0].as<VItem>(), dn + 0, blk[0].as<uint64_t>(), dq + 0, lcap, dcap,
+                                               count_items ? dp : nullptr, count_items ? dp + 4 : nullptr,
                                                b0, e0, heavy[0].as<HeavyRow>(), hn + 0, HEAVY_CAP, heavy_t);
       GEM_LAUNCH_CHECK("k_vext<write>");
     }
     if (b1 < e1) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_FINAL : -1);
-      k_vext<true, OOC><<<grd * (VB / vthreads), vthreads, lds, s>>>(items[1].as<VItem>(), dn + 1, blk[1].as<uint64_t>(), dq + WQ_WORDS, max_nb,
-                                              max_ndup, count_items ? dp + 1 : nullptr, nullptr, b1, e1,
+      k_vext<true, OOC><<<std::min(most, grid[1]), VB, lds, s>>>(items[1].as<VItem>(), dn + 1, blk[1].as<uint64_t>(), dq + WQ_WORDS, lcap, dcap,
+                                              count_items ? dp + 1 : nullptr, nullptr, b1, e1,
                                               heavy[1].as<HeavyRow>(), hn + 1, HEAVY_CAP, heavy_t);
       GEM_LAUNCH_CHECK("k_vext<final>");
     }
     if (b2 < e2) {
       ProfLaunch pl(c, prof_kernels ? K_VCOUNT1 : -1);
-      k_vcount1<OOC><<<grd, VB, 0, s>>>(items[2].as<VItem>(), dn + 2, blk[2].as<uint64_t>(), dq + 2 * WQ_WORDS, b2, e2);
+      k_vcount1<OOC><<<std::min(most, grid[2]), VB, 0, s>>>(items[2].as<VItem>(), dn + 2, blk[2].as<uint64_t>(), dq + 2 * WQ_WORDS, b2, e2);
       GEM_LAUNCH_CHECK("k_vcount1");
     }
     if (b0 < e0) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_HEAVY_WRITE : -1);
       k_heavy_scan<<<1, 1024, 0, s>>>(heavy[0].as<HeavyRow>(), hn + 0, HEAVY_CAP, heavy_chunk, hpre[0].as<uint64_t>());
       GEM_LAUNCH_CHECK("k_heavy_scan");
-      k_vext_heavy<false, OOC><<<grd, VB, 0, s>>>(items[0].as<VItem>(), heavy[0].as<HeavyRow>(), hn + 0, HEAVY_CAP,
+      k_vext_heavy<false, OOC><<<std::min(most, grid[3]), VB, 0, s>>>(items[0].as<VItem>(), heavy[0].as<HeavyRow>(), hn + 0, HEAVY_CAP,
                                                    hpre[0].as<uint64_t>(), hq + 0, heavy_chunk,
                                                    count_items ? dp + 2 : nullptr, count_items ? dp + 5 : nullptr);
       GEM_LAUNCH_CHECK("k_vext_heavy<write>");
@@ -904,7 +1155,7 @@ struct ExtSlot {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_HEAVY_FINAL : -1);
       k_heavy_scan<<<1, 1024, 0, s>>>(heavy[1].as<HeavyRow>(), hn + 1, HEAVY_CAP, heavy_chunk, hpre[1].as<uint64_t>());
       GEM_LAUNCH_CHECK("k_heavy_scan");
-      k_vext_heavy<true, OOC><<<grd, VB, 0, s>>>(items[1].as<VItem>(), heavy[1].as<HeavyRow>(), hn + 1, HEAVY_CAP,
+      k_vext_heavy<true, OOC><<<std::min(most, grid[4]), VB, 0, s>>>(items[1].as<VItem>(), heavy[1].as<HeavyRow>(), hn + 1, HEAVY_CAP,
                                                   hpre[1].as<uint64_t>(), hq + WQ_WORDS, heavy_chunk,
                                                   count_items ? dp + 3 : nullptr, nullptr);
       GEM_LAUNCH_CHECK("k_vext_heavy<final>");
@@ -966,7 +1217,7 @@ struct ExtSlot {
           }
         }
         const uint64_t most = std::max(hi[0] - lo[0], std::max(hi[1] - lo[1], hi[2] - lo[2]));
-        const uint32_t grd = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(grid, most));
+        const uint32_t grd = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(~0u, most));
         // per group: 3 main queues, 2 heavy queues, 2 heavy-row counts
         unsigned int *gq = q + (size_t)GROUP_WORDS * g;
         launch_kernels<true>(c, grd, dn, gq, gq + 3 * WQ_WORDS, gq + 5 * WQ_WORDS, prof, prof, lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]);
@@ -1009,8 +1260,8 @@ namespace {
 // caching allocator, length passes, extend steps through the fixed launch
 // buffers of the run (eager, captured as a hipGraph, or with streamed tables).
 struct HipSchedBackend {
-  using Buf = DevBuf;
-  using Item = gemh::SItem<DevBuf>;
+  using Buf = LevelBuf;
+  using Item = gemh::SItem<LevelBuf>;
   gem_ctx *c;
   std::vector<VQueryState *> &qs;
   ExtSlot &slot;
@@ -1023,16 +1274,16 @@ struct HipSchedBackend {
   double t_len = 0, t_ext = 0;
   uint64_t ext_tasks = 0;
 
-  static uint64_t buf_bytes(const DevBuf &b) { return b.bytes; }
+  static uint64_t buf_bytes(const LevelBuf &b) { return b.bytes; }
 
-  std::shared_ptr<DevBuf> alloc(uint64_t bytes) {
-    auto b = std::make_shared<DevBuf>();
+  std::shared_ptr<LevelBuf> alloc(uint64_t bytes) {
+    auto b = std::make_shared<LevelBuf>();
     b->alloc(bytes, c->stream);
     return b;
   }
 
-  std::shared_ptr<DevBuf> shrink(const std::shared_ptr<DevBuf> &from, uint64_t bytes) {
-    auto b = std::make_shared<DevBuf>();
+  std::shared_ptr<LevelBuf> shrink(const std::shared_ptr<LevelBuf> &from, uint64_t bytes) {
+    auto b = std::make_shared<LevelBuf>();
     b->alloc(bytes, c->stream);
     GEM_HIP_CHECK(hipMemcpyAsync(b->p, from->p, bytes, hipMemcpyDeviceToDevice, c->stream));
     return b;
@@ -1056,7 +1307,9 @@ struct HipSchedBackend {
     DevLaunch D;
     upload(c, L, D);
     const uint64_t nblk = L.blk.back(), nunit = nblk * VW;
-    DevBuf bu, bp;
+    DevBuf bu;
+    auto kept = std::make_shared<DevBuf>();  // the unit prefix, which the levels keep for their write walks
+    DevBuf &bp = *kept;
     bu.alloc(nunit * 8, s);
     bp.alloc((nunit + 1) * 8, s);
     {
@@ -1066,6 +1319,11 @@ struct HipSchedBackend {
       GEM_LAUNCH_CHECK("k_vlen");
     }
     scan_u64(c, bu.as<uint64_t>(), bp.as<uint64_t>(), nunit);
+    for (size_t t = 0; t < items.size(); ++t) {
+      items[t].rows->units = kept;
+      items[t].rows->unit0 = L.blk[t] * VW - items[t].row_begin / gemh::SCHED_UNIT;
+    }
+    if (!prefix) return;
     uint64_t *pref = pinned<uint64_t>(c, nunit + 1);
     GEM_HIP_CHECK(hipMemcpyAsync(pref, bp.p, (nunit + 1) * 8, hipMemcpyDeviceToHost, s));
     GEM_HIP_CHECK(hipStreamSynchronize(s));
@@ -1083,6 +1341,20 @@ struct HipSchedBackend {
     t_len += std::chrono::duration<double>(clk::now() - t0).count();
   }
 
+  // Unit prefixes of chunks whose level came back from host memory without
+  // them; they are dropped again by extend (they cover the chunk only).
+  std::vector<const LevelBuf *> remeasure(const std::vector<Item> &wr_items) {
+    std::vector<Item> need;
+    std::vector<const LevelBuf *> bufs;
+    for (const Item &x : wr_items)
+      if (!x.rows->units) {
+        need.push_back(x);
+        bufs.push_back(x.rows);
+      }
+    if (!need.empty()) length_pass(need, nullptr);
+    return bufs;
+  }
+
   void extend(const std::vector<Item> &wr_items, const std::vector<Item> &fin_items, std::vector<uint64_t> *got_wr,
               std::vector<uint64_t> *got_fin) {
     const auto t0 = clk::now();
@@ -1092,12 +1364,34 @@ struct HipSchedBackend {
     Launch wr, fin, fin1;
     std::vector<std::pair<int, size_t>> fin_at(fin_items.size());
     size_t nctr = 0;
+    // counters / work queues / walked-entry counts travel zeroed in the copy
+    std::memset(slot.h_hdr + ExtSlot::HDR_HEAVYN, 0, slot.hdr_bytes - ExtSlot::HDR_HEAVYN);
+    auto units_of = [](const Item &x) { return (x.row_end - x.row_begin + gemh::SCHED_UNIT - 1) / gemh::SCHED_UNIT; };
+    // runs of the write walks (see unit_range): CLAIMS per wave of the grid by
+    // cost, an entry of a level with other lists costing its searches too
+    auto weight = [&](const Item &x) { return 4ull * qs[x.q]->max_nb[x.level] - 3; };
+    uint64_t run_cost = 0;
+    std::vector<const LevelBuf *> once;
+    if (!tc) {
+      uint64_t cost = 0;
+      for (const Item &x : wr_items) cost += (x.out_rows + UNIT_COST * units_of(x)) * weight(x);
+      run_cost = cost / ((uint64_t)slot.grid[0] * VW * CLAIMS) + 1;
+      once = remeasure(wr_items);
+    }
     for (const Item &x : wr_items) {
       VItem it = vitem(x);
       it.out = x.out->as<uint32_t>();
       it.out_cap = x.out_rows;
       it.counter = slot.dev_counter(nctr++);
-      wr.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level]);
+      if (run_cost) {
+        it.units = x.rows->units->as<uint64_t>() + x.rows->unit0 + x.row_begin / gemh::SCHED_UNIT;
+        it.nunits = (uint32_t)units_of(x);
+        it.run_cost = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(run_cost / weight(x), 4 * UNIT_COST), RUN_COST);
+        wr.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level],
+               (x.out_rows + UNIT_COST * units_of(x) - 1) / it.run_cost + 1);
+      } else {
+        wr.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level]);
+      }
     }
     std::vector<size_t> fin_ctr(fin_items.size());
     for (size_t t = 0; t < fin_items.size(); ++t) {
@@ -1121,8 +1415,6 @@ struct HipSchedBackend {
       *slot.nitems(i) = (uint32_t)L.items.size();
       ext_tasks += L.blk.empty() ? 0 : L.blk.back();
     }
-    // counters / work queues / walked-entry counts travel zeroed in the copy
-    std::memset(slot.h_hdr + ExtSlot::HDR_HEAVYN, 0, slot.hdr_bytes - ExtSlot::HDR_HEAVYN);
     const bool prof = c->prof.on;
     if (tc)
       slot.launch_streamed(c, *tc);
@@ -1130,6 +1422,7 @@ struct HipSchedBackend {
       slot.launch(c, c->use_graph && !prof);
     GEM_HIP_CHECK(hipStreamSynchronize(s));
     if (tc) tc->finish();
+    for (const LevelBuf *b : once) b->units.reset();
     got_wr->resize(wr_items.size());
     got_fin->resize(fin_items.size());
     for (size_t t = 0; t < wr_items.size(); ++t) {
@@ -1162,7 +1455,7 @@ struct HipSchedBackend {
   // the context stream (the device buffer goes back to the pool at once: its
   // next user is ordered after the copy).  A host buffer is freed after the
   // stream has drained, so no copy still reads or writes it.
-  std::shared_ptr<void> swap_out(const DevBuf &b, uint64_t bytes) {
+  std::shared_ptr<void> swap_out(const LevelBuf &b, uint64_t bytes) {
     void *h = nullptr;
     GEM_HIP_CHECK(hipHostMalloc(&h, std::max<uint64_t>(bytes, 1), hipHostMallocDefault));
     hipStream_t s = c->stream;
@@ -1173,8 +1466,8 @@ struct HipSchedBackend {
     GEM_HIP_CHECK(hipMemcpyAsync(h, b.p, bytes, hipMemcpyDeviceToHost, s));
     return hp;
   }
-  std::shared_ptr<DevBuf> swap_in(const std::shared_ptr<void> &h, uint64_t bytes) {
-    auto b = std::make_shared<DevBuf>();
+  std::shared_ptr<LevelBuf> swap_in(const std::shared_ptr<void> &h, uint64_t bytes) {
+    auto b = std::make_shared<LevelBuf>();
     b->alloc(bytes, c->stream);
     GEM_HIP_CHECK(hipMemcpyAsync(b->p, h.get(), bytes, hipMemcpyHostToDevice, c->stream));
     return b;
@@ -1262,7 +1555,7 @@ struct HipSchedBackend {
   // Its limit becomes what it has spent plus 1.5 times that estimate.
   bool prolong(uint32_t qi) {
     VQueryState &V = *qs[qi];
-    gemh::SQuery<DevBuf> &Q = V.s;
+    gemh::SQuery<LevelBuf> &Q = V.s;
     if (!cap_ || Q.count < cap_ / 4 || Q.count == 0) return false;
     const uint64_t spent = Q.work - Q.attempt_start;
     const double need = (double)spent * ((double)(cap_ + 1) / (double)Q.count - 1.0);
@@ -1281,7 +1574,7 @@ struct HipSchedBackend {
   // the next ranked order, with the next attempt's limit.
   bool restart(uint32_t qi) {
     VQueryState &V = *qs[qi];
-    gemh::SQuery<DevBuf> &Q = V.s;
+    gemh::SQuery<LevelBuf> &Q = V.s;
     if (!attempt_limit(V, 0)) return false;
     const uint32_t a = Q.attempts + 1;
     if (V.max_attempts && a >= V.max_attempts) return false;
@@ -1383,11 +1676,11 @@ void VBatchRunner::run(std::vector<VQueryState *> &qs) {
   }
   // queries are seeded with the identity level of their first vertex when
   // the scheduler starts them (HipSchedBackend::admit)
-  std::vector<gemh::SQuery<DevBuf> *> sq;
+  std::vector<gemh::SQuery<LevelBuf> *> sq;
   for (VQueryState *S : qs) {
-    gemh::SQuery<DevBuf> &Q = S->s;
+    gemh::SQuery<LevelBuf> &Q = S->s;
     const int64_t partner = Q.partner;
-    Q = gemh::SQuery<DevBuf>{};
+    Q = gemh::SQuery<LevelBuf>{};
     Q.partner = partner;
     // (a pending state's query may still be being prepared: its vertex count
     // was recorded when the state was made)

@@ -178,32 +178,32 @@ __device__ __forceinline__ void contains_pair(const uint32_t *a0, uint32_t n0, u
 // Four membership tests at once (contains_pair for four values): v[g] in
 // sorted a[g][0..n[g]); k[g] enters as "still wanted" and leaves as the
 // result.  The four searches advance in lockstep, so up to four loads of one
-// lane are in flight at every stage.
+// lane are in flight at every stage.  A search that has ended goes on loading
+// from `any` (one readable word) instead of masking its lane off: the steps are
+// selects and not branches (with four branches a step, the walk kernel ran
+// more scalar than vector instructions).
 __device__ __forceinline__ void contains_quad(const uint32_t *const a[4], const uint32_t n_in[4],
-                                              const uint32_t v[4], bool k[4]) {
-  uint32_t lo[4], n[4];
+                                              const uint32_t v[4], bool k[4], const uint32_t *any) {
+  const uint32_t *p[4];
+  uint32_t n[4];
   bool f[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    lo[g] = 0;
+    p[g] = a[g];
     n[g] = k[g] ? n_in[g] : 0;
     f[g] = false;
   }
-  while (n[0] | n[1] | n[2] | n[3]) {
+  while (__any(n[0] | n[1] | n[2] | n[3])) {
     uint32_t x[4];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) x[g] = n[g] ? ldg(a[g] + lo[g] + (n[g] >> 1)) : 0;
+    for (int g = 0; g < 4; ++g) x[g] = ldg(n[g] ? p[g] + (n[g] >> 1) : any);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      if (!n[g]) continue;
       const uint32_t h = n[g] >> 1;
-      if (x[g] < v[g]) {
-        lo[g] += h + 1;
-        n[g] -= h + 1;
-      } else {
-        f[g] |= x[g] == v[g];
-        n[g] = h;
-      }
+      const bool less = x[g] < v[g];
+      f[g] = f[g] || (n[g] && x[g] == v[g]);
+      p[g] += less ? h + 1 : 0;
+      n[g] = !n[g] ? 0 : less ? n[g] - h - 1 : h;
     }
   }
 #pragma unroll

@@ -340,6 +340,20 @@ int make_vertex_plan(const QueryInfo &q, const std::vector<uint32_t> &vorder, Ve
   return GEM_OK;
 }
 
+void live_columns(const VertexPlan &plan, std::vector<std::vector<uint32_t>> *live) {
+  const uint32_t nv = (uint32_t)plan.vorder.size();
+  std::vector<uint32_t> last(nv, 0);  // the last level that reads a column
+  for (uint32_t i = 1; i < nv; ++i) {
+    const VLevelPlan &L = plan.levels[i];
+    for (uint32_t j = 0; j < L.nb; ++j) last[L.key_col[j]] = i;
+    for (uint32_t d = 0; d < L.ndup; ++d) last[L.dup_col[d]] = i;
+  }
+  live->assign(nv, {});
+  for (uint32_t i = 1; i < nv; ++i)
+    for (uint32_t c = 0; c < i; ++c)
+      if (last[c] >= i) (*live)[i].push_back(c);
+}
+
 static int32_t q16(double x) { return (int32_t)std::llround(16.0 * std::log2(1.0 + std::max(0.0, x))); }
 
 // fanout of the table w -> u: average row length

@@ -116,6 +116,10 @@ struct VertexPlan {
 int vertex_order_from_edges(const QueryInfo &q, const uint32_t *edge_order, std::vector<uint32_t> *vorder);
 // Requires vorder[0] to be a non-leaf and every later vertex to have an
 // earlier neighbour.
+// live[i] (i >= 1): the vertex-order positions below i that level i or a later
+// one reads, as the key of a backward list or as an equal-label column,
+// ascending.  Level i's input rows hold these columns only.
+void live_columns(const VertexPlan &plan, std::vector<std::vector<uint32_t>> *live);
 int make_vertex_plan(const QueryInfo &q, const std::vector<uint32_t> &vorder, VertexPlan *plan);
 
 // ------------------------------------------------------- learned ordering

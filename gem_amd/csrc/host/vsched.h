@@ -22,6 +22,11 @@
 // so the charged bytes never exceed
 //   budget + (levels - 1) * max(force_chunk, largest unit bound).
 //
+// Rows are charged at 4 bytes per earlier query vertex.  A level may hold fewer
+// columns (SQuery::width) and then takes less memory than it is charged; the
+// chunks, and with them the order in which a capped query is searched, do not
+// depend on that.
+//
 // Restarts.  A query may carry a limit on the work of its current attempt
 // (attempt_limit).  When an attempt goes past it, its pending levels are
 // dropped and the backend may start the query again (another vertex order, a
@@ -107,6 +112,8 @@ template <class Buf>
 struct SQuery {
   uint32_t nv = 0;
   std::vector<uint32_t> nb;  // backward lists of each level (nb[i], i >= 1)
+  std::vector<uint32_t> width;  // columns of each level's input rows (empty: one per earlier vertex)
+  uint32_t cols(uint32_t level) const { return width.empty() ? level : width[level]; }
   std::vector<SLevel<Buf>> stack;
   std::vector<uint64_t> level_rows;  // rows after each level
   uint64_t count = 0, processed = 0;
@@ -129,7 +136,7 @@ struct SQuery {
 
 // One unit of a launch: rows [row_begin, row_end) of a pending level of
 // query `q`, extended to `level`; `out` (write items) receives at most
-// out_rows rows of k + 1 columns.
+// out_rows rows of the next level's columns.
 template <class Buf>
 struct SItem {
   uint32_t q = 0, level = 0, k = 0;
@@ -247,10 +254,15 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
   using Buf = typename BE::Buf;
   using Item = SItem<Buf>;
   const uint64_t budget = cfg.budget;
+  auto charge = [](const SQuery<Buf> &S, const SLevel<Buf> &L) -> uint64_t {
+    if (!L.rows) return 0;
+    const uint32_t cols = S.cols(L.level);
+    return cols == L.level ? BE::buf_bytes(*L.rows) : BE::buf_bytes(*L.rows) / cols * L.level;
+  };
   auto live_bytes = [&]() {
     uint64_t b = 0;
     for (SQuery<Buf> *S : qs)
-      for (const SLevel<Buf> &L : S->stack) b += L.rows ? BE::buf_bytes(*L.rows) : 0;
+      for (const SLevel<Buf> &L : S->stack) b += charge(*S, L);
     return b;
   };
   std::vector<uint8_t> started(qs.size(), 0);
@@ -370,8 +382,8 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
       const uint64_t nu = top.nunits();
       if (top.level + 1 != S.nv) {
         uint64_t mine = 0;
-        for (const SLevel<Buf> &L : S.stack) mine += L.rows ? BE::buf_bytes(*L.rows) : 0;
-        cand.push_back(ChunkCand{&top.unit_u, top.cursor, nu, 4ull * (top.k + 1), top.level, mine, quota,
+        for (const SLevel<Buf> &L : S.stack) mine += charge(S, L);
+        cand.push_back(ChunkCand{&top.unit_u, top.cursor, nu, 4ull * (top.level + 1), top.level, mine, quota,
                                  S.nv - 1 - top.level});
         cand_owner.push_back(qi);
         continue;
@@ -434,7 +446,7 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
         continue;
       }
       const uint64_t ub = top.unit_u[b1] - top.unit_u[b0];
-      const uint64_t rb = 4ull * (top.k + 1);
+      const uint64_t rb = 4ull * (top.level + 1);
       Item it;
       it.q = qi;
       it.level = top.level;
@@ -447,7 +459,7 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
       top.cursor = b1;
       if (ub) {
         keep_alive.push_back(top.rows);
-        std::shared_ptr<Buf> out = be.alloc(ub * rb);
+        std::shared_ptr<Buf> out = be.alloc(ub * 4ull * S.cols(top.level + 1));
         charged += ub * rb;
         it.out = out.get();
         it.out_rows = ub;
@@ -478,13 +490,13 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
         // than half of those rows survived, they move to a buffer of their
         // size, and the bound-sized one goes back at once (pending rows are
         // what the budget is charged with)
-        const uint64_t rb = 4ull * (it.k + 1);
+        const uint64_t rb = 4ull * S.cols(it.level + 1);
         if (2 * got <= it.out_rows && it.out_rows * rb >= cfg.shrink_min) rows = be.shrink(rows, got * rb);
         SLevel<Buf> L;
         L.level = it.level + 1;
         L.rows = std::move(rows);
         L.nrows = got;
-        L.k = it.k + 1;
+        L.k = S.cols(it.level + 1);
         L.last_use = st->iterations;
         S.stack.push_back(std::move(L));
       }
@@ -528,13 +540,13 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
     if (cfg.swap_bytes) {
       uint64_t dev = live_bytes();
       if (dev > budget) {
-        std::vector<SLevel<Buf> *> cands;
+        std::vector<std::pair<SLevel<Buf> *, uint64_t>> cands;  // level, its charge
         for (SQuery<Buf> *S : qs)
           for (size_t i = 0; i + 1 < S->stack.size(); ++i)
-            if (S->stack[i].rows) cands.push_back(&S->stack[i]);
+            if (S->stack[i].rows) cands.push_back({&S->stack[i], charge(*S, S->stack[i])});
         std::stable_sort(cands.begin(), cands.end(),
-                         [](const SLevel<Buf> *a, const SLevel<Buf> *b) { return a->last_use < b->last_use; });
-        for (SLevel<Buf> *L : cands) {
+                         [](const auto &a, const auto &b) { return a.first->last_use < b.first->last_use; });
+        for (auto [L, charged_bytes] : cands) {
           if (dev <= budget) break;
           const uint64_t b = BE::buf_bytes(*L->rows);
           if (host_used + b > cfg.swap_bytes) continue;
@@ -542,7 +554,7 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
           L->host_bytes = b;
           L->rows.reset();
           host_used += b;
-          dev -= b;
+          dev -= charged_bytes;
           ++st->swaps_out;
           st->swap_bytes_out += b;
         }
