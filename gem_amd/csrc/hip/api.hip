@@ -216,11 +216,16 @@ int gem_hip_load_data_csr(gem_ctx *c, const gem_csr_view *g) {
     G = GraphDev();
     G.n = g->num_v;
     G.slots = g->num_slots;
+    std::vector<uint32_t> heavy, hubs;
     for (uint32_t v = 0; v < g->num_v; ++v) {
       if (g->offsets[v + 1] < g->offsets[v]) throw Error{GEM_E_INVALID, "offsets not monotone"};
-      G.max_deg = std::max<uint64_t>(G.max_deg, g->offsets[v + 1] - g->offsets[v]);
-      if (g->offsets[v + 1] - g->offsets[v] > gemd::FILTER_HUB_DEG) ++G.n_hub;
+      const uint64_t deg = g->offsets[v + 1] - g->offsets[v];
+      G.max_deg = std::max<uint64_t>(G.max_deg, deg);
+      if (deg > gemd::FILTER_LIGHT_DEG) (deg > gemd::FILTER_HUB_DEG ? hubs : heavy).push_back(v);
     }
+    G.n_heavy = (uint32_t)heavy.size();
+    G.n_hub = (uint32_t)hubs.size();
+    heavy.insert(heavy.end(), hubs.begin(), hubs.end());
     // dense label ids in first-seen order
     std::vector<uint32_t> dense(g->num_v);
     for (uint32_t v = 0; v < g->num_v; ++v) {
@@ -231,16 +236,27 @@ int gem_hip_load_data_csr(gem_ctx *c, const gem_csr_view *g) {
         G.label_id.emplace(g->labels[v], id);
         G.label_freq.push_back(0);
         G.label_deg.push_back(0);
+        G.label_long.push_back(0);
+        G.label_chunks.push_back(0);
       } else {
         id = it->second;
       }
       G.label_freq[id]++;
-      G.label_deg[id] += g->offsets[v + 1] - g->offsets[v];
+      const uint64_t deg = g->offsets[v + 1] - g->offsets[v];
+      G.label_deg[id] += deg;
+      if (deg > gemd::TABLE_HEAVY_ROW) {
+        G.label_long[id]++;
+        G.label_chunks[id] += (deg + gemd::TABLE_CHUNK - 1) / gemd::TABLE_CHUNK;
+      }
       dense[v] = id;
     }
     G.lab8 = G.label_freq.size() <= 255;
     hipStream_t s = c->stream;
     G.off.alloc(((uint64_t)G.n + 1) * 8, s);
+    if (!heavy.empty()) {
+      G.heavy.alloc(heavy.size() * 4, s);
+      GEM_HIP_CHECK(hipMemcpyAsync(G.heavy.p, heavy.data(), heavy.size() * 4, hipMemcpyHostToDevice, s));
+    }
     GEM_HIP_CHECK(hipMemcpyAsync(G.off.p, g->offsets, ((uint64_t)G.n + 1) * 8, hipMemcpyHostToDevice, s));
     if (c->graph_host) {
       // Host-resident graph: the neighbour array (all but 12 B per vertex of
@@ -259,6 +275,7 @@ int gem_hip_load_data_csr(gem_ctx *c, const gem_csr_view *g) {
       std::vector<uint8_t> l8(dense.begin(), dense.end());
       G.lab.alloc(std::max<uint64_t>(G.n, 1), s);
       GEM_HIP_CHECK(hipMemcpyAsync(G.lab.p, l8.data(), G.n, hipMemcpyHostToDevice, s));
+      make_slot_labels(c, G);
       GEM_HIP_CHECK(hipStreamSynchronize(s));
     } else {
       G.lab.alloc(std::max<uint64_t>(G.n, 1) * 4, s);

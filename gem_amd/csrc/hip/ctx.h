@@ -148,24 +148,34 @@ struct GraphDev {
   uint32_t n = 0;
   uint64_t slots = 0;
   uint64_t max_deg = 0;
-  uint32_t n_hub = 0;  // vertices of degree > FILTER_HUB_DEG
+  // vertices of degree in (FILTER_LIGHT_DEG, FILTER_HUB_DEG] and above, and
+  // their ids: u32[n_heavy + n_hub], the hubs last
+  uint32_t n_heavy = 0, n_hub = 0;
+  DevBuf heavy;
   DevBuf off;     // u64[n + 1]
   DevBuf nbr;     // u32[slots] in HBM, or
   PinnedBuf nbr_host;  // u32[slots] in mapped pinned host memory (host-resident graph)
   const uint32_t *nbr_mapped = nullptr;  // device address of nbr_host
   DevBuf lab;     // u8[n] or u32[n] dense label ids
+  DevBuf nbr_lab; // u8[slots + 16] label of each adjacency slot's neighbour (byte labels; none if it does not fit)
   bool lab8 = true;
   std::unordered_map<uint32_t, uint32_t> label_id;  // original -> dense
   std::vector<uint64_t> label_freq;                 // dense id -> #vertices
   std::vector<uint64_t> label_deg;                  // dense id -> sum of degrees
+  // dense id -> vertices of degree > TABLE_HEAVY_ROW, and their adjacency in
+  // pieces of TABLE_CHUNK slots
+  std::vector<uint64_t> label_long, label_chunks;
   // Neighbour array as the kernels address it: HBM, or host memory read over
   // PCIe by the filter and table kernels.
   const uint32_t *nbr_dev() const { return nbr_mapped ? nbr_mapped : nbr.as<uint32_t>(); }
 };
 
-// The filter walks the adjacency of vertices of larger degree than this in
-// chunks of this many entries spread over waves.
-constexpr uint32_t FILTER_HUB_DEG = 4096;
+// The filter counts the neighbours of a vertex up to this degree in one lane,
+// up to that in one wave, beyond in one block.
+constexpr uint32_t FILTER_LIGHT_DEG = 64, FILTER_HUB_DEG = 4096;
+// The table build walks candidates of larger degree than this in chunks of
+// this many adjacency slots spread over waves.
+constexpr uint32_t TABLE_HEAVY_ROW = 256, TABLE_CHUNK = 2048;
 
 // Query description consumed by the filter kernel (device copy).
 struct FilterQuery {
@@ -199,8 +209,6 @@ struct QueryDev {
   DevBuf can;                          // u32 candidate lists (sorted)
   DevBuf bitmap;                       // u64[nv * W]
   DevBuf rank;                         // u32[nv * (W + 1)]: exclusive popcount prefix
-  DevBuf fq;                           // FilterQuery
-  DevBuf slot_of;                      // u8[num data labels]: dense label -> query slot
   std::vector<TableDev> tab;           // per directed edge
   bool streamed = false;               // table values live in host_vals
   PinnedBuf host_vals;
@@ -286,6 +294,7 @@ struct gem_ctx {
   uint64_t stream_slot_bytes = 1ull << 20;
   gem_stream_stats sstats{};
   void *pinned = nullptr;                   // small pinned staging area
+  void *pinned_map = nullptr;               // its device address
   size_t pinned_bytes = 0;
   gemd::Prof prof;
   // the last batched run's level budget and scheduler statistics
@@ -361,19 +370,30 @@ template <class T>
 T *pinned(gem_ctx *c, size_t n) {
   size_t need = n * sizeof(T);
   if (need > c->pinned_bytes) {
+    GEM_HIP_CHECK(hipStreamSynchronize(c->stream));  // copies from or to the old one
     if (c->pinned) (void)hipHostFree(c->pinned);
     c->pinned = nullptr;
+    c->pinned_bytes = 0;
     size_t sz = std::max<size_t>(need, 1 << 20);
-    GEM_HIP_CHECK(hipHostMalloc(&c->pinned, sz, hipHostMallocDefault));
+    GEM_HIP_CHECK(hipHostMalloc(&c->pinned, sz, hipHostMallocMapped));
+    GEM_HIP_CHECK(hipHostGetDevicePointer(&c->pinned_map, c->pinned, 0));
     c->pinned_bytes = sz;
   }
   return reinterpret_cast<T *>(c->pinned);
+}
+// Device address of a place in the staging area: a kernel may write its
+// result there, which the host reads after a synchronisation.
+template <class T>
+T *pinned_dev(gem_ctx *c, T *h) {
+  return reinterpret_cast<T *>(static_cast<char *>(c->pinned_map) + (reinterpret_cast<char *>(h) - static_cast<char *>(c->pinned)));
 }
 
 // ---------------------------------------------------------------- phases
 // The data graph a context's filter and table kernels read.
 inline const GraphDev &graph(const gem_ctx *c) { return c->gsrc ? *c->gsrc : c->g; }
 
+// Labels of the adjacency slots of a loaded graph (when they fit).
+void make_slot_labels(gem_ctx *c, GraphDev &G);
 void run_filter(gem_ctx *c, const gem_query_view *qv, uint32_t T);
 void run_tables(gem_ctx *c);
 // the same phases on an explicit per-query state (several queries resident)
@@ -433,8 +453,5 @@ struct ScanSeg {
   uint64_t n;
 };
 void scan_many_u64(gem_ctx *c, const ScanSeg *d_segs, const ScanSeg *h_segs, uint32_t nseg, uint64_t *d_totals);
-// Segmented exclusive scan of u32 counts: nseg segments of length len each,
-// out has len + 1 entries per segment (last = segment total).
-void scan_segments_u32(gem_ctx *c, const uint32_t *d_in, uint32_t *d_out, uint32_t nseg, uint64_t len);
 
 }  // namespace gemd

@@ -9,17 +9,24 @@
 //
 // Layout: one wave owns a tile of 64 consecutive data vertices (lane = vertex)
 // and writes, for every query vertex u, one 64-bit word of u's candidate bitmap
-// (ballot of the lanes that pass) plus that word's popcount.  A per-u scan of
-// the popcounts gives rank[u][tile] = #candidates before the tile, so
+// (ballot of the lanes that pass).  A per-u scan of the words' popcounts gives
+// rank[u][tile] = #candidates before the tile, so
 //   pos_u(v) = rank[u][v/64] + popcount(bitmap[u][v/64] & below(v % 64))
 // equals lower_bound(Can(u), v): the value the reference's cuckoo hash returns
 // (unifiedTrie.cuh:84-125, unifiedTrie.cu:54-101), in one cache line, with no
-// build retries.  Can(u) is then compacted from the bitmap in ascending order.
+// build retries.  The same pass writes Can(u) in ascending order.
 //
-// Neighbour-label counts: a vertex of degree <= 64 is counted by its own lane
-// into a private LDS column (label-major, lane-minor: conflict-free); a
-// higher-degree vertex is counted by the whole wave, 64 neighbours per step,
-// one ballot + popcount per query label (no atomics).
+// Neighbour labels are read as one byte per adjacency slot (GraphDev::nbr_lab,
+// made once per data graph): contiguous bytes in place of a neighbour id and a
+// gather of its label.  A lane counts its neighbours into an LDS column of its
+// own, four 8-bit counts to a word (label slot s: word s / 4, byte s % 4), with
+// LDS adds that return nothing.  Vertices of degree <= 64 take one lane, larger
+// ones a wave, those past FILTER_HUB_DEG a block; which is which depends on
+// the data graph alone, so the two lists are made with it.
+// All kernels of a 16-vertex query on the 2^22-vertex R-MAT graph (65 M slots):
+// 215 us, against 1,060 with a gather per neighbour, lists made per query and
+// one-block scans; k_filter (103 us) reads 100 MB and is bound by the LDS adds
+// of its longest lanes, k_filter_heavy (88) by the block of the largest hub.
 #include <mutex>
 #include <string>
 
@@ -28,242 +35,294 @@
 
 namespace gemd {
 
-constexpr uint32_t FILTER_WAVES = 4;
-constexpr uint32_t LIGHT_DEG = 64;
+constexpr uint32_t FILTER_WAVES = 4, HEAVY_WAVES = 8;
+constexpr uint32_t HIST_WORDS = GEM_MAX_QV / 4 + 1;  // the last word takes labels outside the query
+constexpr uint32_t OUT_SLOT = GEM_MAX_QV;
 
-template <class LabT>
-__global__ void __launch_bounds__(FILTER_WAVES * 64)
-k_filter(const uint64_t *__restrict__ off, const uint32_t *__restrict__ nbr, const LabT *__restrict__ lab, uint32_t n,
-         const FilterQuery *__restrict__ fqp, const uint8_t *__restrict__ slot_of, uint64_t *__restrict__ bitmap,
-         uint32_t *__restrict__ tile_count, uint32_t *__restrict__ heavy_list, uint32_t *__restrict__ heavy_n) {
-  __shared__ FilterQuery fq;
-  __shared__ uint32_t hist[FILTER_WAVES][GEM_MAX_QV][64];
-  {
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(fqp);
-    uint32_t *dst = reinterpret_cast<uint32_t *>(&fq);
-    for (uint32_t i = threadIdx.x; i < sizeof(FilterQuery) / 4; i += blockDim.x) dst[i] = src[i];
-  }
+// The query and, for byte labels, its label -> slot table, as a kernel argument.
+struct FilterArgs {
+  FilterQuery fq;
+  uint8_t slot_of[256];
+};
+
+// Query and slot table in LDS.
+struct FilterLds {
+  FilterQuery fq;
+  uint8_t tab[256];
+};
+__device__ __forceinline__ void load_args(const FilterArgs &a, FilterLds &s) {
+  static_assert(sizeof(FilterArgs) % 4 == 0 && sizeof(FilterLds) == sizeof(FilterArgs), "copied by words");
+  const uint32_t *src = reinterpret_cast<const uint32_t *>(&a);
+  uint32_t *dst = reinterpret_cast<uint32_t *>(&s);
+  for (uint32_t i = threadIdx.x; i < sizeof(FilterArgs) / 4; i += blockDim.x) dst[i] = src[i];
   __syncthreads();
-  const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
-  const uint32_t tile = blockIdx.x * FILTER_WAVES + w;
-  if (tile >= fq.W) return;  // whole wave; no block barrier follows
-  const uint64_t v = (uint64_t)tile * 64 + l;
-  const uint32_t nslots = fq.nslots, T = fq.T;
-  uint32_t (*h)[64] = hist[w];
+}
 
-  uint32_t slot = NO_SLOT;
-  uint64_t o0 = 0, deg = 0;
-  uint32_t cmask = 0;
-  if (v < n) {
-    slot = slot_of[lab[v]];
-    if (slot != NO_SLOT) {
-      o0 = off[v];
-      deg = off[v + 1] - o0;
-      uint32_t g = fq.group[slot];
-      while (g) {
-        uint32_t u = __builtin_ctz(g);
-        g &= g - 1;
-        if ((uint64_t)fq.qdeg[u] <= deg + T) cmask |= 1u << u;
+// The graph as the filter reads it.  nl (NL): labels of the adjacency slots,
+// readable to 16 bytes past the last; slot_of (LabT = u32): label -> slot.
+template <class LabT>
+struct FilterGraph {
+  const uint64_t *off;
+  const uint32_t *nbr;
+  const uint8_t *nl;
+  const LabT *lab;
+  const uint8_t *slot_of;
+  uint32_t n;
+};
+template <class LabT>
+__device__ __forceinline__ uint32_t label_slot(const FilterGraph<LabT> &G, const FilterLds &A, LabT x) {
+  const uint32_t s = sizeof(LabT) == 1 ? A.tab[x] : G.slot_of[x];
+  return s == NO_SLOT ? OUT_SLOT : s;
+}
+
+typedef uint64_t u64u __attribute__((aligned(1)));
+
+// Adds adjacency slots j, j + step, ... < end to the lane's column: 8 slots
+// at a time (NL; j and step are then in units of slots but multiples of 8
+// from the list's start), or one neighbour's label at a time.
+template <class LabT, bool NL>
+__device__ __forceinline__ void count_slots(const FilterGraph<LabT> &G, const FilterLds &A, uint64_t o0, uint64_t j,
+                                            uint64_t end, uint64_t step, uint32_t *col, uint32_t stride) {
+  auto add = [&](uint32_t s) { atomicAdd(&col[(s >> 2) * stride], 1u << ((s & 3) * 8)); };
+  for (; j < end; j += step) {
+    if (NL) {
+      const uint64_t x = *reinterpret_cast<const u64u *>(G.nl + o0 + j);
+      const uint32_t m = end - j < 8 ? (uint32_t)(end - j) : 8;
+#pragma unroll
+      for (uint32_t b = 0; b < 8; ++b) {
+        const uint32_t s = A.tab[(x >> (8 * b)) & 0xFF];
+        add(b < m && s != NO_SLOT ? s : OUT_SLOT);
       }
-    }
-  }
-  for (uint32_t s = 0; s < nslots; ++s) h[s][l] = 0;
-  uint32_t pass = 0;
-  // light vertices: own lane, private LDS column
-  if (cmask && deg <= LIGHT_DEG) {
-    // four neighbours at a time: four independent neighbour -> label -> slot
-    // chains in flight instead of one
-    uint64_t j = 0;
-    for (; j + 4 <= deg; j += 4) {
-      const uint32_t a0 = nbr[o0 + j], a1 = nbr[o0 + j + 1], a2 = nbr[o0 + j + 2], a3 = nbr[o0 + j + 3];
-      const uint32_t b0 = lab[a0], b1 = lab[a1], b2 = lab[a2], b3 = lab[a3];
-      const uint32_t s0 = slot_of[b0], s1 = slot_of[b1], s2 = slot_of[b2], s3 = slot_of[b3];
-      if (s0 != NO_SLOT) h[s0][l] += 1;
-      if (s1 != NO_SLOT) h[s1][l] += 1;
-      if (s2 != NO_SLOT) h[s2][l] += 1;
-      if (s3 != NO_SLOT) h[s3][l] += 1;
-    }
-    for (; j < deg; ++j) {
-      uint32_t s = slot_of[lab[nbr[o0 + j]]];
-      if (s != NO_SLOT) h[s][l] += 1;
-    }
-    uint32_t g = cmask;
-    while (g) {
-      uint32_t u = __builtin_ctz(g);
-      g &= g - 1;
-      uint32_t deficit = 0;
-      for (uint32_t r = 0; r < fq.nreq[u]; ++r) {
-        uint32_t need = fq.req_cnt[u][r], have = h[fq.req_slot[u][r]][l];
-        deficit += need > have ? need - have : 0;
-      }
-      if (deficit <= T) pass |= 1u << u;
-    }
-  }
-  // heavy vertices are deferred to k_filter_heavy (one wave each), so a tile
-  // full of hubs does not hold its wave for thousands of steps
-  const uint64_t heavy = __ballot(cmask != 0 && deg > LIGHT_DEG);
-  if (heavy) {
-    uint32_t base = 0;
-    if (l == 0) base = atomicAdd(heavy_n, (uint32_t)__popcll(heavy));
-    base = readlane_u32(base, 0);
-    if ((heavy >> l) & 1ull) heavy_list[base + rank_below(heavy)] = (uint32_t)v;
-  }
-  const uint32_t W = fq.W;
-  for (uint32_t u = 0; u < fq.nv; ++u) {
-    uint64_t m = __ballot((pass >> u) & 1u);
-    if (l == 0) {
-      bitmap[(uint64_t)u * W + tile] = m;
-      tile_count[(uint64_t)u * W + tile] = (uint32_t)__popcll(m);
+    } else {
+      add(label_slot(G, A, G.lab[G.nbr[o0 + j]]));
     }
   }
 }
 
-// Query vertex u's decision for data vertex v of degree deg whose neighbour
-// label counts (per query label slot) are cnt: lane u sets v's bit.
+// Tiles of 64 vertices, those of degree <= FILTER_LIGHT_DEG counted here.
+template <class LabT, bool NL>
+__global__ void __launch_bounds__(FILTER_WAVES * 64)
+k_filter(const FilterGraph<LabT> G, const FilterArgs args, uint64_t *__restrict__ bitmap) {
+  __shared__ FilterLds A;
+  __shared__ uint32_t hist[FILTER_WAVES][HIST_WORDS][64];
+  load_args(args, A);
+  const FilterQuery &fq = A.fq;
+  const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
+  const uint32_t T = fq.T, W = fq.W, nw = (fq.nslots + 3) / 4;
+  uint32_t *col = &hist[w][0][l];
+  for (uint32_t tile = blockIdx.x * FILTER_WAVES + w; tile < W; tile += gridDim.x * FILTER_WAVES) {
+    const uint64_t v = (uint64_t)tile * 64 + l;
+    uint64_t o0 = 0, deg = 0;
+    uint32_t cmask = 0, pass = 0;
+    if (v < G.n) {
+      const uint32_t slot = label_slot(G, A, G.lab[v]);
+      if (slot != OUT_SLOT) {
+        o0 = G.off[v];
+        deg = G.off[v + 1] - o0;
+        uint32_t g = deg <= FILTER_LIGHT_DEG ? fq.group[slot] : 0;
+        while (g) {
+          const uint32_t u = __builtin_ctz(g);
+          g &= g - 1;
+          if ((uint64_t)fq.qdeg[u] <= deg + T) cmask |= 1u << u;
+        }
+      }
+    }
+    if (cmask) {
+      for (uint32_t s = 0; s < nw; ++s) col[s * 64] = 0;
+      count_slots<LabT, NL>(G, A, o0, 0, deg, NL ? 8 : 1, col, 64);
+      uint32_t g = cmask;
+      while (g) {
+        const uint32_t u = __builtin_ctz(g);
+        g &= g - 1;
+        uint32_t deficit = 0;
+        for (uint32_t r = 0; r < fq.nreq[u]; ++r) {
+          const uint32_t need = fq.req_cnt[u][r], s = fq.req_slot[u][r];
+          const uint32_t have = (col[(s >> 2) * 64] >> ((s & 3) * 8)) & 0xFF;
+          deficit += need > have ? need - have : 0;
+        }
+        if (deficit <= T) pass |= 1u << u;
+      }
+    }
+    uint64_t mine = 0;  // lane u: u's word
+    for (uint32_t u = 0; u < fq.nv; ++u) {
+      const uint64_t m = __ballot((pass >> u) & 1u);
+      if (l == u) mine = m;
+    }
+    if (l < fq.nv) bitmap[(uint64_t)l * W + tile] = mine;
+  }
+}
+
+// Label counts of a wave's columns (each lane's at most 255): cnt[s] += the
+// sum over lanes; the columns are cleared.
+__device__ __forceinline__ void sum_columns(uint32_t *col, uint32_t nslots, uint32_t l, uint32_t *cnt) {
+  for (uint32_t w = 0; w < (nslots + 3) / 4; ++w) {
+    uint32_t e = col[w * 64] & 0x00FF00FFu, o = (col[w * 64] >> 8) & 0x00FF00FFu;
+    col[w * 64] = 0;
+#pragma unroll
+    for (uint32_t d = 32; d >= 1; d >>= 1) {
+      e += __shfl_xor(e, d, 64);
+      o += __shfl_xor(o, d, 64);
+    }
+    // slots 4 w ...: e low, o low, e high, o high
+    const uint32_t x = l & 1 ? o : e, y = l & 2 ? x >> 16 : x & 0xFFFFu;
+    if (l < 4 && 4 * w + l < nslots) atomicAdd(&cnt[4 * w + l], y);
+  }
+}
+
+// Query vertex l's decision for data vertex v of degree deg whose neighbour
+// label counts are cnt: lane l sets v's bit.
 __device__ __forceinline__ void filter_decide(const FilterQuery &fq, uint32_t l, uint32_t v, uint64_t deg, uint32_t g,
-                                              const uint32_t *cnt, unsigned long long *bitmap,
-                                              uint32_t *tile_count) {
+                                              const uint32_t *cnt, unsigned long long *bitmap) {
   if (l < fq.nv && ((g >> l) & 1u) && (uint64_t)fq.qdeg[l] <= deg + fq.T) {
     uint32_t deficit = 0;
     for (uint32_t r = 0; r < fq.nreq[l]; ++r) {
       const uint32_t need = fq.req_cnt[l][r], have = cnt[fq.req_slot[l][r]];
       deficit += need > have ? need - have : 0;
     }
-    if (deficit <= fq.T) {
-      atomicOr(&bitmap[(uint64_t)l * fq.W + (v >> 6)], 1ull << (v & 63));
-      atomicAdd(&tile_count[(uint64_t)l * fq.W + (v >> 6)], 1u);
-    }
+    if (deficit <= fq.T) atomicOr(&bitmap[(uint64_t)l * fq.W + (v >> 6)], 1ull << (v & 63));
   }
 }
 
-// Vertices of degree in (LIGHT_DEG, FILTER_HUB_DEG]: one wave per vertex
-// (persistent grid over the list k_filter built); larger ones are passed on to
-// the hub list for k_filter_hub.  Neighbour labels are counted 64 at a time,
-// one ballot + popcount per query label (lane s keeps label s's count); lane u
-// then decides query vertex u and sets its bit with an atomic OR.
-template <class LabT>
-__global__ void __launch_bounds__(FILTER_WAVES * 64)
-k_filter_heavy(const uint64_t *__restrict__ off, const uint32_t *__restrict__ nbr, const LabT *__restrict__ lab,
-               const FilterQuery *__restrict__ fqp, const uint8_t *__restrict__ slot_of,
-               unsigned long long *__restrict__ bitmap, uint32_t *__restrict__ tile_count,
-               const uint32_t *__restrict__ heavy_list, const uint32_t *__restrict__ heavy_n,
-               uint32_t *__restrict__ hub_list, uint32_t *__restrict__ hub_n, uint32_t hub_cap) {
-  __shared__ FilterQuery fq;
-  __shared__ uint32_t cnt[FILTER_WAVES][GEM_MAX_QV];
-  {
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(fqp);
-    uint32_t *dst = reinterpret_cast<uint32_t *>(&fq);
-    for (uint32_t i = threadIdx.x; i < sizeof(FilterQuery) / 4; i += blockDim.x) dst[i] = src[i];
-  }
+// The graph's vertices past FILTER_LIGHT_DEG, after k_filter wrote the words:
+// blocks [0, n_hub) take one hub each (all waves), the waves of the others the
+// list of the rest.
+template <class LabT, bool NL>
+__global__ void __launch_bounds__(HEAVY_WAVES * 64)
+k_filter_heavy(const FilterGraph<LabT> G, const FilterArgs args, const uint32_t *__restrict__ heavy, uint32_t n_heavy,
+               const uint32_t *__restrict__ hubs, uint32_t n_hub, unsigned long long *__restrict__ bitmap) {
+  __shared__ FilterLds A;
+  __shared__ uint32_t hist[HEAVY_WAVES][HIST_WORDS][64];
+  __shared__ uint32_t cnt[HEAVY_WAVES][GEM_MAX_QV];
+  load_args(args, A);
+  const FilterQuery &fq = A.fq;
+  const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64, per = NL ? 8 : 1;
+  uint32_t *col = &hist[w][0][l];
+  for (uint32_t s = 0; s < (fq.nslots + 3) / 4; ++s) col[s * 64] = 0;
+  if (l < GEM_MAX_QV) cnt[w][l] = 0;
   __syncthreads();
-  const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
-  const uint32_t nh = *heavy_n;
-  const uint32_t nslots = fq.nslots;
-  for (uint32_t i = blockIdx.x * FILTER_WAVES + w; i < nh; i += gridDim.x * FILTER_WAVES) {
-    const uint32_t v = heavy_list[i];
-    const uint64_t o0 = off[v], deg = off[v + 1] - o0;
-    if (deg > FILTER_HUB_DEG) {
-      if (l == 0) {
-        const uint32_t h = atomicAdd(hub_n, 1u);
-        if (h < hub_cap) hub_list[h] = v;  // hub_cap = all such vertices of the graph
-      }
-      continue;
+  if (blockIdx.x < n_hub) {
+    const uint32_t v = hubs[blockIdx.x];
+    const uint32_t slot = label_slot(G, A, G.lab[v]);
+    if (slot == OUT_SLOT) return;
+    const uint64_t o0 = G.off[v], deg = G.off[v + 1] - o0;
+    // a lane's 8-bit counts hold 248 slots
+    const uint64_t round = (uint64_t)HEAVY_WAVES * 64 * 248;
+    for (uint64_t j0 = 0; j0 < deg; j0 += round) {
+      const uint64_t end = deg - j0 < round ? deg : j0 + round;
+      count_slots<LabT, NL>(G, A, o0, j0 + (uint64_t)threadIdx.x * per, end, (uint64_t)HEAVY_WAVES * 64 * per, col, 64);
+      sum_columns(col, fq.nslots, l, cnt[0]);
     }
-    const uint32_t g = fq.group[slot_of[lab[v]]];
-    uint32_t acc = 0;
-    for (uint64_t j = 0; j < deg; j += 128) {
-      // two 64-entry groups: both neighbour -> label -> slot chains in flight
-      const bool i0 = j + l < deg, i1 = j + 64 + l < deg;
-      const uint32_t a0 = i0 ? nbr[o0 + j + l] : 0, a1 = i1 ? nbr[o0 + j + 64 + l] : 0;
-      const uint32_t b0 = i0 ? (uint32_t)lab[a0] : 0, b1 = i1 ? (uint32_t)lab[a1] : 0;
-      const uint32_t s0 = i0 ? slot_of[b0] : NO_SLOT, s1 = i1 ? slot_of[b1] : NO_SLOT;
-      for (uint32_t q = 0; q < nslots; ++q) {
-        const uint32_t c = (uint32_t)__popcll(__ballot(s0 == q)) + (uint32_t)__popcll(__ballot(s1 == q));
-        if (l == q) acc += c;
-      }
-    }
-    if (l < nslots) cnt[w][l] = acc;
+    __syncthreads();
+    if (w == 0) filter_decide(fq, l, v, deg, fq.group[slot], cnt[0], bitmap);
+    return;
+  }
+  for (uint32_t i = (blockIdx.x - n_hub) * HEAVY_WAVES + w; i < n_heavy; i += (gridDim.x - n_hub) * HEAVY_WAVES) {
+    const uint32_t v = heavy[i];
+    const uint32_t slot = label_slot(G, A, G.lab[v]);
+    if (slot == OUT_SLOT) continue;
+    const uint64_t o0 = G.off[v], deg = G.off[v + 1] - o0;
+    count_slots<LabT, NL>(G, A, o0, (uint64_t)l * per, deg, 64 * per, col, 64);
+    sum_columns(col, fq.nslots, l, cnt[w]);
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    filter_decide(fq, l, v, deg, g, cnt[w], bitmap, tile_count);
+    filter_decide(fq, l, v, deg, fq.group[slot], cnt[w], bitmap);
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (l < GEM_MAX_QV) cnt[w][l] = 0;
   }
 }
 
-// Hubs (degree > FILTER_HUB_DEG): task t = (hub t / maxc, chunk t % maxc) of
-// FILTER_HUB_DEG adjacency entries; label counts are added into
-// hub_cnt[hub][slot] (zeroed by the host).  maxc = chunks of the largest degree.
-template <class LabT>
-__global__ void __launch_bounds__(FILTER_WAVES * 64)
-k_filter_hub(const uint64_t *__restrict__ off, const uint32_t *__restrict__ nbr, const LabT *__restrict__ lab,
-             const FilterQuery *__restrict__ fqp, const uint8_t *__restrict__ slot_of,
-             const uint32_t *__restrict__ hub_list, const uint32_t *__restrict__ hub_n, uint32_t hub_cap,
-             uint32_t maxc, uint32_t *__restrict__ hub_cnt) {
-  const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
-  const uint32_t nslots = fqp->nslots;
-  const uint32_t nh = *hub_n < hub_cap ? *hub_n : hub_cap;
-  const uint64_t ntask = (uint64_t)nh * maxc;
-  for (uint64_t t = (uint64_t)blockIdx.x * FILTER_WAVES + w; t < ntask; t += (uint64_t)gridDim.x * FILTER_WAVES) {
-    const uint32_t h = (uint32_t)(t / maxc), ch = (uint32_t)(t % maxc);
-    const uint32_t v = hub_list[h];
-    const uint64_t o0 = off[v], deg = off[v + 1] - o0;
-    const uint64_t j0 = (uint64_t)ch * FILTER_HUB_DEG;
-    if (j0 >= deg) continue;
-    const uint64_t j1 = j0 + FILTER_HUB_DEG < deg ? j0 + FILTER_HUB_DEG : deg;
-    uint32_t acc = 0;
-    for (uint64_t j = j0; j < j1; j += 128) {
-      const bool i0 = j + l < j1, i1 = j + 64 + l < j1;
-      const uint32_t a0 = i0 ? nbr[o0 + j + l] : 0, a1 = i1 ? nbr[o0 + j + 64 + l] : 0;
-      const uint32_t b0 = i0 ? (uint32_t)lab[a0] : 0, b1 = i1 ? (uint32_t)lab[a1] : 0;
-      const uint32_t s0 = i0 ? slot_of[b0] : NO_SLOT, s1 = i1 ? slot_of[b1] : NO_SLOT;
-      for (uint32_t q = 0; q < nslots; ++q) {
-        const uint32_t c = (uint32_t)__popcll(__ballot(s0 == q)) + (uint32_t)__popcll(__ballot(s1 == q));
-        if (l == q) acc += c;
-      }
-    }
-    if (l < nslots && acc) atomicAdd(&hub_cnt[(uint64_t)h * GEM_MAX_QV + l], acc);
+// Ranks and candidate lists in chunks of RANK_CHUNK bitmap words: chunk sums
+// (left out when one chunk holds all), then each block adds up the sums before
+// its own and scans it.  Wave w of a block holds words [w, w + 1) * 1024 of the
+// chunk, lane = word modulo 64.  With one block per query vertex scanning all
+// words, and a launch of its own for the lists, the ranks of the 2^22-vertex
+// graph took 108 us and its lists 63.
+constexpr uint32_t RANK_STEPS = 16, RANK_CHUNK = 4 * 64 * RANK_STEPS;
+
+__global__ void __launch_bounds__(256) k_rank_sums(const uint64_t *__restrict__ bitmap, uint32_t W,
+                                                  uint32_t *__restrict__ sums) {
+  __shared__ uint32_t sm[4];
+  const uint32_t u = blockIdx.y, w0 = blockIdx.x * RANK_CHUNK;
+  uint32_t x = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < RANK_STEPS; ++i) {
+    const uint32_t word = w0 + i * 256 + threadIdx.x;
+    if (word < W) x += (uint32_t)__popcll(bitmap[(uint64_t)u * W + word]);
   }
+  x = (uint32_t)wave_sum_u64(x);
+  if (threadIdx.x % 64 == 0) sm[threadIdx.x / 64] = x;
+  __syncthreads();
+  if (threadIdx.x == 0) sums[u * gridDim.x + blockIdx.x] = sm[0] + sm[1] + sm[2] + sm[3];
 }
 
-// One wave per hub: the filter decision from the summed label counts.
-template <class LabT>
-__global__ void __launch_bounds__(FILTER_WAVES * 64)
-k_filter_hub_decide(const uint64_t *__restrict__ off, const LabT *__restrict__ lab,
-                    const FilterQuery *__restrict__ fqp, const uint8_t *__restrict__ slot_of,
-                    const uint32_t *__restrict__ hub_list, const uint32_t *__restrict__ hub_n, uint32_t hub_cap,
-                    const uint32_t *__restrict__ hub_cnt, unsigned long long *__restrict__ bitmap,
-                    uint32_t *__restrict__ tile_count) {
-  __shared__ FilterQuery fq;
-  {
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(fqp);
-    uint32_t *dst = reinterpret_cast<uint32_t *>(&fq);
-    for (uint32_t i = threadIdx.x; i < sizeof(FilterQuery) / 4; i += blockDim.x) dst[i] = src[i];
+struct CanOffsets {
+  uint64_t at[GEM_MAX_QV + 1];
+};
+// can == null: counts and ranks only.  ncan[u] = |Can(u)| (device or mapped
+// host memory).
+__global__ void __launch_bounds__(256) k_rank_lists(const uint64_t *__restrict__ bitmap, uint32_t W,
+                                                   const uint32_t *__restrict__ sums, uint32_t *__restrict__ rank,
+                                                   const CanOffsets can_off, uint32_t *__restrict__ can,
+                                                   uint32_t *__restrict__ ncan) {
+  __shared__ uint32_t sm[4], before[4];
+  const uint32_t u = blockIdx.y, w = threadIdx.x / 64, l = threadIdx.x % 64;
+  const uint32_t w0 = blockIdx.x * RANK_CHUNK + w * 64 * RANK_STEPS;
+  uint64_t m[RANK_STEPS];
+  uint32_t x = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < RANK_STEPS; ++i) {
+    const uint32_t word = w0 + i * 64 + l;
+    m[i] = word < W ? bitmap[(uint64_t)u * W + word] : 0;
+    x += (uint32_t)__popcll(m[i]);
+  }
+  uint32_t y = 0;  // candidates of the chunks before
+  for (uint32_t c = threadIdx.x; c < blockIdx.x; c += 256) y += sums[u * gridDim.x + c];
+  x = (uint32_t)wave_sum_u64(x);
+  y = (uint32_t)wave_sum_u64(y);
+  if (l == 0) {
+    sm[w] = x;
+    before[w] = y;
   }
   __syncthreads();
-  const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
-  const uint32_t nh = *hub_n < hub_cap ? *hub_n : hub_cap;
-  for (uint32_t h = blockIdx.x * FILTER_WAVES + w; h < nh; h += gridDim.x * FILTER_WAVES) {
-    const uint32_t v = hub_list[h];
-    const uint64_t deg = off[v + 1] - off[v];
-    filter_decide(fq, l, v, deg, fq.group[slot_of[lab[v]]], hub_cnt + (uint64_t)h * GEM_MAX_QV, bitmap, tile_count);
+  uint32_t run = before[0] + before[1] + before[2] + before[3];
+  for (uint32_t i = 0; i < w; ++i) run += sm[i];
+  if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 192) {  // the last wave's first lane
+    ncan[u] = run + sm[3];
+    rank[(uint64_t)u * (W + 1) + W] = run + sm[3];
+  }
+  uint32_t *out = can ? can + can_off.at[u] : nullptr;
+#pragma unroll
+  for (uint32_t i = 0; i < RANK_STEPS; ++i) {
+    if (w0 + i * 64 >= W) break;
+    const uint32_t word = w0 + i * 64 + l, c = (uint32_t)__popcll(m[i]);
+    const uint32_t incl = wave_incl_scan_u32(c);
+    uint32_t r = run + incl - c;
+    if (word < W) rank[(uint64_t)u * (W + 1) + word] = r;
+    if (out)
+      for (uint64_t b = m[i]; b; b &= b - 1) out[r++] = word * 64 + (uint32_t)__builtin_ctzll(b);
+    run += readlane_u32(incl, 63);
   }
 }
 
-// Compaction: Can(u) ascending from the bitmap and ranks.
-__global__ void __launch_bounds__(256) k_compact(const uint64_t *__restrict__ bitmap, const uint32_t *__restrict__ rank,
-                                               uint32_t nv, uint32_t W, const uint64_t *__restrict__ can_off,
-                                               uint32_t *__restrict__ can) {
-  const uint32_t tile = blockIdx.x * 4 + threadIdx.x / 64, l = threadIdx.x % 64;
-  if (tile >= W) return;
-  for (uint32_t u = 0; u < nv; ++u) {
-    const uint64_t m = bitmap[(uint64_t)u * W + tile];
-    if (!m) continue;
-    if (m >> l & 1ull) {
-      const uint32_t r = rank[(uint64_t)u * (W + 1) + tile] + rank_below(m);
-      can[can_off[u] + r] = tile * 64 + l;
-    }
+// Labels of the adjacency slots (255, no label, for a neighbour out of range).
+__global__ void k_slot_labels(const uint32_t *__restrict__ nbr, uint64_t slots, const uint8_t *__restrict__ lab,
+                              uint32_t n, uint8_t *__restrict__ nl) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < slots; i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t v = nbr[i];
+    nl[i] = v < n ? lab[v] : 255;
   }
+}
+
+void make_slot_labels(gem_ctx *c, GraphDev &G) {
+  // a quarter of the free memory at most: a larger graph keeps the gathers
+  size_t free_b = 0, total_b = 0;
+  GEM_HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+  if (!G.lab8 || !G.slots || G.slots > (free_b + pool_reusable_bytes()) / 4) return;
+  G.nbr_lab.alloc(G.slots + 16, c->stream);
+  k_slot_labels<<<(uint32_t)std::min<uint64_t>((G.slots + 255) / 256, 16384), 256, 0, c->stream>>>(
+      G.nbr_dev(), G.slots, G.lab.as<uint8_t>(), G.n, G.nbr_lab.as<uint8_t>());
+  GEM_LAUNCH_CHECK("k_slot_labels");
 }
 
 __global__ void k_position_lookup(const uint64_t *__restrict__ bitmap, const uint32_t *__restrict__ rank, uint32_t W,
@@ -284,19 +343,12 @@ __global__ void k_position_lookup(const uint64_t *__restrict__ bitmap, const uin
 // Device buffers of one filter run (library-owned, or carved from the
 // no-allocation scratch array).
 struct FilterBufs {
-  FilterQuery *fq = nullptr;
-  uint8_t *slot_of = nullptr;
-  uint64_t *bitmap = nullptr;      // u64[nv * W]
-  uint32_t *tile_count = nullptr;  // u32[nv * W]
-  uint32_t *rank = nullptr;        // u32[nv * (W + 1)]
-  uint32_t *can = nullptr;         // candidate lists at can_off[u]
-  const uint64_t *can_off = nullptr;
-  uint32_t *heavy_list = nullptr;  // u32[n]
-  uint32_t *heavy_n = nullptr;     // u32
-  uint32_t *hub_list = nullptr;    // u32[hub_cap]
-  uint32_t *hub_n = nullptr;       // u32
-  uint32_t *hub_cnt = nullptr;     // u32[hub_cap * GEM_MAX_QV]
-  uint32_t hub_cap = 1;
+  const uint8_t *slot_of = nullptr;  // label -> slot, when labels are not bytes
+  uint64_t *bitmap = nullptr;        // u64[nv * W]
+  uint32_t *sums = nullptr;          // u32[nv * chunks]
+  uint32_t *rank = nullptr;          // u32[nv * (W + 1)]
+  uint32_t *can = nullptr;           // candidate lists at can_off[u]
+  uint32_t *ncan = nullptr;          // u32[nv]
 };
 
 // Host side of a filter run: the query's label slots and per-vertex label
@@ -304,7 +356,7 @@ struct FilterBufs {
 // bound per list = frequency of the vertex's label) and the adjacency slots of
 // label-matching vertices (for the algorithmic bytes).
 struct FilterPrep {
-  FilterQuery fq{};
+  FilterArgs args{};
   std::vector<uint8_t> slot_of;
   std::vector<uint64_t> can_off;
   double adj = 0;
@@ -313,8 +365,8 @@ struct FilterPrep {
 static void filter_prepare(const GraphDev &G, const gemh::QueryInfo &Q, uint32_t T, uint32_t W, FilterPrep *P) {
   const uint32_t nv = Q.nv;
   // query label slots in first-seen order (in-core/lib/io/src/io.cu:135-161)
-  FilterQuery &fq = P->fq;
-  fq = FilterQuery{};
+  P->args = FilterArgs{};
+  FilterQuery &fq = P->args.fq;
   fq.nv = nv;
   fq.T = T;
   fq.W = W;
@@ -346,6 +398,10 @@ static void filter_prepare(const GraphDev &G, const gemh::QueryInfo &Q, uint32_t
     auto it = G.label_id.find(slot_label[s]);
     if (it != G.label_id.end()) P->slot_of[it->second] = (uint8_t)s;
   }
+  if (G.lab8) {
+    std::fill(std::begin(P->args.slot_of), std::end(P->args.slot_of), (uint8_t)NO_SLOT);
+    std::copy(P->slot_of.begin(), P->slot_of.end(), P->args.slot_of);
+  }
   // candidate storage: upper bound = frequency of u's label
   P->can_off.assign(nv + 1, 0);
   for (uint32_t u = 0; u < nv; ++u) {
@@ -360,86 +416,51 @@ static void filter_prepare(const GraphDev &G, const gemh::QueryInfo &Q, uint32_t
   }
 }
 
-// |Can(u)| = rank[u][W] for every u.
-__global__ void k_gather_counts(const uint32_t *__restrict__ rank, uint32_t nv, uint32_t W, uint32_t *__restrict__ out) {
-  for (uint32_t u = threadIdx.x; u < nv; u += blockDim.x) out[u] = rank[(uint64_t)u * (W + 1) + W];
-}
-
-__global__ void k_zero_u32(uint32_t *p, uint64_t n) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-    p[i] = 0;
-}
-
-// The filter's kernels on the context stream: per-tile bitmaps and counts
-// (light vertices in k_filter, heavy ones in k_filter_heavy, hubs in chunks),
-// the rank scan, and the compaction of Can(u).  No allocation; the counters
-// are cleared by a kernel (no memset node when a caller captures the stream).
-static void filter_launch(gem_ctx *c, uint32_t nv, uint32_t W, const FilterBufs &B) {
+// The filter's kernels on the context stream.  No allocation, no copy (a
+// caller may capture the stream).
+template <class LabT, bool NL>
+static void filter_launch_as(gem_ctx *c, uint32_t W, const FilterPrep &P, const FilterBufs &B) {
   const GraphDev &G = graph(c);
   hipStream_t s = c->stream;
-  k_zero_u32<<<1, 64, 0, s>>>(B.heavy_n, 1);
-  k_zero_u32<<<1, 64, 0, s>>>(B.hub_n, 1);
-  if (G.n_hub)
-    k_zero_u32<<<(uint32_t)std::min<uint64_t>(((uint64_t)B.hub_cap * GEM_MAX_QV + 255) / 256, 1024), 256, 0, s>>>(
-        B.hub_cnt, (uint64_t)B.hub_cap * GEM_MAX_QV);
-  GEM_LAUNCH_CHECK("k_zero_u32");
-  const uint32_t blocks = (W + FILTER_WAVES - 1) / FILTER_WAVES;
+  const FilterGraph<LabT> g{G.off.as<uint64_t>(), G.nbr_dev(), G.nbr_lab.as<uint8_t>(), G.lab.as<LabT>(), B.slot_of, G.n};
   {
     ProfLaunch pl(c, K_FILTER);
-    if (G.lab8)
-      k_filter<uint8_t><<<blocks, FILTER_WAVES * 64, 0, s>>>(G.off.as<uint64_t>(), G.nbr_dev(),
-                                                             G.lab.as<uint8_t>(), G.n, B.fq, B.slot_of, B.bitmap,
-                                                             B.tile_count, B.heavy_list, B.heavy_n);
-    else
-      k_filter<uint32_t><<<blocks, FILTER_WAVES * 64, 0, s>>>(G.off.as<uint64_t>(), G.nbr_dev(),
-                                                              G.lab.as<uint32_t>(), G.n, B.fq, B.slot_of, B.bitmap,
-                                                              B.tile_count, B.heavy_list, B.heavy_n);
+    k_filter<LabT, NL><<<std::min<uint32_t>((W + FILTER_WAVES - 1) / FILTER_WAVES, 4096), FILTER_WAVES * 64, 0, s>>>(
+        g, P.args, B.bitmap);
     GEM_LAUNCH_CHECK("k_filter");
   }
-  const uint32_t maxc = (uint32_t)((G.max_deg + FILTER_HUB_DEG - 1) / FILTER_HUB_DEG);
-  auto *bm = reinterpret_cast<unsigned long long *>(B.bitmap);
-  {
+  if (G.n_heavy + G.n_hub) {
     ProfLaunch pl(c, K_FILTER_HEAVY);
-    const uint32_t hb = 1024;  // persistent: 4096 waves walk the heavy list
-    if (G.lab8)
-      k_filter_heavy<uint8_t><<<hb, FILTER_WAVES * 64, 0, s>>>(G.off.as<uint64_t>(), G.nbr_dev(),
-                                                               G.lab.as<uint8_t>(), B.fq, B.slot_of, bm, B.tile_count,
-                                                               B.heavy_list, B.heavy_n, B.hub_list, B.hub_n,
-                                                               B.hub_cap);
-    else
-      k_filter_heavy<uint32_t><<<hb, FILTER_WAVES * 64, 0, s>>>(G.off.as<uint64_t>(), G.nbr_dev(),
-                                                                G.lab.as<uint32_t>(), B.fq, B.slot_of, bm,
-                                                                B.tile_count, B.heavy_list, B.heavy_n, B.hub_list,
-                                                                B.hub_n, B.hub_cap);
+    const uint32_t blocks = G.n_hub + std::min<uint32_t>((G.n_heavy + HEAVY_WAVES - 1) / HEAVY_WAVES, 2048);
+    k_filter_heavy<LabT, NL><<<blocks, HEAVY_WAVES * 64, 0, s>>>(g, P.args, G.heavy.as<uint32_t>(), G.n_heavy,
+                                                                 G.heavy.as<uint32_t>() + G.n_heavy, G.n_hub,
+                                                                 reinterpret_cast<unsigned long long *>(B.bitmap));
     GEM_LAUNCH_CHECK("k_filter_heavy");
-    if (G.n_hub) {
-      const uint32_t tb = (uint32_t)std::min<uint64_t>(((uint64_t)G.n_hub * maxc + FILTER_WAVES - 1) / FILTER_WAVES,
-                                                       2048);
-      const uint32_t db = (G.n_hub + FILTER_WAVES - 1) / FILTER_WAVES;
-      if (G.lab8) {
-        k_filter_hub<uint8_t><<<tb, FILTER_WAVES * 64, 0, s>>>(G.off.as<uint64_t>(), G.nbr_dev(),
-                                                               G.lab.as<uint8_t>(), B.fq, B.slot_of, B.hub_list,
-                                                               B.hub_n, B.hub_cap, maxc, B.hub_cnt);
-        k_filter_hub_decide<uint8_t><<<db, FILTER_WAVES * 64, 0, s>>>(G.off.as<uint64_t>(), G.lab.as<uint8_t>(), B.fq,
-                                                                      B.slot_of, B.hub_list, B.hub_n, B.hub_cap,
-                                                                      B.hub_cnt, bm, B.tile_count);
-      } else {
-        k_filter_hub<uint32_t><<<tb, FILTER_WAVES * 64, 0, s>>>(G.off.as<uint64_t>(), G.nbr_dev(),
-                                                                G.lab.as<uint32_t>(), B.fq, B.slot_of, B.hub_list,
-                                                                B.hub_n, B.hub_cap, maxc, B.hub_cnt);
-        k_filter_hub_decide<uint32_t><<<db, FILTER_WAVES * 64, 0, s>>>(G.off.as<uint64_t>(), G.lab.as<uint32_t>(),
-                                                                       B.fq, B.slot_of, B.hub_list, B.hub_n,
-                                                                       B.hub_cap, B.hub_cnt, bm, B.tile_count);
-      }
-      GEM_LAUNCH_CHECK("k_filter_hub");
-    }
   }
-  scan_segments_u32(c, B.tile_count, B.rank, nv, W);
-  if (B.can) {
-    ProfLaunch pl(c, K_COMPACT);
-    k_compact<<<(W + 3) / 4, 256, 0, s>>>(B.bitmap, B.rank, nv, W, B.can_off, B.can);
-    GEM_LAUNCH_CHECK("k_compact");
+}
+
+static uint32_t rank_chunks(uint32_t W) { return (W + RANK_CHUNK - 1) / RANK_CHUNK; }
+
+static void filter_launch(gem_ctx *c, uint32_t nv, uint32_t W, const FilterPrep &P, const uint64_t *can_off,
+                          const FilterBufs &B) {
+  const GraphDev &G = graph(c);
+  hipStream_t s = c->stream;
+  if (!G.lab8)
+    filter_launch_as<uint32_t, false>(c, W, P, B);
+  else if (G.nbr_lab.p)
+    filter_launch_as<uint8_t, true>(c, W, P, B);
+  else
+    filter_launch_as<uint8_t, false>(c, W, P, B);
+  const dim3 grid(rank_chunks(W), nv);
+  CanOffsets co{};
+  std::copy(can_off, can_off + nv + 1, co.at);
+  ProfLaunch pl(c, K_COMPACT);
+  if (grid.x > 1) {
+    k_rank_sums<<<grid, 256, 0, s>>>(B.bitmap, W, B.sums);
+    GEM_LAUNCH_CHECK("k_rank_sums");
   }
+  k_rank_lists<<<grid, 256, 0, s>>>(B.bitmap, W, B.sums, B.rank, co, B.can, B.ncan);
+  GEM_LAUNCH_CHECK("k_rank_lists");
 }
 
 void run_filter(gem_ctx *c, const gem_query_view *qv, uint32_t T) { run_filter(c, c->q, qv, T); }
@@ -461,51 +482,28 @@ void run_filter(gem_ctx *c, QueryDev &Qd, const gem_query_view *qv, uint32_t T) 
 
   hipStream_t s = c->stream;
   GEM_HIP_CHECK(hipEventRecord(c->ev[0], s));
-  Qd.fq.alloc(sizeof(FilterQuery), s);
-  Qd.slot_of.alloc(P.slot_of.size(), s);
-  GEM_HIP_CHECK(hipMemcpyAsync(Qd.fq.p, &P.fq, sizeof(FilterQuery), hipMemcpyHostToDevice, s));
-  GEM_HIP_CHECK(hipMemcpyAsync(Qd.slot_of.p, P.slot_of.data(), P.slot_of.size(), hipMemcpyHostToDevice, s));
+  FilterBufs B;
+  DevBuf slot_of, sums;
+  if (!G.lab8) {
+    slot_of.alloc(P.slot_of.size(), s);
+    GEM_HIP_CHECK(hipMemcpyAsync(slot_of.p, P.slot_of.data(), P.slot_of.size(), hipMemcpyHostToDevice, s));
+  }
   Qd.bitmap.alloc((uint64_t)nv * W * 8, s);
-  DevBuf tile_count;
-  tile_count.alloc((uint64_t)nv * W * 4, s);
   Qd.rank.alloc((uint64_t)nv * (W + 1) * 4, s);
   Qd.can.alloc(std::max<uint64_t>(Qd.can_off[nv], 1) * 4, s);
-  DevBuf can_off;
-  can_off.alloc((nv + 1) * 8, s);
-  GEM_HIP_CHECK(hipMemcpyAsync(can_off.p, Qd.can_off.data(), (nv + 1) * 8, hipMemcpyHostToDevice, s));
-  DevBuf heavy_list, heavy_n, hub_list, hub_n, hub_cnt;
-  heavy_list.alloc(std::max<uint64_t>(G.n, 1) * 4, s);
-  heavy_n.alloc(4, s);
-  const uint32_t hub_cap = std::max<uint32_t>(G.n_hub, 1);
-  hub_list.alloc((uint64_t)hub_cap * 4, s);
-  hub_n.alloc(4, s);
-  hub_cnt.alloc((uint64_t)hub_cap * GEM_MAX_QV * 4, s);
-  FilterBufs B;
-  B.fq = Qd.fq.as<FilterQuery>();
-  B.slot_of = Qd.slot_of.as<uint8_t>();
+  sums.alloc((uint64_t)nv * rank_chunks(W) * 4, s);
+  B.slot_of = slot_of.as<uint8_t>();
   B.bitmap = Qd.bitmap.as<uint64_t>();
-  B.tile_count = tile_count.as<uint32_t>();
+  B.sums = sums.as<uint32_t>();
   B.rank = Qd.rank.as<uint32_t>();
   B.can = Qd.can.as<uint32_t>();
-  B.can_off = can_off.as<uint64_t>();
-  B.heavy_list = heavy_list.as<uint32_t>();
-  B.heavy_n = heavy_n.as<uint32_t>();
-  B.hub_list = hub_list.as<uint32_t>();
-  B.hub_n = hub_n.as<uint32_t>();
-  B.hub_cnt = hub_cnt.as<uint32_t>();
-  B.hub_cap = hub_cap;
-  filter_launch(c, nv, W, B);
+  uint32_t *h = pinned<uint32_t>(c, nv);  // written by the last kernel
+  B.ncan = pinned_dev(c, h);
+  filter_launch(c, nv, W, P, Qd.can_off.data(), B);
   // algorithmic bytes: 16 B per vertex (label, degree, offset pair), 8 B per
-  // adjacency slot of a label-matching vertex (neighbour id + its label), the
-  // candidate bitmaps and per-tile counts written
-  prof_bytes(c, K_FILTER, 16.0 * G.n + 8.0 * P.adj + nv * (double)W * 8 + nv * (double)W * 4);
-  // |Can(u)| = rank[u][W], gathered by one kernel and copied back at once
-  DevBuf dn;
-  dn.alloc(4ull * nv, s);
-  k_gather_counts<<<1, 64, 0, s>>>(Qd.rank.as<uint32_t>(), nv, W, dn.as<uint32_t>());
-  GEM_LAUNCH_CHECK("k_gather_counts");
-  uint32_t *h = pinned<uint32_t>(c, nv);
-  GEM_HIP_CHECK(hipMemcpyAsync(h, dn.p, 4ull * nv, hipMemcpyDeviceToHost, s));
+  // adjacency slot of a label-matching vertex (neighbour id + its label; 1 B
+  // with slot labels), the candidate bitmaps written
+  prof_bytes(c, K_FILTER, 16.0 * G.n + (G.nbr_lab.p ? 1.0 : 8.0) * P.adj + nv * (double)W * 8);
   GEM_HIP_CHECK(hipEventRecord(c->ev[1], s));
   GEM_HIP_CHECK(hipStreamSynchronize(s));
   Qd.ncan.assign(h, h + nv);
@@ -581,7 +579,7 @@ void run_filter_noalloc(gem_ctx *c, const gem_query_view *qv, uint32_t T, uint32
     can_off[u] = (uint64_t)u * can_pitch;
   }
   can_off[nv] = (uint64_t)nv * can_pitch;
-  // carve the scratch array
+  // carve the scratch array (its layout takes less than the limit above)
   unsigned char *base = g_scratch_ptr[c->device];
   uint64_t at = 0;
   auto take = [&](uint64_t bytes) {
@@ -589,30 +587,19 @@ void run_filter_noalloc(gem_ctx *c, const gem_query_view *qv, uint32_t T, uint32
     at += (bytes + 255) / 256 * 256;
     return p;
   };
-  const uint32_t hub_cap = std::max<uint32_t>(G.n_hub, 1);
   FilterBufs B;
-  B.fq = reinterpret_cast<FilterQuery *>(take(sizeof(FilterQuery)));
-  B.slot_of = take(P.slot_of.size());
-  uint64_t *d_can_off = reinterpret_cast<uint64_t *>(take(8ull * (nv + 1)));
-  B.can_off = d_can_off;
+  uint8_t *d_slot_of = take(P.slot_of.size());
+  B.slot_of = d_slot_of;
   B.bitmap = reinterpret_cast<uint64_t *>(take(8ull * nv * W));
-  B.tile_count = reinterpret_cast<uint32_t *>(take(4ull * nv * W));
+  B.sums = reinterpret_cast<uint32_t *>(take(4ull * nv * std::max<uint32_t>(rank_chunks(W), 1)));
   B.rank = reinterpret_cast<uint32_t *>(take(4ull * nv * (W + 1)));
-  B.heavy_list = reinterpret_cast<uint32_t *>(take(4ull * std::max<uint32_t>(G.n, 1)));
-  B.heavy_n = reinterpret_cast<uint32_t *>(take(4));
-  B.hub_list = reinterpret_cast<uint32_t *>(take(4ull * hub_cap));
-  B.hub_n = reinterpret_cast<uint32_t *>(take(4));
-  B.hub_cnt = reinterpret_cast<uint32_t *>(take(4ull * hub_cap * GEM_MAX_QV));
-  B.hub_cap = hub_cap;
   if (at > FILTER_SCRATCH_BYTES) throw Error{GEM_E_STATE, "scratch layout exceeds its size"};
-  B.can = d_can;  // null: counts only (no compaction)
+  B.can = d_can;  // null: counts only
+  B.ncan = d_num_can;
   hipStream_t s = c->stream;
-  GEM_HIP_CHECK(hipMemcpyAsync(B.fq, &P.fq, sizeof(FilterQuery), hipMemcpyHostToDevice, s));
-  GEM_HIP_CHECK(hipMemcpyAsync(B.slot_of, P.slot_of.data(), P.slot_of.size(), hipMemcpyHostToDevice, s));
-  GEM_HIP_CHECK(hipMemcpyAsync(d_can_off, can_off.data(), 8ull * (nv + 1), hipMemcpyHostToDevice, s));
-  filter_launch(c, nv, W, B);
-  k_gather_counts<<<1, 64, 0, s>>>(B.rank, nv, W, d_num_can);
-  GEM_LAUNCH_CHECK("k_gather_counts");
+  if (!G.lab8)
+    GEM_HIP_CHECK(hipMemcpyAsync(d_slot_of, P.slot_of.data(), P.slot_of.size(), hipMemcpyHostToDevice, s));
+  filter_launch(c, nv, W, P, can_off.data(), B);
   // the host arrays above are read by the copies: wait before they go
   GEM_HIP_CHECK(hipStreamSynchronize(s));
 }

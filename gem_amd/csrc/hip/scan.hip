@@ -135,27 +135,4 @@ void scan_many_u64(gem_ctx *c, const ScanSeg *d_segs, const ScanSeg *h_segs, uin
   }
 }
 
-// One block per segment: exclusive scan of len u32 counts, out[len] = total.
-__global__ void __launch_bounds__(1024) k_scan_segments_u32(const uint32_t *in, uint32_t *out, uint64_t len) {
-  __shared__ uint64_t sm[16];
-  const uint32_t *src = in + (uint64_t)blockIdx.x * len;
-  uint32_t *dst = out + (uint64_t)blockIdx.x * (len + 1);
-  uint64_t carry = 0;
-  for (uint64_t b = 0; b < len; b += blockDim.x) {
-    uint64_t idx = b + threadIdx.x;
-    uint64_t x = idx < len ? src[idx] : 0;
-    uint64_t ex;
-    uint64_t tot = block_excl_scan_u64(x, &ex, sm);
-    if (idx < len) dst[idx] = (uint32_t)(carry + ex);
-    carry += tot;
-  }
-  if (threadIdx.x == 0) dst[len] = (uint32_t)carry;
-}
-
-void scan_segments_u32(gem_ctx *c, const uint32_t *d_in, uint32_t *d_out, uint32_t nseg, uint64_t len) {
-  if (nseg == 0) return;
-  k_scan_segments_u32<<<nseg, 1024, 0, c->stream>>>(d_in, d_out, len);
-  GEM_LAUNCH_CHECK("k_scan_segments_u32");
-}
-
 }  // namespace gemd
