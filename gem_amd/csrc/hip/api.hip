@@ -33,7 +33,7 @@ int guard(gem_ctx *c, F &&f) {
 // Filter, tables and GEM's edge order of q (the plain pipeline before the join).
 std::vector<uint32_t> plain_prepare(gem_ctx *c, const gem_query_view *q) {
   run_filter(c, q, 0);
-  run_tables(c);
+  run_tables(c, c->q);
   const gemh::QueryInfo &Q = c->q.Q;
   std::vector<uint64_t> sz(Q.ne);
   for (uint32_t e = 0; e < Q.ne; ++e) {

@@ -128,6 +128,7 @@ void run_match_batch(gem_ctx *c, const gem_query_view *qs, uint32_t nq, const ui
   float ms = 0;
   GEM_HIP_CHECK(hipEventElapsedTime(&ms, c->ev[6], c->ev[7]));
   c->times.join_ms = ms;
+  settle_times(c);
   prof_flush(c);
   // the run's level buffers and tables are gone: empty segments beyond half
   // of the device memory go back to the driver (the rest stays for the next
@@ -425,7 +426,7 @@ class Preparer {
           const auto ta = clk::now();
           run_filter(shadow_, qd[i], views[i], 0);
           const auto tb = clk::now();
-          run_tables(shadow_, qd[i]);
+          run_tables(shadow_, qd[i], true);  // the batch stream reads them
           t_filter += std::chrono::duration<double>(tb - ta).count();
           t_tables += std::chrono::duration<double>(clk::now() - tb).count();
           run.candidates(shadow_, i);
@@ -465,6 +466,7 @@ static void end_run(gem_ctx *c, double sum_filter, double sum_tables) {
   float ms = 0;
   GEM_HIP_CHECK(hipEventElapsedTime(&ms, c->ev[6], c->ev[7]));
   c->times.join_ms = ms;
+  c->tables_timed = false;
   // wall time of the whole run's filter and table passes (host clock)
   c->times.filter_ms = sum_filter * 1e3;
   c->times.tables_ms = sum_tables * 1e3;
@@ -620,6 +622,7 @@ void run_vjoin(gem_ctx *c, const uint32_t *vorder, uint64_t cap, gem_join_result
   std::vector<VQueryState *> ptrs{&S};
   VBatchRunner runner(c, cap, c->work_limit_rows, c->level_budget_bytes);
   runner.run(ptrs);
+  settle_times(c);
   fill_result(S, cap, out, level_rows);
   prof_flush(c);
 }

@@ -270,6 +270,7 @@ struct gem_ctx {
   gemd::GraphDev g;
   gemd::QueryDev q;
   gem_phase_times times{};
+  bool tables_timed = false;                // ev[2], ev[3] hold a table build not yet in `times`
   uint64_t level_budget_bytes = 1ull << 31;  // per join level buffer
   uint64_t work_limit_rows = 0;             // 0 = none
   uint32_t persistent_blocks = 2048;        // grid of the batched path's persistent kernels
@@ -388,6 +389,16 @@ T *pinned_dev(gem_ctx *c, T *h) {
   return reinterpret_cast<T *>(static_cast<char *>(c->pinned_map) + (reinterpret_cast<char *>(h) - static_cast<char *>(c->pinned)));
 }
 
+// Times of phases whose events were recorded without a wait (call after a
+// stream synchronisation).
+inline void settle_times(gem_ctx *c) {
+  if (!c->tables_timed) return;
+  c->tables_timed = false;
+  float ms = 0;
+  GEM_HIP_CHECK(hipEventElapsedTime(&ms, c->ev[2], c->ev[3]));
+  c->times.tables_ms = ms;
+}
+
 // ---------------------------------------------------------------- phases
 // The data graph a context's filter and table kernels read.
 inline const GraphDev &graph(const gem_ctx *c) { return c->gsrc ? *c->gsrc : c->g; }
@@ -405,7 +416,9 @@ void filter_scratch_init(int device);
 uint64_t filter_scratch_bytes(const GraphDev &G, uint32_t nv);
 void run_filter_noalloc(gem_ctx *c, const gem_query_view *qv, uint32_t T, uint32_t *d_num_can, uint32_t *d_can,
                         uint64_t can_pitch);
-void run_tables(gem_ctx *c, QueryDev &Qd);
+// wait: return when the tables stand (else their write pass may still run on
+// the context stream).
+void run_tables(gem_ctx *c, QueryDev &Qd, bool wait = false);
 void run_position_lookup(gem_ctx *c, uint32_t u, const uint32_t *h_vertices, uint64_t n, uint32_t *h_pos);
 
 struct JoinOut {
@@ -447,11 +460,14 @@ void run_match_relaxed(gem_ctx *c, const gem_query_view *q, uint32_t threshold,
 // out[n] = total.  Returns nothing; caller reads out[n] if needed.
 void scan_u64(gem_ctx *c, const uint64_t *d_in, uint64_t *d_out, uint64_t n);
 // Independent in-place exclusive scans of u64 arrays p[0..n) (the total goes
-// to p[n] and to d_totals[i]); d_segs is the device copy of h_segs.
+// to p[n] and to d_totals[i], device or mapped host memory); first_chunk: the
+// chunks (scan_chunks) of the segments before, `chunks` those of all.
 struct ScanSeg {
   uint64_t *p;
   uint64_t n;
+  uint32_t first_chunk;
 };
-void scan_many_u64(gem_ctx *c, const ScanSeg *d_segs, const ScanSeg *h_segs, uint32_t nseg, uint64_t *d_totals);
+uint32_t scan_chunks(uint64_t n);
+void scan_segments_u64(gem_ctx *c, const ScanSeg *d_segs, uint32_t nseg, uint32_t chunks, uint64_t *d_totals);
 
 }  // namespace gemd

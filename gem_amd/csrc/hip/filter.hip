@@ -315,10 +315,14 @@ __global__ void k_slot_labels(const uint32_t *__restrict__ nbr, uint64_t slots, 
 }
 
 void make_slot_labels(gem_ctx *c, GraphDev &G) {
-  // a quarter of the free memory at most: a larger graph keeps the gathers
-  size_t free_b = 0, total_b = 0;
-  GEM_HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
-  if (!G.lab8 || !G.slots || G.slots > (free_b + pool_reusable_bytes()) / 4) return;
+  if (!G.lab8 || !G.slots) return;
+  // a quarter of the free memory at most (asked for when it could matter): a
+  // larger graph keeps the gathers
+  if (G.slots > (1ull << 28)) {
+    size_t free_b = 0, total_b = 0;
+    GEM_HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    if (G.slots > (free_b + pool_reusable_bytes()) / 4) return;
+  }
   G.nbr_lab.alloc(G.slots + 16, c->stream);
   k_slot_labels<<<(uint32_t)std::min<uint64_t>((G.slots + 255) / 256, 16384), 256, 0, c->stream>>>(
       G.nbr_dev(), G.slots, G.lab.as<uint8_t>(), G.n, G.nbr_lab.as<uint8_t>());

@@ -605,6 +605,7 @@ void run_join_sink(gem_ctx *c, const uint32_t *order, uint64_t cap, JoinOut *out
   float ms = 0;
   GEM_HIP_CHECK(hipEventElapsedTime(&ms, c->ev[4], c->ev[5]));
   c->times.join_ms = ms;
+  settle_times(c);
   prof_flush(c);
 }
 

@@ -10,12 +10,18 @@
 //
 // One pass over adjacency serves all of u's tables: a wave takes 64
 // consecutive candidates of one u, flattens their adjacency lists into one
-// item range (wave scan of degrees) and walks it 64 items per step; item ->
+// item range (wave scan of degrees) and walks it 64 items per group; item ->
 // row by binary lifting over the 64 row starts in LDS; membership of w in each
-// Can(u_j) is one bit of u_j's bitmap (L2-resident); per-row counts and
-// in-row ranks come from ballots restricted to the row's lane segment, with
-// one carried count for the row that spans two steps.  Count pass -> per-table
-// exclusive scan -> write pass.
+// Can(u_j) is one bit of u_j's bitmap (L2-resident), looked up only where w's
+// label (one byte per adjacency slot, GraphDev::nbr_lab) is u_j's; per-row
+// counts and in-row ranks come from ballots restricted to the row's lane
+// segment, with one carried count for the row that spans two groups.  Count
+// pass -> per-table exclusive scan -> write pass; candidates of degree above
+// TABLE_HEAVY_ROW are walked in pieces of TABLE_CHUNK slots by other waves.
+// The count pass hands out the pieces itself, so that nothing between the
+// parameters' upload and the table sizes waits for the host.  Tables of a
+// 16-vertex query on the 2^22-vertex R-MAT graph: 0.71 ms of kernels, against
+// 1.42 with a bitmap word per neighbour and table and one-block scans.
 #include "ctx.h"
 #include "wave.h"
 
@@ -35,8 +41,27 @@ struct TableJob {
 
 struct TableDesc {
   uint32_t val_u;
+  uint32_t lab;  // dense label of val_u
   uint64_t *off;
   uint32_t *val;
+};
+
+// A heavy row: candidate i of the ju-th keyed vertex, its pieces [c0, c0 + n).
+struct HeavyTab {
+  uint32_t ju, i, c0, n;
+};
+
+// Device counters of one build (uploaded as zeros with the descriptors).
+struct TableCtr {
+  uint32_t rows, pieces;
+  unsigned long long adj_len[GEM_MAX_QV];  // light and heavy slots walked per keyed vertex (profiling)
+};
+
+// The graph as the table kernels read it.
+struct TableGraph {
+  const uint64_t *off;
+  const uint32_t *nbr;
+  const uint8_t *nl;  // labels of the adjacency slots (NL)
 };
 
 __device__ __forceinline__ uint64_t lane_range(uint32_t a, uint32_t b) {  // bits [a, b], a <= b < 64
@@ -44,17 +69,18 @@ __device__ __forceinline__ uint64_t lane_range(uint32_t a, uint32_t b) {  // bit
   return hi & ~((1ull << a) - 1);
 }
 
-// Rows longer than HEAVY_ROW are walked by k_tables_heavy in fixed-size
-// chunks spread over waves, so that neither a wave of 64 hub rows nor one
-// hub's row can become a straggler.
-constexpr uint32_t HEAVY_ROW = 256;
+// Is neighbour wv (label lw, when known) to be looked up in a table whose
+// value vertex has label lab?
+template <bool NL>
+__device__ __forceinline__ bool wanted(bool iv, uint32_t lw, uint32_t lab) {
+  return iv && (!NL || lw == lab);
+}
 
-template <bool WRITE>
+template <bool WRITE, bool NL>
 __global__ void __launch_bounds__(TAB_WAVES * 64)
-k_tables(const uint64_t *__restrict__ goff, const uint32_t *__restrict__ gnbr, const uint32_t *__restrict__ can,
-         const uint64_t *__restrict__ bitmap, const uint32_t *__restrict__ rank, const TableJob job,
-         const TableDesc *__restrict__ desc, unsigned long long *__restrict__ adj_len,
-         uint64_t *__restrict__ heavy_list, uint32_t *__restrict__ heavy_n) {
+k_tables(const TableGraph G, const uint32_t *__restrict__ can, const uint64_t *__restrict__ bitmap,
+         const uint32_t *__restrict__ rank, const TableJob job, const TableDesc *__restrict__ desc,
+         TableCtr *__restrict__ ctr, HeavyTab *__restrict__ heavy, uint32_t *__restrict__ piece_row, int prof) {
   __shared__ uint32_t st[TAB_WAVES][65];
   __shared__ uint64_t ob[TAB_WAVES][64];
   const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
@@ -70,22 +96,27 @@ k_tables(const uint64_t *__restrict__ goff, const uint32_t *__restrict__ gnbr, c
   uint32_t len = 0, full_len = 0;
   if (valid) {
     const uint32_t v = can[job.can_off[ju] + i];
-    o0 = goff[v];
-    full_len = (uint32_t)(goff[v + 1] - o0);
-    len = full_len > HEAVY_ROW ? 0u : full_len;
+    o0 = G.off[v];
+    full_len = (uint32_t)(G.off[v + 1] - o0);
+    len = full_len > TABLE_HEAVY_ROW ? 0u : full_len;
   }
   if (!WRITE) {
-    const uint64_t hv = __ballot(full_len > HEAVY_ROW);
+    const uint64_t hv = __ballot(full_len > TABLE_HEAVY_ROW);
     if (hv) {
-      uint32_t base = 0;
-      if (l == 0) base = atomicAdd(heavy_n, (uint32_t)__popcll(hv));
-      base = readlane_u32(base, 0);
-      if ((hv >> l) & 1ull) heavy_list[base + rank_below(hv)] = ((uint64_t)ju << 32) | i;
+      const uint32_t n = full_len > TABLE_HEAVY_ROW ? (full_len + TABLE_CHUNK - 1) / TABLE_CHUNK : 0;
+      const uint32_t incl = wave_incl_scan_u32(n);
+      uint32_t r = 0, c = 0;
+      if (l == 0) r = atomicAdd(&ctr->rows, (uint32_t)__popcll(hv));
+      if (l == 63) c = atomicAdd(&ctr->pieces, incl);
+      r = readlane_u32(r, 0) + rank_below(hv);
+      c = readlane_u32(c, 63) + incl - n;
+      if (n) heavy[r] = HeavyTab{ju, i, c, n};
+      for (uint32_t x = 0; x < n; ++x) piece_row[c + x] = r;
     }
   }
   const uint32_t incl = wave_incl_scan_u32(len);
   const uint32_t total = readlane_u32(incl, 63);
-  if (!WRITE && l == 0 && total) atomicAdd(adj_len + ju, (unsigned long long)total);
+  if (!WRITE && prof && l == 0 && total) atomicAdd(&ctr->adj_len[ju], (unsigned long long)total);
   st[w][l] = incl - len;
   ob[w][l] = o0;
   if (l == 63) st[w][64] = total;
@@ -95,21 +126,22 @@ k_tables(const uint64_t *__restrict__ goff, const uint32_t *__restrict__ gnbr, c
   if (!WRITE && valid && full_len == 0)
     for (uint32_t j = 0; j < nd; ++j) desc[t0 + j].off[i] = 0;
   const uint32_t W = job.W;
-  // lane j < nd holds table j: value vertex, row offsets, values
-  uint32_t my_vu = 0;
+  // lane j < nd holds table j: value vertex and its label, row offsets, values
+  uint32_t my_vu = 0, my_lab = 0;
   uint64_t my_off = 0, my_val = 0;
   if (l < nd) {
     const TableDesc d = desc[t0 + l];
     my_vu = d.val_u;
+    my_lab = d.lab;
     my_off = reinterpret_cast<uint64_t>(d.off);
     my_val = reinterpret_cast<uint64_t>(d.val);
   }
   uint32_t carry_reg = 0;  // lane j: hits of the row carried into the next group, table j
-  // One 64-item group of the flattened adjacency: the lane's row, its value,
-  // and the lane range of its row inside the group.
+  // One 64-item group of the flattened adjacency: the lane's row, its value
+  // and label, and the lane range of its row inside the group.
   struct Grp {
     bool iv, row_done;
-    uint32_t row, wv, last, row0, seg_hi;
+    uint32_t row, wv, lw, last, row0, seg_hi;
     uint64_t seg_mask, below_mask;
   };
   auto group = [&](uint32_t t) {
@@ -118,7 +150,9 @@ k_tables(const uint64_t *__restrict__ goff, const uint32_t *__restrict__ gnbr, c
     g.iv = item < total;
     g.row = g.iv ? seg_of(st[w], item) : 63;
     const uint32_t rs = st[w][g.row], re = st[w][g.row + 1];
-    g.wv = g.iv ? gnbr[ob[w][g.row] + (item - rs)] : 0;
+    const uint64_t at = ob[w][g.row] + (item - rs);
+    g.wv = g.iv ? G.nbr[at] : 0;
+    g.lw = NL && g.iv ? G.nl[at] : 0;
     g.last = min(63u, total - 1 - t);
     g.row0 = readlane_u32(g.row, 0);
     const uint32_t seg_lo = rs > t ? rs - t : 0;
@@ -142,10 +176,10 @@ k_tables(const uint64_t *__restrict__ goff, const uint32_t *__restrict__ gnbr, c
         const uint32_t r = before + (uint32_t)__popcll(m & g.below_mask);
         const uint32_t p = rank[(uint64_t)vu * (W + 1) + (g.wv >> 6)] +
                            (uint32_t)__popcll(word & ((1ull << (g.wv & 63)) - 1));
-        val[off[row_base + g.row] + r] = p;
+        stg(val + ldg(off + row_base + g.row) + r, p);
       }
     } else {
-      if (g.iv && l == g.seg_hi && g.row_done) off[row_base + g.row] = tot_row;
+      if (g.iv && l == g.seg_hi && g.row_done) stg(off + row_base + g.row, (uint64_t)tot_row);
     }
     return readlane_u32(g.row_done ? 0u : tot_row, g.last);
   };
@@ -156,10 +190,10 @@ k_tables(const uint64_t *__restrict__ goff, const uint32_t *__restrict__ gnbr, c
     const Grp A = group(t);
     const Grp B = two ? group(t + 64) : A;
     for (uint32_t j = 0; j < nd; ++j) {
-      const uint32_t vu = readlane_u32(my_vu, j);
+      const uint32_t vu = readlane_u32(my_vu, j), lab = readlane_u32(my_lab, j);
       const uint64_t *bm = bitmap + (uint64_t)vu * W;
-      const uint64_t wa = A.iv ? bm[A.wv >> 6] : 0;
-      const uint64_t wb = two && B.iv ? bm[B.wv >> 6] : 0;
+      const uint64_t wa = wanted<NL>(A.iv, A.lw, lab) ? bm[A.wv >> 6] : 0;
+      const uint64_t wb = two && wanted<NL>(B.iv, B.lw, lab) ? bm[B.wv >> 6] : 0;
       uint32_t carry = apply(A, j, vu, wa, readlane_u32(carry_reg, j));
       if (two) carry = apply(B, j, vu, wb, carry);
       if (l == j) carry_reg = carry;
@@ -167,133 +201,150 @@ k_tables(const uint64_t *__restrict__ goff, const uint32_t *__restrict__ gnbr, c
   }
 }
 
-// Heavy rows are walked in chunks of TCH adjacency entries, one wave task per
-// chunk, so that a hub's row is spread over many waves.  The count pass stores
-// each chunk's hit count per table (ccnt[chunk * ndmax + j]); k_theavy_bases
-// turns those into each chunk's offset inside its row (exclusive over the
-// row's chunks) and writes the rows' totals; the write pass starts each
-// chunk's hits at that offset, so values stay in adjacency order.
-constexpr uint32_t TCH = 2048;
-
-// Chunk prefix of the heavy rows: cpre[h] = chunks of rows before h,
-// cpre[n] = *total = all chunks (one block).
-__global__ void __launch_bounds__(1024) k_theavy_prefix(const uint64_t *__restrict__ goff,
-                                                       const uint32_t *__restrict__ can, const TableJob job,
-                                                       const uint64_t *__restrict__ heavy_list,
-                                                       const uint32_t *__restrict__ heavy_n, uint64_t *__restrict__ cpre,
-                                                       uint64_t *__restrict__ total) {
-  __shared__ uint64_t sm[16];
-  const uint32_t n = *heavy_n;
-  uint64_t carry = 0;
-  for (uint32_t b = 0; b < n; b += blockDim.x) {
-    const uint32_t h = b + threadIdx.x;
-    uint64_t x = 0;
-    if (h < n) {
-      const uint64_t e = heavy_list[h];
-      const uint32_t v = can[job.can_off[(uint32_t)(e >> 32)] + (uint32_t)e];
-      x = (goff[v + 1] - goff[v] + TCH - 1) / TCH;
-    }
-    uint64_t ex;
-    const uint64_t tot = block_excl_scan_u64(x, &ex, sm);
-    if (h < n) cpre[h] = carry + ex;
-    carry += tot;
-  }
-  if (threadIdx.x == 0) {
-    cpre[n] = carry;
-    *total = carry;
-  }
-}
-
-// Persistent grid over the chunks; lane j carries table j's running count.
-template <bool WRITE>
+// Persistent grid over the heavy rows' pieces; lane j carries table j's
+// running count.  The count pass stores each piece's hits per table
+// (ccnt[piece * ndmax + j]); k_theavy_bases turns those into each piece's
+// offset inside its row and writes the rows' totals; the write pass starts
+// each piece's hits at that offset, so values stay in adjacency order.  Four
+// groups of 64 slots per step: their loads, and then the bitmap words of each
+// table for the slots of its label, are in flight together.
+template <bool WRITE, bool NL>
 __global__ void __launch_bounds__(TAB_WAVES * 64)
-k_tables_heavy(const uint64_t *__restrict__ goff, const uint32_t *__restrict__ gnbr, const uint32_t *__restrict__ can,
-               const uint64_t *__restrict__ bitmap, const uint32_t *__restrict__ rank, const TableJob job,
-               const TableDesc *__restrict__ desc, unsigned long long *__restrict__ adj_len,
-               const uint64_t *__restrict__ heavy_list, const uint32_t *__restrict__ heavy_n,
-               const uint64_t *__restrict__ cpre, uint32_t *__restrict__ ccnt, uint32_t ndmax) {
+k_tables_heavy(const TableGraph G, const uint32_t *__restrict__ can, const uint64_t *__restrict__ bitmap,
+               const uint32_t *__restrict__ rank, const TableJob job, const TableDesc *__restrict__ desc,
+               TableCtr *__restrict__ ctr, const HeavyTab *__restrict__ heavy, const uint32_t *__restrict__ piece_row,
+               uint32_t *__restrict__ ccnt, uint32_t ndmax, int prof) {
+  constexpr int GR = 4;
   const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
-  const uint32_t nh = *heavy_n, W = job.W;
-  const uint64_t nchunks = cpre[nh];
-  for (uint64_t c = (uint64_t)blockIdx.x * TAB_WAVES + w; c < nchunks; c += (uint64_t)gridDim.x * TAB_WAVES) {
-    uint32_t lo = 0, hi = nh;  // the chunk's row: largest h with cpre[h] <= c
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (cpre[mid] <= c)
-        lo = mid;
-      else
-        hi = mid;
-    }
-    const uint64_t e = heavy_list[lo];
-    const uint32_t ju = (uint32_t)(e >> 32), i = (uint32_t)e;
-    const uint32_t v = can[job.can_off[ju] + i];
-    const uint64_t o0 = goff[v], len = goff[v + 1] - o0;
-    const uint64_t t0 = (c - cpre[lo]) * TCH, t1 = t0 + TCH < len ? t0 + TCH : len;
-    if (!WRITE && l == 0) atomicAdd(adj_len + ju, (unsigned long long)(t1 - t0));
-    const uint32_t nd = job.nd[ju], tb = job.tab0[ju];
-    // lane j < nd holds table j: its value vertex, (write) the address of the
-    // row's first value, and its running count in the row
-    uint32_t my_vu = 0, run_reg = 0;
+  const uint32_t W = job.W, pieces = ctr->pieces;
+  for (uint32_t c = blockIdx.x * TAB_WAVES + w; c < pieces; c += gridDim.x * TAB_WAVES) {
+    const HeavyTab e = heavy[piece_row[c]];
+    const uint32_t v = can[job.can_off[e.ju] + e.i];
+    const uint64_t o0 = G.off[v], len = G.off[v + 1] - o0;
+    const uint64_t t0 = (uint64_t)(c - e.c0) * TABLE_CHUNK, t1 = t0 + TABLE_CHUNK < len ? t0 + TABLE_CHUNK : len;
+    if (!WRITE && prof && l == 0) atomicAdd(&ctr->adj_len[e.ju], (unsigned long long)(t1 - t0));
+    const uint32_t nd = job.nd[e.ju], tb = job.tab0[e.ju];
+    // lane j < nd holds table j: its value vertex and label, (write) the
+    // address of the row's first value, and its running count in the row
+    uint32_t my_vu = 0, my_lab = 0, run_reg = 0;
     uint64_t my_dst = 0;
     if (l < nd) {
       const TableDesc d = desc[tb + l];
       my_vu = d.val_u;
+      my_lab = d.lab;
       if (WRITE) {
-        my_dst = reinterpret_cast<uint64_t>(d.val + d.off[i]);
-        run_reg = ccnt[c * ndmax + l];
+        my_dst = reinterpret_cast<uint64_t>(d.val + d.off[e.i]);
+        run_reg = ccnt[(uint64_t)c * ndmax + l];
       }
     }
-    // two 64-entry groups per step: both groups' loads are in flight before
-    // either group's ballots
-    for (uint64_t t = t0; t < t1; t += 128) {
-      const bool iv0 = t + l < t1, iv1 = t + 64 + l < t1;
-      const uint32_t wv0 = iv0 ? gnbr[o0 + t + l] : 0;
-      const uint32_t wv1 = iv1 ? gnbr[o0 + t + 64 + l] : 0;
+    for (uint64_t t = t0; t < t1; t += 64 * GR) {
+      uint32_t wv[GR], lw[GR];
+      bool iv[GR];
+#pragma unroll
+      for (int g = 0; g < GR; ++g) {
+        const uint64_t x = t + 64 * g + l;
+        iv[g] = x < t1;
+        wv[g] = iv[g] ? G.nbr[o0 + x] : 0;
+        lw[g] = NL && iv[g] ? G.nl[o0 + x] : 0;
+      }
       for (uint32_t j = 0; j < nd; ++j) {
-        const uint32_t vu = readlane_u32(my_vu, j);
+        const uint32_t vu = readlane_u32(my_vu, j), lab = readlane_u32(my_lab, j);
         const uint64_t *bm = bitmap + (uint64_t)vu * W;
-        const uint64_t word0 = iv0 ? bm[wv0 >> 6] : 0, word1 = iv1 ? bm[wv1 >> 6] : 0;
-        const bool hit0 = (word0 >> (wv0 & 63)) & 1ull, hit1 = (word1 >> (wv1 & 63)) & 1ull;
-        const uint64_t m0 = __ballot(hit0), m1 = __ballot(hit1);
-        const uint32_t run = readlane_u32(run_reg, j);
-        if (WRITE && (hit0 || hit1)) {
-          uint32_t *dst = reinterpret_cast<uint32_t *>(readlane_u64(my_dst, j));
-          const uint32_t *rk = rank + (uint64_t)vu * (W + 1);
-          if (hit0) dst[run + rank_below(m0)] = rk[wv0 >> 6] + (uint32_t)__popcll(word0 & ((1ull << (wv0 & 63)) - 1));
-          if (hit1)
-            dst[run + (uint32_t)__popcll(m0) + rank_below(m1)] =
-                rk[wv1 >> 6] + (uint32_t)__popcll(word1 & ((1ull << (wv1 & 63)) - 1));
+        const uint32_t *rk = rank + (uint64_t)vu * (W + 1);
+        uint64_t word[GR];
+        uint32_t r[GR];
+#pragma unroll
+        for (int g = 0; g < GR; ++g) {
+          const bool want = wanted<NL>(iv[g], lw[g], lab);
+          word[g] = want ? bm[wv[g] >> 6] : 0;
+          if (WRITE) r[g] = want ? rk[wv[g] >> 6] : 0;
         }
-        if (l == j) run_reg = run + (uint32_t)__popcll(m0) + (uint32_t)__popcll(m1);
+        uint32_t run = readlane_u32(run_reg, j);
+        uint32_t *dst = reinterpret_cast<uint32_t *>(readlane_u64(my_dst, j));
+#pragma unroll
+        for (int g = 0; g < GR; ++g) {
+          const bool hit = (word[g] >> (wv[g] & 63)) & 1ull;
+          const uint64_t m = __ballot(hit);
+          if (WRITE && hit)
+            stg(dst + run + rank_below(m), r[g] + (uint32_t)__popcll(word[g] & ((1ull << (wv[g] & 63)) - 1)));
+          run += (uint32_t)__popcll(m);
+        }
+        if (l == j) run_reg = run;
       }
     }
-    if (!WRITE && l < nd) ccnt[c * ndmax + l] = run_reg;
+    if (!WRITE && l < nd) ccnt[(uint64_t)c * ndmax + l] = run_reg;
   }
 }
 
-// One thread per (heavy row, table slot): chunk counts -> chunk offsets inside
+// One thread per (heavy row, table slot): piece counts -> piece offsets inside
 // the row, and the row's total as its count.
-__global__ void k_theavy_bases(const TableJob job, const TableDesc *__restrict__ desc,
-                               const uint64_t *__restrict__ heavy_list, const uint32_t *__restrict__ heavy_n,
-                               const uint64_t *__restrict__ cpre, uint32_t *__restrict__ ccnt, uint32_t ndmax) {
-  const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= (uint64_t)(*heavy_n) * ndmax) return;
-  const uint32_t h = (uint32_t)(x / ndmax), j = (uint32_t)(x % ndmax);
-  const uint64_t e = heavy_list[h];
-  const uint32_t ju = (uint32_t)(e >> 32), i = (uint32_t)e;
-  if (j >= job.nd[ju]) return;
-  uint32_t run = 0;
-  for (uint64_t c = cpre[h]; c < cpre[h + 1]; ++c) {
-    const uint32_t n = ccnt[c * ndmax + j];
-    ccnt[c * ndmax + j] = run;
-    run += n;
+__global__ void __launch_bounds__(256) k_theavy_bases(const TableJob job, const TableDesc *__restrict__ desc,
+                                                     const TableCtr *__restrict__ ctr,
+                                                     const HeavyTab *__restrict__ heavy, uint32_t *__restrict__ ccnt,
+                                                     uint32_t ndmax) {
+  const uint64_t n = (uint64_t)ctr->rows * ndmax;
+  for (uint64_t x = (uint64_t)blockIdx.x * 256 + threadIdx.x; x < n; x += (uint64_t)gridDim.x * 256) {
+    const HeavyTab e = heavy[x / ndmax];
+    const uint32_t j = (uint32_t)(x % ndmax);
+    if (j >= job.nd[e.ju]) continue;
+    uint32_t run = 0;
+    for (uint32_t c = e.c0; c < e.c0 + e.n; ++c) {
+      const uint32_t h = ccnt[(uint64_t)c * ndmax + j];
+      ccnt[(uint64_t)c * ndmax + j] = run;
+      run += h;
+    }
+    stg(desc[job.tab0[e.ju] + j].off + e.i, (uint64_t)run);
   }
-  desc[job.tab0[ju] + j].off[i] = run;
 }
 
-void run_tables(gem_ctx *c) { run_tables(c, c->q); }
+void run_tables(gem_ctx *c) { run_tables(c, c->q, true); }
 
-void run_tables(gem_ctx *c, QueryDev &Qd) {
+// The launches over the build's parameters; passes by `write`.
+struct TableRun {
+  gem_ctx *c;
+  const GraphDev &G;
+  QueryDev &Qd;
+  TableJob job{};
+  uint32_t waves = 0, ndmax = 1;
+  uint64_t rows_bound = 0, pieces_bound = 0;  // heavy rows and pieces there can be
+  DevBuf params, heavy, piece_row, ccnt;
+  TableDesc *desc = nullptr;
+  TableCtr *ctr = nullptr;
+
+  template <bool WRITE, bool NL>
+  void pass_as() {
+    hipStream_t s = c->stream;
+    const TableGraph g{G.off.as<uint64_t>(), G.nbr_dev(), G.nbr_lab.as<uint8_t>()};
+    const int prof = c->prof.on;
+    if (waves) {
+      k_tables<WRITE, NL><<<(waves + TAB_WAVES - 1) / TAB_WAVES, TAB_WAVES * 64, 0, s>>>(
+          g, Qd.can.as<uint32_t>(), Qd.bitmap.as<uint64_t>(), Qd.rank.as<uint32_t>(), job, desc, ctr,
+          heavy.as<HeavyTab>(), piece_row.as<uint32_t>(), prof);
+      GEM_LAUNCH_CHECK("k_tables");
+    }
+    if (waves && rows_bound) {
+      const uint32_t hb = (uint32_t)std::min<uint64_t>((pieces_bound + TAB_WAVES - 1) / TAB_WAVES, 2048);
+      k_tables_heavy<WRITE, NL><<<hb, TAB_WAVES * 64, 0, s>>>(
+          g, Qd.can.as<uint32_t>(), Qd.bitmap.as<uint64_t>(), Qd.rank.as<uint32_t>(), job, desc, ctr,
+          heavy.as<HeavyTab>(), piece_row.as<uint32_t>(), ccnt.as<uint32_t>(), ndmax, prof);
+      GEM_LAUNCH_CHECK("k_tables_heavy");
+      if (!WRITE) {
+        k_theavy_bases<<<(uint32_t)std::min<uint64_t>((rows_bound * ndmax + 255) / 256, 1024), 256, 0, s>>>(
+            job, desc, ctr, heavy.as<HeavyTab>(), ccnt.as<uint32_t>(), ndmax);
+        GEM_LAUNCH_CHECK("k_theavy_bases");
+      }
+    }
+  }
+  void pass(bool write) {
+    ProfLaunch pl(c, write ? K_TABLES_WRITE : K_TABLES_COUNT);
+    if (G.nbr_lab.p)
+      write ? pass_as<true, true>() : pass_as<false, true>();
+    else
+      write ? pass_as<true, false>() : pass_as<false, false>();
+  }
+};
+
+void run_tables(gem_ctx *c, QueryDev &Qd, bool wait) {
   if (!Qd.filtered) throw Error{GEM_E_STATE, "filter has not run"};
   const gemh::QueryInfo &Q = Qd.Q;
   const GraphDev &G = graph(c);
@@ -301,14 +352,14 @@ void run_tables(gem_ctx *c, QueryDev &Qd) {
   GEM_HIP_CHECK(hipEventRecord(c->ev[2], s));
   Qd.tab.clear();
   Qd.tab.resize(2 * Q.ne);
-  TableJob job{};
+  TableRun R{c, G, Qd};
+  TableJob &job = R.job;
   job.W = Qd.W;
   std::vector<uint32_t> desc_tab;  // TableDesc index -> directed edge
-  uint32_t waves = 0;
   for (uint32_t u = 0; u < Q.nv; ++u) {
     if (Q.deg[u] == 1) continue;  // leaves key no table (unifiedTrie.cu:1045,1095)
     const uint32_t ju = job.nu++;
-    job.wave_start[ju] = waves;
+    job.wave_start[ju] = R.waves;
     job.ncan[ju] = Qd.ncan[u];
     job.can_off[ju] = Qd.can_off[u];
     job.tab0[ju] = (uint32_t)desc_tab.size();
@@ -322,138 +373,81 @@ void run_tables(gem_ctx *c, QueryDev &Qd) {
       desc_tab.push_back(d);
       job.nd[ju]++;
     }
-    waves += (Qd.ncan[u] + 63) / 64;
-  }
-  job.wave_start[job.nu] = waves;
-  std::vector<TableDesc> desc(desc_tab.size());
-  auto fill_desc = [&]() {
-    for (size_t k = 0; k < desc_tab.size(); ++k) {
-      TableDev &T = Qd.tab[desc_tab[k]];
-      desc[k] = TableDesc{T.val_u, T.off.as<uint64_t>(), T.val.as<uint32_t>()};
+    R.ndmax = std::max(R.ndmax, job.nd[ju]);
+    R.waves += (Qd.ncan[u] + 63) / 64;
+    auto it = G.label_id.find(Q.lab[u]);
+    if (it != G.label_id.end()) {
+      R.rows_bound += std::min<uint64_t>(G.label_long[it->second], Qd.ncan[u]);
+      R.pieces_bound += G.label_chunks[it->second];
     }
-  };
-  fill_desc();
-  DevBuf ddesc;
-  ddesc.alloc(std::max<size_t>(desc.size(), 1) * sizeof(TableDesc), s);
-  GEM_HIP_CHECK(hipMemcpyAsync(ddesc.p, desc.data(), desc.size() * sizeof(TableDesc), hipMemcpyHostToDevice, s));
-  const uint32_t blocks = (waves + TAB_WAVES - 1) / TAB_WAVES;
-  DevBuf adj_len, heavy_list, heavy_n;
-  adj_len.alloc(GEM_MAX_QV * 8, s);
-  GEM_HIP_CHECK(hipMemsetAsync(adj_len.p, 0, GEM_MAX_QV * 8, s));
-  uint64_t rows_total = 0;
-  for (uint32_t ju = 0; ju < job.nu; ++ju) rows_total += job.ncan[ju];
-  heavy_list.alloc(std::max<uint64_t>(rows_total, 1) * 8, s);
-  heavy_n.alloc(4, s);
-  GEM_HIP_CHECK(hipMemsetAsync(heavy_n.p, 0, 4, s));
-  uint32_t ndmax = 1;
-  for (uint32_t ju = 0; ju < job.nu; ++ju) ndmax = std::max(ndmax, job.nd[ju]);
-  DevBuf cpre, ccnt;
-  cpre.alloc((std::max<uint64_t>(rows_total, 1) + 2) * 8, s);
-  uint64_t *d_chunks = cpre.as<uint64_t>() + std::max<uint64_t>(rows_total, 1) + 1;
-  uint32_t nh = 0;
-  uint64_t nchunks = 0;
-  auto launch_light = [&](bool write) {
-    if (!blocks) return;
-    if (write)
-      k_tables<true><<<blocks, TAB_WAVES * 64, 0, s>>>(
-          G.off.as<uint64_t>(), G.nbr_dev(), Qd.can.as<uint32_t>(), Qd.bitmap.as<uint64_t>(),
-          Qd.rank.as<uint32_t>(), job, ddesc.as<TableDesc>(), adj_len.as<unsigned long long>(),
-          heavy_list.as<uint64_t>(), heavy_n.as<uint32_t>());
-    else
-      k_tables<false><<<blocks, TAB_WAVES * 64, 0, s>>>(
-          G.off.as<uint64_t>(), G.nbr_dev(), Qd.can.as<uint32_t>(), Qd.bitmap.as<uint64_t>(),
-          Qd.rank.as<uint32_t>(), job, ddesc.as<TableDesc>(), adj_len.as<unsigned long long>(),
-          heavy_list.as<uint64_t>(), heavy_n.as<uint32_t>());
-    GEM_LAUNCH_CHECK(write ? "k_tables<write>" : "k_tables<count>");
-  };
-  auto launch_heavy = [&](bool write) {
-    if (!nchunks) return;
-    const uint32_t hb = (uint32_t)std::min<uint64_t>((nchunks + TAB_WAVES - 1) / TAB_WAVES, 2048);
-    if (write)
-      k_tables_heavy<true><<<hb, TAB_WAVES * 64, 0, s>>>(
-          G.off.as<uint64_t>(), G.nbr_dev(), Qd.can.as<uint32_t>(), Qd.bitmap.as<uint64_t>(),
-          Qd.rank.as<uint32_t>(), job, ddesc.as<TableDesc>(), adj_len.as<unsigned long long>(),
-          heavy_list.as<uint64_t>(), heavy_n.as<uint32_t>(), cpre.as<uint64_t>(), ccnt.as<uint32_t>(), ndmax);
-    else
-      k_tables_heavy<false><<<hb, TAB_WAVES * 64, 0, s>>>(
-          G.off.as<uint64_t>(), G.nbr_dev(), Qd.can.as<uint32_t>(), Qd.bitmap.as<uint64_t>(),
-          Qd.rank.as<uint32_t>(), job, ddesc.as<TableDesc>(), adj_len.as<unsigned long long>(),
-          heavy_list.as<uint64_t>(), heavy_n.as<uint32_t>(), cpre.as<uint64_t>(), ccnt.as<uint32_t>(), ndmax);
-    GEM_LAUNCH_CHECK(write ? "k_tables_heavy<write>" : "k_tables_heavy<count>");
-  };
-  {
-    ProfLaunch pl(c, K_TABLES_COUNT);
-    launch_light(false);
-    // rows longer than HEAVY_ROW: chunk prefix, then (sizes known) the chunked count
-    k_theavy_prefix<<<1, 1024, 0, s>>>(G.off.as<uint64_t>(), Qd.can.as<uint32_t>(), job, heavy_list.as<uint64_t>(),
-                                       heavy_n.as<uint32_t>(), cpre.as<uint64_t>(), d_chunks);
-    GEM_LAUNCH_CHECK("k_theavy_prefix");
   }
-  {
-    uint64_t *hh = pinned<uint64_t>(c, 2);
-    hh[0] = 0;
-    GEM_HIP_CHECK(hipMemcpyAsync(hh, heavy_n.p, 4, hipMemcpyDeviceToHost, s));
-    GEM_HIP_CHECK(hipMemcpyAsync(hh + 1, d_chunks, 8, hipMemcpyDeviceToHost, s));
-    GEM_HIP_CHECK(hipStreamSynchronize(s));
-    nh = (uint32_t)hh[0];
-    nchunks = hh[1];
-  }
-  if (nchunks) {
-    ccnt.alloc(nchunks * ndmax * 4, s);
-    ProfLaunch pl(c, K_TABLES_COUNT);
-    launch_heavy(false);
-    const uint64_t nthreads = (uint64_t)nh * ndmax;
-    k_theavy_bases<<<(uint32_t)((nthreads + 255) / 256), 256, 0, s>>>(
-        job, ddesc.as<TableDesc>(), heavy_list.as<uint64_t>(), heavy_n.as<uint32_t>(), cpre.as<uint64_t>(),
-        ccnt.as<uint32_t>(), ndmax);
-    GEM_LAUNCH_CHECK("k_theavy_bases");
-  }
-  // row counts -> offsets for every table in one launch (the larger ones by
-  // the multi-block scan), then the table sizes and adjacency lengths in one
-  // copy back
+  job.wave_start[job.nu] = R.waves;
+  // Parameters of the build: one staging block, one device block: the tables,
+  // the scan segments (and, before them on the host, the sizes that the scan
+  // writes), the counters.
   const size_t nt = desc_tab.size();
-  std::vector<ScanSeg> segs(nt);
+  const size_t at_seg = nt * sizeof(TableDesc), at_ctr = at_seg + nt * sizeof(ScanSeg);
+  const size_t bytes = at_ctr + sizeof(TableCtr);
+  uint64_t *sizes = pinned<uint64_t>(c, nt + (bytes + 7) / 8);
+  unsigned char *stage = reinterpret_cast<unsigned char *>(sizes + nt);
+  TableDesc *hdesc = reinterpret_cast<TableDesc *>(stage);
+  ScanSeg *hseg = reinterpret_cast<ScanSeg *>(stage + at_seg);
+  uint32_t chunks = 0;
   for (size_t k = 0; k < nt; ++k) {
-    TableDev &T = Qd.tab[desc_tab[k]];
-    segs[k] = ScanSeg{T.off.as<uint64_t>(), (uint64_t)Qd.ncan[T.key_u]};
+    const TableDev &T = Qd.tab[desc_tab[k]];
+    auto it = G.label_id.find(Q.lab[T.val_u]);
+    hdesc[k] = TableDesc{T.val_u, it == G.label_id.end() ? ~0u : it->second, T.off.as<uint64_t>(), nullptr};
+    hseg[k] = ScanSeg{T.off.as<uint64_t>(), (uint64_t)Qd.ncan[T.key_u], chunks};
+    chunks += scan_chunks(Qd.ncan[T.key_u]);
   }
-  DevBuf dsegs, dtot;
-  dsegs.alloc(std::max<size_t>(nt, 1) * sizeof(ScanSeg), s);
-  dtot.alloc((nt + GEM_MAX_QV) * 8, s);
-  if (nt) GEM_HIP_CHECK(hipMemcpyAsync(dsegs.p, segs.data(), nt * sizeof(ScanSeg), hipMemcpyHostToDevice, s));
-  scan_many_u64(c, dsegs.as<ScanSeg>(), segs.data(), (uint32_t)nt, dtot.as<uint64_t>());
-  GEM_HIP_CHECK(hipMemcpyAsync(dtot.as<uint64_t>() + nt, adj_len.p, GEM_MAX_QV * 8, hipMemcpyDeviceToDevice, s));
-  uint64_t *h = pinned<uint64_t>(c, nt + GEM_MAX_QV);
-  GEM_HIP_CHECK(hipMemcpyAsync(h, dtot.p, (nt + GEM_MAX_QV) * 8, hipMemcpyDeviceToHost, s));
+  *reinterpret_cast<TableCtr *>(stage + at_ctr) = TableCtr{};
+  R.params.alloc(bytes, s);
+  unsigned char *dev = R.params.as<unsigned char>();
+  R.desc = reinterpret_cast<TableDesc *>(dev);
+  R.ctr = reinterpret_cast<TableCtr *>(dev + at_ctr);
+  GEM_HIP_CHECK(hipMemcpyAsync(dev, stage, bytes, hipMemcpyHostToDevice, s));
+  if (R.rows_bound) {
+    R.heavy.alloc(R.rows_bound * sizeof(HeavyTab), s);
+    R.piece_row.alloc(R.pieces_bound * 4, s);
+    R.ccnt.alloc(R.pieces_bound * R.ndmax * 4, s);
+  }
+  R.pass(false);
+  // row counts -> offsets of every table, the sizes straight to the host
+  scan_segments_u64(c, reinterpret_cast<ScanSeg *>(dev + at_seg), (uint32_t)nt, chunks, pinned_dev(c, sizes));
   GEM_HIP_CHECK(hipStreamSynchronize(s));
-  // algorithmic bytes: per keyed u, its candidates (4 B), offset pairs (8 B)
-  // and adjacency (4 B per slot) once for all its tables; per table the value
-  // vertex's bitmap (|V|/8) and the row counts / offsets (8 B per row)
-  double shared_bytes = 0, count_bytes = 0, write_bytes = 0;
-  for (uint32_t ju = 0; ju < job.nu; ++ju) shared_bytes += 12.0 * job.ncan[ju] + 4.0 * (double)h[nt + ju];
   for (size_t k = 0; k < nt; ++k) {
     TableDev &T = Qd.tab[desc_tab[k]];
-    T.size = h[k];
-    count_bytes += 8.0 * Qd.W + 8.0 * Qd.ncan[T.key_u];
-    write_bytes += 12.0 * Qd.W + 8.0 * Qd.ncan[T.key_u] + 4.0 * (double)T.size;
+    T.size = sizes[k];
     T.val.alloc(std::max<uint64_t>(T.size, 1) * 4, s);
+    hdesc[k].val = T.val.as<uint32_t>();
   }
-  prof_bytes(c, K_TABLES_COUNT, shared_bytes + count_bytes);
-  prof_bytes(c, K_TABLES_WRITE, shared_bytes + write_bytes);
-  fill_desc();
-  GEM_HIP_CHECK(hipMemcpyAsync(ddesc.p, desc.data(), desc.size() * sizeof(TableDesc), hipMemcpyHostToDevice, s));
-  {
-    ProfLaunch pl(c, K_TABLES_WRITE);
-    launch_light(true);
-    launch_heavy(true);
+  if (c->prof.on) {
+    // algorithmic bytes: per keyed u, its candidates (4 B), offset pairs (8 B)
+    // and adjacency (4 B per slot) once for all its tables; per table the value
+    // vertex's bitmap (|V|/8) and the row counts / offsets (8 B per row)
+    TableCtr h;
+    GEM_HIP_CHECK(hipMemcpyAsync(&h, R.ctr, sizeof(h), hipMemcpyDeviceToHost, s));
+    GEM_HIP_CHECK(hipStreamSynchronize(s));
+    double shared_bytes = 0, count_bytes = 0, write_bytes = 0;
+    for (uint32_t ju = 0; ju < job.nu; ++ju) shared_bytes += 12.0 * job.ncan[ju] + 4.0 * (double)h.adj_len[ju];
+    for (size_t k = 0; k < nt; ++k) {
+      const TableDev &T = Qd.tab[desc_tab[k]];
+      count_bytes += 8.0 * Qd.W + 8.0 * Qd.ncan[T.key_u];
+      write_bytes += 12.0 * Qd.W + 8.0 * Qd.ncan[T.key_u] + 4.0 * (double)T.size;
+    }
+    prof_bytes(c, K_TABLES_COUNT, shared_bytes + count_bytes);
+    prof_bytes(c, K_TABLES_WRITE, shared_bytes + write_bytes);
   }
+  GEM_HIP_CHECK(hipMemcpyAsync(dev, stage, nt * sizeof(TableDesc), hipMemcpyHostToDevice, s));
+  R.pass(true);
   GEM_HIP_CHECK(hipEventRecord(c->ev[3], s));
-  GEM_HIP_CHECK(hipStreamSynchronize(s));
-  prof_flush(c);
-  float ms = 0;
-  GEM_HIP_CHECK(hipEventElapsedTime(&ms, c->ev[2], c->ev[3]));
-  c->times.tables_ms = ms;
+  c->tables_timed = true;
   Qd.tabled = true;
+  if (wait || c->prof.on) {
+    GEM_HIP_CHECK(hipStreamSynchronize(s));
+    prof_flush(c);
+    settle_times(c);
+  }
 }
 
 }  // namespace gemd

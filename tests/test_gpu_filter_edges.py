@@ -49,3 +49,24 @@ def test_candidates_and_positions(num_labels):
                 want = np.searchsorted(lists[0], probe)
                 hit = np.isin(probe, lists[0])
                 assert np.array_equal(ctx.position_lookup(0, probe), np.where(hit, want, 0xFFFFFFFF))
+
+
+@pytest.mark.parametrize("num_labels", [3, 300])
+def test_edge_tables(num_labels):
+    """Offsets and values over several scan chunks (lists past 4,096
+    candidates) and rows of one to 64 pieces."""
+    g = _graph(num_labels)
+    with GemContext(0) as ctx:
+        ctx.load_data(g)
+        q = next(_queries(num_labels))
+        num, _ = ctx.filter(q, want_lists=False)
+        sizes = ctx.build_edge_tables()
+        assert np.array_equal(sizes, oracle.table_sizes(g, q))
+        for d in range(2 * q.num_e):
+            u = int(q.edges[d // 2][d % 2])
+            ref = oracle.edge_table(g, q, d, int(num[u]), int(sizes[d]))
+            if ref is None:  # keyed on a leaf
+                assert sizes[d] == 0
+                continue
+            off, val = ctx.read_edge_table(d, int(num[u]), int(sizes[d]))
+            assert np.array_equal(off, ref[0]) and np.array_equal(val, ref[2])
