@@ -29,9 +29,16 @@ namespace gemd {
 
 constexpr uint32_t TAB_WAVES = 4;
 
+// Candidates a wave of k_tables takes: a list of 64 rows of up to 256 slots is
+// walked in up to 128 dependent steps, so builds of few candidates take fewer
+// rows per wave until the chip has waves enough (about 8 per SIMD).  64 rows
+// per wave: 68 us a pass for queries of a few thousand candidates on 2^18.
+constexpr uint32_t MIN_ROWS = 8, ENOUGH_WAVES = 8192;
+
 struct TableJob {
   uint32_t nu;
   uint32_t W;
+  uint32_t rows;  // candidates per wave
   uint32_t wave_start[GEM_MAX_QV + 1];
   uint32_t ncan[GEM_MAX_QV];
   uint64_t can_off[GEM_MAX_QV];
@@ -88,10 +95,10 @@ k_tables(const TableGraph G, const uint32_t *__restrict__ can, const uint64_t *_
   if (gw >= job.wave_start[job.nu]) return;
   uint32_t ju = 0;
   while (job.wave_start[ju + 1] <= gw) ++ju;
-  const uint32_t row_base = (gw - job.wave_start[ju]) * 64;
+  const uint32_t row_base = (gw - job.wave_start[ju]) * job.rows;
   const uint32_t ncan = job.ncan[ju];
   const uint32_t i = row_base + l;
-  const bool valid = i < ncan;
+  const bool valid = l < job.rows && i < ncan;
   uint64_t o0 = 0;
   uint32_t len = 0, full_len = 0;
   if (valid) {
@@ -359,7 +366,6 @@ void run_tables(gem_ctx *c, QueryDev &Qd, bool wait) {
   for (uint32_t u = 0; u < Q.nv; ++u) {
     if (Q.deg[u] == 1) continue;  // leaves key no table (unifiedTrie.cu:1045,1095)
     const uint32_t ju = job.nu++;
-    job.wave_start[ju] = R.waves;
     job.ncan[ju] = Qd.ncan[u];
     job.can_off[ju] = Qd.can_off[u];
     job.tab0[ju] = (uint32_t)desc_tab.size();
@@ -374,12 +380,19 @@ void run_tables(gem_ctx *c, QueryDev &Qd, bool wait) {
       job.nd[ju]++;
     }
     R.ndmax = std::max(R.ndmax, job.nd[ju]);
-    R.waves += (Qd.ncan[u] + 63) / 64;
     auto it = G.label_id.find(Q.lab[u]);
     if (it != G.label_id.end()) {
       R.rows_bound += std::min<uint64_t>(G.label_long[it->second], Qd.ncan[u]);
       R.pieces_bound += G.label_chunks[it->second];
     }
+  }
+  for (job.rows = 64;; job.rows /= 2) {
+    R.waves = 0;
+    for (uint32_t ju = 0; ju < job.nu; ++ju) {
+      job.wave_start[ju] = R.waves;
+      R.waves += (job.ncan[ju] + job.rows - 1) / job.rows;
+    }
+    if (job.rows == MIN_ROWS || R.waves >= ENOUGH_WAVES / 2) break;
   }
   job.wave_start[job.nu] = R.waves;
   // Parameters of the build: one staging block, one device block: the tables,
