@@ -51,6 +51,8 @@ struct Error {
 // cached block and empty segment and retries.
 void *pool_alloc(size_t n, hipStream_t s, size_t *cls);
 void pool_free(void *p, size_t cls, hipStream_t s);
+// The block's size after all but its first n bytes went back (large blocks).
+size_t pool_shrink(void *p, size_t cls, size_t n, hipStream_t s);
 // hipFree every cached block of stream s (its work must have finished).
 void pool_release(hipStream_t s);
 // Bytes the allocator holds that no buffer uses and that a large request can
@@ -88,6 +90,12 @@ struct DevBuf {
     s = stream;
     if (n == 0) return;
     p = pool_alloc(n, stream, &cls);
+    bytes = n;
+  }
+  // Keep the first n bytes, in place.
+  void shrink(size_t n) {
+    if (!p || n >= bytes) return;
+    cls = pool_shrink(p, cls, n, s);
     bytes = n;
   }
   void reset() {

@@ -77,6 +77,11 @@ gemh::PoolStats pool_stats(bool reset_peak) {
   return st;
 }
 
+size_t pool_shrink(void *p, size_t cls, size_t n, hipStream_t s) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  return core().shrink(p, cls, n, s);
+}
+
 void pool_release(hipStream_t s) {
   std::lock_guard<std::mutex> lk(g_mu);
   core().release_stream(s);

@@ -841,13 +841,26 @@ __global__ void __launch_bounds__(VB) k_vmark(const VItem *__restrict__ items, u
     CLevel &L = *(CLevel *)it.lv;
     const uint64_t r = it.row_begin + (g - blk_prefix[t]) * VB + threadIdx.x;
     // k_vcount1 reads list values only to remove equal-label columns
-    if (r >= it.row_end || (count_only && L.ndup == 0)) continue;
+    if (count_only && L.ndup == 0) continue;
+    const bool valid = r < it.row_end;
     const uint32_t *row = it.rows + r * it.k;
     const uint32_t gt = (uint32_t)(base + g - wa);
     for (uint32_t j = 0; j < L.nb; ++j) {
-      const uint32_t b = L.gblk[j] + (ldg(row + L.key_col[j]) >> L.kshift[j]);
-      if (first[b] > gt) atomicMin(&first[b], gt);
-      if (last[b] < gt) atomicMax(&last[b], gt);
+      const uint32_t b = valid ? L.gblk[j] + (ldg(row + L.key_col[j]) >> L.kshift[j]) : 0;
+      // one lane per distinct block of the wave's rows marks it (rows of one
+      // parent mostly share theirs), and only where the mark moves
+      uint64_t rest = __ballot(valid);
+      bool lead = false;
+      while (rest) {
+        const uint32_t x = (uint32_t)__builtin_ctzll(rest);
+        const uint64_t same = __ballot(valid && b == readlane_u32(b, x));
+        if (threadIdx.x % 64 == x) lead = true;
+        rest &= ~same;
+      }
+      if (lead) {
+        if (__hip_atomic_load(&first[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > gt) atomicMin(&first[b], gt);
+        if (__hip_atomic_load(&last[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < gt) atomicMax(&last[b], gt);
+      }
     }
   }
 }
@@ -1283,10 +1296,8 @@ struct HipSchedBackend {
   }
 
   std::shared_ptr<LevelBuf> shrink(const std::shared_ptr<LevelBuf> &from, uint64_t bytes) {
-    auto b = std::make_shared<LevelBuf>();
-    b->alloc(bytes, c->stream);
-    GEM_HIP_CHECK(hipMemcpyAsync(b->p, from->p, bytes, hipMemcpyDeviceToDevice, c->stream));
-    return b;
+    from->shrink(bytes);
+    return from;
   }
 
   VItem vitem(const Item &x) const {

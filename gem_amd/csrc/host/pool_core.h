@@ -6,7 +6,8 @@
 //     at least), freed blocks parked on a free list per (stream, class);
 //   * larger requests: segments of `seg` bytes (or one of the request's size
 //     when larger, or when a whole segment is refused) carved best-fit in
-//     `unit`-byte units, freed ranges merged with their free neighbours.
+//     `unit`-byte units, freed ranges merged with their free neighbours; an
+//     allocation may give back its tail in place (shrink).
 // Memory freed by one stream is only reused by that stream (all device work
 // of a context runs on its one stream, so a range freed after its last use
 // was enqueued can serve later work there without a wait).  When the backing
@@ -109,9 +110,9 @@ class PoolCore {
     return p;
   }
 
-  void free(void *ptr, size_t cls, const void *stream) {
+  void free(void *ptr, size_t cls, const void *stream, bool carved = false) {
     if (!ptr) return;
-    if (cls < big_) {
+    if (cls < big_ && !carved) {
       st_.in_use -= cls;
       small_[{stream, cls}].push_back(ptr);
       st_.cached_small += cls;
@@ -141,6 +142,15 @@ class PoolCore {
       }
     }
     g.add_free(off, len);
+  }
+
+  // Keep the first n bytes of a carved allocation and free the rest of its
+  // range; the block's new size (cls unchanged: nothing to give back).
+  size_t shrink(void *ptr, size_t cls, size_t n, const void *stream) {
+    const size_t c = std::max(big_, (n + unit_ - 1) / unit_ * unit_);
+    if (!ptr || cls < big_ || c >= cls) return cls;
+    free(static_cast<char *>(ptr) + c, cls - c, stream, true);
+    return c;
   }
 
   // Return parked small blocks and empty segments to the backing allocator

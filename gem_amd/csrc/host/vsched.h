@@ -62,7 +62,7 @@ struct SchedConfig {
   uint64_t max_chunk = 4ull << 30;       // largest output buffer of one query in one iteration
   uint64_t force_chunk = 0;              // past the budget (see above); 0 = budget / 32
   uint64_t final_piece = 1ull << 26;     // least output bound of a capped final-level piece
-  uint64_t shrink_min = 4ull << 20;      // outputs at least this large move when half unused
+  uint64_t shrink_min = 4ull << 20;      // outputs at least this large are cut when half unused
   // queries running at once (0 = all): the others wait in index order and
   // start as running ones end (continuous admission; a query's first level
   // is seeded when it starts)
@@ -224,7 +224,8 @@ inline int plan_chunks(const std::vector<ChunkCand> &cand, uint64_t left, uint64
 //   // rows written per write item, embeddings counted per final item
 //   void extend(const std::vector<SItem<Buf>> &wr, const std::vector<SItem<Buf>> &fin,
 //               std::vector<uint64_t> *got_wr, std::vector<uint64_t> *got_fin);
-//   // a buffer of `bytes` holding the first `bytes` of `from`
+//   // a buffer of `bytes` holding the first `bytes` of `from` (which is not
+//   // used again; it may be `from` itself, cut short)
 //   std::shared_ptr<Buf> shrink(const std::shared_ptr<Buf> &from, uint64_t bytes);
 //   void on_iteration(uint64_t iter, size_t active, uint64_t live, uint64_t budget);
 //   // query q's attempt went past its limit and its stack is empty: seed it
@@ -487,9 +488,9 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
         std::shared_ptr<Buf> rows = std::move(outs[t]);
         if (!got) continue;  // the buffer goes back now
         // the output was allocated for the length pass's bound; when fewer
-        // than half of those rows survived, they move to a buffer of their
-        // size, and the bound-sized one goes back at once (pending rows are
-        // what the budget is charged with)
+        // than half of those rows survived, it is cut to their size, and the
+        // rest goes back at once (pending rows are what the budget is charged
+        // with)
         const uint64_t rb = 4ull * S.cols(it.level + 1);
         if (2 * got <= it.out_rows && it.out_rows * rb >= cfg.shrink_min) rows = be.shrink(rows, got * rb);
         SLevel<Buf> L;
