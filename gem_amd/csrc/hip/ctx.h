@@ -443,6 +443,9 @@ struct JoinOut {
 struct EmbSink {
   virtual ~EmbSink() = default;
   virtual bool put(const uint32_t *rows, uint64_t n, uint32_t nv) = 0;
+  // Where the sink wants the next n rows (put is then called with that
+  // address); null: anywhere.
+  virtual uint32_t *place(uint64_t, uint32_t) { return nullptr; }
 };
 // The plain join with its final rows going to `sink` (count cap off); null
 // sink: count only, capped at cap.
@@ -465,8 +468,9 @@ void run_match_relaxed(gem_ctx *c, const gem_query_view *q, uint32_t threshold,
 
 // ------------------------------------------------------------------ scans
 // Exclusive scan of n u64 values in place-free form: out[i] = sum(in[0..i)),
-// out[n] = total.  Returns nothing; caller reads out[n] if needed.
-void scan_u64(gem_ctx *c, const uint64_t *d_in, uint64_t *d_out, uint64_t n);
+// out[n] = total, which also goes to *d_total when given (device or mapped host
+// memory).
+void scan_u64(gem_ctx *c, const uint64_t *d_in, uint64_t *d_out, uint64_t n, uint64_t *d_total = nullptr);
 // Independent in-place exclusive scans of u64 arrays p[0..n) (the total goes
 // to p[n] and to d_totals[i], device or mapped host memory); first_chunk: the
 // chunks (scan_chunks) of the segments before, `chunks` those of all.

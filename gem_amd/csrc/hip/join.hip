@@ -19,7 +19,10 @@
 // Count pass (one thread per row, 256-row blocks) -> block scan -> write pass
 // (waves walk their 64 rows' lists 64 items per step, ballot compaction).  A
 // level whose output would exceed the level budget is split into block ranges
-// and each range is finished depth-first, so memory stays bounded.
+// and each range is finished depth-first, so memory stays bounded.  When only
+// the count is wanted, a level's rows hold only the columns that a later step
+// reads, and the steps run as one chain of launches with the row counts on the
+// device (k_chain), as far as the levels stay below CHAIN_ROWS rows.
 #include <algorithm>
 #include <cstring>
 #include <functional>
@@ -32,10 +35,14 @@ namespace gemd {
 constexpr uint32_t JB = 256;  // rows per block
 constexpr uint32_t JW = JB / 64;
 
+constexpr uint8_t JCOL_NEW = 0xFF;
+
 struct StepArgs {
-  const uint32_t *rows;
+  const uint32_t *rows;  // null: row r is the single column r
   uint64_t nrows;
   uint32_t k;        // input row width
+  uint32_t ko;       // output row width, and the input column each output
+  uint8_t src[GEM_MAX_QV];  // column is copied from (JCOL_NEW: the new position)
   uint32_t key_col;  // column whose position keys the table
   uint32_t val_col;  // select: tested column
   const uint64_t *toff;
@@ -64,19 +71,22 @@ __device__ __forceinline__ uint64_t search_bytes(uint64_t len) {
   return 4ull * (cl + 1);
 }
 
+__device__ __forceinline__ uint32_t col_of(const StepArgs &a, uint64_t r, uint32_t c) {
+  return a.rows ? a.rows[r * a.k + c] : (uint32_t)r;
+}
+
 // Count of row r's expansion: list length minus equal-label columns that occur
 // in the list.  Also returns the list start/length, (optionally) the dup
 // positions, and the search bytes spent.
 __device__ __forceinline__ uint64_t expand_count_row(const StepArgs &a, uint64_t r, uint64_t *o0, uint64_t *len,
                                                      uint32_t *dup_pos, uint64_t *sbytes) {
-  const uint32_t *row = a.rows + r * a.k;
-  const uint32_t p = row[a.key_col];
+  const uint32_t p = col_of(a, r, a.key_col);
   const uint64_t b = a.toff[p], e = a.toff[p + 1];
   *o0 = b;
   *len = e - b;
   uint64_t cnt = e - b;
   for (uint32_t c = 0; c < a.ndup; ++c) {
-    const uint32_t vid = a.dup_can[c][row[a.dup_col[c]]];
+    const uint32_t vid = a.dup_can[c][col_of(a, r, a.dup_col[c])];
     const uint32_t pos = position_in(a.bm_new, a.rank_new, vid);
     if (dup_pos) dup_pos[c] = pos;
     if (pos != NOT_FOUND) {
@@ -88,8 +98,7 @@ __device__ __forceinline__ uint64_t expand_count_row(const StepArgs &a, uint64_t
 }
 
 __device__ __forceinline__ bool select_row(const StepArgs &a, uint64_t r, uint64_t *len) {
-  const uint32_t *row = a.rows + r * a.k;
-  const uint32_t p = row[a.key_col], v = row[a.val_col];
+  const uint32_t p = col_of(a, r, a.key_col), v = col_of(a, r, a.val_col);
   const uint64_t b = a.toff[p], e = a.toff[p + 1];
   *len = e - b;
   return sorted_contains(a.tval + b, e - b, v);
@@ -165,15 +174,56 @@ __global__ void __launch_bounds__(JB) k_select_write(const StepArgs a, const uin
   const uint64_t ex = block_excl_u64(keep ? 1 : 0, sm);
   if (keep) {
     const uint64_t o = block_off[b] - out_base + ex;
-    const uint32_t *src = a.rows + r * a.k;
-    uint32_t *dst = out + o * a.k;
-    for (uint32_t c = 0; c < a.k; ++c) dst[c] = src[c];
+    uint32_t *dst = out + o * a.ko;
+    for (uint32_t c = 0; c < a.ko; ++c) dst[c] = col_of(a, r, a.src[c]);
   }
 }
 
 __device__ __forceinline__ uint64_t lanes_between(uint32_t lo, uint32_t hi) {  // bits [lo, hi]
   const uint64_t h = (hi >= 63) ? ~0ull : ((1ull << (hi + 1)) - 1);
   return h & ~((1ull << lo) - 1);
+}
+
+// A wave writes the extensions of its 64 rows [row0, row0 + 64): the lists are
+// walked 64 items per group; st = starts of the rows' lists in the flattened
+// range (st[64] = total), ob = their first entries, ro = their first output
+// rows, dups = the equal-label columns' positions (ndup per row).  Row order
+// and list order are kept.
+__device__ __forceinline__ void write_extensions(const StepArgs &a, uint64_t row0, const uint32_t *st,
+                                                 const uint64_t *ob, const uint64_t *ro, const uint32_t *dups,
+                                                 uint32_t *out) {
+  const uint32_t l = lane_id(), total = st[64];
+  uint32_t carry = 0;
+  for (uint32_t t = 0; t < total; t += 64) {
+    const uint32_t item = t + l;
+    const bool iv = item < total;
+    const uint32_t row = iv ? seg_of(st, item) : 63;
+    const uint32_t rs = st[row], re = st[row + 1];
+    const uint32_t last = min(63u, total - 1 - t);
+    const uint32_t first = readlane_u32(row, 0);
+    bool keep = false;
+    uint32_t val = 0;
+    if (iv) {
+      val = a.tval[ob[row] + (item - rs)];
+      keep = true;
+      const uint32_t *rdp = dups + (uint64_t)row * a.ndup;
+      for (uint32_t c = 0; c < a.ndup; ++c)
+        if (rdp[c] == val) keep = false;
+    }
+    const uint64_t m = __ballot(keep);
+    const uint32_t seg_lo = rs > t ? rs - t : 0;
+    const uint32_t seg_hi = (re < t + 64 ? re - t : 64) - 1;
+    const bool row_done = re <= t + 64;
+    const uint32_t before = (row == first) ? carry : 0;
+    if (keep) {
+      const uint64_t below = lanes_between(seg_lo, l) & ~(1ull << l);
+      const uint64_t o = ro[row] + before + (uint64_t)__popcll(m & below);
+      uint32_t *dst = out + o * a.ko;
+      for (uint32_t c = 0; c < a.ko; ++c) dst[c] = a.src[c] == JCOL_NEW ? val : col_of(a, row0 + row, a.src[c]);
+    }
+    const uint32_t tot_row = iv ? before + (uint32_t)__popcll(m & lanes_between(seg_lo, seg_hi)) : 0;
+    carry = readlane_u32(row_done ? 0u : tot_row, last);
+  }
 }
 
 // Expand write.  Dynamic LDS: JW * 64 * ndup u32 dup positions.
@@ -201,41 +251,82 @@ __global__ void __launch_bounds__(JB) k_expand_write(const StepArgs a, const uin
   ob[w][l] = o0;
   ro[w][l] = block_off[b] - out_base + ex;
   __syncthreads();
-  const uint64_t wave_row0 = (uint64_t)b * JB + w * 64;
-  const uint32_t k = a.k;
-  uint32_t carry = 0;
-  for (uint32_t t = 0; t < total; t += 64) {
-    const uint32_t item = t + l;
-    const bool iv = item < total;
-    const uint32_t row = iv ? seg_of(st[w], item) : 63;
-    const uint32_t rs = st[w][row], re = st[w][row + 1];
-    const uint32_t last = min(63u, total - 1 - t);
-    const uint32_t row0 = readlane_u32(row, 0);
-    bool keep = false;
-    uint32_t val = 0;
-    if (iv) {
-      val = a.tval[ob[w][row] + (item - rs)];
-      keep = true;
-      const uint32_t *rdp = dup_lds + (uint64_t)(w * 64 + row) * a.ndup;
-      for (uint32_t c = 0; c < a.ndup; ++c)
-        if (rdp[c] == val) keep = false;
+  write_extensions(a, (uint64_t)b * JB + w * 64, st[w], ob[w], ro[w], dup_lds + (uint64_t)w * 64 * a.ndup, out);
+}
+
+// One step of the count-only chain: the level's row count comes from the step
+// before (*n_in) and goes to the next (*n_out); output places are handed out by
+// one atomic per 64 rows (a count does not depend on row order).  A level past
+// its room (cap_in, cap_out rows) is counted but not written whole, and the
+// steps after it do nothing: the host goes on from it with the count / scan /
+// write passes.  A step of those costs three launches, a copy and two waits,
+// 40 us however few the rows; a chained one 5 to 8 us.  (A 5-vertex query on
+// 10,000 vertices: 246 us, chained 128.)
+// FINAL: *n_out += the count.  Dynamic LDS as k_expand_write (expand).
+constexpr uint32_t CHAIN_BLOCKS = 1024;
+constexpr uint64_t CHAIN_ROWS = 1ull << 18, CHAIN_LEAST = 1ull << 13;
+template <bool SELECT, bool FINAL>
+__global__ void __launch_bounds__(JB) k_chain(const StepArgs a, const unsigned long long *__restrict__ n_in,
+                                             uint64_t cap_in, unsigned long long *__restrict__ n_out,
+                                             uint64_t cap_out, uint32_t *__restrict__ out) {
+  __shared__ uint32_t st[JW][65];
+  __shared__ uint64_t ob[JW][64];
+  __shared__ uint64_t ro[JW][64];
+  extern __shared__ uint32_t dup_lds[];
+  const uint64_t n = *n_in;
+  if (n > cap_in) return;
+  const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
+  uint64_t sum = 0;
+  for (uint64_t row0 = ((uint64_t)blockIdx.x * JW + w) * 64; row0 < n; row0 += (uint64_t)gridDim.x * JB) {
+    const uint64_t r = row0 + l;
+    uint64_t cnt = 0, o0 = 0, len = 0, sb = 0;
+    uint32_t *dp = dup_lds + (uint64_t)(w * 64 + l) * a.ndup;
+    if (r < n) {
+      if (SELECT)
+        cnt = select_row(a, r, &len) ? 1 : 0;
+      else
+        cnt = expand_count_row(a, r, &o0, &len, FINAL ? nullptr : dp, &sb);
     }
-    const uint64_t m = __ballot(keep);
-    const uint32_t seg_lo = rs > t ? rs - t : 0;
-    const uint32_t seg_hi = (re < t + 64 ? re - t : 64) - 1;
-    const bool row_done = re <= t + 64;
-    const uint32_t before = (row == row0) ? carry : 0;
-    if (keep) {
-      const uint64_t below = lanes_between(seg_lo, l) & ~(1ull << l);
-      const uint64_t o = ro[w][row] + before + (uint64_t)__popcll(m & below);
-      const uint32_t *src = a.rows + (wave_row0 + row) * k;
-      uint32_t *dst = out + o * (k + 1);
-      for (uint32_t c = 0; c < k; ++c) dst[c] = src[c];
-      dst[k] = val;
+    if (FINAL) {
+      sum += cnt;
+      continue;
     }
-    const uint32_t tot_row = iv ? before + (uint32_t)__popcll(m & lanes_between(seg_lo, seg_hi)) : 0;
-    carry = readlane_u32(row_done ? 0u : tot_row, last);
+    const uint64_t incl = wave_incl_scan_u64(cnt), all = readlane_u64(incl, 63);
+    if (!all) continue;
+    uint64_t base = 0;
+    if (l == 0) base = atomicAdd(n_out, (unsigned long long)all);
+    base = readlane_u64(base, 0);
+    if (base + all > cap_out) continue;
+    if (SELECT) {
+      if (cnt) {
+        uint32_t *dst = out + (base + incl - 1) * a.ko;
+        for (uint32_t c = 0; c < a.ko; ++c) dst[c] = col_of(a, r, a.src[c]);
+      }
+      continue;
+    }
+    const uint32_t il = wave_incl_scan_u32((uint32_t)len);
+    st[w][l] = il - (uint32_t)len;
+    if (l == 63) st[w][64] = il;
+    ob[w][l] = o0;
+    ro[w][l] = base + incl - cnt;
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    write_extensions(a, row0, st[w], ob[w], ro[w], dup_lds + (uint64_t)w * 64 * a.ndup, out);
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   }
+  if (FINAL) {
+    sum = wave_sum_u64(sum);
+    if (l == 0 && sum) atomicAdd(n_out, (unsigned long long)sum);
+  }
+}
+
+// Level counts of a chain: n[0] = first, the rest zero; and to the host.
+__global__ void k_chain_init(unsigned long long *n, uint32_t steps, uint64_t first) {
+  for (uint32_t i = threadIdx.x; i <= steps; i += blockDim.x) n[i] = i ? 0 : first;
+}
+__global__ void k_chain_done(const unsigned long long *__restrict__ n, uint32_t steps, uint64_t *__restrict__ host) {
+  for (uint32_t i = threadIdx.x; i <= steps; i += blockDim.x) host[i] = n[i];
 }
 
 // Final rows (positions) -> vertex ids in query-vertex order.
@@ -249,17 +340,15 @@ __global__ void k_rows_to_ids(const uint32_t *__restrict__ rows, uint64_t nrows,
   out[r * nv + col_u[c]] = col_can[c][rows[i]];
 }
 
-__global__ void k_iota(uint32_t *p, uint64_t n) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = (uint32_t)i;
-}
-
 struct JStep {
   bool select;
   uint32_t table;  // directed edge
   uint32_t key_col, val_col, new_u;
   uint32_t ndup;
   uint32_t dup_col[GEM_MAX_QV];
+  // query columns of the rows the step reads, and of those it writes
+  uint32_t ncols;
+  std::vector<uint32_t> in, out;
 };
 
 class JoinRunner {
@@ -284,6 +373,25 @@ class JoinRunner {
       for (uint32_t i = 0; i < ps.num_dup; ++i) s.dup_col[i] = ps.dup_cols[i];
       steps_.push_back(s);
     }
+    // columns each step's rows hold: all of them for a sink, else those that
+    // this step or a later one reads
+    std::vector<uint32_t> last(plan.col_u.size(), 0);
+    for (uint32_t i = 0; i < steps_.size(); ++i) {
+      const JStep &st = steps_[i];
+      last[st.key_col] = i;
+      if (st.select) last[st.val_col] = i;
+      for (uint32_t d = 0; d < st.ndup; ++d) last[st.dup_col[d]] = i;
+    }
+    uint32_t ncols = 1;
+    for (uint32_t i = 0; i < steps_.size(); ++i) {
+      JStep &st = steps_[i];
+      st.ncols = ncols;
+      for (uint32_t c = 0; c < ncols; ++c)
+        if (sink_ || last[c] >= i) st.in.push_back(c);
+      if (!st.select) ++ncols;
+      for (uint32_t c = 0; c < ncols; ++c)
+        if (sink_ || last[c] > i) st.out.push_back(c);
+    }
     col_u_ = plan.col_u;
     rows_.assign(steps_.size(), 0);
     ms_.assign(steps_.size(), 0.0f);
@@ -294,20 +402,20 @@ class JoinRunner {
   void run(JoinOut *out) {
     hipStream_t s = c_->stream;
     d_aux_.alloc(24, s);
-    GEM_HIP_CHECK(hipMemsetAsync(d_aux_.p, 0, 24, s));
-    GEM_HIP_CHECK(hipEventCreate(&e0_));
-    GEM_HIP_CHECK(hipEventCreate(&e1_));
+    if (log_) {
+      GEM_HIP_CHECK(hipEventCreate(&e0_));
+      GEM_HIP_CHECK(hipEventCreate(&e1_));
+    }
     const uint32_t a = col_u_[0];
     const uint64_t n0 = Qd_.ncan[a];
-    DevBuf lvl;
-    lvl.alloc(std::max<uint64_t>(n0, 1) * 4, s);
     if (n0) {
-      k_iota<<<(uint32_t)((n0 + 255) / 256), 256, 0, s>>>(lvl.as<uint32_t>(), n0);
-      GEM_LAUNCH_CHECK("k_iota");
-      level(0, lvl.as<uint32_t>(), n0, 1);
+      if (!log_ && !sink_ && !c_->prof.on)
+        chain(n0);
+      else
+        level(0, nullptr, n0);
     }
-    (void)hipEventDestroy(e0_);
-    (void)hipEventDestroy(e1_);
+    if (e0_) (void)hipEventDestroy(e0_);
+    if (e1_) (void)hipEventDestroy(e1_);
     out->count = saturated_ ? cap_ : final_total_;
     out->saturated = saturated_;
     out->emb_written = emb_rows_;
@@ -353,13 +461,16 @@ class JoinRunner {
   std::vector<uint32_t> host_rows_;
   hipEvent_t e0_{}, e1_{};
 
-  StepArgs args(const JStep &st, const uint32_t *rows, uint64_t n, uint32_t k) {
+  StepArgs args(const JStep &st, const uint32_t *rows, uint64_t n) {
     StepArgs a{};
     a.rows = rows;
     a.nrows = n;
-    a.k = k;
-    a.key_col = st.key_col;
-    a.val_col = st.val_col;
+    a.k = (uint32_t)st.in.size();
+    a.ko = (uint32_t)st.out.size();
+    auto at = [&](uint32_t col) { return (uint32_t)(std::lower_bound(st.in.begin(), st.in.end(), col) - st.in.begin()); };
+    for (uint32_t c = 0; c < a.ko; ++c) a.src[c] = st.out[c] == st.ncols ? JCOL_NEW : (uint8_t)at(st.out[c]);
+    a.key_col = at(st.key_col);
+    if (st.select) a.val_col = at(st.val_col);
     const TableDev &T = Qd_.tab[st.table];
     if (!T.present) throw Error{GEM_E_STATE, "join step uses a table that was not built"};
     a.toff = T.off.as<uint64_t>();
@@ -370,22 +481,19 @@ class JoinRunner {
       a.bm_new = Qd_.bitmap.as<uint64_t>() + (uint64_t)st.new_u * Qd_.W;
       a.rank_new = Qd_.rank.as<uint32_t>() + (uint64_t)st.new_u * (Qd_.W + 1);
       for (uint32_t i = 0; i < st.ndup; ++i) {
-        a.dup_col[i] = st.dup_col[i];
+        a.dup_col[i] = at(st.dup_col[i]);
         a.dup_can[i] = Qd_.can.as<uint32_t>() + Qd_.can_off[col_u_[st.dup_col[i]]];
       }
     }
     return a;
   }
 
-  uint64_t read_u64(const uint64_t *d) {
-    uint64_t *h = pinned<uint64_t>(c_, 1);
-    GEM_HIP_CHECK(hipMemcpyAsync(h, d, 8, hipMemcpyDeviceToHost, c_->stream));
-    GEM_HIP_CHECK(hipStreamSynchronize(c_->stream));
-    return *h;
+  // Step times are taken for a log only (each waits for its step).
+  void time_begin() {
+    if (log_) GEM_HIP_CHECK(hipEventRecord(e0_, c_->stream));
   }
-
-  void time_begin() { GEM_HIP_CHECK(hipEventRecord(e0_, c_->stream)); }
   void time_end(uint32_t s) {
+    if (!log_) return;
     GEM_HIP_CHECK(hipEventRecord(e1_, c_->stream));
     GEM_HIP_CHECK(hipEventSynchronize(e1_));
     float ms = 0;
@@ -403,9 +511,73 @@ class JoinRunner {
     out3[2] = h[2];
   }
 
-  void final_count(uint32_t si, const uint32_t *rows, uint64_t n, uint32_t k) {
+  // Did the rows read so far, with n more, pass the work limit?
+  bool over_limit(uint64_t n) {
+    processed_ += n;
+    if (!work_limit_ || processed_ <= work_limit_) return false;
+    work_limited_ = true;
+    stop_ = true;
+    return true;
+  }
+
+  // The steps as one chain of launches from the identity rows of the first
+  // column, with one wait at its end; from the first level without room on
+  // (CHAIN_ROWS rows, or the level budget), level() takes over.
+  void chain(uint64_t n0) {
+    hipStream_t s = c_->stream;
+    const uint32_t ns = (uint32_t)steps_.size();
+    // rows a level has room for: many times its estimate by the tables' mean
+    // list lengths, so that small queries take small buffers
+    std::vector<uint64_t> cap(ns + 1, ~0ull);
+    size_t words[2] = {0, 0};
+    double est = (double)n0;
+    for (uint32_t i = 0; i + 1 < ns; ++i) {
+      const JStep &st = steps_[i];
+      const TableDev &T = Qd_.tab[st.table];
+      if (!st.select) est *= (double)T.size / std::max<double>(1, Qd_.ncan[T.key_u]);
+      cap[i + 1] = std::min<uint64_t>(CHAIN_ROWS, budget_ / (4ull * (st.select ? st.ncols : st.ncols + 1)));
+      cap[i + 1] = std::min<uint64_t>(cap[i + 1], std::max<uint64_t>(CHAIN_LEAST, (uint64_t)std::min(16 * est, 1e9)));
+      words[i & 1] = std::max<size_t>(words[i & 1], cap[i + 1] * st.out.size());
+    }
+    DevBuf buf[2], dn;
+    for (int i = 0; i < 2; ++i) buf[i].alloc(words[i] * 4, s);
+    dn.alloc((ns + 1) * 8, s);
+    auto *n = dn.as<unsigned long long>();
+    k_chain_init<<<1, 64, 0, s>>>(n, ns, n0);
+    for (uint32_t i = 0; i < ns; ++i) {
+      const JStep &st = steps_[i];
+      const uint32_t *rows = i ? buf[(i - 1) & 1].as<uint32_t>() : nullptr;
+      uint32_t *out = buf[i & 1].as<uint32_t>();
+      const StepArgs a = args(st, rows, 0);
+      const bool last = i + 1 == ns;
+      const size_t lds = last || st.select ? 0 : (size_t)JW * 64 * st.ndup * 4;
+      const uint64_t most = i ? cap[i] : n0;
+      const uint32_t grid = (uint32_t)std::min<uint64_t>((most + JB - 1) / JB, CHAIN_BLOCKS);
+      auto kernel = st.select ? (last ? k_chain<true, true> : k_chain<true, false>)
+                              : (last ? k_chain<false, true> : k_chain<false, false>);
+      kernel<<<grid, JB, lds, s>>>(a, n + i, cap[i], n + i + 1, cap[i + 1], out);
+    }
+    uint64_t *h = pinned<uint64_t>(c_, ns + 1);
+    k_chain_done<<<1, 64, 0, s>>>(n, ns, pinned_dev(c_, h));
+    GEM_LAUNCH_CHECK("k_chain");
+    GEM_HIP_CHECK(hipStreamSynchronize(s));
+    const std::vector<uint64_t> got(h, h + ns + 1);
+    for (uint32_t i = 0; i < ns; ++i) {
+      if (!got[i]) return;
+      if (got[i + 1] > cap[i + 1]) {  // no room: step i again, the other way
+        level(i, i ? buf[(i - 1) & 1].as<uint32_t>() : nullptr, got[i]);
+        return;
+      }
+      if (over_limit(got[i])) return;
+    }
+    final_total_ = got[ns];
+    if (cap_ && final_total_ > cap_) saturated_ = true;
+  }
+
+  void final_count(uint32_t si, const uint32_t *rows, uint64_t n) {
     const JStep &st = steps_[si];
-    StepArgs a = args(st, rows, n, k);
+    StepArgs a = args(st, rows, n);
+    const uint32_t k = a.k;
     const uint32_t nb = (uint32_t)((n + JB - 1) / JB);
     const int prof = c_->prof.on ? 1 : 0;
     time_begin();
@@ -449,33 +621,32 @@ class JoinRunner {
     k_rows_to_ids<<<(uint32_t)((tot + 255) / 256), 256, 0, s>>>(rows, n, k, dcc.as<const uint32_t *>(),
                                                                  dcu.as<uint32_t>(), nv, dout.as<uint32_t>());
     GEM_LAUNCH_CHECK("k_rows_to_ids");
-    host_rows_.resize(n * nv);
-    GEM_HIP_CHECK(hipMemcpyAsync(host_rows_.data(), dout.p, n * nv * 4, hipMemcpyDeviceToHost, s));
+    uint32_t *host = sink_->place(n, nv);
+    if (!host) {
+      host_rows_.resize(n * nv);
+      host = host_rows_.data();
+    }
+    GEM_HIP_CHECK(hipMemcpyAsync(host, dout.p, n * nv * 4, hipMemcpyDeviceToHost, s));
     GEM_HIP_CHECK(hipStreamSynchronize(s));
     emb_rows_ += n;
-    if (!sink_->put(host_rows_.data(), n, nv)) {
+    if (!sink_->put(host, n, nv)) {
       sink_stopped_ = true;
       stop_ = true;
     }
   }
 
-  // Apply step si to `n` rows of width k.
-  void level(uint32_t si, const uint32_t *rows, uint64_t n, uint32_t k) {
-    if (stop_ || n == 0) return;
-    processed_ += n;
-    if (work_limit_ && processed_ > work_limit_) {
-      work_limited_ = true;
-      stop_ = true;
-      return;
-    }
+  // Apply step si to `n` rows.
+  void level(uint32_t si, const uint32_t *rows, uint64_t n) {
+    if (stop_ || n == 0 || over_limit(n)) return;
     const JStep &st = steps_[si];
     const bool last = si + 1 == steps_.size();
     if (last && !sink_) {
-      final_count(si, rows, n, k);
+      final_count(si, rows, n);
       return;
     }
     hipStream_t s = c_->stream;
-    StepArgs a = args(st, rows, n, k);
+    StepArgs a = args(st, rows, n);
+    const uint32_t k = a.k;
     const uint32_t nb = (uint32_t)((n + JB - 1) / JB);
     const int prof = c_->prof.on ? 1 : 0;
     time_begin();
@@ -491,12 +662,15 @@ class JoinRunner {
         k_step_count<false, false><<<nb, JB, 0, s>>>(a, bc.as<uint64_t>(), d_aux_.as<unsigned long long>(), prof);
       GEM_LAUNCH_CHECK("k_step_count");
     }
-    scan_u64(c_, bc.as<uint64_t>(), bo.as<uint64_t>(), nb);
-    const uint64_t total = read_u64(bo.as<uint64_t>() + nb);
+    uint64_t *htot = pinned<uint64_t>(c_, 1);
+    scan_u64(c_, bc.as<uint64_t>(), bo.as<uint64_t>(), nb, pinned_dev(c_, htot));
+    GEM_HIP_CHECK(hipStreamSynchronize(s));
+    const uint64_t total = *htot;
     bc.reset();
     rows_[si] += total;
-    const uint32_t ko = st.select ? k : k + 1;
-    const uint64_t row_bytes = (uint64_t)ko * 4;
+    // the budget is charged for every column, held or not (so the chunks do
+    // not depend on which are)
+    const uint64_t row_bytes = 4ull * (st.select ? st.ncols : st.ncols + 1), out_bytes = 4ull * a.ko;
     double search_per_row = 0;
     if (prof) {
       uint64_t aux[3];
@@ -535,7 +709,7 @@ class JoinRunner {
       if (cnt == 0) continue;
       if (timed) time_begin();
       DevBuf outb;
-      outb.alloc(cnt * row_bytes, s);
+      outb.alloc(cnt * out_bytes, s);
       const uint32_t g = b1 - b0;
       if (prof) GEM_HIP_CHECK(hipMemsetAsync(d_aux_.p, 0, 24, s));
       {
@@ -556,15 +730,15 @@ class JoinRunner {
         read_aux(aux);
         const double nr = (double)std::min<uint64_t>((uint64_t)(b1 - b0) * JB, n - (uint64_t)b0 * JB);
         prof_bytes(c_, st.select ? K_SELECT_WRITE : K_EXPAND_WRITE,
-                   (4.0 * k + 8.0 + search_per_row) * nr + 4.0 * (double)aux[1] + (double)row_bytes * cnt);
+                   (4.0 * k + 8.0 + search_per_row) * nr + 4.0 * (double)aux[1] + (double)out_bytes * cnt);
       }
       time_end(si);
       timed = true;
       if (last) {
-        emit_rows(outb.as<uint32_t>(), cnt, ko);
+        emit_rows(outb.as<uint32_t>(), cnt, a.ko);
         final_total_ += cnt;
       } else {
-        level(si + 1, outb.as<uint32_t>(), cnt, ko);
+        level(si + 1, outb.as<uint32_t>(), cnt);
       }
     }
     if (!timed) time_end(si);
@@ -578,12 +752,16 @@ struct ArraySink : EmbSink {
   uint64_t cap, rows = 0;
   bool overflow = false;
   ArraySink(uint32_t *o, uint64_t c) : out(o), cap(c) {}
+  // rows that fit are copied from the device to their place in the array
+  uint32_t *place(uint64_t n, uint32_t nv) override {
+    return overflow || rows + n > cap ? nullptr : out + rows * nv;
+  }
   bool put(const uint32_t *r, uint64_t n, uint32_t nv) override {
     if (overflow || rows + n > cap) {
       overflow = true;
       return true;
     }
-    std::memcpy(out + rows * nv, r, n * nv * 4);
+    if (r != out + rows * nv) std::memcpy(out + rows * nv, r, n * nv * 4);
     rows += n;
     return true;
   }

@@ -24,8 +24,9 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_tile_sums_u64(const uint64_t *
   if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
-// one block: exclusive scan of m values, out[m] = total
-__global__ void __launch_bounds__(1024) k_scan_small_u64(const uint64_t *in, uint64_t m, uint64_t *out) {
+// one block: exclusive scan of m values, out[m] = total (and *total, when given)
+__global__ void __launch_bounds__(1024) k_scan_small_u64(const uint64_t *in, uint64_t m, uint64_t *out,
+                                                        uint64_t *total) {
   __shared__ uint64_t sm[16];
   uint64_t carry = 0;
   for (uint64_t b = 0; b < m; b += blockDim.x) {
@@ -36,7 +37,10 @@ __global__ void __launch_bounds__(1024) k_scan_small_u64(const uint64_t *in, uin
     if (idx < m) out[idx] = carry + ex;
     carry += tot;
   }
-  if (threadIdx.x == 0) out[m] = carry;
+  if (threadIdx.x == 0) {
+    out[m] = carry;
+    if (total) *total = carry;
+  }
 }
 
 __global__ void __launch_bounds__(SCAN_THREADS) k_tile_scan_u64(const uint64_t *in, uint64_t n, const uint64_t *tile_base,
@@ -64,9 +68,9 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_tile_scan_u64(const uint64_t *
   }
 }
 
-void scan_u64(gem_ctx *c, const uint64_t *d_in, uint64_t *d_out, uint64_t n) {
+void scan_u64(gem_ctx *c, const uint64_t *d_in, uint64_t *d_out, uint64_t n, uint64_t *d_total) {
   if (n <= 4 * 1024 * 16) {
-    k_scan_small_u64<<<1, 1024, 0, c->stream>>>(d_in, n, d_out);
+    k_scan_small_u64<<<1, 1024, 0, c->stream>>>(d_in, n, d_out, d_total);
     GEM_LAUNCH_CHECK("k_scan_small_u64");
     return;
   }
@@ -77,9 +81,9 @@ void scan_u64(gem_ctx *c, const uint64_t *d_in, uint64_t *d_out, uint64_t n) {
   k_tile_sums_u64<<<(uint32_t)tiles, SCAN_THREADS, 0, c->stream>>>(d_in, n, sums.as<uint64_t>());
   GEM_LAUNCH_CHECK("k_tile_sums_u64");
   if (tiles > 4 * 1024 * 16) {
-    scan_u64(c, sums.as<uint64_t>(), base.as<uint64_t>(), tiles);
+    scan_u64(c, sums.as<uint64_t>(), base.as<uint64_t>(), tiles, d_total);
   } else {
-    k_scan_small_u64<<<1, 1024, 0, c->stream>>>(sums.as<uint64_t>(), tiles, base.as<uint64_t>());
+    k_scan_small_u64<<<1, 1024, 0, c->stream>>>(sums.as<uint64_t>(), tiles, base.as<uint64_t>(), d_total);
     GEM_LAUNCH_CHECK("k_scan_small_u64");
   }
   k_tile_scan_u64<<<(uint32_t)tiles, SCAN_THREADS, 0, c->stream>>>(d_in, n, base.as<uint64_t>(), d_out);
