@@ -13,11 +13,11 @@ namespace gemd {
 // of the earlier vertices that this level or a later one reads (as the key of
 // a list or an equal-label column), in vertex-order; column numbers are places
 // in that row.  Device copy, one per (query, level).
-constexpr uint8_t COL_NEW = 0xFF;
+constexpr uint32_t COL_NEW = 0xFF;
 struct VLevel {
   uint32_t nb, ndup;
   uint32_t kout;             // columns of an output row:
-  uint8_t src[GEM_MAX_QV];   // the input column each is copied from, or COL_NEW for the new position
+  uint32_t src[GEM_MAX_QV];  // the input column each is copied from, or COL_NEW for the new position
   uint32_t key_col[GEM_MAX_QV];
   const uint64_t *toff[GEM_MAX_QV];
   const uint32_t *tval[GEM_MAX_QV];  // in-HBM tables
@@ -55,16 +55,29 @@ struct LevelBuf : DevBuf {
   mutable uint64_t unit0 = 0;
 };
 
-// A row whose driving list is too long for one wave: walked in chunks by
-// k_vext_heavy (t = item of the launch, r = row of the item's level).
+// A row whose driving list is too long for one wave: walked in pieces by
+// k_vext_heavy (t = item of the launch, r = row of the item's level, piece0 =
+// its first piece in the launch's piece table).
 struct HeavyRow {
   uint32_t t, len;
   uint64_t r;
+  uint32_t piece0, pad;
+};
+
+// The heavy rows of a walking launch: rows, the row of every piece (or
+// NOT_FOUND), and how many of each were asked for (more than the tables hold,
+// when rows were refused for lack of room).
+struct HeavyOut {
+  HeavyRow *rows;
+  uint32_t *piece_row;
+  unsigned int *ctr;  // rows, pieces
+  uint32_t threshold, piece;  // a list longer than `threshold` entries is cut into pieces of `piece`
 };
 
 // A work queue of the persistent kernels: WQ counters a cache line apart.
 constexpr uint32_t WQ = 8, WQ_STRIDE = 16, WQ_WORDS = WQ * WQ_STRIDE;
-// Counters of one task group of a streamed launch: 5 queues, 2 heavy-row counts.
+// Counters of one task group of a streamed launch: 5 queues, heavy rows and
+// pieces of two launches.
 constexpr uint32_t GROUP_WORDS = 5 * WQ_WORDS + WQ_STRIDE;
 
 struct VQueryState {

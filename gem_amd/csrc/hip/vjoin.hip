@@ -157,6 +157,21 @@ struct Runs {
   }
 };
 
+// Up to four consecutive words in one store.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3), aligned(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ void st_words(uint32_t *p, u32x4 x, uint32_t n) {
+  if (n == 4)
+    *(__attribute__((address_space(1))) u32x4 *)p = x;
+  else if (n == 3)
+    *(__attribute__((address_space(1))) u32x3 *)p = u32x3{x[0], x[1], x[2]};
+  else if (n == 2)
+    *(__attribute__((address_space(1))) u32x2 *)p = u32x2{x[0], x[1]};
+  else
+    stg(p, x[0]);
+}
+
 // Device address of the list of key p in backward table j (b = its first
 // offset): in HBM, or through the streamed tables' block map.
 template <bool OOC>
@@ -230,6 +245,29 @@ __device__ __forceinline__ void row_dups(CLevel &L, const uint32_t *row, uint32_
 // CU's 32 waves.
 constexpr uint32_t LDS_LISTS = 2, LDS_DUPS = 8;
 
+// Rows whose driving list has more than the threshold's entries go to
+// k_vext_heavy; at most HEAVY_CAP rows and PIECE_CAP pieces per launch (a row
+// that finds no room is walked by its own wave).
+constexpr uint32_t HEAVY_CAP = 1u << 20, PIECE_CAP = 1u << 22;
+
+// Sets aside the rows of the lanes that ask (want; list of len entries, row r
+// of item t); returns the lanes whose row was taken.  Rows and pieces are
+// numbered by two atomics per wave; pieces of refused rows are marked.
+__device__ __forceinline__ uint64_t set_aside(const HeavyOut &H, bool want, uint32_t t, uint32_t len, uint64_t r) {
+  const uint64_t m = __ballot(want);
+  if (!m) return 0;
+  const uint32_t n = want ? (len - 1) / H.piece + 1 : 0, incl = wave_incl_scan_u32(n);
+  uint32_t h = 0, c = 0;
+  if (lane_id() == 0) h = atomicAdd(&H.ctr[0], (uint32_t)__popcll(m));
+  if (lane_id() == 63) c = atomicAdd(&H.ctr[1], incl);
+  h = readlane_u32(h, 0) + rank_below(m);
+  c = readlane_u32(c, 63) + incl - n;
+  const bool taken = want && h < HEAVY_CAP && c <= PIECE_CAP && n <= PIECE_CAP - c;
+  if (taken) H.rows[h] = HeavyRow{t, len, r, c, 0};
+  for (uint32_t x = 0; x < n && c < PIECE_CAP && x < PIECE_CAP - c; ++x) H.piece_row[c + x] = taken ? h : NOT_FOUND;
+  return __ballot(taken);
+}
+
 // Each wave takes runs of 64-row units on its own (no block barrier): of equal
 // cost by the length pass's unit prefix, so that a run's rows are reserved
 // together however many units that takes, and no wave is left with a run of
@@ -255,15 +293,13 @@ __global__ void __launch_bounds__(VB) __attribute__((amdgpu_waves_per_eu(6)))
 k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, const uint64_t *__restrict__ blk_prefix,
        unsigned int *__restrict__ queue, uint32_t lcap, uint32_t dcap,
        unsigned long long *__restrict__ prof_items, unsigned long long *__restrict__ prof_out, uint64_t g_begin,
-       uint64_t g_end, HeavyRow *__restrict__ heavy, unsigned int *__restrict__ heavy_n, uint32_t heavy_cap,
-       uint32_t heavy_t) {
+       uint64_t g_end, const HeavyOut heavy) {
   const uint32_t nitems = *nitems_p;
   const uint64_t total = blk_prefix[nitems] < g_end ? blk_prefix[nitems] : g_end;
   if (g_begin >= total) return;
   __shared__ uint32_t st[VW][65];
   __shared__ uint64_t drv[VW][64];         // address of each row's driving list
   __shared__ uint8_t drv_j[VW][64];        // which of the row's lists drives
-  __shared__ uint8_t src[VW][GEM_MAX_QV];  // the item's output columns (VLevel::src)
   __shared__ uint64_t aside[VW][MAX_RUN];  // counted runs: rows of each task set aside as heavy
   __shared__ uint32_t sv_row[VW][VSTAGE];  // staged survivors: row in the item's range
   __shared__ uint32_t sv_val[VW][VSTAGE];  // and new value
@@ -280,15 +316,15 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
   const VLevel *lv = nullptr;
   const uint32_t *in = nullptr;  // first row of the item's range
   uint64_t nrow = 0;
-  uint32_t k = 1, ko = 1, inv = 0;  // columns read and written, 2^32 / ko rounded up
+  uint32_t k = 1, ko = 1;  // columns read and written
   uint64_t survivors = 0;  // final level: survivors of the item in hand
   uint32_t pend = 0;       // survivors staged in LDS, not yet written
   bool counted = false;    // output rows already reserved, from `cursor` on
   uint64_t cursor = 0;
-  // write the staged survivors: one reservation for all of them, then
-  // their rows as one run of consecutive words (word q is column q % ko of
-  // survivor q / ko: a parent column or the value), four words per lane in
-  // flight.  q / ko by the reciprocal rounded up: exact while q * ko < 2^32.
+  // Write the staged survivors: one reservation for all of them, then a lane
+  // per survivor copies its columns, up to four at a time and two survivors in
+  // flight.  (A lane per output word, whose column and survivor it looked up,
+  // spent 18 vector instructions a word.)
   auto flush = [&]() {
     CItem &I = ((CItem *)items)[t];
     if (FINAL) {
@@ -304,22 +340,33 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
       base = readlane_u64(base, 0);
     }
     const uint64_t room = I.out_cap > base ? I.out_cap - base : 0;
-    const uint32_t n = (pend < room ? pend : (uint32_t)room) * ko;
+    const uint32_t n = pend < room ? pend : (uint32_t)room;
+    CLevel &L = *(CLevel *)lv;
     uint32_t *dst = I.out + base * ko;
-    written += (uint64_t)n * 4;
-    for (uint32_t b = 0; b < n; b += 256) {
-      uint32_t x[4];
+    written += (uint64_t)n * 4 * ko;
+    for (uint32_t b = 0; b < n; b += 128) {
+      uint32_t v[2];
+      const uint32_t *row[2];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const uint32_t q = b + 64 * g + l < n ? b + 64 * g + l : n - 1;
-        const uint32_t i = ko > 1 ? __umulhi(q, inv) : q;
-        const uint32_t c = src[w][q - i * ko];
-        x[g] = ldg(in + (uint64_t)sv_row[w][i] * k + (c == COL_NEW ? 0 : c));
-        if (c == COL_NEW) x[g] = sv_val[w][i];
+      for (int g = 0; g < 2; ++g) {
+        const uint32_t i = b + 64 * g + l < n ? b + 64 * g + l : n - 1;
+        v[g] = sv_val[w][i];
+        row[g] = in + (uint64_t)sv_row[w][i] * k;
       }
+      for (uint32_t c = 0; c < ko; c += 4) {
+        const uint32_t m = ko - c < 4 ? ko - c : 4;
+        u32x4 x[2];
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        if (b + 64 * g + l < n) stg(dst + b + 64 * g + l, x[g]);
+        for (int e = 0; e < 4; ++e)
+          if (e < m) {
+            const uint32_t from = L.src[c + e];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) x[g][e] = from == COL_NEW ? v[g] : ldg(row[g] + from);
+          }
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+          if (b + 64 * g + l < n) st_words(dst + (size_t)(b + 64 * g + l) * ko + c, x[g], m);
+      }
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -333,14 +380,7 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
     CItem &I = ((CItem *)items)[t];
     lv = I.lv;
     k = I.k;
-    if (!FINAL) {
-      CLevel &L = *(CLevel *)lv;
-      ko = L.kout;
-      inv = 0xFFFFFFFFu / ko + 1;
-      if (l < ko) src[w][l] = L.src[l];
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    }
+    if (!FINAL) ko = ((CLevel *)lv)->kout;
     in = I.rows + I.row_begin * k;
     nrow = I.row_end - I.row_begin;
   };
@@ -366,19 +406,8 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
           len = (uint32_t)(o.y - o.x);
           addr = list_addr<OOC>(L, 0, p, o.x);
         }
-        const uint64_t hv = heavy ? __ballot(len > heavy_t) : 0;
-        uint64_t taken = 0;
-        if (hv) {
-          uint32_t h = 0;
-          if (l == 0) h = atomicAdd(heavy_n, (uint32_t)__popcll(hv));
-          h = readlane_u32(h, 0) + rank_below(hv);
-          const bool mine = ((hv >> l) & 1ull) && h < heavy_cap;
-          if (mine) {
-            heavy[h] = HeavyRow{t, len, ((CItem *)items)[t].row_begin + r};
-            len = 0;  // walked by k_vext_heavy
-          }
-          taken = __ballot(mine);
-        }
+        const uint64_t taken = set_aside(heavy, len > heavy.threshold, t, len, ((CItem *)items)[t].row_begin + r);
+        if ((taken >> l) & 1ull) len = 0;  // walked by k_vext_heavy
         if (l == 0) aside[w][j - j0] = taken;
         cnt += len;
         if (len)
@@ -426,17 +455,11 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
       }
       if (i < nb) row_lists<1>(L, row, i, take);
     }
-    const uint64_t hv = heavy && !counted ? __ballot(dlen > heavy_t) : 0;
-    if (!FINAL && counted && ((aside[w][j - j0] >> l) & 1ull)) dlen = 0;
-    if (hv) {
-      uint32_t h = 0;
-      if (l == 0) h = atomicAdd(heavy_n, (uint32_t)__popcll(hv));
-      h = readlane_u32(h, 0) + rank_below(hv);
-      if (((hv >> l) & 1ull) && h < heavy_cap) {
-        heavy[h] = HeavyRow{t, dlen, ((CItem *)items)[t].row_begin + rbase + l};
-        dlen = 0;  // walked by k_vext_heavy
-      }
-    }
+    const uint64_t taken =
+        !FINAL && counted
+            ? aside[w][j - j0]
+            : set_aside(heavy, dlen > heavy.threshold, t, dlen, ((CItem *)items)[t].row_begin + rbase + l);
+    if ((taken >> l) & 1ull) dlen = 0;  // walked by k_vext_heavy
     // a row with nothing to walk here (empty driving list, or set aside as a
     // heavy row) owns no item of the steps below, so its equal-label columns
     // are never read: skip their loads
@@ -576,25 +599,6 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
   if (prof_out && l == 0 && written) atomicAdd(prof_out, (unsigned long long)written);
 }
 
-// One block: chunk prefix of the heavy rows, pre[i] = sum over rows before i
-// of ceil(len / chunk), pre[n] = total, n = min(heavy_n, heavy_cap).
-__global__ void __launch_bounds__(1024) k_heavy_scan(const HeavyRow *__restrict__ heavy,
-                                                    const unsigned int *__restrict__ heavy_n, uint32_t heavy_cap,
-                                                    uint32_t chunk, uint64_t *__restrict__ pre) {
-  __shared__ uint64_t sm[16];
-  const uint32_t n = *heavy_n < heavy_cap ? *heavy_n : heavy_cap;
-  uint64_t carry = 0;
-  for (uint32_t b = 0; b < n; b += blockDim.x) {
-    const uint32_t i = b + threadIdx.x;
-    const uint64_t x = i < n ? (heavy[i].len + chunk - 1) / chunk : 0;
-    uint64_t ex;
-    const uint64_t tot = block_excl_scan_u64(x, &ex, sm);
-    if (i < n) pre[i] = carry + ex;
-    carry += tot;
-  }
-  if (threadIdx.x == 0) pre[n] = carry;
-}
-
 // Entries of a staged window of the first other list (k_vext_heavy).
 constexpr uint32_t HWIN = 512;
 
@@ -604,26 +608,24 @@ constexpr uint32_t HWIN = 512;
 // to the row's item output like the main pass's.
 template <bool FINAL, bool OOC>
 __global__ void __launch_bounds__(VB) __attribute__((amdgpu_waves_per_eu(8)))
-k_vext_heavy(const VItem *__restrict__ items, const HeavyRow *__restrict__ heavy,
-             const unsigned int *__restrict__ heavy_n, uint32_t heavy_cap, const uint64_t *__restrict__ pre,
-             unsigned int *__restrict__ queue, uint32_t chunk, unsigned long long *__restrict__ prof_items,
-             unsigned long long *__restrict__ prof_out) {
+k_vext_heavy(const VItem *__restrict__ items, const HeavyOut heavy, unsigned int *__restrict__ queue,
+             unsigned long long *__restrict__ prof_items, unsigned long long *__restrict__ prof_out) {
   __shared__ uint64_t oaddr[VW][GEM_MAX_QV];
   __shared__ uint32_t olen[VW][GEM_MAX_QV], dpos[VW][GEM_MAX_QV];
   __shared__ uint32_t wend[VW][64];   // window ends in the first other list
   __shared__ uint32_t win[VW][HWIN];  // staged window
   __shared__ uint32_t prow[VW][GEM_MAX_QV], hsv[VW][VSTAGE];  // parent row, staged surviving values
   const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64;
-  const uint32_t n = *heavy_n < heavy_cap ? *heavy_n : heavy_cap;
-  const uint64_t total = pre[n];
+  const uint32_t total = heavy.ctr[1] < PIECE_CAP ? heavy.ctr[1] : PIECE_CAP, chunk = heavy.piece;
   if (!total) return;
   uint64_t walked = 0, written = 0;
   const uint32_t bw = blockDim.x / 64;
   Runs runs(total, blockIdx.x * bw + w, gridDim.x * bw, 1, queue);  // a piece is long enough to ask for one at a time
   for (; runs.valid(); runs.next()) {
-    const uint64_t wt = runs.begin();
-    const uint32_t h = find_item(pre, n, wt);
-    const HeavyRow e = heavy[h];
+    const uint32_t wt = runs.begin();
+    const uint32_t h = __builtin_amdgcn_readfirstlane(heavy.piece_row[wt]);
+    if (h == NOT_FOUND) continue;
+    const HeavyRow e = heavy.rows[h];
     const VItem it = items[e.t];
     CLevel &L = *(CLevel *)it.lv;
     const uint32_t nb = L.nb, ndup = L.ndup;
@@ -665,17 +667,30 @@ k_vext_heavy(const VItem *__restrict__ items, const HeavyRow *__restrict__ heavy
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const uint64_t s0 = (uint64_t)(wt - pre[h]) * chunk;
+    const uint64_t s0 = (uint64_t)(wt - e.piece0) * chunk;
     const uint64_t s1 = s0 + chunk < dlen ? s0 + chunk : dlen;
     walked += s1 - s0;
     uint64_t survivors = 0;
     uint32_t pend = 0;  // surviving values staged, not yet written
+    // With no other list the piece's rows are known before it is walked, all
+    // entries but the equal-label columns' (as in k_vext): one reservation.
+    uint64_t cursor = 0;
+    const bool counted = !FINAL && nb == 1;
+    if (counted) {
+      const bool gone = l < ndup && dpos[w][l] != NOT_FOUND && sorted_contains(dlist + s0, s1 - s0, dpos[w][l]);
+      const uint64_t n = s1 - s0 - __popcll(__ballot(gone));
+      if (l == 0) cursor = atomicAdd(it.counter, (unsigned long long)n);
+      cursor = readlane_u64(cursor, 0);
+    }
     // the staged rows share the parent row: pend * ko consecutive words
     // of the output, reserved by one atomic, written by consecutive lanes
     auto flush = [&]() {
-      uint64_t base = 0;
-      if (l == 0) base = atomicAdd(it.counter, (unsigned long long)pend);
-      base = readlane_u64(base, 0);
+      uint64_t base = cursor;
+      cursor += pend;
+      if (!counted) {
+        if (l == 0) base = atomicAdd(it.counter, (unsigned long long)pend);
+        base = readlane_u64(base, 0);
+      }
       const uint32_t inv = 0xFFFFFFFFu / ko + 1;
       written += (uint64_t)pend * 4 * ko;
       for (uint32_t q = l; q < pend * ko; q += 64) {
@@ -902,7 +917,7 @@ void build_vlevels(gem_ctx *c, VQueryState &S) {
     }
     if (i + 1 < nv) {
       L.kout = (uint32_t)live[i + 1].size();
-      for (uint32_t x = 0; x < L.kout; ++x) L.src[x] = live[i + 1][x] == i ? COL_NEW : (uint8_t)at(live[i + 1][x]);
+      for (uint32_t x = 0; x < L.kout; ++x) L.src[x] = live[i + 1][x] == i ? COL_NEW : at(live[i + 1][x]);
     }
     L.can_new = Qd.can.as<uint32_t>() + Qd.can_off[u];
     L.bm_new = Qd.bitmap.as<uint64_t>() + (uint64_t)u * Qd.W;
@@ -1020,24 +1035,18 @@ uint32_t resident_blocks(const void *kernel, size_t lds) {
   return (uint32_t)std::max(1, per_cu * cus);
 }
 
-// Rows whose driving list has more entries than the context's heavy_t are
-// walked by k_vext_heavy, heavy_chunk entries per wave task; at most HEAVY_CAP
-// such rows per launch (a row that finds the list full is walked by its own
-// wave).
-constexpr uint32_t HEAVY_CAP = 1u << 20;
-
 // Fixed buffers for the extend step of every iteration of one run: item
 // tables and block prefixes of the three launches (write, final walk, final
 // single-list count), the heavy-row lists of the two walking launches, and a
 // header with the item counts, work queues, heavy-row counts, walked-entry
 // counts and per-task result counters.  Host side: pinned mirrors.  Because
 // every pointer, grid and LDS size is fixed for the run, the step
-//   H2D header, items, prefixes -> 3 kernels -> 2 x (heavy scan, heavy walk)
+//   H2D header, items, prefixes -> 3 kernels -> 2 heavy walks
 //   -> D2H header
 // is captured once as a hipGraph and replayed each iteration (no memset node:
 // the zeroed counters travel in the header copy).
 struct ExtSlot {
-  // header: item counts [3], heavy-row counts [2], profile counters [6] (u64:
+  // header: item counts [3], heavy rows and pieces [2 x 2], profile counters [6] (u64:
   // entries walked by the write / final / heavy write / heavy final kernels,
   // bytes written by the write / heavy write kernels), queues [3 main + 2
   // heavy] of WQ_WORDS words, result counters [cap] (u64, a cache line each:
@@ -1046,7 +1055,7 @@ struct ExtSlot {
                           HDR_CTR = HDR_QUEUE + 5 * 4 * WQ_WORDS, CTR_STRIDE = 8;
   uint32_t cap = 0;  // items per launch = counters
   DevBuf items[3], blk[3], hdr;
-  DevBuf heavy[2], hpre[2];  // heavy rows and their chunk prefix, per walking launch
+  DevBuf heavy[2], pieces[2];  // heavy rows and the rows of their pieces, per walking launch
   VItem *h_items[3] = {};
   uint64_t *h_blk[3] = {};
   unsigned char *h_hdr = nullptr;
@@ -1078,7 +1087,7 @@ struct ExtSlot {
     hdr.alloc(hdr_bytes, s);
     for (int i = 0; i < 2; ++i) {
       heavy[i].alloc(sizeof(HeavyRow) * HEAVY_CAP, s);
-      hpre[i].alloc(8ull * (HEAVY_CAP + 1), s);
+      pieces[i].alloc(4ull * PIECE_CAP, s);
     }
     GEM_HIP_CHECK(hipHostMalloc((void **)&h_hdr, hdr_bytes, hipHostMallocDefault));
     for (int i = 0; i < 3; ++i) {
@@ -1127,9 +1136,13 @@ struct ExtSlot {
     GEM_HIP_CHECK(hipMemcpyAsync(h_hdr, d, hdr_bytes, hipMemcpyDeviceToHost, s));
   }
 
+  HeavyOut heavy_out(int i, unsigned int *hn) const {
+    return HeavyOut{heavy[i].as<HeavyRow>(), pieces[i].as<uint32_t>(), hn + 2 * i, heavy_t, heavy_chunk};
+  }
+
   // (At most `most` blocks each.)  The three kernels over task ranges [b_i, e_i) of launch i (queues
   // dq, WQ_WORDS words each), then the heavy rows the two walking launches set
-  // aside (queues hq, row counts hn[0..1]; everything starts at zero).
+  // aside (queues hq, rows and pieces hn[0..3]; everything starts at zero).
   template <bool OOC>
   void launch_kernels(gem_ctx *c, uint32_t most, const uint32_t *dn, unsigned int *dq, unsigned int *hq,
                       unsigned int *hn, bool prof_kernels, bool count_items, uint64_t b0, uint64_t e0, uint64_t b1,
@@ -1140,14 +1153,14 @@ struct ExtSlot {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_WRITE : -1);
       k_vext<false, OOC><<<std::min(most, grid[0]), VB, lds, s>>>(items[0].as<VItem>(), dn + 0, blk[0].as<uint64_t>(), dq + 0, lcap, dcap,
                                                count_items ? dp : nullptr, count_items ? dp + 4 : nullptr,
-                                               b0, e0, heavy[0].as<HeavyRow>(), hn + 0, HEAVY_CAP, heavy_t);
+                                               b0, e0, heavy_out(0, hn));
       GEM_LAUNCH_CHECK("k_vext<write>");
     }
     if (b1 < e1) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_FINAL : -1);
       k_vext<true, OOC><<<std::min(most, grid[1]), VB, lds, s>>>(items[1].as<VItem>(), dn + 1, blk[1].as<uint64_t>(), dq + WQ_WORDS, lcap, dcap,
                                               count_items ? dp + 1 : nullptr, nullptr, b1, e1,
-                                              heavy[1].as<HeavyRow>(), hn + 1, HEAVY_CAP, heavy_t);
+                                              heavy_out(1, hn));
       GEM_LAUNCH_CHECK("k_vext<final>");
     }
     if (b2 < e2) {
@@ -1157,20 +1170,16 @@ struct ExtSlot {
     }
     if (b0 < e0) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_HEAVY_WRITE : -1);
-      k_heavy_scan<<<1, 1024, 0, s>>>(heavy[0].as<HeavyRow>(), hn + 0, HEAVY_CAP, heavy_chunk, hpre[0].as<uint64_t>());
-      GEM_LAUNCH_CHECK("k_heavy_scan");
-      k_vext_heavy<false, OOC><<<std::min(most, grid[3]), VB, 0, s>>>(items[0].as<VItem>(), heavy[0].as<HeavyRow>(), hn + 0, HEAVY_CAP,
-                                                   hpre[0].as<uint64_t>(), hq + 0, heavy_chunk,
-                                                   count_items ? dp + 2 : nullptr, count_items ? dp + 5 : nullptr);
+      k_vext_heavy<false, OOC><<<std::min(most, grid[3]), VB, 0, s>>>(items[0].as<VItem>(), heavy_out(0, hn), hq + 0,
+                                                                      count_items ? dp + 2 : nullptr,
+                                                                      count_items ? dp + 5 : nullptr);
       GEM_LAUNCH_CHECK("k_vext_heavy<write>");
     }
     if (b1 < e1) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_HEAVY_FINAL : -1);
-      k_heavy_scan<<<1, 1024, 0, s>>>(heavy[1].as<HeavyRow>(), hn + 1, HEAVY_CAP, heavy_chunk, hpre[1].as<uint64_t>());
-      GEM_LAUNCH_CHECK("k_heavy_scan");
-      k_vext_heavy<true, OOC><<<std::min(most, grid[4]), VB, 0, s>>>(items[1].as<VItem>(), heavy[1].as<HeavyRow>(), hn + 1, HEAVY_CAP,
-                                                  hpre[1].as<uint64_t>(), hq + WQ_WORDS, heavy_chunk,
-                                                  count_items ? dp + 3 : nullptr, nullptr);
+      k_vext_heavy<true, OOC><<<std::min(most, grid[4]), VB, 0, s>>>(items[1].as<VItem>(), heavy_out(1, hn),
+                                                                     hq + WQ_WORDS, count_items ? dp + 3 : nullptr,
+                                                                     nullptr);
       GEM_LAUNCH_CHECK("k_vext_heavy<final>");
     }
   }
@@ -1231,7 +1240,7 @@ struct ExtSlot {
         }
         const uint64_t most = std::max(hi[0] - lo[0], std::max(hi[1] - lo[1], hi[2] - lo[2]));
         const uint32_t grd = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(~0u, most));
-        // per group: 3 main queues, 2 heavy queues, 2 heavy-row counts
+        // per group: 3 main queues, 2 heavy queues, heavy rows and pieces
         unsigned int *gq = q + (size_t)GROUP_WORDS * g;
         launch_kernels<true>(c, grd, dn, gq, gq + 3 * WQ_WORDS, gq + 5 * WQ_WORDS, prof, prof, lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]);
         tc.done(g);
