@@ -47,12 +47,15 @@ struct VItem {
   unsigned long long *counter;
 };
 
-// Rows of a pending level.  Once measured they know the device prefix of
-// their units' output bounds (from entry unit0 on; one buffer holds those of
-// all levels measured together).
+// Rows of a pending level, with the device prefix of the output bounds of the
+// units [lo, hi) measured last (unit u's at entry unit0 + u; one buffer holds
+// those of all levels measured together).
 struct LevelBuf : DevBuf {
-  mutable std::shared_ptr<DevBuf> units;
-  mutable uint64_t unit0 = 0;
+  struct Units {
+    std::shared_ptr<DevBuf> prefix;
+    uint64_t unit0 = 0, lo = 0, hi = 0;
+  };
+  mutable Units units;
 };
 
 // A row whose driving list is too long for one wave: walked in pieces by

@@ -1017,6 +1017,11 @@ void upload(gem_ctx *c, const Launch &L, DevLaunch &D) {
   GEM_HIP_CHECK(hipMemcpyAsync(D.blk.p, L.blk.data(), 8 * L.blk.size(), hipMemcpyHostToDevice, s));
 }
 
+// Units of a level that a capped run measures at first (see SchedConfig): of
+// the levels of 16 queries of up to 24 vertices under a cap of 1e9 (2^20 R-MAT),
+// 27 times as many units were measured as walked, half the pass.
+constexpr uint64_t MEASURE_UNITS = 4096;
+
 // persistent grid: enough blocks to fill the chip (tunable cap), never more
 // than the tasks
 uint32_t g_persistent_blocks = 2048;
@@ -1340,8 +1345,8 @@ struct HipSchedBackend {
     }
     scan_u64(c, bu.as<uint64_t>(), bp.as<uint64_t>(), nunit);
     for (size_t t = 0; t < items.size(); ++t) {
-      items[t].rows->units = kept;
-      items[t].rows->unit0 = L.blk[t] * VW - items[t].row_begin / gemh::SCHED_UNIT;
+      const uint64_t lo = items[t].row_begin / gemh::SCHED_UNIT;
+      items[t].rows->units = LevelBuf::Units{kept, L.blk[t] * VW - lo, lo, lo + units_of(items[t])};
     }
     if (!prefix) return;
     uint64_t *pref = pinned<uint64_t>(c, nunit + 1);
@@ -1361,18 +1366,25 @@ struct HipSchedBackend {
     t_len += std::chrono::duration<double>(clk::now() - t0).count();
   }
 
-  // Unit prefixes of chunks whose level came back from host memory without
-  // them; they are dropped again by extend (they cover the chunk only).
-  std::vector<const LevelBuf *> remeasure(const std::vector<Item> &wr_items) {
+  static uint64_t units_of(const Item &x) {
+    return (x.row_end - x.row_begin + gemh::SCHED_UNIT - 1) / gemh::SCHED_UNIT;
+  }
+
+  // Unit prefixes of chunks that the last measurement of their level does not
+  // hold (the level came back from host memory without them).  Returns what
+  // they replace, which extend puts back.
+  std::vector<std::pair<const LevelBuf *, LevelBuf::Units>> remeasure(const std::vector<Item> &wr_items) {
     std::vector<Item> need;
-    std::vector<const LevelBuf *> bufs;
-    for (const Item &x : wr_items)
-      if (!x.rows->units) {
-        need.push_back(x);
-        bufs.push_back(x.rows);
-      }
+    std::vector<std::pair<const LevelBuf *, LevelBuf::Units>> old;
+    for (const Item &x : wr_items) {
+      const uint64_t lo = x.row_begin / gemh::SCHED_UNIT;
+      const LevelBuf::Units &u = x.rows->units;
+      if (u.prefix && lo >= u.lo && lo + units_of(x) <= u.hi) continue;
+      need.push_back(x);
+      old.push_back({x.rows, u});
+    }
     if (!need.empty()) length_pass(need, nullptr);
-    return bufs;
+    return old;
   }
 
   void extend(const std::vector<Item> &wr_items, const std::vector<Item> &fin_items, std::vector<uint64_t> *got_wr,
@@ -1386,17 +1398,16 @@ struct HipSchedBackend {
     size_t nctr = 0;
     // counters / work queues / walked-entry counts travel zeroed in the copy
     std::memset(slot.h_hdr + ExtSlot::HDR_HEAVYN, 0, slot.hdr_bytes - ExtSlot::HDR_HEAVYN);
-    auto units_of = [](const Item &x) { return (x.row_end - x.row_begin + gemh::SCHED_UNIT - 1) / gemh::SCHED_UNIT; };
     // runs of the write walks (see unit_range): CLAIMS per wave of the grid by
     // cost, an entry of a level with other lists costing its searches too
     auto weight = [&](const Item &x) { return 4ull * qs[x.q]->max_nb[x.level] - 3; };
     uint64_t run_cost = 0;
-    std::vector<const LevelBuf *> once;
+    std::vector<std::pair<const LevelBuf *, LevelBuf::Units>> replaced;
     if (!tc) {
       uint64_t cost = 0;
       for (const Item &x : wr_items) cost += (x.out_rows + UNIT_COST * units_of(x)) * weight(x);
       run_cost = cost / ((uint64_t)slot.grid[0] * VW * CLAIMS) + 1;
-      once = remeasure(wr_items);
+      replaced = remeasure(wr_items);
     }
     for (const Item &x : wr_items) {
       VItem it = vitem(x);
@@ -1404,7 +1415,7 @@ struct HipSchedBackend {
       it.out_cap = x.out_rows;
       it.counter = slot.dev_counter(nctr++);
       if (run_cost) {
-        it.units = x.rows->units->as<uint64_t>() + x.rows->unit0 + x.row_begin / gemh::SCHED_UNIT;
+        it.units = x.rows->units.prefix->as<uint64_t>() + x.rows->units.unit0 + x.row_begin / gemh::SCHED_UNIT;
         it.nunits = (uint32_t)units_of(x);
         it.run_cost = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(run_cost / weight(x), 4 * UNIT_COST), RUN_COST);
         wr.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level],
@@ -1442,7 +1453,7 @@ struct HipSchedBackend {
       slot.launch(c, c->use_graph && !prof);
     GEM_HIP_CHECK(hipStreamSynchronize(s));
     if (tc) tc->finish();
-    for (const LevelBuf *b : once) b->units.reset();
+    for (auto &r : replaced) r.first->units = r.second;
     got_wr->resize(wr_items.size());
     got_fin->resize(fin_items.size());
     for (size_t t = 0; t < wr_items.size(); ++t) {
@@ -1720,6 +1731,7 @@ void VBatchRunner::run(std::vector<VQueryState *> &qs) {
   cfg.max_active = c_->max_active;
   cfg.primaries = primaries_;
   cfg.swap_bytes = c_->swap_bytes;
+  if (cap_) cfg.measure_units = MEASURE_UNITS;
   const auto t0 = std::chrono::steady_clock::now();
   stats_ = gemh::SchedStats{};
   gemh::run_schedule(be, sq, cfg, &stats_);

@@ -73,6 +73,10 @@ struct SchedConfig {
   // not count as waiting for the quotas
   uint32_t primaries = 0;
   uint64_t swap_bytes = 0;  // host memory pending levels may move to (0 = none)
+  // units of a level measured at first, four times as many each time that these
+  // do not fill what the query may take of it (0 = the whole level at once):
+  // a capped query seldom comes back to the rest of a level
+  uint64_t measure_units = 0;
 };
 
 struct SchedStats {
@@ -97,7 +101,10 @@ struct SLevel {
   std::shared_ptr<Buf> rows;
   uint64_t nrows = 0;
   uint32_t k = 0;                 // columns per row
-  std::vector<uint64_t> unit_u;   // prefix of per-unit output bounds (nunits + 1) once measured
+  // prefix of the output bounds of units [unit_base, measured_to), from where the
+  // cursor stood when they were measured
+  std::vector<uint64_t> unit_u;
+  uint64_t unit_base = 0, measured_to = 0;
   uint64_t cursor = 0;            // next unit
   bool measured = false;
   // swapping: the rows in host memory (rows null meanwhile), their bytes, and
@@ -106,6 +113,8 @@ struct SLevel {
   uint64_t host_bytes = 0;
   uint64_t last_use = 0;
   uint64_t nunits() const { return (nrows + SCHED_UNIT - 1) / SCHED_UNIT; }
+  // output bound of units [a, b)
+  uint64_t bound(uint64_t a, uint64_t b) const { return unit_u[b - unit_base] - unit_u[a - unit_base]; }
 };
 
 template <class Buf>
@@ -219,7 +228,8 @@ inline int plan_chunks(const std::vector<ChunkCand> &cand, uint64_t left, uint64
 //   using Buf = ...;
 //   static uint64_t buf_bytes(const Buf &);
 //   std::shared_ptr<Buf> alloc(uint64_t bytes);
-//   // per item, the prefix of per-unit output bounds over its rows
+//   // per item, the prefix of per-unit output bounds over its rows (a level's,
+//   // or with measure_units, those of its next units)
 //   void length_pass(const std::vector<SItem<Buf>> &items, std::vector<std::vector<uint64_t>> *prefix);
 //   // rows written per write item, embeddings counted per final item
 //   void extend(const std::vector<SItem<Buf>> &wr, const std::vector<SItem<Buf>> &fin,
@@ -326,46 +336,6 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
     const uint64_t live = live_bytes();
     be.on_iteration(st->iterations, act.size(), live, budget);
 
-    // ---- length pass: output bounds of every unmeasured top level (final
-    // levels only when they walk lists under a cap: their units are then
-    // counted a cap-sized piece at a time)
-    {
-      std::vector<Item> items;
-      std::vector<uint32_t> owner;
-      for (uint32_t qi : act) {
-        SQuery<Buf> &S = *qs[qi];
-        SLevel<Buf> &top = S.stack.back();
-        const bool final_level = top.level + 1 == S.nv;
-        if (top.measured || (final_level && (S.nb[top.level] == 1 || !cfg.cap))) continue;
-        Item it;
-        it.q = qi;
-        it.level = top.level;
-        it.k = top.k;
-        it.rows = top.rows.get();
-        it.row_begin = 0;
-        it.row_end = top.nrows;
-        items.push_back(it);
-        owner.push_back(qi);
-      }
-      if (!items.empty()) {
-        ++st->length_passes;
-        std::vector<std::vector<uint64_t>> pref;
-        be.length_pass(items, &pref);
-        for (size_t t = 0; t < owner.size(); ++t) {
-          SLevel<Buf> &top = qs[owner[t]]->stack.back();
-          top.unit_u = std::move(pref[t]);
-          top.measured = true;
-        }
-      }
-    }
-
-    // ---- count-only pieces of final levels (no output memory)
-    std::vector<Item> wr, fin;
-    std::vector<std::shared_ptr<Buf>> keep_alive, outs;
-    std::vector<uint32_t> wr_owner, fin_owner;
-    std::vector<uint64_t> fin_bounds;  // output bound of each measured final piece (0: unmeasured)
-    std::vector<ChunkCand> cand;
-    std::vector<uint32_t> cand_owner;
     // quotas: budget / max_active while queries wait to start; then the
     // budget over the queries still running, at most tail_growth times the
     // first quota (the last queries take larger chunks, so they do not crawl
@@ -377,41 +347,105 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
       shares = next < nprim ? cfg.max_active
                             : std::max<uint64_t>(shares, cfg.max_active / std::max<uint32_t>(cfg.tail_growth, 1));
     const uint64_t quota = budget / std::max<uint64_t>(shares, 1);
+    // what the pending levels of a query hold, and the share of its free quota
+    // that its next chunk may take
+    auto held = [&](const SQuery<Buf> &S) {
+      uint64_t b = 0;
+      for (const SLevel<Buf> &L : S.stack) b += charge(S, L);
+      return b;
+    };
+    // A piece of a final level whose output bound should just exceed the cap:
+    // what is still missing, over the share of bounds that earlier pieces
+    // turned into embeddings (1 before any), plus 10% (at least final_piece
+    // list entries of work).
+    auto final_target = [&](const SQuery<Buf> &S) {
+      const uint64_t need = cfg.cap + 1 > S.count ? cfg.cap + 1 - S.count : 1;
+      const double ratio = S.fin_bound >= (1ull << 20) && S.fin_got
+                               ? std::min(1.0, (double)S.fin_got / (double)S.fin_bound)
+                               : 1.0;
+      const double want = 1.1 * (double)need / ratio;
+      return std::max<uint64_t>(want >= 1.8e19 ? ~0ull : (uint64_t)want, cfg.final_piece);
+    };
+
+    // ---- length passes: output bounds of the next units of every top level,
+    // as many as this iteration can use (final levels only when they walk
+    // lists under a cap: their units are then counted a cap-sized piece at a
+    // time)
+    for (;;) {
+      std::vector<Item> items;
+      std::vector<uint32_t> owner;
+      for (uint32_t qi : act) {
+        SQuery<Buf> &S = *qs[qi];
+        SLevel<Buf> &top = S.stack.back();
+        const bool final_level = top.level + 1 == S.nv;
+        if (final_level && (S.nb[top.level] == 1 || !cfg.cap)) continue;
+        const uint64_t nu = top.nunits();
+        uint64_t seg = cfg.measure_units ? cfg.measure_units : nu;  // a longer one starts at the cursor again
+        if (top.measured) {
+          if (top.measured_to >= nu) continue;
+          const uint64_t rows = top.bound(top.cursor, top.measured_to);
+          if (final_level) {
+            if (rows >= final_target(S)) continue;
+          } else {
+            const uint64_t mine = held(S), free_q = quota > mine ? quota - mine : 0;
+            const uint64_t share = std::min(cfg.max_chunk, free_q / std::max<uint64_t>(S.nv - 1 - top.level, 1));
+            if (top.measured_to > top.cursor && rows * 4 * (top.level + 1) > share) continue;
+          }
+          seg = 4 * std::max(seg, top.measured_to - top.cursor);
+        }
+        Item it;
+        it.q = qi;
+        it.level = top.level;
+        it.k = top.k;
+        it.rows = top.rows.get();
+        it.row_begin = top.cursor * SCHED_UNIT;
+        it.row_end = std::min<uint64_t>((top.cursor + std::min(seg, nu - top.cursor)) * SCHED_UNIT, top.nrows);
+        items.push_back(it);
+        owner.push_back(qi);
+      }
+      if (items.empty()) break;
+      ++st->length_passes;
+      std::vector<std::vector<uint64_t>> pref;
+      be.length_pass(items, &pref);
+      for (size_t t = 0; t < owner.size(); ++t) {
+        SLevel<Buf> &top = qs[owner[t]]->stack.back();
+        top.unit_u = std::move(pref[t]);
+        top.unit_base = top.cursor;
+        top.measured_to = top.cursor + top.unit_u.size() - 1;
+        top.measured = true;
+      }
+    }
+
+    // ---- count-only pieces of final levels (no output memory)
+    std::vector<Item> wr, fin;
+    std::vector<std::shared_ptr<Buf>> keep_alive, outs;
+    std::vector<uint32_t> wr_owner, fin_owner;
+    std::vector<uint64_t> fin_bounds;  // output bound of each measured final piece (0: unmeasured)
+    std::vector<ChunkCand> cand;
+    std::vector<uint32_t> cand_owner;
     for (uint32_t qi : act) {
       SQuery<Buf> &S = *qs[qi];
       SLevel<Buf> &top = S.stack.back();
       const uint64_t nu = top.nunits();
       if (top.level + 1 != S.nv) {
-        uint64_t mine = 0;
-        for (const SLevel<Buf> &L : S.stack) mine += charge(S, L);
-        cand.push_back(ChunkCand{&top.unit_u, top.cursor, nu, 4ull * (top.level + 1), top.level, mine, quota,
-                                 S.nv - 1 - top.level});
+        cand.push_back(ChunkCand{&top.unit_u, top.cursor - top.unit_base, top.measured_to - top.unit_base,
+                                 4ull * (top.level + 1), top.level, held(S), quota, S.nv - 1 - top.level});
         cand_owner.push_back(qi);
         continue;
       }
       uint64_t b1 = nu, piece_bound = 0;
       if (top.measured) {
-        // a piece whose output bound should just exceed the cap: what is
-        // still missing, over the share of bounds that earlier pieces turned
-        // into embeddings (1 before any), plus 10% (at least final_piece
-        // list entries of work)
-        const uint64_t need = cfg.cap + 1 > S.count ? cfg.cap + 1 - S.count : 1;
-        const double ratio = S.fin_bound >= (1ull << 20) && S.fin_got
-                                 ? std::min(1.0, (double)S.fin_got / (double)S.fin_bound)
-                                 : 1.0;
-        const double want = 1.1 * (double)need / ratio;
-        const uint64_t target = std::max<uint64_t>(want >= 1.8e19 ? ~0ull : (uint64_t)want, cfg.final_piece);
-        const std::vector<uint64_t> &P = top.unit_u;
-        uint64_t lo = top.cursor + 1, hi = nu;  // smallest b1 with P[b1] - P[cursor] >= target, else nu
+        const uint64_t target = final_target(S), known = top.measured_to;
+        uint64_t lo = top.cursor + 1, hi = known;  // smallest b1 with bound(cursor, b1) >= target, else all known
         while (lo < hi) {
           const uint64_t mid = lo + (hi - lo) / 2;
-          if (P[mid] - P[top.cursor] >= target)
+          if (top.bound(top.cursor, mid) >= target)
             hi = mid;
           else
             lo = mid + 1;
         }
         b1 = lo;
-        piece_bound = P[b1] - P[top.cursor];
+        piece_bound = top.bound(top.cursor, b1);
         S.work += piece_bound;
       }
       Item it;
@@ -441,12 +475,12 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
       const uint32_t qi = cand_owner[c];
       SQuery<Buf> &S = *qs[qi];
       SLevel<Buf> &top = S.stack.back();
-      const uint64_t b0 = top.cursor, b1 = end[c];
+      const uint64_t b0 = top.cursor, b1 = top.unit_base + end[c];
       if (b1 == b0) {
         ++st->waits;
         continue;
       }
-      const uint64_t ub = top.unit_u[b1] - top.unit_u[b0];
+      const uint64_t ub = top.bound(b0, b1);
       const uint64_t rb = 4ull * (top.level + 1);
       Item it;
       it.q = qi;
