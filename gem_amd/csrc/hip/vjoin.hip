@@ -67,6 +67,7 @@ __device__ __forceinline__ uint32_t vposition_in(const uint64_t *bm, const uint3
 #define GEM_CONST const __attribute__((address_space(4)))
 using CLevel = GEM_CONST VLevel;
 using CItem = GEM_CONST VItem;
+using CWord = GEM_CONST uint64_t;
 
 // Two neighbouring offsets (start and end of a list) in one 16-byte load.
 typedef uint64_t u64x2 __attribute__((ext_vector_type(2), aligned(8)));
@@ -185,9 +186,17 @@ __device__ __forceinline__ uint64_t list_addr(CLevel &L, uint32_t j, uint32_t p,
 // setup.  A run of a write walk has at most RUN_COST of it.
 constexpr uint32_t UNIT_COST = 256, RUN_COST = UNIT_COST * MAX_RUN;
 
-// The units [*j0, *j1) of an item of n units whose cost starts in
-// [at, at + run): cost(j) = units[j] - units[0] + UNIT_COST * j, at < cost(n),
-// run <= RUN_COST (so they are at most MAX_RUN).  The first is searched 64
+// A unit that costs more than this part of a run is cut between its rows: row
+// i starts at the unit's cost plus UNIT_COST / 64 a row and the entries of the
+// rows before it, and belongs to the run that holds its start.  (With units
+// whole, one unit of 64 rows of up to 1024 entries kept a wave for 1.0 to 2.8 ms
+// of launches of 1.5 to 3 ms, whose waves were busy 58% of the time.)
+__device__ __forceinline__ bool unit_is_cut(uint64_t cost, uint32_t run) { return cost > run / 2; }
+
+// The units [*j0, *j1) of an item of n units that a run looks at: those whose
+// cost starts in [at, at + run) and the one before when it is cut and reaches
+// into the run: cost(j) = units[j] - units[0] + UNIT_COST * j, at < cost(n),
+// run <= RUN_COST (so they are at most MAX_RUN + 1).  The first is searched 64
 // places at a time, the end looked up in one step.
 __device__ __forceinline__ void unit_range(const uint64_t *units, uint32_t n, uint64_t at, uint32_t run, uint32_t *j0,
                                            uint32_t *j1) {
@@ -210,8 +219,12 @@ __device__ __forceinline__ void unit_range(const uint64_t *units, uint32_t n, ui
   const uint64_t x = (uint64_t)b + lane_id();
   bool past = x >= n;
   if (!past) past = ldg(units + x) - first + (uint64_t)UNIT_COST * x >= at + run;
-  *j0 = b;
   *j1 = b + (uint32_t)__builtin_ctzll(__ballot(past));
+  if (b) {
+    const u64x2 c = ld_pair(units + b - 1);
+    if (unit_is_cut(c.y - c.x + UNIT_COST, run) && c.y - first + (uint64_t)UNIT_COST * b > at) --b;
+  }
+  *j0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
 }
 
 // Loads of N lists (N equal-label columns) of one row at a time, so that a
@@ -300,7 +313,7 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
   __shared__ uint32_t st[VW][65];
   __shared__ uint64_t drv[VW][64];         // address of each row's driving list
   __shared__ uint8_t drv_j[VW][64];        // which of the row's lists drives
-  __shared__ uint64_t aside[VW][MAX_RUN];  // counted runs: rows of each task set aside as heavy
+  __shared__ uint64_t aside[VW][MAX_RUN + 1];  // counted runs: rows of each task set aside as heavy
   __shared__ uint32_t sv_row[VW][VSTAGE];  // staged survivors: row in the item's range
   __shared__ uint32_t sv_val[VW][VSTAGE];  // and new value
   extern __shared__ unsigned char vlds[];
@@ -384,8 +397,19 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
     in = I.rows + I.row_begin * k;
     nrow = I.row_end - I.row_begin;
   };
-  // walk units [j0, j1) of the item in hand (at most MAX_RUN of them)
-  auto walk = [&](uint64_t j0, uint64_t j1) {
+  // is the lane's row, of len entries, of unit j the run's that starts at `at`?
+  auto owned = [&](uint64_t j, uint32_t len, uint64_t at) {
+    CItem &I = ((CItem *)items)[t];
+    CWord *u = (CWord *)I.units;
+    const uint64_t a = u[j], b = u[j + 1];
+    if (!unit_is_cut(b - a + UNIT_COST, I.run_cost)) return true;
+    const uint32_t n = len < (1u << 25) ? len : 1u << 25;
+    const uint64_t c = a - u[0] + UNIT_COST * j + wave_incl_scan_u32(n) - n + UNIT_COST / 64 * l;
+    return c >= at && c - at < I.run_cost;
+  };
+  // walk units [j0, j1) of the item in hand (at most MAX_RUN of them; a write
+  // walk's run that starts at cost `at`: MAX_RUN + 1)
+  auto walk = [&](uint64_t j0, uint64_t j1, uint64_t at = 0) {
     CLevel &L = *(CLevel *)lv;
     const uint32_t nb = L.nb, ndup = L.ndup;
     if (!FINAL && nb == 1) {
@@ -406,6 +430,7 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
           len = (uint32_t)(o.y - o.x);
           addr = list_addr<OOC>(L, 0, p, o.x);
         }
+        if (!FINAL && !OOC && !owned(j, len, at)) len = 0;
         const uint64_t taken = set_aside(heavy, len > heavy.threshold, t, len, ((CItem *)items)[t].row_begin + r);
         if ((taken >> l) & 1ull) len = 0;  // walked by k_vext_heavy
         if (l == 0) aside[w][j - j0] = taken;
@@ -455,6 +480,7 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
       }
       if (i < nb) row_lists<1>(L, row, i, take);
     }
+    if (!FINAL && !OOC && !owned(j, dlen, at)) dlen = 0;
     const uint64_t taken =
         !FINAL && counted
             ? aside[w][j - j0]
@@ -581,8 +607,8 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
         q = qn;
       }
   } else {
-    // tasks are runs of units of about equal cost: run i of an item holds the
-    // units whose cost starts in [i, i + 1) * run_cost (the item's)
+    // tasks are runs of units of about equal cost: run i of an item holds what
+    // starts in [i, i + 1) * run_cost (the item's)
     Runs runs(total - g_begin, blockIdx.x * bw + w, gridDim.x * bw, 1, queue);
     for (; runs.valid(); runs.next()) {
       const uint64_t g = g_begin + runs.begin();
@@ -590,8 +616,9 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
       if (x != t) open(x);
       CItem &I = ((CItem *)items)[t];
       uint32_t j0, j1;
-      unit_range(I.units, I.nunits, (g - blk_prefix[t]) * I.run_cost, I.run_cost, &j0, &j1);
-      if (j0 < j1) walk(j0, j1);
+      const uint64_t at = (g - blk_prefix[t]) * I.run_cost;
+      unit_range(I.units, I.nunits, at, I.run_cost, &j0, &j1);
+      if (j0 < j1) walk(j0, j1, at);
     }
   }
   if (t != NOT_FOUND) flush();
