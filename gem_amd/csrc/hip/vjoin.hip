@@ -310,9 +310,11 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
   const uint32_t nitems = *nitems_p;
   const uint64_t total = blk_prefix[nitems] < g_end ? blk_prefix[nitems] : g_end;
   if (g_begin >= total) return;
-  __shared__ uint32_t st[VW][65];
+  __shared__ uint32_t st[VW][64];          // first item of each row
   __shared__ uint64_t drv[VW][64];         // address of each row's driving list
   __shared__ uint8_t drv_j[VW][64];        // which of the row's lists drives
+  __shared__ uint8_t full_row[VW][64];     // the unit's rows that have entries
+  __shared__ uint32_t marks[VW][8];        // bit i: a row's entries start at item i of the step
   __shared__ uint64_t aside[VW][MAX_RUN + 1];  // counted runs: rows of each task set aside as heavy
   __shared__ uint32_t sv_row[VW][VSTAGE];  // staged survivors: row in the item's range
   __shared__ uint32_t sv_val[VW][VSTAGE];  // and new value
@@ -502,23 +504,41 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
     }
     const uint32_t incl = wave_incl_scan_u32(dlen);
     const uint32_t wtotal = readlane_u32(incl, 63);
-    st[w][l] = incl - dlen;
-    if (l == 63) st[w][64] = wtotal;
+    const uint32_t start = incl - dlen;
+    st[w][l] = start;
     drv[w][l] = daddr;
+    {
+      const uint64_t full = __ballot(dlen);
+      if (dlen) full_row[w][rank_below(full)] = (uint8_t)l;
+    }
     if (nb > 1) drv_j[w][l] = (uint8_t)dj;
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     walked += wtotal;
     // 256 items per step, four per lane (items s + 64 g + l), so that each
-    // lane has four loads in flight at every stage of the probes
+    // lane has four loads in flight at every stage of the probes.  An item's
+    // row is the last one to start at or before it: the rows that start in the
+    // step mark their items, and the marks up to an item are counted (searched
+    // in the starts, the rows took a fifth of the vector instructions).
+    uint32_t rows_before = 0;  // rows with entries that start before the step
     for (uint32_t s = 0; s < wtotal; s += 256) {
       uint32_t val[4], rw[4];
       bool keep[4];
+      if (l < 8) marks[w][l] = 0;
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      if (dlen && start - s < 256) atomicOr(&marks[w][(start - s) / 32], 1u << ((start - s) % 32));
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const uint32_t item = s + 64u * g + l;
         keep[g] = item < wtotal;
-        rw[g] = keep[g] ? seg_of(st[w], item) : 0;
+        const uint32_t mlo = __builtin_amdgcn_readfirstlane(marks[w][2 * g]);
+        const uint32_t mhi = __builtin_amdgcn_readfirstlane(marks[w][2 * g + 1]);
+        const uint64_t m = (uint64_t)mhi << 32 | mlo;
+        rw[g] = full_row[w][rows_before + rank_below(m) + ((m >> l) & 1) - 1];
+        rows_before += (uint32_t)__popcll(m);
         val[g] = keep[g] ? ldg(reinterpret_cast<const uint32_t *>(drv[w][rw[g]]) + (item - st[w][rw[g]])) : 0;
       }
       for (uint32_t j = 0; nb > 1 && j < nb; ++j) {
@@ -762,21 +782,22 @@ k_vext_heavy(const VItem *__restrict__ items, const HeavyOut heavy, unsigned int
           if (dpos[w][c] == val1) keep1 = false;
         }
         if (nb > 1) {
-          const uint32_t a = j ? wend[w][j - 1] : wend[w][63], wn = wend[w][j] - a;
+          const uint32_t a = __builtin_amdgcn_readfirstlane(j ? wend[w][j - 1] : wend[w][63]);
+          const uint32_t wn = __builtin_amdgcn_readfirstlane(wend[w][j]) - a;
           if (wn <= HWIN) {
             for (uint32_t i = l; i < wn; i += 64) win[w][i] = ldg(l0p + a + i);
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            contains_pair<false>(win[w], wn, val0, keep0, win[w], wn, val1, keep1);
+            contains_pair<false>(win[w], wn, val0, keep0, val1, keep1);
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
           } else {
-            contains_pair(l0p + a, wn, val0, keep0, l0p + a, wn, val1, keep1);
+            contains_pair(l0p + a, wn, val0, keep0, val1, keep1);
           }
         }
         for (uint32_t o = 1; o + 1 < nb; ++o) {
           const uint32_t *a = reinterpret_cast<const uint32_t *>(oaddr[w][o]);
-          contains_pair(a, olen[w][o], val0, keep0, a, olen[w][o], val1, keep1);
+          contains_pair(a, __builtin_amdgcn_readfirstlane(olen[w][o]), val0, keep0, val1, keep1);
         }
         const uint64_t m0 = __ballot(keep0), m1 = __ballot(keep1);
         const uint32_t nk0 = (uint32_t)__popcll(m0), nk = nk0 + (uint32_t)__popcll(m1);

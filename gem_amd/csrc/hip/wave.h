@@ -36,14 +36,19 @@ __device__ __forceinline__ uint64_t readlane_u64(uint64_t x, uint32_t lane) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-// Inclusive wave scan (Hillis-Steele over 64 lanes).
+// Inclusive wave scan (all lanes active): within rows of 16 lanes, then the
+// rows' totals handed on, all by DPP moves (shuffles go through LDS).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+}
 __device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t x) {
-  const uint32_t l = lane_id();
-#pragma unroll
-  for (uint32_t d = 1; d < 64; d <<= 1) {
-    uint32_t y = __shfl_up(x, d, 64);
-    if (l >= d) x += y;
-  }
+  x += dpp_or_zero<0x111, 0xf>(x);  // row_shr 1, 2, 4, 8
+  x += dpp_or_zero<0x112, 0xf>(x);
+  x += dpp_or_zero<0x114, 0xf>(x);
+  x += dpp_or_zero<0x118, 0xf>(x);
+  x += dpp_or_zero<0x142, 0xa>(x);  // lane 15 of a row to the next one (rows 1 and 3)
+  x += dpp_or_zero<0x143, 0xc>(x);  // lane 31 to rows 2 and 3
   return x;
 }
 __device__ __forceinline__ uint64_t wave_incl_scan_u64(uint64_t x) {
@@ -133,81 +138,67 @@ __device__ __forceinline__ uint32_t upper_bound_u32(const uint32_t *a, uint32_t 
   return lo;
 }
 
-// Two membership tests at once: is v0 in sorted a0[0..n0) and v1 in
-// a1[0..n1)?  k0 / k1 enter as "still wanted" (a false one is not searched)
-// and leave as the result.  The two lower-bound searches advance in lockstep
-// so their loads are in flight together, and a hit is seen when it is probed
-// (a lower bound i with a[i] == v is always probed: the range's right end
-// only moves onto i by probing it), so no load follows the search.
-// GLOBAL: the lists are in device or mapped host memory (else in LDS).
+// Two membership tests at once in one list (the same in every lane): k0 says
+// whether v0, k1 whether v1 is in sorted a[0..n); false ones stay false.  A
+// search keeps the last place whose value is not above its own, so it is a
+// load, a compare and a select a step, and the lanes step together.
+// GLOBAL: the list is in device or mapped host memory (else in LDS).
 template <bool GLOBAL = true>
-__device__ __forceinline__ void contains_pair(const uint32_t *a0, uint32_t n0, uint32_t v0, bool &k0,
-                                              const uint32_t *a1, uint32_t n1, uint32_t v1, bool &k1) {
-  uint32_t lo0 = 0, lo1 = 0;
-  bool f0 = false, f1 = false;
-  if (!k0) n0 = 0;
-  if (!k1) n1 = 0;
-  while (n0 | n1) {
-    const uint32_t h0 = n0 >> 1, h1 = n1 >> 1;
-    uint32_t x0 = 0, x1 = 0;
-    if (n0) x0 = GLOBAL ? ldg(a0 + lo0 + h0) : a0[lo0 + h0];
-    if (n1) x1 = GLOBAL ? ldg(a1 + lo1 + h1) : a1[lo1 + h1];
-    if (n0) {
-      if (x0 < v0) {
-        lo0 += h0 + 1;
-        n0 -= h0 + 1;
-      } else {
-        f0 |= x0 == v0;
-        n0 = h0;
-      }
-    }
-    if (n1) {
-      if (x1 < v1) {
-        lo1 += h1 + 1;
-        n1 -= h1 + 1;
-      } else {
-        f1 |= x1 == v1;
-        n1 = h1;
-      }
-    }
+__device__ __forceinline__ void contains_pair(const uint32_t *a, uint32_t n, uint32_t v0, bool &k0, uint32_t v1,
+                                              bool &k1) {
+  auto at = [&](uint32_t i) { return GLOBAL ? ldg(a + i) : a[i]; };
+  if (!n) {
+    k0 = k1 = false;
+    return;
   }
-  k0 = k0 && f0;
-  k1 = k1 && f1;
+  uint32_t o0 = 0, o1 = 0;
+  for (; n > 1; n -= n >> 1) {
+    const uint32_t h = n >> 1;
+    const uint32_t x0 = at(o0 + h), x1 = at(o1 + h);
+    o0 += x0 <= v0 ? h : 0;
+    o1 += x1 <= v1 ? h : 0;
+  }
+  const uint32_t x0 = at(o0), x1 = at(o1);
+  k0 = k0 && x0 == v0;
+  k1 = k1 && x1 == v1;
 }
 
-// Four membership tests at once (contains_pair for four values): v[g] in
-// sorted a[g][0..n[g]); k[g] enters as "still wanted" and leaves as the
-// result.  The four searches advance in lockstep, so up to four loads of one
-// lane are in flight at every stage.  A search that has ended goes on loading
-// from `any` (one readable word) instead of masking its lane off: the steps are
-// selects and not branches (with four branches a step, the walk kernel ran
-// more scalar than vector instructions).
+// Four membership tests at once: v[g] in sorted a[g][0..n[g]) (each lane its
+// own lists); k[g] enters as "still wanted" and leaves as the result.  The four
+// searches advance in lockstep, so up to four loads of one lane are in flight
+// at every stage.  A search that has ended or is not wanted goes on loading the
+// place it found, or `any` (one readable word), instead of masking its lane
+// off: the steps are selects and not branches (with four branches a step, the
+// walk kernel ran more scalar than vector instructions), and the last place not
+// above the value is kept instead of a flag for an equal one (8 vector
+// instructions a step instead of 14).
 __device__ __forceinline__ void contains_quad(const uint32_t *const a[4], const uint32_t n_in[4],
                                               const uint32_t v[4], bool k[4], const uint32_t *any) {
   const uint32_t *p[4];
-  uint32_t n[4];
-  bool f[4];
+  uint32_t n[4], o[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    p[g] = a[g];
-    n[g] = k[g] ? n_in[g] : 0;
-    f[g] = false;
+    k[g] = k[g] && n_in[g];
+    p[g] = k[g] ? a[g] : any;
+    n[g] = k[g] ? n_in[g] : 1;
+    o[g] = 0;
   }
-  while (__any(n[0] | n[1] | n[2] | n[3])) {
+  while (__any((n[0] | n[1] | n[2] | n[3]) > 1)) {
     uint32_t x[4];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) x[g] = ldg(n[g] ? p[g] + (n[g] >> 1) : any);
+    for (int g = 0; g < 4; ++g) x[g] = ldg(p[g] + (o[g] + (n[g] >> 1)));
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const uint32_t h = n[g] >> 1;
-      const bool less = x[g] < v[g];
-      f[g] = f[g] || (n[g] && x[g] == v[g]);
-      p[g] += less ? h + 1 : 0;
-      n[g] = !n[g] ? 0 : less ? n[g] - h - 1 : h;
+      o[g] += x[g] <= v[g] ? h : 0;
+      n[g] -= h;
     }
   }
+  uint32_t x[4];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) k[g] = k[g] && f[g];
+  for (int g = 0; g < 4; ++g) x[g] = ldg(p[g] + o[g]);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) k[g] = k[g] && x[g] == v[g];
 }
 
 // Map a hardware workgroup id to a logical one so that consecutive logical
