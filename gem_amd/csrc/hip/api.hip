@@ -100,6 +100,7 @@ void gem_hip_destroy(gem_ctx *c) {
   for (auto &e : c->ev)
     if (e) (void)hipEventDestroy(e);
   if (c->pinned) (void)hipHostFree(c->pinned);
+  if (c->launch_host) (void)hipHostFree(c->launch_host);
   hipStream_t s = c->stream;
   delete c;  // its remaining device buffers go back to the block cache
   if (s) {

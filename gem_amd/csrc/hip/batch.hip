@@ -65,7 +65,7 @@ static void plan_query(gem_ctx *c, VQueryState &S, const QueryDev &Qd, const uin
   else
     vorder = gem_vertex_order(Qd);
   S.qd = &Qd;
-  replan(c, S, vorder);
+  replan(S, vorder);
 }
 
 // Seed of a query's candidate orders: a hash of its labels and edges, so the
@@ -278,7 +278,7 @@ class ItemRun : public LazyStates {
           V.mnd_all = std::max(V.mnd_all, P.levels[l].ndup);
         }
       }
-    replan(c_, V, V.ranked[0]);
+    replan(V, V.ranked[0]);
     V.cur = 0;
   }
 

@@ -305,6 +305,10 @@ struct gem_ctx {
   void *pinned = nullptr;                   // small pinned staging area
   void *pinned_map = nullptr;               // its device address
   size_t pinned_bytes = 0;
+  // pinned mirror of the batched runs' launch buffers, kept from run to run
+  // (up to 1 MiB; a larger one goes back with its run)
+  void *launch_host = nullptr;
+  size_t launch_host_bytes = 0;
   gemd::Prof prof;
   // the last batched run's level budget and scheduler statistics
   uint64_t last_budget = 0;

@@ -208,8 +208,7 @@ void TableCache::bind(VQueryState &S, size_t i) {
       L.gblk[j] = (uint32_t)base_[i][d];
     }
   }
-  GEM_HIP_CHECK(hipMemcpyAsync(S.levels.p, S.hlv.data(), sizeof(VLevel) * S.hlv.size(), hipMemcpyHostToDevice,
-                               c_->stream));
+  S.dlev = nullptr;  // copied again before the query is seeded
 }
 
 void TableCache::reset_marks() {

@@ -56,6 +56,11 @@ struct LevelBuf : DevBuf {
     uint64_t unit0 = 0, lo = 0, hi = 0;
   };
   mutable Units units;
+  // the identity rows of a first level lie in a buffer that all such levels share
+  std::shared_ptr<DevBuf> shared;
+  ~LevelBuf() {
+    if (shared) p = nullptr;
+  }
 };
 
 // A row whose driving list is too long for one wave: walked in pieces by
@@ -91,8 +96,11 @@ struct VQueryState {
   const gemh::QueryInfo *Qp = nullptr;
   const std::vector<uint32_t> *edge_map = nullptr;
   gemh::VertexPlan plan;
-  DevBuf levels;  // VLevel[nv]
-  std::vector<VLevel> hlv;  // host copy of `levels`
+  std::vector<VLevel> hlv;  // VLevel[nv], host side
+  // the same on the device: in a buffer of the run for the states it starts
+  // with, else in `levels`; null when `hlv` is not there yet (see put_levels)
+  const VLevel *dlev = nullptr;
+  DevBuf levels;
   std::vector<uint32_t> max_nb, max_ndup;  // per level
   std::vector<uint32_t> cols_in;           // per level: columns of its input rows
   // depth-first stack of pending level ranges, counts and limits (host/vsched.h)
@@ -139,9 +147,11 @@ struct LazyStates {
   virtual ~LazyStates() = default;
 };
 
-void build_vlevels(gem_ctx *c, VQueryState &S);
-// The vertex plan of `vorder` for S (S.qd set) and its device level table.
-void replan(gem_ctx *c, VQueryState &S, const std::vector<uint32_t> &vorder);
+void build_vlevels(VQueryState &S);
+// Copies S's level table to the device unless it is there.
+void put_levels(gem_ctx *c, VQueryState &S);
+// The vertex plan of `vorder` for S (S.qd set) and its level table.
+void replan(VQueryState &S, const std::vector<uint32_t> &vorder);
 // Work limit of attempt a (0 = none).
 uint64_t attempt_limit(const VQueryState &S, uint32_t a);
 

@@ -935,7 +935,7 @@ __global__ void k_viota(uint32_t *p, uint64_t n) {
 
 // ================================================================== host
 
-void build_vlevels(gem_ctx *c, VQueryState &S) {
+void build_vlevels(VQueryState &S) {
   const QueryDev &Qd = *S.qd;
   const gemh::VertexPlan &P = S.plan;
   const uint32_t nv = Qd.Q.nv;
@@ -971,19 +971,53 @@ void build_vlevels(gem_ctx *c, VQueryState &S) {
     L.bm_new = Qd.bitmap.as<uint64_t>() + (uint64_t)u * Qd.W;
     L.rank_new = Qd.rank.as<uint32_t>() + (uint64_t)u * (Qd.W + 1);
   }
-  S.levels.alloc(sizeof(VLevel) * nv, c->stream);
-  GEM_HIP_CHECK(hipMemcpyAsync(S.levels.p, lv.data(), sizeof(VLevel) * nv, hipMemcpyHostToDevice, c->stream));
   S.max_nb.assign(nv, 0);
   S.max_ndup.assign(nv, 0);
   for (uint32_t i = 1; i < nv; ++i) {
     S.max_nb[i] = lv[i].nb;
     S.max_ndup[i] = lv[i].ndup;
   }
-  // the copy above reads lv asynchronously: keep it in the query state
   S.hlv = std::move(lv);
+  S.dlev = nullptr;
 }
 
-void replan(gem_ctx *c, VQueryState &S, const std::vector<uint32_t> &vorder) {
+void put_levels(gem_ctx *c, VQueryState &S) {
+  if (S.dlev) return;
+  S.levels.alloc(sizeof(VLevel) * S.hlv.size(), c->stream);
+  GEM_HIP_CHECK(
+      hipMemcpyAsync(S.levels.p, S.hlv.data(), sizeof(VLevel) * S.hlv.size(), hipMemcpyHostToDevice, c->stream));
+  S.dlev = S.levels.as<VLevel>();
+}
+
+// The level tables of the states that a run starts with, in one buffer and one
+// copy (a copy takes 8 us of the stream whatever its size: 20 queries' took
+// a twelfth of their batch).
+struct RunLevels {
+  std::vector<VQueryState *> in;
+  std::vector<VLevel> host;
+  DevBuf dev;
+  RunLevels(gem_ctx *c, const std::vector<VQueryState *> &qs) {
+    for (VQueryState *S : qs)
+      if (!S->pending && !S->dlev && !S->hlv.empty()) {
+        in.push_back(S);
+        host.insert(host.end(), S->hlv.begin(), S->hlv.end());
+      }
+    if (in.empty()) return;
+    dev.alloc(sizeof(VLevel) * host.size(), c->stream);
+    GEM_HIP_CHECK(hipMemcpyAsync(dev.p, host.data(), sizeof(VLevel) * host.size(), hipMemcpyHostToDevice, c->stream));
+    const VLevel *at = dev.as<VLevel>();
+    for (VQueryState *S : in) {
+      S->dlev = at;
+      at += S->hlv.size();
+    }
+  }
+  ~RunLevels() {
+    for (VQueryState *S : in)
+      if (S->dlev >= dev.as<VLevel>() && S->dlev < dev.as<VLevel>() + host.size()) S->dlev = nullptr;
+  }
+};
+
+void replan(VQueryState &S, const std::vector<uint32_t> &vorder) {
   if (gemh::make_vertex_plan(S.Qp ? *S.Qp : S.qd->Q, vorder, &S.plan))
     throw Error{GEM_E_INVALID, "invalid vertex order (leaf first, or a vertex without an earlier neighbour)"};
   if (S.edge_map)
@@ -992,7 +1026,7 @@ void replan(gem_ctx *c, VQueryState &S, const std::vector<uint32_t> &vorder) {
       for (uint32_t j = 0; j < lp.nb; ++j)
         lp.directed[j] = 2 * (*S.edge_map)[lp.directed[j] >> 1] + (lp.directed[j] & 1);
     }
-  build_vlevels(c, S);
+  build_vlevels(S);
   S.mnb_all = std::max(S.mnb_all, *std::max_element(S.max_nb.begin(), S.max_nb.end()));
   S.mnd_all = std::max(S.mnd_all, *std::max_element(S.max_ndup.begin(), S.max_ndup.end()));
 }
@@ -1007,9 +1041,11 @@ uint64_t attempt_limit(const VQueryState &S, uint32_t a) {
 }
 
 // (Re)start a query's attempt: the identity level of its first vertex's
-// candidates, no count yet.
-static void seed_query(gem_ctx *c, VQueryState &V) {
+// candidates, no count yet.  Its rows are the first of `identity`, which grows
+// to the longest such level.
+static void seed_query(gem_ctx *c, VQueryState &V, std::shared_ptr<DevBuf> &identity) {
   hipStream_t s = c->stream;
+  put_levels(c, V);
   gemh::SQuery<LevelBuf> &Q = V.s;
   Q.nb = V.max_nb;
   Q.width = V.cols_in;
@@ -1023,10 +1059,17 @@ static void seed_query(gem_ctx *c, VQueryState &V) {
     Q.done = true;
     return;
   }
+  if (!identity || identity->bytes < n0 * 4) {
+    const uint64_t n = std::max<uint64_t>({n0, identity ? identity->bytes / 2 : 0, 1 << 16});
+    identity = std::make_shared<DevBuf>();
+    identity->alloc(n * 4, s);
+    k_viota<<<(uint32_t)((n + 255) / 256), 256, 0, s>>>(identity->as<uint32_t>(), n);
+    GEM_LAUNCH_CHECK("k_viota");
+  }
   auto buf = std::make_shared<LevelBuf>();
-  buf->alloc(n0 * 4, s);
-  k_viota<<<(uint32_t)((n0 + 255) / 256), 256, 0, s>>>(buf->as<uint32_t>(), n0);
-  GEM_LAUNCH_CHECK("k_viota");
+  buf->shared = identity;
+  buf->p = identity->p;
+  buf->bytes = n0 * 4;
   gemh::SLevel<LevelBuf> L;
   L.level = 1;
   L.rows = std::move(buf);
@@ -1051,19 +1094,6 @@ struct Launch {
   }
   bool empty() const { return items.empty(); }
 };
-
-// Upload an item table + block prefix, return device pointers (kept alive by bufs).
-struct DevLaunch {
-  DevBuf items, blk;
-};
-
-void upload(gem_ctx *c, const Launch &L, DevLaunch &D) {
-  hipStream_t s = c->stream;
-  D.items.alloc(sizeof(VItem) * L.items.size(), s);
-  D.blk.alloc(8 * L.blk.size(), s);
-  GEM_HIP_CHECK(hipMemcpyAsync(D.items.p, L.items.data(), sizeof(VItem) * L.items.size(), hipMemcpyHostToDevice, s));
-  GEM_HIP_CHECK(hipMemcpyAsync(D.blk.p, L.blk.data(), 8 * L.blk.size(), hipMemcpyHostToDevice, s));
-}
 
 // Units of a level that a capped run measures at first (see SchedConfig): of
 // the levels of 16 queries of up to 24 vertices under a cap of 1e9 (2^20 R-MAT),
@@ -1094,11 +1124,12 @@ uint32_t resident_blocks(const void *kernel, size_t lds) {
 // header with the item counts, work queues, heavy-row counts, walked-entry
 // counts and per-task result counters.  Host side: pinned mirrors.  Because
 // every pointer, grid and LDS size is fixed for the run, the step
-//   H2D header, items, prefixes -> 3 kernels -> 2 heavy walks
+//   H2D header, prefixes, items -> 3 kernels -> 2 heavy walks
 //   -> D2H header
 // is captured once as a hipGraph and replayed each iteration (no memset node:
 // the zeroed counters travel in the header copy).
 struct ExtSlot {
+  static constexpr size_t KEEP_LAUNCH = 1 << 20;
   // header: item counts [3], heavy rows and pieces [2 x 2], profile counters [6] (u64:
   // entries walked by the write / final / heavy write / heavy final kernels,
   // bytes written by the write / heavy write kernels), queues [3 main + 2
@@ -1107,10 +1138,19 @@ struct ExtSlot {
   static constexpr size_t HDR_NITEMS = 0, HDR_HEAVYN = 16, HDR_PITEMS = 32, HDR_QUEUE = 128,
                           HDR_CTR = HDR_QUEUE + 5 * 4 * WQ_WORDS, CTR_STRIDE = 8;
   uint32_t cap = 0;  // items per launch = counters
-  DevBuf items[3], blk[3], hdr;
+  // one block, on both sides: header, block prefixes [3][cap + 1] and items
+  // [3][cap] of a step, copied at once (in seven copies they took the stream 60
+  // us), then those of a length pass
+  DevBuf block;
+  unsigned char *host = nullptr;
+  size_t step_bytes = 0, len_bytes = 0;
+  bool own_host = false, in_flight = false;
+  hipStream_t stream = nullptr;
+  const VItem *items[4] = {};
+  const uint64_t *blk[4] = {};
   DevBuf heavy[2], pieces[2];  // heavy rows and the rows of their pieces, per walking launch
-  VItem *h_items[3] = {};
-  uint64_t *h_blk[3] = {};
+  VItem *h_items[4] = {};
+  uint64_t *h_blk[4] = {};
   unsigned char *h_hdr = nullptr;
   size_t hdr_bytes = 0;
   uint32_t max_nb = 1, max_ndup = 0;
@@ -1137,47 +1177,77 @@ struct ExtSlot {
     heavy_t = c->heavy_t;
     heavy_chunk = c->heavy_chunk;
     hdr_bytes = HDR_CTR + 8ull * CTR_STRIDE * cap;
-    hdr.alloc(hdr_bytes, s);
     for (int i = 0; i < 2; ++i) {
       heavy[i].alloc(sizeof(HeavyRow) * HEAVY_CAP, s);
       pieces[i].alloc(4ull * PIECE_CAP, s);
     }
-    GEM_HIP_CHECK(hipHostMalloc((void **)&h_hdr, hdr_bytes, hipHostMallocDefault));
-    for (int i = 0; i < 3; ++i) {
-      items[i].alloc(sizeof(VItem) * cap, s);
-      blk[i].alloc(8ull * (cap + 1), s);
-      GEM_HIP_CHECK(hipHostMalloc((void **)&h_items[i], sizeof(VItem) * cap, hipHostMallocDefault));
-      GEM_HIP_CHECK(hipHostMalloc((void **)&h_blk[i], 8ull * (cap + 1), hipHostMallocDefault));
-      std::memset(h_items[i], 0, sizeof(VItem) * cap);
-      std::memset(h_blk[i], 0, 8ull * (cap + 1));
+    const size_t blk_bytes = 8ull * (cap + 1), item_bytes = sizeof(VItem) * cap;
+    len_bytes = blk_bytes + item_bytes;
+    step_bytes = hdr_bytes + 3 * len_bytes;
+    const size_t bytes = step_bytes + len_bytes;
+    block.alloc(bytes, s);
+    stream = s;
+    if (bytes > c->launch_host_bytes) {
+      void *p = nullptr;
+      const size_t n = std::max<size_t>(bytes, KEEP_LAUNCH / 4);
+      GEM_HIP_CHECK(hipHostMalloc(&p, n, hipHostMallocDefault));
+      if (bytes > KEEP_LAUNCH) {
+        own_host = true;
+      } else {
+        if (c->launch_host) (void)hipHostFree(c->launch_host);
+        c->launch_host = p;
+        c->launch_host_bytes = n;
+      }
+      host = static_cast<unsigned char *>(p);
+    } else {
+      host = static_cast<unsigned char *>(c->launch_host);
     }
-    std::memset(h_hdr, 0, hdr_bytes);
+    std::memset(host, 0, bytes);
+    h_hdr = host;
+    for (int i = 0; i < 4; ++i) {
+      const size_t at = i < 3 ? hdr_bytes + i * blk_bytes : step_bytes;
+      const size_t it = i < 3 ? hdr_bytes + 3 * blk_bytes + i * item_bytes : step_bytes + blk_bytes;
+      h_blk[i] = reinterpret_cast<uint64_t *>(host + at);
+      blk[i] = reinterpret_cast<const uint64_t *>(block.as<unsigned char>() + at);
+      h_items[i] = reinterpret_cast<VItem *>(host + it);
+      items[i] = reinterpret_cast<const VItem *>(block.as<unsigned char>() + it);
+    }
+  }
+  // A launch's items and block prefix to the host side of the block.
+  void fill(int i, const Launch &L) {
+    if (L.items.size() > cap) throw Error{GEM_E_STATE, "more vjoin items than launch slots"};
+    std::copy(L.items.begin(), L.items.end(), h_items[i]);
+    std::copy(L.blk.begin(), L.blk.end(), h_blk[i]);
+    if (L.blk.empty()) h_blk[i][0] = 0;
+  }
+  void copy_length_launch() {
+    GEM_HIP_CHECK(hipMemcpyAsync(block.as<unsigned char>() + step_bytes, host + step_bytes, len_bytes,
+                                 hipMemcpyHostToDevice, stream));
+    in_flight = true;
+  }
+  // Waits for everything enqueued so far; the host side may then be filled anew.
+  void wait() {
+    GEM_HIP_CHECK(hipStreamSynchronize(stream));
+    in_flight = false;
   }
   ~ExtSlot() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
-    if (h_hdr) (void)hipHostFree(h_hdr);
-    for (int i = 0; i < 3; ++i) {
-      if (h_items[i]) (void)hipHostFree(h_items[i]);
-      if (h_blk[i]) (void)hipHostFree(h_blk[i]);
-    }
+    if (in_flight) (void)hipStreamSynchronize(stream);  // an error cut the run short
+    if (own_host) (void)hipHostFree(host);
   }
   uint32_t *nitems(int i) { return reinterpret_cast<uint32_t *>(h_hdr + HDR_NITEMS) + i; }
   uint64_t counter(size_t i) { return reinterpret_cast<uint64_t *>(h_hdr + HDR_CTR)[i * CTR_STRIDE]; }
   uint64_t *pitems() { return reinterpret_cast<uint64_t *>(h_hdr + HDR_PITEMS); }
   unsigned long long *dev_counter(size_t i) {
-    return reinterpret_cast<unsigned long long *>(hdr.as<unsigned char>() + HDR_CTR) + i * CTR_STRIDE;
+    return reinterpret_cast<unsigned long long *>(block.as<unsigned char>() + HDR_CTR) + i * CTR_STRIDE;
   }
 
   // The step's work, enqueued on the stream (eagerly or under capture).
   void enqueue(gem_ctx *c, bool captured, bool prof_kernels, bool count_items) {
     hipStream_t s = c->stream;
-    unsigned char *d = hdr.as<unsigned char>();
-    GEM_HIP_CHECK(hipMemcpyAsync(d, h_hdr, hdr_bytes, hipMemcpyHostToDevice, s));
-    for (int i = 0; i < 3; ++i) {
-      GEM_HIP_CHECK(hipMemcpyAsync(items[i].p, h_items[i], sizeof(VItem) * cap, hipMemcpyHostToDevice, s));
-      GEM_HIP_CHECK(hipMemcpyAsync(blk[i].p, h_blk[i], 8ull * (cap + 1), hipMemcpyHostToDevice, s));
-    }
+    unsigned char *d = block.as<unsigned char>();
+    GEM_HIP_CHECK(hipMemcpyAsync(d, host, step_bytes, hipMemcpyHostToDevice, s));
     const uint32_t *dn = reinterpret_cast<const uint32_t *>(d + HDR_NITEMS);
     unsigned int *dq = reinterpret_cast<unsigned int *>(d + HDR_QUEUE);
     unsigned int *hn = reinterpret_cast<unsigned int *>(d + HDR_HEAVYN);
@@ -1201,36 +1271,36 @@ struct ExtSlot {
                       unsigned int *hn, bool prof_kernels, bool count_items, uint64_t b0, uint64_t e0, uint64_t b1,
                       uint64_t e1, uint64_t b2, uint64_t e2) {
     hipStream_t s = c->stream;
-    unsigned long long *dp = reinterpret_cast<unsigned long long *>(hdr.as<unsigned char>() + HDR_PITEMS);
+    unsigned long long *dp = reinterpret_cast<unsigned long long *>(block.as<unsigned char>() + HDR_PITEMS);
     if (b0 < e0) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_WRITE : -1);
-      k_vext<false, OOC><<<std::min(most, grid[0]), VB, lds, s>>>(items[0].as<VItem>(), dn + 0, blk[0].as<uint64_t>(), dq + 0, lcap, dcap,
+      k_vext<false, OOC><<<std::min(most, grid[0]), VB, lds, s>>>(items[0], dn + 0, blk[0], dq + 0, lcap, dcap,
                                                count_items ? dp : nullptr, count_items ? dp + 4 : nullptr,
                                                b0, e0, heavy_out(0, hn));
       GEM_LAUNCH_CHECK("k_vext<write>");
     }
     if (b1 < e1) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_FINAL : -1);
-      k_vext<true, OOC><<<std::min(most, grid[1]), VB, lds, s>>>(items[1].as<VItem>(), dn + 1, blk[1].as<uint64_t>(), dq + WQ_WORDS, lcap, dcap,
+      k_vext<true, OOC><<<std::min(most, grid[1]), VB, lds, s>>>(items[1], dn + 1, blk[1], dq + WQ_WORDS, lcap, dcap,
                                               count_items ? dp + 1 : nullptr, nullptr, b1, e1,
                                               heavy_out(1, hn));
       GEM_LAUNCH_CHECK("k_vext<final>");
     }
     if (b2 < e2) {
       ProfLaunch pl(c, prof_kernels ? K_VCOUNT1 : -1);
-      k_vcount1<OOC><<<std::min(most, grid[2]), VB, 0, s>>>(items[2].as<VItem>(), dn + 2, blk[2].as<uint64_t>(), dq + 2 * WQ_WORDS, b2, e2);
+      k_vcount1<OOC><<<std::min(most, grid[2]), VB, 0, s>>>(items[2], dn + 2, blk[2], dq + 2 * WQ_WORDS, b2, e2);
       GEM_LAUNCH_CHECK("k_vcount1");
     }
     if (b0 < e0) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_HEAVY_WRITE : -1);
-      k_vext_heavy<false, OOC><<<std::min(most, grid[3]), VB, 0, s>>>(items[0].as<VItem>(), heavy_out(0, hn), hq + 0,
+      k_vext_heavy<false, OOC><<<std::min(most, grid[3]), VB, 0, s>>>(items[0], heavy_out(0, hn), hq + 0,
                                                                       count_items ? dp + 2 : nullptr,
                                                                       count_items ? dp + 5 : nullptr);
       GEM_LAUNCH_CHECK("k_vext_heavy<write>");
     }
     if (b1 < e1) {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_HEAVY_FINAL : -1);
-      k_vext_heavy<true, OOC><<<std::min(most, grid[4]), VB, 0, s>>>(items[1].as<VItem>(), heavy_out(1, hn),
+      k_vext_heavy<true, OOC><<<std::min(most, grid[4]), VB, 0, s>>>(items[1], heavy_out(1, hn),
                                                                      hq + WQ_WORDS, count_items ? dp + 3 : nullptr,
                                                                      nullptr);
       GEM_LAUNCH_CHECK("k_vext_heavy<final>");
@@ -1241,13 +1311,12 @@ struct ExtSlot {
   // blocks are copied in while the previous group runs (eager launches only).
   void launch_streamed(gem_ctx *c, TableCache &tc) {
     hipStream_t s = c->stream;
-    unsigned char *d = hdr.as<unsigned char>();
-    GEM_HIP_CHECK(hipMemcpyAsync(d, h_hdr, hdr_bytes, hipMemcpyHostToDevice, s));
+    in_flight = true;
+    unsigned char *d = block.as<unsigned char>();
+    GEM_HIP_CHECK(hipMemcpyAsync(d, host, step_bytes, hipMemcpyHostToDevice, s));
     uint64_t T[3], base[3];
     uint64_t total = 0;
     for (int i = 0; i < 3; ++i) {
-      GEM_HIP_CHECK(hipMemcpyAsync(items[i].p, h_items[i], sizeof(VItem) * cap, hipMemcpyHostToDevice, s));
-      GEM_HIP_CHECK(hipMemcpyAsync(blk[i].p, h_blk[i], 8ull * (cap + 1), hipMemcpyHostToDevice, s));
       T[i] = *nitems(i) ? h_blk[i][*nitems(i)] : 0;
       base[i] = total;
       total += T[i];
@@ -1266,7 +1335,7 @@ struct ExtSlot {
         if (!T[i] || base[i] + T[i] <= wa || base[i] >= wb) continue;
         const uint64_t lo = std::max(wa, base[i]), hi = std::min(wb, base[i] + T[i]);
         k_vmark<<<(uint32_t)std::min<uint64_t>(hi - lo, 4096), VB, 0, s>>>(
-            items[i].as<VItem>(), *nitems(i), blk[i].as<uint64_t>(), base[i], wa, wb, i == 2, tc.d_first(),
+            items[i], *nitems(i), blk[i], base[i], wa, wb, i == 2, tc.d_first(),
             tc.d_last());
         GEM_LAUNCH_CHECK("k_vmark");
       }
@@ -1305,6 +1374,7 @@ struct ExtSlot {
   }
 
   void launch(gem_ctx *c, bool use_graph) {
+    in_flight = true;
     if (!use_graph) {
       enqueue(c, false, c->prof.on, c->prof.on);
       return;
@@ -1348,6 +1418,7 @@ struct HipSchedBackend {
   clk::time_point last_print = clk::now();
   double t_len = 0, t_ext = 0;
   uint64_t ext_tasks = 0;
+  std::shared_ptr<DevBuf> identity;  // 0, 1, 2, ... (see seed_query)
 
   static uint64_t buf_bytes(const LevelBuf &b) { return b.bytes; }
 
@@ -1364,7 +1435,7 @@ struct HipSchedBackend {
 
   VItem vitem(const Item &x) const {
     VItem it{};
-    it.lv = qs[x.q]->levels.as<VLevel>() + x.level;
+    it.lv = qs[x.q]->dlev + x.level;
     it.rows = x.rows->as<uint32_t>();
     it.row_begin = x.row_begin;
     it.row_end = x.row_end;
@@ -1377,8 +1448,8 @@ struct HipSchedBackend {
     hipStream_t s = c->stream;
     Launch L;
     for (const Item &x : items) L.add(vitem(x), qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level]);
-    DevLaunch D;
-    upload(c, L, D);
+    slot.fill(3, L);
+    slot.copy_length_launch();
     const uint64_t nblk = L.blk.back(), nunit = nblk * VW;
     DevBuf bu;
     auto kept = std::make_shared<DevBuf>();  // the unit prefix, which the levels keep for their write walks
@@ -1387,8 +1458,7 @@ struct HipSchedBackend {
     bp.alloc((nunit + 1) * 8, s);
     {
       ProfLaunch pl(c, K_VLEN);
-      k_vlen<<<grid_for(nblk), VB, 0, s>>>(D.items.as<VItem>(), (uint32_t)L.items.size(), D.blk.as<uint64_t>(),
-                                            bu.as<uint64_t>());
+      k_vlen<<<grid_for(nblk), VB, 0, s>>>(slot.items[3], (uint32_t)L.items.size(), slot.blk[3], bu.as<uint64_t>());
       GEM_LAUNCH_CHECK("k_vlen");
     }
     scan_u64(c, bu.as<uint64_t>(), bp.as<uint64_t>(), nunit);
@@ -1399,7 +1469,7 @@ struct HipSchedBackend {
     if (!prefix) return;
     uint64_t *pref = pinned<uint64_t>(c, nunit + 1);
     GEM_HIP_CHECK(hipMemcpyAsync(pref, bp.p, (nunit + 1) * 8, hipMemcpyDeviceToHost, s));
-    GEM_HIP_CHECK(hipStreamSynchronize(s));
+    slot.wait();
     prefix->resize(items.size());
     for (size_t t = 0; t < items.size(); ++t) {
       const Item &x = items[t];
@@ -1438,7 +1508,6 @@ struct HipSchedBackend {
   void extend(const std::vector<Item> &wr_items, const std::vector<Item> &fin_items, std::vector<uint64_t> *got_wr,
               std::vector<uint64_t> *got_fin) {
     const auto t0 = clk::now();
-    hipStream_t s = c->stream;
     // launch tables: write walks, final walks, final single-list counts; one
     // u64 result counter per item, in the device header
     Launch wr, fin, fin1;
@@ -1487,10 +1556,7 @@ struct HipSchedBackend {
     Launch *L3[3] = {&wr, &fin, &fin1};
     for (int i = 0; i < 3; ++i) {
       Launch &L = *L3[i];
-      if (L.items.size() > slot.cap) throw Error{GEM_E_STATE, "more vjoin items than launch slots"};
-      for (size_t t = 0; t < L.items.size(); ++t) slot.h_items[i][t] = L.items[t];
-      for (size_t t = 0; t < L.blk.size(); ++t) slot.h_blk[i][t] = L.blk[t];
-      if (L.blk.empty()) slot.h_blk[i][0] = 0;
+      slot.fill(i, L);
       *slot.nitems(i) = (uint32_t)L.items.size();
       ext_tasks += L.blk.empty() ? 0 : L.blk.back();
     }
@@ -1499,7 +1565,7 @@ struct HipSchedBackend {
       slot.launch_streamed(c, *tc);
     else
       slot.launch(c, c->use_graph && !prof);
-    GEM_HIP_CHECK(hipStreamSynchronize(s));
+    slot.wait();
     if (tc) tc->finish();
     for (auto &r : replaced) r.first->units = r.second;
     got_wr->resize(wr_items.size());
@@ -1609,7 +1675,7 @@ struct HipSchedBackend {
       const uint32_t a = P.s.attempts;
       V.shift = (P.cur + 1 + K - a % K) % K;
       V.cur = (a + V.shift) % K;
-      replan(c, V, V.ranked[V.cur]);
+      replan(V, V.ranked[V.cur]);
       V.s.nb = V.max_nb;
       if (V.mnb_all > slot.max_nb || V.mnd_all > slot.max_ndup)
         throw Error{GEM_E_STATE, "racing order needs more launch LDS than the run was sized for"};
@@ -1622,7 +1688,7 @@ struct HipSchedBackend {
         std::fflush(stderr);
       }
     }
-    seed_query(c, V);
+    seed_query(c, V, identity);
   }
 
   // The attempt of query qi went past its limit with its levels still
@@ -1671,14 +1737,14 @@ struct HipSchedBackend {
         if (V.rate[j] > V.rate[best]) best = j;
       if (V.rate[best] > 0) V.cur = best;
     }
-    replan(c, V, V.ranked[V.cur]);
+    replan(V, V.ranked[V.cur]);
     if (tc) tc->bind(V, qi);
     if (V.mnb_all > slot.max_nb || V.mnd_all > slot.max_ndup)
       throw Error{GEM_E_STATE, "restart order needs more launch LDS than the run was sized for"};
     Q.attempts = a;
     Q.attempt_start = Q.work;
     Q.attempt_limit = attempt_limit(V, a);
-    seed_query(c, V);
+    seed_query(c, V, identity);
     if (verbose) {
       std::fprintf(stderr, "[vjoin] query %u: attempt %u with order %u, limit %.3g\n", qi, a, V.ranked_idx[V.cur],
                    (double)Q.attempt_limit);
@@ -1771,6 +1837,7 @@ void VBatchRunner::run(std::vector<VQueryState *> &qs) {
   }
   const char *verbose_env = std::getenv("GEM_VERBOSE");
   const bool verbose = verbose_env && verbose_env[0] == '1';
+  RunLevels levels(c_, qs);
   HipSchedBackend be{c_, qs, slot, tc.get(), verbose, cap_, lazy_};
   gemh::SchedConfig cfg;
   cfg.cap = cap_;
