@@ -111,12 +111,19 @@ void run_match_batch(gem_ctx *c, const gem_query_view *qs, uint32_t nq, const ui
     std::vector<QueryDev> qd(gn);
     std::vector<VQueryState> st(gn);
     std::vector<VQueryState *> ptrs;
-    for (uint32_t i = 0; i < gn; ++i) {
-      run_filter(c, qd[i], &qs[g0 + i], 0);
-      run_tables(c, qd[i]);
-      plan_query(c, st[i], qd[i], vorders ? vorders[g0 + i] : nullptr);
-      if (streamed) spill_tables(c, qd[i], c->stream_slot_bytes);
-      ptrs.push_back(&st[i]);
+    // (streamed tables leave the device one query at a time)
+    const uint32_t at_once = streamed ? 1 : PREPARE_GROUP;
+    for (uint32_t i0 = 0; i0 < gn; i0 += at_once) {
+      const uint32_t n = std::min(at_once, gn - i0);
+      const gem_query_view *views[PREPARE_GROUP];
+      for (uint32_t i = 0; i < n; ++i) views[i] = &qs[g0 + i0 + i];
+      run_filters(c, &qd[i0], views, n, 0);
+      run_tables(c, &qd[i0], n, false);
+      for (uint32_t i = i0; i < i0 + n; ++i) {
+        plan_query(c, st[i], qd[i], vorders ? vorders[g0 + i] : nullptr);
+        if (streamed) spill_tables(c, qd[i], c->stream_slot_bytes);
+        ptrs.push_back(&st[i]);
+      }
     }
     VBatchRunner runner(c, o.cap, o.work_limit, budget, streamed);
     runner.run(ptrs);
@@ -517,15 +524,17 @@ void run_match_batch_learned(gem_ctx *c, const gem_query_view *qs, uint32_t nq, 
     ItemRun run(c, items, mlp, max_orders, o);
     double t_filter = 0, t_tables = 0;
     const auto t_prep = clk::now();
-    for (uint32_t i = 0; i < eager; ++i) {
+    const uint32_t at_once = streamed ? 1 : PREPARE_GROUP;
+    for (uint32_t i0 = 0; i0 < eager; i0 += at_once) {
+      const uint32_t n = std::min(at_once, eager - i0);
       const auto ta = clk::now();
-      run_filter(c, qd[i], views[i], 0);
+      run_filters(c, &qd[i0], &views[i0], n, 0);
       const auto tb = clk::now();
-      run_tables(c, qd[i]);
-      if (streamed) spill_tables(c, qd[i], c->stream_slot_bytes);
+      run_tables(c, &qd[i0], n, false);
+      if (streamed) spill_tables(c, qd[i0], c->stream_slot_bytes);
       t_filter += secs(ta, tb);
       t_tables += secs(tb, clk::now());
-      run.candidates(c, i);
+      for (uint32_t i = i0; i < i0 + n; ++i) run.candidates(c, i);
     }
     {
       std::unique_ptr<Preparer> prep;

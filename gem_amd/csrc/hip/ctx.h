@@ -419,8 +419,16 @@ inline const GraphDev &graph(const gem_ctx *c) { return c->gsrc ? *c->gsrc : c->
 void make_slot_labels(gem_ctx *c, GraphDev &G);
 void run_filter(gem_ctx *c, const gem_query_view *qv, uint32_t T);
 void run_tables(gem_ctx *c);
-// the same phases on an explicit per-query state (several queries resident)
+// the same phases on an explicit per-query state (several queries resident),
 void run_filter(gem_ctx *c, QueryDev &Qd, const gem_query_view *qv, uint32_t T);
+// and on n of them: enqueued one after the other, waited for once (the waits
+// of a query at a time, with the copies between them, took half of the
+// preparation of 20 small queries)
+void run_filters(gem_ctx *c, QueryDev *Qd, const gem_query_view *const *qv, uint32_t n, uint32_t T);
+void run_tables(gem_ctx *c, QueryDev *Qd, uint32_t n, bool wait);
+// run_filters and run_tables over n queries, at most PREPARE_GROUP at a time
+// (their scratch memory is held meanwhile)
+constexpr uint32_t PREPARE_GROUP = 32;
 // The filter into caller-owned device arrays with the library's fixed scratch
 // array (no allocation); filter_scratch_init finds that array's address on
 // the current device (once per device, at context creation).

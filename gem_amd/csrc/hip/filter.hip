@@ -469,57 +469,77 @@ static void filter_launch(gem_ctx *c, uint32_t nv, uint32_t W, const FilterPrep 
 
 void run_filter(gem_ctx *c, const gem_query_view *qv, uint32_t T) { run_filter(c, c->q, qv, T); }
 
-void run_filter(gem_ctx *c, QueryDev &Qd, const gem_query_view *qv, uint32_t T) {
-  if (!graph(c).loaded) throw Error{GEM_E_STATE, "no data graph loaded"};
-  Qd = QueryDev();
-  std::string why;
-  int st = gemh::analyse_query(qv, &Qd.Q, &why);
-  if (st) throw Error{st, why};
-  const gemh::QueryInfo &Q = Qd.Q;
-  const GraphDev &G = graph(c);
-  const uint32_t nv = Q.nv;
-  const uint32_t W = (G.n + 63) / 64;
-  Qd.W = W;
-  FilterPrep P;
-  filter_prepare(G, Q, T, W, &P);
-  Qd.can_off = P.can_off;
+void run_filter(gem_ctx *c, QueryDev &Qd, const gem_query_view *qv, uint32_t T) { run_filters(c, &Qd, &qv, 1, T); }
 
-  hipStream_t s = c->stream;
-  GEM_HIP_CHECK(hipEventRecord(c->ev[0], s));
-  FilterBufs B;
-  DevBuf slot_of, sums;
-  if (!G.lab8) {
-    slot_of.alloc(P.slot_of.size(), s);
-    GEM_HIP_CHECK(hipMemcpyAsync(slot_of.p, P.slot_of.data(), P.slot_of.size(), hipMemcpyHostToDevice, s));
+void run_filters(gem_ctx *c, QueryDev *Qds, const gem_query_view *const *qv, uint32_t n, uint32_t T) {
+  if (!graph(c).loaded) throw Error{GEM_E_STATE, "no data graph loaded"};
+  const GraphDev &G = graph(c);
+  const uint32_t W = (G.n + 63) / 64;
+  uint32_t nvs = 0;
+  for (uint32_t i = 0; i < n; ++i) {
+    Qds[i] = QueryDev();
+    std::string why;
+    int st = gemh::analyse_query(qv[i], &Qds[i].Q, &why);
+    if (st) throw Error{st, why};
+    nvs += Qds[i].Q.nv;
   }
-  Qd.bitmap.alloc((uint64_t)nv * W * 8, s);
-  Qd.rank.alloc((uint64_t)nv * (W + 1) * 4, s);
-  Qd.can.alloc(std::max<uint64_t>(Qd.can_off[nv], 1) * 4, s);
-  sums.alloc((uint64_t)nv * rank_chunks(W) * 4, s);
-  B.slot_of = slot_of.as<uint8_t>();
-  B.bitmap = Qd.bitmap.as<uint64_t>();
-  B.sums = sums.as<uint32_t>();
-  B.rank = Qd.rank.as<uint32_t>();
-  B.can = Qd.can.as<uint32_t>();
-  uint32_t *h = pinned<uint32_t>(c, nv);  // written by the last kernel
-  B.ncan = pinned_dev(c, h);
-  filter_launch(c, nv, W, P, Qd.can_off.data(), B);
-  // algorithmic bytes: 16 B per vertex (label, degree, offset pair), 8 B per
-  // adjacency slot of a label-matching vertex (neighbour id + its label; 1 B
-  // with slot labels), the candidate bitmaps written
-  prof_bytes(c, K_FILTER, 16.0 * G.n + (G.nbr_lab.p ? 1.0 : 8.0) * P.adj + nv * (double)W * 8);
-  GEM_HIP_CHECK(hipEventRecord(c->ev[1], s));
+  struct Run {
+    FilterPrep P;
+    DevBuf slot_of, sums;
+  };
+  std::vector<Run> runs(n);
+  uint32_t *const h = pinned<uint32_t>(c, nvs);  // |Can(u)|, written by the last kernel of each
+  hipStream_t s = c->stream;
+  uint32_t *hq = h;
+  for (uint32_t i = 0; i < n; ++i) {
+    QueryDev &Qd = Qds[i];
+    const uint32_t nv = Qd.Q.nv;
+    FilterPrep &P = runs[i].P;
+    Qd.W = W;
+    filter_prepare(G, Qd.Q, T, W, &P);
+    Qd.can_off = P.can_off;
+    GEM_HIP_CHECK(hipEventRecord(c->ev[0], s));
+    FilterBufs B;
+    DevBuf &slot_of = runs[i].slot_of, &sums = runs[i].sums;
+    if (!G.lab8) {
+      slot_of.alloc(P.slot_of.size(), s);
+      GEM_HIP_CHECK(hipMemcpyAsync(slot_of.p, P.slot_of.data(), P.slot_of.size(), hipMemcpyHostToDevice, s));
+    }
+    Qd.bitmap.alloc((uint64_t)nv * W * 8, s);
+    Qd.rank.alloc((uint64_t)nv * (W + 1) * 4, s);
+    Qd.can.alloc(std::max<uint64_t>(Qd.can_off[nv], 1) * 4, s);
+    sums.alloc((uint64_t)nv * rank_chunks(W) * 4, s);
+    B.slot_of = slot_of.as<uint8_t>();
+    B.bitmap = Qd.bitmap.as<uint64_t>();
+    B.sums = sums.as<uint32_t>();
+    B.rank = Qd.rank.as<uint32_t>();
+    B.can = Qd.can.as<uint32_t>();
+    B.ncan = pinned_dev(c, hq);
+    hq += nv;
+    filter_launch(c, nv, W, P, Qd.can_off.data(), B);
+    // algorithmic bytes: 16 B per vertex (label, degree, offset pair), 8 B per
+    // adjacency slot of a label-matching vertex (neighbour id + its label; 1 B
+    // with slot labels), the candidate bitmaps written
+    prof_bytes(c, K_FILTER, 16.0 * G.n + (G.nbr_lab.p ? 1.0 : 8.0) * P.adj + nv * (double)W * 8);
+    GEM_HIP_CHECK(hipEventRecord(c->ev[1], s));
+  }
   GEM_HIP_CHECK(hipStreamSynchronize(s));
-  Qd.ncan.assign(h, h + nv);
-  double ncan_sum = 0;
-  for (uint32_t u = 0; u < nv; ++u) ncan_sum += Qd.ncan[u];
-  prof_bytes(c, K_COMPACT, nv * (double)W * 12 + 4.0 * ncan_sum);
+  hq = h;
+  for (uint32_t i = 0; i < n; ++i) {
+    QueryDev &Qd = Qds[i];
+    const uint32_t nv = Qd.Q.nv;
+    Qd.ncan.assign(hq, hq + nv);
+    hq += nv;
+    double ncan_sum = 0;
+    for (uint32_t u = 0; u < nv; ++u) ncan_sum += Qd.ncan[u];
+    prof_bytes(c, K_COMPACT, nv * (double)W * 12 + 4.0 * ncan_sum);
+    Qd.filtered = true;
+  }
   prof_flush(c);
-  float ms = 0;
+  float ms = 0;  // the last query's
   GEM_HIP_CHECK(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
   c->times.filter_ms = ms;
   c->times.index_ms = 0;  // the index (bitmap + rank) is a by-product of the filter
-  Qd.filtered = true;
 }
 
 // ------------------------------------------------ no-allocation variant

@@ -314,9 +314,10 @@ struct TableRun {
   TableJob job{};
   uint32_t waves = 0, ndmax = 1;
   uint64_t rows_bound = 0, pieces_bound = 0;  // heavy rows and pieces there can be
-  DevBuf params, heavy, piece_row, ccnt;
+  DevBuf heavy, piece_row, ccnt;
   TableDesc *desc = nullptr;
   TableCtr *ctr = nullptr;
+  std::vector<uint32_t> desc_tab;  // TableDesc index -> directed edge
 
   template <bool WRITE, bool NL>
   void pass_as() {
@@ -351,32 +352,29 @@ struct TableRun {
   }
 };
 
-void run_tables(gem_ctx *c, QueryDev &Qd, bool wait) {
-  if (!Qd.filtered) throw Error{GEM_E_STATE, "filter has not run"};
-  const gemh::QueryInfo &Q = Qd.Q;
-  const GraphDev &G = graph(c);
-  hipStream_t s = c->stream;
-  GEM_HIP_CHECK(hipEventRecord(c->ev[2], s));
+// The tables of Qd's query, without their values, and its launches' sizes.
+static void plan_tables(TableRun &R) {
+  const gemh::QueryInfo &Q = R.Qd.Q;
+  const GraphDev &G = R.G;
+  QueryDev &Qd = R.Qd;
   Qd.tab.clear();
   Qd.tab.resize(2 * Q.ne);
-  TableRun R{c, G, Qd};
   TableJob &job = R.job;
   job.W = Qd.W;
-  std::vector<uint32_t> desc_tab;  // TableDesc index -> directed edge
   for (uint32_t u = 0; u < Q.nv; ++u) {
     if (Q.deg[u] == 1) continue;  // leaves key no table (unifiedTrie.cu:1045,1095)
     const uint32_t ju = job.nu++;
     job.ncan[ju] = Qd.ncan[u];
     job.can_off[ju] = Qd.can_off[u];
-    job.tab0[ju] = (uint32_t)desc_tab.size();
+    job.tab0[ju] = (uint32_t)R.desc_tab.size();
     for (auto [un, e] : Q.adj[u]) {
       const uint32_t d = 2 * e + (Q.edges[e].first == u ? 0 : 1);
       TableDev &T = Qd.tab[d];
       T.present = true;
       T.key_u = u;
       T.val_u = un;
-      T.off.alloc(((uint64_t)Qd.ncan[u] + 1) * 8, s);
-      desc_tab.push_back(d);
+      T.off.alloc(((uint64_t)Qd.ncan[u] + 1) * 8, R.c->stream);
+      R.desc_tab.push_back(d);
       job.nd[ju]++;
     }
     R.ndmax = std::max(R.ndmax, job.nd[ju]);
@@ -395,67 +393,100 @@ void run_tables(gem_ctx *c, QueryDev &Qd, bool wait) {
     if (job.rows == MIN_ROWS || R.waves >= ENOUGH_WAVES / 2) break;
   }
   job.wave_start[job.nu] = R.waves;
-  // Parameters of the build: one staging block, one device block: the tables,
+}
+
+void run_tables(gem_ctx *c, QueryDev &Qd, bool wait) { run_tables(c, &Qd, 1, wait); }
+
+void run_tables(gem_ctx *c, QueryDev *Qds, uint32_t n, bool wait) {
+  const GraphDev &G = graph(c);
+  hipStream_t s = c->stream;
+  for (uint32_t i = 0; i < n; ++i)
+    if (!Qds[i].filtered) throw Error{GEM_E_STATE, "filter has not run"};
+  GEM_HIP_CHECK(hipEventRecord(c->ev[2], s));
+  std::vector<TableRun> runs;
+  runs.reserve(n);
+  size_t nt = 0;
+  for (uint32_t i = 0; i < n; ++i) {
+    runs.push_back(TableRun{c, G, Qds[i]});
+    plan_tables(runs.back());
+    nt += runs.back().desc_tab.size();
+  }
+  // Parameters of the builds: one staging block, one device block: the tables,
   // the scan segments (and, before them on the host, the sizes that the scan
   // writes), the counters.
-  const size_t nt = desc_tab.size();
   const size_t at_seg = nt * sizeof(TableDesc), at_ctr = at_seg + nt * sizeof(ScanSeg);
-  const size_t bytes = at_ctr + sizeof(TableCtr);
+  const size_t bytes = at_ctr + n * sizeof(TableCtr);
   uint64_t *sizes = pinned<uint64_t>(c, nt + (bytes + 7) / 8);
   unsigned char *stage = reinterpret_cast<unsigned char *>(sizes + nt);
   TableDesc *hdesc = reinterpret_cast<TableDesc *>(stage);
   ScanSeg *hseg = reinterpret_cast<ScanSeg *>(stage + at_seg);
+  DevBuf params;
+  params.alloc(bytes, s);
+  unsigned char *dev = params.as<unsigned char>();
   uint32_t chunks = 0;
-  for (size_t k = 0; k < nt; ++k) {
-    const TableDev &T = Qd.tab[desc_tab[k]];
-    auto it = G.label_id.find(Q.lab[T.val_u]);
-    hdesc[k] = TableDesc{T.val_u, it == G.label_id.end() ? ~0u : it->second, T.off.as<uint64_t>(), nullptr};
-    hseg[k] = ScanSeg{T.off.as<uint64_t>(), (uint64_t)Qd.ncan[T.key_u], chunks};
-    chunks += scan_chunks(Qd.ncan[T.key_u]);
+  size_t k = 0;
+  for (uint32_t i = 0; i < n; ++i) {
+    TableRun &R = runs[i];
+    R.desc = reinterpret_cast<TableDesc *>(dev) + k;
+    R.ctr = reinterpret_cast<TableCtr *>(dev + at_ctr) + i;
+    for (uint32_t d : R.desc_tab) {
+      const TableDev &T = R.Qd.tab[d];
+      auto it = G.label_id.find(R.Qd.Q.lab[T.val_u]);
+      hdesc[k] = TableDesc{T.val_u, it == G.label_id.end() ? ~0u : it->second, T.off.as<uint64_t>(), nullptr};
+      hseg[k] = ScanSeg{T.off.as<uint64_t>(), (uint64_t)R.Qd.ncan[T.key_u], chunks};
+      chunks += scan_chunks(R.Qd.ncan[T.key_u]);
+      ++k;
+    }
+    reinterpret_cast<TableCtr *>(stage + at_ctr)[i] = TableCtr{};
   }
-  *reinterpret_cast<TableCtr *>(stage + at_ctr) = TableCtr{};
-  R.params.alloc(bytes, s);
-  unsigned char *dev = R.params.as<unsigned char>();
-  R.desc = reinterpret_cast<TableDesc *>(dev);
-  R.ctr = reinterpret_cast<TableCtr *>(dev + at_ctr);
   GEM_HIP_CHECK(hipMemcpyAsync(dev, stage, bytes, hipMemcpyHostToDevice, s));
-  if (R.rows_bound) {
-    R.heavy.alloc(R.rows_bound * sizeof(HeavyTab), s);
-    R.piece_row.alloc(R.pieces_bound * 4, s);
-    R.ccnt.alloc(R.pieces_bound * R.ndmax * 4, s);
+  for (TableRun &R : runs) {
+    if (R.rows_bound) {
+      R.heavy.alloc(R.rows_bound * sizeof(HeavyTab), s);
+      R.piece_row.alloc(R.pieces_bound * 4, s);
+      R.ccnt.alloc(R.pieces_bound * R.ndmax * 4, s);
+    }
+    R.pass(false);
   }
-  R.pass(false);
   // row counts -> offsets of every table, the sizes straight to the host
   scan_segments_u64(c, reinterpret_cast<ScanSeg *>(dev + at_seg), (uint32_t)nt, chunks, pinned_dev(c, sizes));
   GEM_HIP_CHECK(hipStreamSynchronize(s));
-  for (size_t k = 0; k < nt; ++k) {
-    TableDev &T = Qd.tab[desc_tab[k]];
-    T.size = sizes[k];
-    T.val.alloc(std::max<uint64_t>(T.size, 1) * 4, s);
-    hdesc[k].val = T.val.as<uint32_t>();
-  }
-  if (c->prof.on) {
-    // algorithmic bytes: per keyed u, its candidates (4 B), offset pairs (8 B)
-    // and adjacency (4 B per slot) once for all its tables; per table the value
-    // vertex's bitmap (|V|/8) and the row counts / offsets (8 B per row)
-    TableCtr h;
-    GEM_HIP_CHECK(hipMemcpyAsync(&h, R.ctr, sizeof(h), hipMemcpyDeviceToHost, s));
-    GEM_HIP_CHECK(hipStreamSynchronize(s));
-    double shared_bytes = 0, count_bytes = 0, write_bytes = 0;
-    for (uint32_t ju = 0; ju < job.nu; ++ju) shared_bytes += 12.0 * job.ncan[ju] + 4.0 * (double)h.adj_len[ju];
-    for (size_t k = 0; k < nt; ++k) {
-      const TableDev &T = Qd.tab[desc_tab[k]];
-      count_bytes += 8.0 * Qd.W + 8.0 * Qd.ncan[T.key_u];
-      write_bytes += 12.0 * Qd.W + 8.0 * Qd.ncan[T.key_u] + 4.0 * (double)T.size;
+  k = 0;
+  for (TableRun &R : runs) {
+    const size_t k0 = k;
+    for (uint32_t d : R.desc_tab) {
+      TableDev &T = R.Qd.tab[d];
+      T.size = sizes[k];
+      T.val.alloc(std::max<uint64_t>(T.size, 1) * 4, s);
+      hdesc[k++].val = T.val.as<uint32_t>();
     }
-    prof_bytes(c, K_TABLES_COUNT, shared_bytes + count_bytes);
-    prof_bytes(c, K_TABLES_WRITE, shared_bytes + write_bytes);
+    if (c->prof.on) {
+      // algorithmic bytes: per keyed u, its candidates (4 B), offset pairs (8 B)
+      // and adjacency (4 B per slot) once for all its tables; per table the value
+      // vertex's bitmap (|V|/8) and the row counts / offsets (8 B per row)
+      TableCtr h;
+      GEM_HIP_CHECK(hipMemcpyAsync(&h, R.ctr, sizeof(h), hipMemcpyDeviceToHost, s));
+      GEM_HIP_CHECK(hipStreamSynchronize(s));
+      const TableJob &job = R.job;
+      const QueryDev &Qd = R.Qd;
+      double shared_bytes = 0, count_bytes = 0, write_bytes = 0;
+      for (uint32_t ju = 0; ju < job.nu; ++ju) shared_bytes += 12.0 * job.ncan[ju] + 4.0 * (double)h.adj_len[ju];
+      for (size_t x = k0; x < k; ++x) {
+        const TableDev &T = Qd.tab[R.desc_tab[x - k0]];
+        count_bytes += 8.0 * Qd.W + 8.0 * Qd.ncan[T.key_u];
+        write_bytes += 12.0 * Qd.W + 8.0 * Qd.ncan[T.key_u] + 4.0 * (double)T.size;
+      }
+      prof_bytes(c, K_TABLES_COUNT, shared_bytes + count_bytes);
+      prof_bytes(c, K_TABLES_WRITE, shared_bytes + write_bytes);
+    }
   }
   GEM_HIP_CHECK(hipMemcpyAsync(dev, stage, nt * sizeof(TableDesc), hipMemcpyHostToDevice, s));
-  R.pass(true);
+  for (TableRun &R : runs) {
+    R.pass(true);
+    R.Qd.tabled = true;
+  }
   GEM_HIP_CHECK(hipEventRecord(c->ev[3], s));
   c->tables_timed = true;
-  Qd.tabled = true;
   if (wait || c->prof.on) {
     GEM_HIP_CHECK(hipStreamSynchronize(s));
     prof_flush(c);
