@@ -69,13 +69,6 @@ using CLevel = GEM_CONST VLevel;
 using CItem = GEM_CONST VItem;
 using CWord = GEM_CONST uint64_t;
 
-// Two neighbouring offsets (start and end of a list) in one 16-byte load.
-typedef uint64_t u64x2 __attribute__((ext_vector_type(2), aligned(8)));
-__device__ __forceinline__ u64x2 ld_pair(const uint64_t *p) {
-  return *(const __attribute__((address_space(1))) u64x2 *)p;
-}
-
-// task g (global block index of the launch) -> item t, row block within item
 __device__ __forceinline__ uint32_t find_item(const uint64_t *blk_prefix, uint32_t nitems, uint64_t g) {
   uint32_t lo = 0, hi = nitems;  // largest t with blk_prefix[t] <= g
   while (hi - lo > 1) {
@@ -157,21 +150,6 @@ struct Runs {
     run = (given + readlane_u32(c, 0)) * nq + sub;
   }
 };
-
-// Up to four consecutive words in one store.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint32_t u32x3 __attribute__((ext_vector_type(3), aligned(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2), aligned(4)));
-__device__ __forceinline__ void st_words(uint32_t *p, u32x4 x, uint32_t n) {
-  if (n == 4)
-    *(__attribute__((address_space(1))) u32x4 *)p = x;
-  else if (n == 3)
-    *(__attribute__((address_space(1))) u32x3 *)p = u32x3{x[0], x[1], x[2]};
-  else if (n == 2)
-    *(__attribute__((address_space(1))) u32x2 *)p = u32x2{x[0], x[1]};
-  else
-    stg(p, x[0]);
-}
 
 // Device address of the list of key p in backward table j (b = its first
 // offset): in HBM, or through the streamed tables' block map.

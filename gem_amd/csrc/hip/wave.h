@@ -23,6 +23,28 @@ __device__ __forceinline__ void stg(T *p, T v) {
   *(__attribute__((address_space(1))) T *)p = v;
 }
 
+// Two neighbouring offsets (start and end of a list) in one 16-byte load.
+typedef uint64_t u64x2 __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ u64x2 ld_pair(const uint64_t *p) {
+  return *(const __attribute__((address_space(1))) u64x2 *)p;
+}
+
+// task g (global block index of the launch) -> item t, row block within item
+// Up to four consecutive words in one store.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3), aligned(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ void st_words(uint32_t *p, u32x4 x, uint32_t n) {
+  if (n == 4)
+    *(__attribute__((address_space(1))) u32x4 *)p = x;
+  else if (n == 3)
+    *(__attribute__((address_space(1))) u32x3 *)p = u32x3{x[0], x[1], x[2]};
+  else if (n == 2)
+    *(__attribute__((address_space(1))) u32x2 *)p = u32x2{x[0], x[1]};
+  else
+    stg(p, x[0]);
+}
+
 // popcount of the bits of `m` below this lane (v_mbcnt_lo/hi)
 __device__ __forceinline__ uint32_t rank_below(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
