@@ -182,8 +182,9 @@ struct GraphDev {
 // up to that in one wave, beyond in one block.
 constexpr uint32_t FILTER_LIGHT_DEG = 64, FILTER_HUB_DEG = 4096;
 // The table build walks candidates of larger degree than this in chunks of
-// this many adjacency slots spread over waves.
-constexpr uint32_t TABLE_HEAVY_ROW = 256, TABLE_CHUNK = 2048;
+// this many adjacency slots spread over waves (2048 slots: 22 and 17 us a write
+// and count pass on 2^18 vertices, 145 and 92 on 2^22; 512: 9 and 7, 116 and 81).
+constexpr uint32_t TABLE_HEAVY_ROW = 256, TABLE_CHUNK = 512;
 
 // Query description consumed by the filter kernel (device copy).
 struct FilterQuery {

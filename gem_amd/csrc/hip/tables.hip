@@ -31,9 +31,11 @@ constexpr uint32_t TAB_WAVES = 4;
 
 // Candidates a wave of k_tables takes: a list of 64 rows of up to 256 slots is
 // walked in up to 128 dependent steps, so builds of few candidates take fewer
-// rows per wave until the chip has waves enough (about 8 per SIMD).  64 rows
-// per wave: 68 us a pass for queries of a few thousand candidates on 2^18.
-constexpr uint32_t MIN_ROWS = 8, ENOUGH_WAVES = 8192;
+// rows per wave until the chip has waves enough (about 8 per SIMD, twice).  64
+// rows per wave: 68 us a pass for queries of a few thousand candidates on 2^18;
+// on 2^22 (4 * 10^5 candidates) count / write passes of 119 / 136 us with two groups of 64
+// slots a step and 8192 waves enough, 111 / 114 with 16384, 101 / 117 with four.
+constexpr uint32_t MIN_ROWS = 8, ENOUGH_WAVES = 16384, STEP = 4;
 
 struct TableJob {
   uint32_t nu;
@@ -60,7 +62,7 @@ struct HeavyTab {
 
 // Device counters of one build (uploaded as zeros with the descriptors).
 struct TableCtr {
-  uint32_t rows, pieces;
+  unsigned long long rows_pieces;  // heavy rows (low word) and their pieces
   unsigned long long adj_len[GEM_MAX_QV];  // light and heavy slots walked per keyed vertex (profiling)
 };
 
@@ -92,9 +94,8 @@ k_tables(const TableGraph G, const uint32_t *__restrict__ can, const uint64_t *_
   __shared__ uint64_t ob[TAB_WAVES][64];
   const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
   const uint32_t gw = blockIdx.x * TAB_WAVES + w;
-  if (gw >= job.wave_start[job.nu]) return;
   uint32_t ju = 0;
-  while (job.wave_start[ju + 1] <= gw) ++ju;
+  while (ju + 1 < job.nu && job.wave_start[ju + 1] <= gw) ++ju;
   const uint32_t row_base = (gw - job.wave_start[ju]) * job.rows;
   const uint32_t ncan = job.ncan[ju];
   const uint32_t i = row_base + l;
@@ -108,15 +109,30 @@ k_tables(const TableGraph G, const uint32_t *__restrict__ can, const uint64_t *_
     len = full_len > TABLE_HEAVY_ROW ? 0u : full_len;
   }
   if (!WRITE) {
+    // One atomic a block numbers its heavy rows and their pieces (two a wave
+    // were 12,400 on one address, the 240 us of a pass over 4 * 10^5 candidates).
+    __shared__ uint32_t wrows[TAB_WAVES], wpieces[TAB_WAVES];
+    __shared__ unsigned long long first;
     const uint64_t hv = __ballot(full_len > TABLE_HEAVY_ROW);
+    const uint32_t n = full_len > TABLE_HEAVY_ROW ? (full_len + TABLE_CHUNK - 1) / TABLE_CHUNK : 0;
+    const uint32_t incl = wave_incl_scan_u32(n);
+    if (l == 63) {
+      wrows[w] = (uint32_t)__popcll(hv);
+      wpieces[w] = incl;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      unsigned long long sum = 0;
+      for (uint32_t x = 0; x < TAB_WAVES; ++x) sum += (unsigned long long)wpieces[x] << 32 | wrows[x];
+      first = sum ? atomicAdd(&ctr->rows_pieces, sum) : 0;
+    }
+    __syncthreads();
     if (hv) {
-      const uint32_t n = full_len > TABLE_HEAVY_ROW ? (full_len + TABLE_CHUNK - 1) / TABLE_CHUNK : 0;
-      const uint32_t incl = wave_incl_scan_u32(n);
-      uint32_t r = 0, c = 0;
-      if (l == 0) r = atomicAdd(&ctr->rows, (uint32_t)__popcll(hv));
-      if (l == 63) c = atomicAdd(&ctr->pieces, incl);
-      r = readlane_u32(r, 0) + rank_below(hv);
-      c = readlane_u32(c, 63) + incl - n;
+      uint32_t r = (uint32_t)first + rank_below(hv), c = (uint32_t)(first >> 32) + incl - n;
+      for (uint32_t x = 0; x < w; ++x) {
+        r += wrows[x];
+        c += wpieces[x];
+      }
       if (n) heavy[r] = HeavyTab{ju, i, c, n};
       for (uint32_t x = 0; x < n; ++x) piece_row[c + x] = r;
     }
@@ -160,7 +176,7 @@ k_tables(const TableGraph G, const uint32_t *__restrict__ can, const uint64_t *_
     const uint64_t at = ob[w][g.row] + (item - rs);
     g.wv = g.iv ? G.nbr[at] : 0;
     g.lw = NL && g.iv ? G.nl[at] : 0;
-    g.last = min(63u, total - 1 - t);
+    g.last = t < total ? min(63u, total - 1 - t) : 0;
     g.row0 = readlane_u32(g.row, 0);
     const uint32_t seg_lo = rs > t ? rs - t : 0;
     g.seg_hi = (re < t + 64 ? re - t : 64) - 1;
@@ -190,19 +206,22 @@ k_tables(const TableGraph G, const uint32_t *__restrict__ can, const uint64_t *_
     }
     return readlane_u32(g.row_done ? 0u : tot_row, g.last);
   };
-  // two groups per step: both groups' loads are in flight before either
+  // STEP groups per step: all their loads are in flight before the first
   // group's ballots
-  for (uint32_t t = 0; t < total; t += 128) {
-    const bool two = t + 64 < total;
-    const Grp A = group(t);
-    const Grp B = two ? group(t + 64) : A;
+  for (uint32_t t = 0; t < total; t += 64 * STEP) {
+    Grp g[STEP];
+#pragma unroll
+    for (uint32_t x = 0; x < STEP; ++x) g[x] = group(t + 64 * x);
     for (uint32_t j = 0; j < nd; ++j) {
       const uint32_t vu = readlane_u32(my_vu, j), lab = readlane_u32(my_lab, j);
       const uint64_t *bm = bitmap + (uint64_t)vu * W;
-      const uint64_t wa = wanted<NL>(A.iv, A.lw, lab) ? bm[A.wv >> 6] : 0;
-      const uint64_t wb = two && wanted<NL>(B.iv, B.lw, lab) ? bm[B.wv >> 6] : 0;
-      uint32_t carry = apply(A, j, vu, wa, readlane_u32(carry_reg, j));
-      if (two) carry = apply(B, j, vu, wb, carry);
+      uint64_t word[STEP];
+#pragma unroll
+      for (uint32_t x = 0; x < STEP; ++x) word[x] = wanted<NL>(g[x].iv, g[x].lw, lab) ? bm[g[x].wv >> 6] : 0;
+      uint32_t carry = readlane_u32(carry_reg, j);
+#pragma unroll
+      for (uint32_t x = 0; x < STEP; ++x)
+        if (t + 64 * x < total) carry = apply(g[x], j, vu, word[x], carry);
       if (l == j) carry_reg = carry;
     }
   }
@@ -223,7 +242,7 @@ k_tables_heavy(const TableGraph G, const uint32_t *__restrict__ can, const uint6
                uint32_t *__restrict__ ccnt, uint32_t ndmax, int prof) {
   constexpr int GR = 4;
   const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
-  const uint32_t W = job.W, pieces = ctr->pieces;
+  const uint32_t W = job.W, pieces = (uint32_t)(ctr->rows_pieces >> 32);
   for (uint32_t c = blockIdx.x * TAB_WAVES + w; c < pieces; c += gridDim.x * TAB_WAVES) {
     const HeavyTab e = heavy[piece_row[c]];
     const uint32_t v = can[job.can_off[e.ju] + e.i];
@@ -289,16 +308,22 @@ __global__ void __launch_bounds__(256) k_theavy_bases(const TableJob job, const 
                                                      const TableCtr *__restrict__ ctr,
                                                      const HeavyTab *__restrict__ heavy, uint32_t *__restrict__ ccnt,
                                                      uint32_t ndmax) {
-  const uint64_t n = (uint64_t)ctr->rows * ndmax;
+  const uint64_t n = (uint64_t)(uint32_t)ctr->rows_pieces * ndmax;
   for (uint64_t x = (uint64_t)blockIdx.x * 256 + threadIdx.x; x < n; x += (uint64_t)gridDim.x * 256) {
     const HeavyTab e = heavy[x / ndmax];
     const uint32_t j = (uint32_t)(x % ndmax);
     if (j >= job.nd[e.ju]) continue;
     uint32_t run = 0;
-    for (uint32_t c = e.c0; c < e.c0 + e.n; ++c) {
-      const uint32_t h = ccnt[(uint64_t)c * ndmax + j];
-      ccnt[(uint64_t)c * ndmax + j] = run;
-      run += h;
+    for (uint32_t c = 0; c < e.n; c += 8) {  // eight loads in flight
+      uint32_t h[8];
+      uint32_t *at = ccnt + (uint64_t)(e.c0 + c) * ndmax + j;
+#pragma unroll
+      for (uint32_t x = 0; x < 8; ++x) h[x] = c + x < e.n ? at[x * ndmax] : 0;
+#pragma unroll
+      for (uint32_t x = 0; x < 8; ++x) {
+        if (c + x < e.n) at[x * ndmax] = run;
+        run += h[x];
+      }
     }
     stg(desc[job.tab0[e.ju] + j].off + e.i, (uint64_t)run);
   }
