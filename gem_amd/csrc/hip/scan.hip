@@ -1,7 +1,7 @@
 // Exclusive prefix sums used by the filter (candidate ranks), the edge tables
 // (row offsets) and the join (output offsets).  Reduce-then-scan: per-tile sums,
-// a one-block scan of the tile sums, then a tile-local scan with the carried
-// base.  Integer adds only, so results are exact and order-independent.
+// then a tile-local scan whose blocks add up the sums before theirs.  Integer
+// adds only, so results are exact and order-independent.
 #include "ctx.h"
 #include "wave.h"
 
@@ -24,72 +24,69 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_tile_sums_u64(const uint64_t *
   if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
-// one block: exclusive scan of m values, out[m] = total (and *total, when given)
-__global__ void __launch_bounds__(1024) k_scan_small_u64(const uint64_t *in, uint64_t m, uint64_t *out,
-                                                        uint64_t *total) {
-  __shared__ uint64_t sm[16];
-  uint64_t carry = 0;
-  for (uint64_t b = 0; b < m; b += blockDim.x) {
-    uint64_t idx = b + threadIdx.x;
-    uint64_t x = idx < m ? in[idx] : 0;
-    uint64_t ex;
-    uint64_t tot = block_excl_scan_u64(x, &ex, sm);
-    if (idx < m) out[idx] = carry + ex;
-    carry += tot;
+// Tile-local scan: wave w of a block holds entries [w, w + 1) * 64 * SCAN_ITEMS
+// of its tile, lane = entry modulo 64.  SUMS: `before` holds the tiles' sums and
+// a block adds up those before its own, else it holds their exclusive scan.
+// The last tile's block writes the total to out[n] (and *total, when given).
+template <bool SUMS>
+__global__ void __launch_bounds__(SCAN_THREADS) k_tile_scan_u64(const uint64_t *in, uint64_t n, const uint64_t *before,
+                                                              uint64_t *out, uint64_t *total) {
+  __shared__ uint64_t sm[4], pre[4];
+  const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
+  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + w * 64 * SCAN_ITEMS;
+  uint64_t v[SCAN_ITEMS], x = 0, y = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < SCAN_ITEMS; ++i) {
+    const uint64_t at = base + i * 64 + l;
+    v[i] = at < n ? in[at] : 0;
+    x += v[i];
   }
-  if (threadIdx.x == 0) {
-    out[m] = carry;
-    if (total) *total = carry;
+  if (SUMS)
+    for (uint32_t c = threadIdx.x; c < blockIdx.x; c += SCAN_THREADS) y += before[c];
+  x = wave_sum_u64(x);
+  y = wave_sum_u64(y);
+  if (l == 0) {
+    sm[w] = x;
+    pre[w] = y;
+  }
+  __syncthreads();
+  uint64_t run = SUMS ? pre[0] + pre[1] + pre[2] + pre[3] : before[blockIdx.x];
+  for (uint32_t i = 0; i < w; ++i) run += sm[i];
+  if (blockIdx.x + 1 == gridDim.x && threadIdx.x == SCAN_THREADS - 64) {  // the last wave
+    out[n] = run + sm[3];
+    if (total) *total = run + sm[3];
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < SCAN_ITEMS; ++i) {
+    if (base + i * 64 >= n) break;
+    const uint64_t at = base + i * 64 + l, incl = wave_incl_scan_u64(v[i]);
+    if (at < n) out[at] = run + incl - v[i];
+    run += readlane_u64(incl, 63);
   }
 }
 
-__global__ void __launch_bounds__(SCAN_THREADS) k_tile_scan_u64(const uint64_t *in, uint64_t n, const uint64_t *tile_base,
-                                                              uint64_t *out) {
-  __shared__ uint64_t sm[8];
-  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
-  // each thread owns SCAN_ITEMS consecutive elements
-  uint64_t v[SCAN_ITEMS];
-  uint64_t acc = 0;
-  const uint64_t my = base + (uint64_t)threadIdx.x * SCAN_ITEMS;
-#pragma unroll
-  for (uint32_t i = 0; i < SCAN_ITEMS; ++i) {
-    uint64_t idx = my + i;
-    v[i] = idx < n ? in[idx] : 0;
-    acc += v[i];
-  }
-  uint64_t ex;
-  block_excl_scan_u64(acc, &ex, sm);
-  uint64_t run = tile_base[blockIdx.x] + ex;
-#pragma unroll
-  for (uint32_t i = 0; i < SCAN_ITEMS; ++i) {
-    uint64_t idx = my + i;
-    if (idx < n) out[idx] = run;
-    run += v[i];
-  }
-}
+// One launch up to a tile, two up to ADD_TILES tiles (blocks adding up the sums
+// before theirs read ADD_TILES^2 / 2 of them at most, 64 MiB); beyond, the sums
+// are scanned in turn.  (One block that scanned up to 65,536 values by itself
+// took 43 us on average and up to 110 in the length passes of capped batches.)
+constexpr uint64_t ADD_TILES = 4096;
 
 void scan_u64(gem_ctx *c, const uint64_t *d_in, uint64_t *d_out, uint64_t n, uint64_t *d_total) {
-  if (n <= 4 * 1024 * 16) {
-    k_scan_small_u64<<<1, 1024, 0, c->stream>>>(d_in, n, d_out, d_total);
-    GEM_LAUNCH_CHECK("k_scan_small_u64");
-    return;
-  }
-  const uint64_t tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
+  const uint64_t tiles = std::max<uint64_t>(1, (n + SCAN_TILE - 1) / SCAN_TILE);
   DevBuf sums, base;
-  sums.alloc(tiles * 8, c->stream);
-  base.alloc((tiles + 1) * 8, c->stream);
-  k_tile_sums_u64<<<(uint32_t)tiles, SCAN_THREADS, 0, c->stream>>>(d_in, n, sums.as<uint64_t>());
-  GEM_LAUNCH_CHECK("k_tile_sums_u64");
-  if (tiles > 4 * 1024 * 16) {
-    scan_u64(c, sums.as<uint64_t>(), base.as<uint64_t>(), tiles, d_total);
-  } else {
-    k_scan_small_u64<<<1, 1024, 0, c->stream>>>(sums.as<uint64_t>(), tiles, base.as<uint64_t>(), d_total);
-    GEM_LAUNCH_CHECK("k_scan_small_u64");
+  if (tiles > 1) {
+    sums.alloc(tiles * 8, c->stream);
+    k_tile_sums_u64<<<(uint32_t)tiles, SCAN_THREADS, 0, c->stream>>>(d_in, n, sums.as<uint64_t>());
+    GEM_LAUNCH_CHECK("k_tile_sums_u64");
   }
-  k_tile_scan_u64<<<(uint32_t)tiles, SCAN_THREADS, 0, c->stream>>>(d_in, n, base.as<uint64_t>(), d_out);
+  if (tiles > ADD_TILES) {
+    base.alloc((tiles + 1) * 8, c->stream);
+    scan_u64(c, sums.as<uint64_t>(), base.as<uint64_t>(), tiles);
+    k_tile_scan_u64<false><<<(uint32_t)tiles, SCAN_THREADS, 0, c->stream>>>(d_in, n, base.as<uint64_t>(), d_out, d_total);
+  } else {
+    k_tile_scan_u64<true><<<(uint32_t)tiles, SCAN_THREADS, 0, c->stream>>>(d_in, n, sums.as<uint64_t>(), d_out, d_total);
+  }
   GEM_LAUNCH_CHECK("k_tile_scan_u64");
-  // out[n] = total
-  GEM_HIP_CHECK(hipMemcpyAsync(d_out + n, base.as<uint64_t>() + tiles, 8, hipMemcpyDeviceToDevice, c->stream));
 }
 
 // Many independent in-place scans: segments in chunks of SEG_CHUNK entries,

@@ -1237,8 +1237,14 @@ struct ExtSlot {
     GEM_HIP_CHECK(hipMemcpyAsync(h_hdr, d, hdr_bytes, hipMemcpyDeviceToHost, s));
   }
 
-  HeavyOut heavy_out(int i, unsigned int *hn) const {
-    return HeavyOut{heavy[i].as<HeavyRow>(), pieces[i].as<uint32_t>(), hn + 2 * i, heavy_t, heavy_chunk};
+  // A write walk over resident tables cuts its units between rows, so a row is
+  // long for it from twice the threshold on (write walks and their heavy rows in
+  // a capped batch, at 1024, 2048 and 4096: 70, 66 and 75 ms on 2^20 vertices, 82, 79
+  // and 76 on 2^22).  Streamed and final walks take whole units: 2048 cost a
+  // streamed batch 20%.
+  HeavyOut heavy_out(int i, unsigned int *hn, bool cut = false) const {
+    return HeavyOut{heavy[i].as<HeavyRow>(), pieces[i].as<uint32_t>(), hn + 2 * i, cut ? 2 * heavy_t : heavy_t,
+                    heavy_chunk};
   }
 
   // (At most `most` blocks each.)  The three kernels over task ranges [b_i, e_i) of launch i (queues
@@ -1254,7 +1260,7 @@ struct ExtSlot {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_WRITE : -1);
       k_vext<false, OOC><<<std::min(most, grid[0]), VB, lds, s>>>(items[0], dn + 0, blk[0], dq + 0, lcap, dcap,
                                                count_items ? dp : nullptr, count_items ? dp + 4 : nullptr,
-                                               b0, e0, heavy_out(0, hn));
+                                               b0, e0, heavy_out(0, hn, !OOC));
       GEM_LAUNCH_CHECK("k_vext<write>");
     }
     if (b1 < e1) {
