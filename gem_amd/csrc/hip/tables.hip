@@ -63,7 +63,6 @@ struct HeavyTab {
 // Device counters of one build (uploaded as zeros with the descriptors).
 struct TableCtr {
   unsigned long long rows_pieces;  // heavy rows (low word) and their pieces
-  unsigned long long adj_len[GEM_MAX_QV];  // light and heavy slots walked per keyed vertex (profiling)
 };
 
 // The graph as the table kernels read it.
@@ -89,7 +88,7 @@ template <bool WRITE, bool NL>
 __global__ void __launch_bounds__(TAB_WAVES * 64)
 k_tables(const TableGraph G, const uint32_t *__restrict__ can, const uint64_t *__restrict__ bitmap,
          const uint32_t *__restrict__ rank, const TableJob job, const TableDesc *__restrict__ desc,
-         TableCtr *__restrict__ ctr, HeavyTab *__restrict__ heavy, uint32_t *__restrict__ piece_row, int prof) {
+         TableCtr *__restrict__ ctr, HeavyTab *__restrict__ heavy, uint32_t *__restrict__ piece_row) {
   __shared__ uint32_t st[TAB_WAVES][65];
   __shared__ uint64_t ob[TAB_WAVES][64];
   const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
@@ -139,7 +138,6 @@ k_tables(const TableGraph G, const uint32_t *__restrict__ can, const uint64_t *_
   }
   const uint32_t incl = wave_incl_scan_u32(len);
   const uint32_t total = readlane_u32(incl, 63);
-  if (!WRITE && prof && l == 0 && total) atomicAdd(&ctr->adj_len[ju], (unsigned long long)total);
   st[w][l] = incl - len;
   ob[w][l] = o0;
   if (l == 63) st[w][64] = total;
@@ -239,7 +237,7 @@ __global__ void __launch_bounds__(TAB_WAVES * 64)
 k_tables_heavy(const TableGraph G, const uint32_t *__restrict__ can, const uint64_t *__restrict__ bitmap,
                const uint32_t *__restrict__ rank, const TableJob job, const TableDesc *__restrict__ desc,
                TableCtr *__restrict__ ctr, const HeavyTab *__restrict__ heavy, const uint32_t *__restrict__ piece_row,
-               uint32_t *__restrict__ ccnt, uint32_t ndmax, int prof) {
+               uint32_t *__restrict__ ccnt, uint32_t ndmax) {
   constexpr int GR = 4;
   const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
   const uint32_t W = job.W, pieces = (uint32_t)(ctr->rows_pieces >> 32);
@@ -248,7 +246,6 @@ k_tables_heavy(const TableGraph G, const uint32_t *__restrict__ can, const uint6
     const uint32_t v = can[job.can_off[e.ju] + e.i];
     const uint64_t o0 = G.off[v], len = G.off[v + 1] - o0;
     const uint64_t t0 = (uint64_t)(c - e.c0) * TABLE_CHUNK, t1 = t0 + TABLE_CHUNK < len ? t0 + TABLE_CHUNK : len;
-    if (!WRITE && prof && l == 0) atomicAdd(&ctr->adj_len[e.ju], (unsigned long long)(t1 - t0));
     const uint32_t nd = job.nd[e.ju], tb = job.tab0[e.ju];
     // lane j < nd holds table j: its value vertex and label, (write) the
     // address of the row's first value, and its running count in the row
@@ -348,18 +345,17 @@ struct TableRun {
   void pass_as() {
     hipStream_t s = c->stream;
     const TableGraph g{G.off.as<uint64_t>(), G.nbr_dev(), G.nbr_lab.as<uint8_t>()};
-    const int prof = c->prof.on;
     if (waves) {
       k_tables<WRITE, NL><<<(waves + TAB_WAVES - 1) / TAB_WAVES, TAB_WAVES * 64, 0, s>>>(
           g, Qd.can.as<uint32_t>(), Qd.bitmap.as<uint64_t>(), Qd.rank.as<uint32_t>(), job, desc, ctr,
-          heavy.as<HeavyTab>(), piece_row.as<uint32_t>(), prof);
+          heavy.as<HeavyTab>(), piece_row.as<uint32_t>());
       GEM_LAUNCH_CHECK("k_tables");
     }
     if (waves && rows_bound) {
       const uint32_t hb = (uint32_t)std::min<uint64_t>((pieces_bound + TAB_WAVES - 1) / TAB_WAVES, 2048);
       k_tables_heavy<WRITE, NL><<<hb, TAB_WAVES * 64, 0, s>>>(
           g, Qd.can.as<uint32_t>(), Qd.bitmap.as<uint64_t>(), Qd.rank.as<uint32_t>(), job, desc, ctr,
-          heavy.as<HeavyTab>(), piece_row.as<uint32_t>(), ccnt.as<uint32_t>(), ndmax, prof);
+          heavy.as<HeavyTab>(), piece_row.as<uint32_t>(), ccnt.as<uint32_t>(), ndmax);
       GEM_LAUNCH_CHECK("k_tables_heavy");
       if (!WRITE) {
         k_theavy_bases<<<(uint32_t)std::min<uint64_t>((rows_bound * ndmax + 255) / 256, 1024), 256, 0, s>>>(
@@ -376,6 +372,30 @@ struct TableRun {
       write ? pass_as<true, false>() : pass_as<false, false>();
   }
 };
+
+// Sum of the degrees of n vertices (for the algorithmic bytes, while profiling;
+// counted by the build itself it is an atomic a wave and heavy piece, which
+// were half of a profiled count pass).
+__global__ void __launch_bounds__(256) k_degree_sum(const uint64_t *__restrict__ off, const uint32_t *__restrict__ v,
+                                                   uint32_t n, unsigned long long *__restrict__ out) {
+  __shared__ uint64_t sm[4];
+  uint64_t x = 0;
+  for (uint32_t i = threadIdx.x; i < n; i += 256) x += off[v[i] + 1] - off[v[i]];
+  x = wave_sum_u64(x);
+  if (threadIdx.x % 64 == 0) sm[threadIdx.x / 64] = x;
+  __syncthreads();
+  if (threadIdx.x == 0) *out = sm[0] + sm[1] + sm[2] + sm[3];
+}
+static uint64_t degree_sum(gem_ctx *c, const GraphDev &G, const uint32_t *v, uint32_t n) {
+  DevBuf d;
+  d.alloc(8, c->stream);
+  k_degree_sum<<<1, 256, 0, c->stream>>>(G.off.as<uint64_t>(), v, n, d.as<unsigned long long>());
+  GEM_LAUNCH_CHECK("k_degree_sum");
+  uint64_t h = 0;
+  GEM_HIP_CHECK(hipMemcpyAsync(&h, d.p, 8, hipMemcpyDeviceToHost, c->stream));
+  GEM_HIP_CHECK(hipStreamSynchronize(c->stream));
+  return h;
+}
 
 // The tables of Qd's query, without their values, and its launches' sizes.
 static void plan_tables(TableRun &R) {
@@ -489,13 +509,12 @@ void run_tables(gem_ctx *c, QueryDev *Qds, uint32_t n, bool wait) {
       // algorithmic bytes: per keyed u, its candidates (4 B), offset pairs (8 B)
       // and adjacency (4 B per slot) once for all its tables; per table the value
       // vertex's bitmap (|V|/8) and the row counts / offsets (8 B per row)
-      TableCtr h;
-      GEM_HIP_CHECK(hipMemcpyAsync(&h, R.ctr, sizeof(h), hipMemcpyDeviceToHost, s));
-      GEM_HIP_CHECK(hipStreamSynchronize(s));
       const TableJob &job = R.job;
       const QueryDev &Qd = R.Qd;
       double shared_bytes = 0, count_bytes = 0, write_bytes = 0;
-      for (uint32_t ju = 0; ju < job.nu; ++ju) shared_bytes += 12.0 * job.ncan[ju] + 4.0 * (double)h.adj_len[ju];
+      for (uint32_t ju = 0; ju < job.nu; ++ju)
+        shared_bytes += 12.0 * job.ncan[ju] +
+                        4.0 * (double)degree_sum(c, G, Qd.can.as<uint32_t>() + job.can_off[ju], job.ncan[ju]);
       for (size_t x = k0; x < k; ++x) {
         const TableDev &T = Qd.tab[R.desc_tab[x - k0]];
         count_bytes += 8.0 * Qd.W + 8.0 * Qd.ncan[T.key_u];
