@@ -284,10 +284,14 @@ __global__ void __launch_bounds__(VB) __attribute__((amdgpu_waves_per_eu(6)))
 k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, const uint64_t *__restrict__ blk_prefix,
        unsigned int *__restrict__ queue, uint32_t lcap, uint32_t dcap,
        unsigned long long *__restrict__ prof_items, unsigned long long *__restrict__ prof_out, uint64_t g_begin,
-       uint64_t g_end, const HeavyOut heavy) {
+       uint64_t g_end, const HeavyOut heavy_in) {
   const uint32_t nitems = *nitems_p;
   const uint64_t total = blk_prefix[nitems] < g_end ? blk_prefix[nitems] : g_end;
   if (g_begin >= total) return;
+  // final walks of measured pieces take runs of equal cost too (all of a launch)
+  const bool by_cost = !OOC && (!FINAL || ((CItem *)items)[0].run_cost);
+  HeavyOut heavy = heavy_in;
+  if (by_cost) heavy.threshold *= 2;  // see ExtSlot::heavy_out
   __shared__ uint32_t st[VW][64];          // first item of each row
   __shared__ uint64_t drv[VW][64];         // address of each row's driving list
   __shared__ uint8_t drv_j[VW][64];        // which of the row's lists drives
@@ -410,7 +414,7 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
           len = (uint32_t)(o.y - o.x);
           addr = list_addr<OOC>(L, 0, p, o.x);
         }
-        if (!FINAL && !OOC && !owned(j, len, at)) len = 0;
+        if (!OOC && !owned(j, len, at)) len = 0;
         const uint64_t taken = set_aside(heavy, len > heavy.threshold, t, len, ((CItem *)items)[t].row_begin + r);
         if ((taken >> l) & 1ull) len = 0;  // walked by k_vext_heavy
         if (l == 0) aside[w][j - j0] = taken;
@@ -460,7 +464,7 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
       }
       if (i < nb) row_lists<1>(L, row, i, take);
     }
-    if (!FINAL && !OOC && !owned(j, dlen, at)) dlen = 0;
+    if (by_cost && !owned(j, dlen, at)) dlen = 0;
     const uint64_t taken =
         !FINAL && counted
             ? aside[w][j - j0]
@@ -589,7 +593,7 @@ k_vext(const VItem *__restrict__ items, const uint32_t *__restrict__ nitems_p, c
   }
   };
   const uint32_t bw = blockDim.x / 64;
-  if (FINAL || OOC) {
+  if (!by_cost) {
     // tasks are 64-row units, numbered through the launch
     Runs runs((total - g_begin) * VW, blockIdx.x * bw + w, gridDim.x * bw, FINAL ? 4 : 8, queue);
     for (; runs.valid(); runs.next())
@@ -1237,14 +1241,13 @@ struct ExtSlot {
     GEM_HIP_CHECK(hipMemcpyAsync(h_hdr, d, hdr_bytes, hipMemcpyDeviceToHost, s));
   }
 
-  // A write walk over resident tables cuts its units between rows, so a row is
-  // long for it from twice the threshold on (write walks and their heavy rows in
-  // a capped batch, at 1024, 2048 and 4096: 70, 66 and 75 ms on 2^20 vertices, 82, 79
-  // and 76 on 2^22).  Streamed and final walks take whole units: 2048 cost a
-  // streamed batch 20%.
-  HeavyOut heavy_out(int i, unsigned int *hn, bool cut = false) const {
-    return HeavyOut{heavy[i].as<HeavyRow>(), pieces[i].as<uint32_t>(), hn + 2 * i, cut ? 2 * heavy_t : heavy_t,
-                    heavy_chunk};
+  // A walk in runs of equal cost cuts its units between rows, so a row is long
+  // for it from twice the threshold on (write walks and their heavy rows in a
+  // capped batch, at 1024, 2048 and 4096: 70, 66 and 75 ms on 2^20 vertices, 82, 79
+  // and 76 on 2^22).  Streamed walks take whole units: 2048 cost a streamed batch
+  // 20%.
+  HeavyOut heavy_out(int i, unsigned int *hn) const {
+    return HeavyOut{heavy[i].as<HeavyRow>(), pieces[i].as<uint32_t>(), hn + 2 * i, heavy_t, heavy_chunk};
   }
 
   // (At most `most` blocks each.)  The three kernels over task ranges [b_i, e_i) of launch i (queues
@@ -1260,7 +1263,7 @@ struct ExtSlot {
       ProfLaunch pl(c, prof_kernels ? K_VEXT_WRITE : -1);
       k_vext<false, OOC><<<std::min(most, grid[0]), VB, lds, s>>>(items[0], dn + 0, blk[0], dq + 0, lcap, dcap,
                                                count_items ? dp : nullptr, count_items ? dp + 4 : nullptr,
-                                               b0, e0, heavy_out(0, hn, !OOC));
+                                               b0, e0, heavy_out(0, hn));
       GEM_LAUNCH_CHECK("k_vext<write>");
     }
     if (b1 < e1) {
@@ -1489,6 +1492,15 @@ struct HipSchedBackend {
     return old;
   }
 
+  // Item x to a launch whose waves take runs of about `cost` of it.
+  void add_by_cost(Launch &L, VItem it, const Item &x, uint64_t cost) {
+    it.units = x.rows->units.prefix->as<uint64_t>() + x.rows->units.unit0 + x.row_begin / gemh::SCHED_UNIT;
+    it.nunits = (uint32_t)units_of(x);
+    it.run_cost = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(cost, 4 * UNIT_COST), RUN_COST);
+    L.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level],
+          (x.out_rows + UNIT_COST * units_of(x) - 1) / it.run_cost + 1);
+  }
+
   void extend(const std::vector<Item> &wr_items, const std::vector<Item> &fin_items, std::vector<uint64_t> *got_wr,
               std::vector<uint64_t> *got_fin) {
     const auto t0 = clk::now();
@@ -1502,28 +1514,39 @@ struct HipSchedBackend {
     // runs of the write walks (see unit_range): CLAIMS per wave of the grid by
     // cost, an entry of a level with other lists costing its searches too
     auto weight = [&](const Item &x) { return 4ull * qs[x.q]->max_nb[x.level] - 3; };
-    uint64_t run_cost = 0;
+    uint64_t run_cost = 0, fin_cost = 0;
     std::vector<std::pair<const LevelBuf *, LevelBuf::Units>> replaced;
+    // final walks: when all their pieces are measured (they are under a cap)
+    std::vector<Item> walked;
+    bool measured = !tc;
+    for (const Item &x : fin_items)
+      if (qs[x.q]->max_nb[x.level] > 1) {
+        walked.push_back(x);
+        measured = measured && x.out_rows;
+      }
+    if (measured && !walked.empty()) {
+      uint64_t cost = 0;
+      for (const Item &x : walked) cost += (x.out_rows + UNIT_COST * units_of(x)) * weight(x);
+      fin_cost = cost / ((uint64_t)slot.grid[1] * VW * CLAIMS) + 1;
+    } else {
+      walked.clear();
+    }
     if (!tc) {
       uint64_t cost = 0;
       for (const Item &x : wr_items) cost += (x.out_rows + UNIT_COST * units_of(x)) * weight(x);
       run_cost = cost / ((uint64_t)slot.grid[0] * VW * CLAIMS) + 1;
-      replaced = remeasure(wr_items);
+      walked.insert(walked.end(), wr_items.begin(), wr_items.end());
+      replaced = remeasure(walked);
     }
     for (const Item &x : wr_items) {
       VItem it = vitem(x);
       it.out = x.out->as<uint32_t>();
       it.out_cap = x.out_rows;
       it.counter = slot.dev_counter(nctr++);
-      if (run_cost) {
-        it.units = x.rows->units.prefix->as<uint64_t>() + x.rows->units.unit0 + x.row_begin / gemh::SCHED_UNIT;
-        it.nunits = (uint32_t)units_of(x);
-        it.run_cost = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(run_cost / weight(x), 4 * UNIT_COST), RUN_COST);
-        wr.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level],
-               (x.out_rows + UNIT_COST * units_of(x) - 1) / it.run_cost + 1);
-      } else {
+      if (run_cost)
+        add_by_cost(wr, it, x, run_cost / weight(x));
+      else
         wr.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level]);
-      }
     }
     std::vector<size_t> fin_ctr(fin_items.size());
     for (size_t t = 0; t < fin_items.size(); ++t) {
@@ -1533,6 +1556,8 @@ struct HipSchedBackend {
       it.counter = slot.dev_counter(nctr++);
       if (qs[x.q]->max_nb[x.level] == 1)
         fin1.add(it, 1, qs[x.q]->max_ndup[x.level]);
+      else if (fin_cost)
+        add_by_cost(fin, it, x, fin_cost / weight(x));
       else
         fin.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level]);
     }

@@ -455,6 +455,7 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
       it.rows = top.rows.get();
       it.row_begin = top.cursor * SCHED_UNIT;
       it.row_end = std::min<uint64_t>(b1 * SCHED_UNIT, top.nrows);
+      it.out_rows = piece_bound;
       keep_alive.push_back(top.rows);
       S.processed += it.row_end - it.row_begin;
       S.work += it.row_end - it.row_begin;

@@ -38,3 +38,22 @@ def test_cut_units(case, blocks, heavy):
         for q, r, ref in zip(qs, ctx.match_batch(qs), refs):
             assert r["count"] == ref["count"]
             assert np.array_equal(r["level_rows"], ref["level_rows"])
+
+
+@pytest.mark.parametrize("blocks", [1, 2048])
+@pytest.mark.parametrize("heavy", [(1024, 1024), (48, 64)])
+def test_capped_final_walks(case, blocks, heavy):
+    # under a cap that no query reaches, final levels are measured and walked in
+    # runs of equal cost too
+    g, qs, refs = case
+    with GemContext(0) as ctx:
+        ctx.load_data(g)
+        ctx.set_persistent_blocks(blocks)
+        ctx.set_heavy_split(*heavy)
+        for graph in (False, True):
+            ctx.set_graph(graph)
+            for q, r, ref in zip(qs, ctx.match_batch(qs, cap=10 ** 8), refs):
+                assert not r["saturated"] and r["count"] == ref["count"]
+        for q, r, ref in zip(qs, ctx.match_batch(qs, cap=30000), refs):
+            assert r["saturated"] == (ref["count"] > 30000)
+            assert r["count"] == min(ref["count"], 30000)
