@@ -372,8 +372,9 @@ int gem_hip_set_persistent_blocks(gem_ctx *ctx, uint32_t blocks);
 /* Load balance of the batched path's walks: a row whose driving (shortest)
  * list has more than `threshold` entries is set aside and walked `chunk`
  * entries per wave task by a second kernel instead of by the wave holding the
- * row (a walk that writes rows from resident tables shares long rows out by
- * itself and sets them aside from twice the threshold on; defaults 1024 and 1024; threshold in [32, 2^24], chunk in
+ * row (walks over resident tables that write rows, or count under a cap, share
+ * long rows out by themselves and set them aside from twice the threshold on;
+ * defaults 1024 and 1024; threshold in [32, 2^24], chunk in
  * [64, 2^20]).  Counts do not depend on either.  Set by the autotuner. */
 int gem_hip_set_heavy_split(gem_ctx *ctx, uint32_t threshold, uint32_t chunk);
 /* on != 0: the batched path's per-iteration extend step (table uploads, three
