@@ -265,10 +265,11 @@ __device__ __forceinline__ uint64_t set_aside(const HeavyOut &H, bool want, uint
 // long lists (runs of a fixed number of units: the longest launch took 18 ms
 // instead of 5; final walks under a cap with their heavy rows: 0.47 ms a launch,
 // by cost 0.40).  Uncapped final walks and streamed ones are not measured, or are
-// cut into task groups, and take runs of whole units.  For each of its rows the shortest backward list drives; a row whose driving list is
-// longer than heavy_t is not walked here but appended to the heavy-row list
-// (when it has room), which k_vext_heavy then walks in fixed-size chunks spread
-// over all waves: a hub row no longer holds one wave for the whole launch.
+// cut into task groups, and take runs of whole units.  For each of its rows the
+// shortest backward list drives; a row whose driving list is longer than the
+// threshold is not walked here but appended to the heavy-row list (when it has
+// room), which k_vext_heavy then walks in fixed-size chunks spread over all
+// waves: a hub row no longer holds one wave for the whole launch.
 // Dynamic LDS per wave: lists (lcap x 64 x (u64 address + u32 length)) and
 // vertices of equal-label columns (dcap x 64 u32).
 // An item (row, value) survives when its value is in the row's other lists and
