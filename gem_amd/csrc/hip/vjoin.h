@@ -4,6 +4,7 @@
 #include <memory>
 #include <vector>
 
+#include "../host/heavy_pieces.h"
 #include "../host/vsched.h"
 #include "ctx.h"
 
@@ -78,7 +79,7 @@ struct HeavyRow {
 struct HeavyOut {
   HeavyRow *rows;
   uint32_t *piece_row;
-  unsigned int *ctr;  // rows, pieces
+  gemh::HeavyCounters *ctr;
   uint32_t threshold, piece;  // a list longer than `threshold` entries is cut into pieces of `piece`
 };
 
@@ -87,6 +88,7 @@ constexpr uint32_t WQ = 8, WQ_STRIDE = 16, WQ_WORDS = WQ * WQ_STRIDE;
 // Counters of one task group of a streamed launch: 5 queues, heavy rows and
 // pieces of two launches.
 constexpr uint32_t GROUP_WORDS = 5 * WQ_WORDS + WQ_STRIDE;
+static_assert(2 * sizeof(gemh::HeavyCounters) <= 4 * WQ_STRIDE && GROUP_WORDS % 2 == 0, "counters of a group, aligned");
 
 struct VQueryState {
   const QueryDev *qd = nullptr;

@@ -236,26 +236,22 @@ __device__ __forceinline__ void row_dups(CLevel &L, const uint32_t *row, uint32_
 // CU's 32 waves.
 constexpr uint32_t LDS_LISTS = 2, LDS_DUPS = 8;
 
-// Rows whose driving list has more than the threshold's entries go to
-// k_vext_heavy; at most HEAVY_CAP rows and PIECE_CAP pieces per launch (a row
-// that finds no room is walked by its own wave).
-constexpr uint32_t HEAVY_CAP = 1u << 20, PIECE_CAP = 1u << 22;
-
 // Sets aside the rows of the lanes that ask (want; list of len entries, row r
-// of item t); returns the lanes whose row was taken.  Rows and pieces are
-// numbered by two atomics per wave; pieces of refused rows are marked.
+// of item t) for k_vext_heavy; returns the lanes whose row was taken.  Rows and
+// pieces are numbered by two atomics per wave; pieces of refused rows are marked.
 __device__ __forceinline__ uint64_t set_aside(const HeavyOut &H, bool want, uint32_t t, uint32_t len, uint64_t r) {
   const uint64_t m = __ballot(want);
   if (!m) return 0;
-  const uint32_t n = want ? (len - 1) / H.piece + 1 : 0, incl = wave_incl_scan_u32(n);
-  uint32_t h = 0, c = 0;
-  if (lane_id() == 0) h = atomicAdd(&H.ctr[0], (uint32_t)__popcll(m));
-  if (lane_id() == 63) c = atomicAdd(&H.ctr[1], incl);
-  h = readlane_u32(h, 0) + rank_below(m);
-  c = readlane_u32(c, 63) + incl - n;
-  const bool taken = want && h < HEAVY_CAP && c <= PIECE_CAP && n <= PIECE_CAP - c;
-  if (taken) H.rows[h] = HeavyRow{t, len, r, c, 0};
-  for (uint32_t x = 0; x < n && c < PIECE_CAP && x < PIECE_CAP - c; ++x) H.piece_row[c + x] = taken ? h : NOT_FOUND;
+  const uint32_t n = want ? gemh::heavy_pieces(len, H.piece) : 0, incl = wave_incl_scan_u32(n);
+  uint64_t h = 0, c = 0;
+  if (lane_id() == 0) h = atomicAdd(&H.ctr->rows, (unsigned long long)__popcll(m));
+  if (lane_id() == 63) c = atomicAdd(&H.ctr->pieces, (unsigned long long)incl);
+  h = readlane_u64(h, 0) + rank_below(m);
+  c = readlane_u64(c, 63) + incl - n;
+  const bool taken = want && gemh::heavy_taken(h, c, n);
+  if (taken) H.rows[h] = HeavyRow{t, len, r, (uint32_t)c, 0};
+  const uint32_t entries = gemh::heavy_entries(c, n);
+  for (uint32_t x = 0; x < entries; ++x) H.piece_row[c + x] = taken ? (uint32_t)h : NOT_FOUND;
   return __ballot(taken);
 }
 
@@ -648,7 +644,8 @@ k_vext_heavy(const VItem *__restrict__ items, const HeavyOut heavy, unsigned int
   __shared__ uint32_t win[VW][HWIN];  // staged window
   __shared__ uint32_t prow[VW][GEM_MAX_QV], hsv[VW][VSTAGE];  // parent row, staged surviving values
   const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64;
-  const uint32_t total = heavy.ctr[1] < PIECE_CAP ? heavy.ctr[1] : PIECE_CAP, chunk = heavy.piece;
+  const uint64_t asked = heavy.ctr->pieces;
+  const uint32_t total = asked < gemh::PIECE_CAP ? (uint32_t)asked : gemh::PIECE_CAP, chunk = heavy.piece;
   if (!total) return;
   uint64_t walked = 0, written = 0;
   const uint32_t bw = blockDim.x / 64;
@@ -1115,12 +1112,12 @@ uint32_t resident_blocks(const void *kernel, size_t lds) {
 // the zeroed counters travel in the header copy).
 struct ExtSlot {
   static constexpr size_t KEEP_LAUNCH = 1 << 20;
-  // header: item counts [3], heavy rows and pieces [2 x 2], profile counters [6] (u64:
+  // header: item counts [3], heavy rows and pieces [2], profile counters [6] (u64:
   // entries walked by the write / final / heavy write / heavy final kernels,
   // bytes written by the write / heavy write kernels), queues [3 main + 2
   // heavy] of WQ_WORDS words, result counters [cap] (u64, a cache line each:
   // the waves of one launch add to several of them at once)
-  static constexpr size_t HDR_NITEMS = 0, HDR_HEAVYN = 16, HDR_PITEMS = 32, HDR_QUEUE = 128,
+  static constexpr size_t HDR_NITEMS = 0, HDR_HEAVYN = 16, HDR_PITEMS = 64, HDR_QUEUE = 128,
                           HDR_CTR = HDR_QUEUE + 5 * 4 * WQ_WORDS, CTR_STRIDE = 8;
   uint32_t cap = 0;  // items per launch = counters
   // one block, on both sides: header, block prefixes [3][cap + 1] and items
@@ -1163,8 +1160,8 @@ struct ExtSlot {
     heavy_chunk = c->heavy_chunk;
     hdr_bytes = HDR_CTR + 8ull * CTR_STRIDE * cap;
     for (int i = 0; i < 2; ++i) {
-      heavy[i].alloc(sizeof(HeavyRow) * HEAVY_CAP, s);
-      pieces[i].alloc(4ull * PIECE_CAP, s);
+      heavy[i].alloc(sizeof(HeavyRow) * gemh::HEAVY_CAP, s);
+      pieces[i].alloc(4ull * gemh::PIECE_CAP, s);
     }
     const size_t blk_bytes = 8ull * (cap + 1), item_bytes = sizeof(VItem) * cap;
     len_bytes = blk_bytes + item_bytes;
@@ -1235,7 +1232,7 @@ struct ExtSlot {
     GEM_HIP_CHECK(hipMemcpyAsync(d, host, step_bytes, hipMemcpyHostToDevice, s));
     const uint32_t *dn = reinterpret_cast<const uint32_t *>(d + HDR_NITEMS);
     unsigned int *dq = reinterpret_cast<unsigned int *>(d + HDR_QUEUE);
-    unsigned int *hn = reinterpret_cast<unsigned int *>(d + HDR_HEAVYN);
+    auto *hn = reinterpret_cast<gemh::HeavyCounters *>(d + HDR_HEAVYN);
     // a captured step holds every kernel (one without items ends at once);
     // an eager one launches those that have items
     uint64_t e[3];
@@ -1249,16 +1246,16 @@ struct ExtSlot {
   // capped batch, at 1024, 2048 and 4096: 70, 66 and 75 ms on 2^20 vertices, 82, 79
   // and 76 on 2^22).  Streamed walks take whole units: 2048 cost a streamed batch
   // 20%.
-  HeavyOut heavy_out(int i, unsigned int *hn) const {
-    return HeavyOut{heavy[i].as<HeavyRow>(), pieces[i].as<uint32_t>(), hn + 2 * i, heavy_t, heavy_chunk};
+  HeavyOut heavy_out(int i, gemh::HeavyCounters *hn) const {
+    return HeavyOut{heavy[i].as<HeavyRow>(), pieces[i].as<uint32_t>(), hn + i, heavy_t, heavy_chunk};
   }
 
   // (At most `most` blocks each.)  The three kernels over task ranges [b_i, e_i) of launch i (queues
   // dq, WQ_WORDS words each), then the heavy rows the two walking launches set
-  // aside (queues hq, rows and pieces hn[0..3]; everything starts at zero).
+  // aside (queues hq, rows and pieces hn[0..1]; everything starts at zero).
   template <bool OOC>
   void launch_kernels(gem_ctx *c, uint32_t most, const uint32_t *dn, unsigned int *dq, unsigned int *hq,
-                      unsigned int *hn, bool prof_kernels, bool count_items, uint64_t b0, uint64_t e0, uint64_t b1,
+                      gemh::HeavyCounters *hn, bool prof_kernels, bool count_items, uint64_t b0, uint64_t e0, uint64_t b1,
                       uint64_t e1, uint64_t b2, uint64_t e2) {
     hipStream_t s = c->stream;
     unsigned long long *dp = reinterpret_cast<unsigned long long *>(block.as<unsigned char>() + HDR_PITEMS);
@@ -1354,7 +1351,9 @@ struct ExtSlot {
         const uint32_t grd = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(~0u, most));
         // per group: 3 main queues, 2 heavy queues, heavy rows and pieces
         unsigned int *gq = q + (size_t)GROUP_WORDS * g;
-        launch_kernels<true>(c, grd, dn, gq, gq + 3 * WQ_WORDS, gq + 5 * WQ_WORDS, prof, prof, lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]);
+        auto *hn = reinterpret_cast<gemh::HeavyCounters *>(gq + 5 * WQ_WORDS);
+        launch_kernels<true>(c, grd, dn, gq, gq + 3 * WQ_WORDS, hn, prof, prof, lo[0], hi[0], lo[1], hi[1], lo[2],
+                             hi[2]);
         tc.done(g);
       }
       wa = wb;
