@@ -367,13 +367,39 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
       return std::max<uint64_t>(want >= 1.8e19 ? ~0ull : (uint64_t)want, cfg.final_piece);
     };
 
+    // Measures the next units of the top levels of these queries (query, units
+    // from its cursor on).
+    auto measure = [&](const std::vector<std::pair<uint32_t, uint64_t>> &next_units) {
+      std::vector<Item> items;
+      for (auto [qi, n] : next_units) {
+        const SLevel<Buf> &top = qs[qi]->stack.back();
+        Item it;
+        it.q = qi;
+        it.level = top.level;
+        it.k = top.k;
+        it.rows = top.rows.get();
+        it.row_begin = top.cursor * SCHED_UNIT;
+        it.row_end = std::min<uint64_t>((top.cursor + std::min(n, top.nunits() - top.cursor)) * SCHED_UNIT, top.nrows);
+        items.push_back(it);
+      }
+      ++st->length_passes;
+      std::vector<std::vector<uint64_t>> pref;
+      be.length_pass(items, &pref);
+      for (size_t t = 0; t < items.size(); ++t) {
+        SLevel<Buf> &top = qs[items[t].q]->stack.back();
+        top.unit_u = std::move(pref[t]);
+        top.unit_base = top.cursor;
+        top.measured_to = top.cursor + top.unit_u.size() - 1;
+        top.measured = true;
+      }
+    };
+
     // ---- length passes: output bounds of the next units of every top level,
     // as many as this iteration can use (final levels only when they walk
     // lists under a cap: their units are then counted a cap-sized piece at a
     // time)
     for (;;) {
-      std::vector<Item> items;
-      std::vector<uint32_t> owner;
+      std::vector<std::pair<uint32_t, uint64_t>> more;
       for (uint32_t qi : act) {
         SQuery<Buf> &S = *qs[qi];
         SLevel<Buf> &top = S.stack.back();
@@ -393,27 +419,10 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
           }
           seg = 4 * std::max(seg, top.measured_to - top.cursor);
         }
-        Item it;
-        it.q = qi;
-        it.level = top.level;
-        it.k = top.k;
-        it.rows = top.rows.get();
-        it.row_begin = top.cursor * SCHED_UNIT;
-        it.row_end = std::min<uint64_t>((top.cursor + std::min(seg, nu - top.cursor)) * SCHED_UNIT, top.nrows);
-        items.push_back(it);
-        owner.push_back(qi);
+        more.push_back({qi, seg});
       }
-      if (items.empty()) break;
-      ++st->length_passes;
-      std::vector<std::vector<uint64_t>> pref;
-      be.length_pass(items, &pref);
-      for (size_t t = 0; t < owner.size(); ++t) {
-        SLevel<Buf> &top = qs[owner[t]]->stack.back();
-        top.unit_u = std::move(pref[t]);
-        top.unit_base = top.cursor;
-        top.measured_to = top.cursor + top.unit_u.size() - 1;
-        top.measured = true;
-      }
+      if (more.empty()) break;
+      measure(more);
     }
 
     // ---- count-only pieces of final levels (no output memory)
@@ -468,9 +477,22 @@ void run_schedule(BE &be, std::vector<SQuery<typename BE::Buf> *> &qs, const Sch
 
     // ---- output chunks under the budget
     const uint64_t left = budget > live ? budget - live : 0;
+    const uint64_t force = cfg.force_chunk ? cfg.force_chunk : budget / 32;
     std::vector<uint64_t> end;
-    const int forced = plan_chunks(cand, left, cfg.max_chunk, cfg.force_chunk ? cfg.force_chunk : budget / 32,
-                                   !fin.empty(), &end);
+    int forced = plan_chunks(cand, left, cfg.max_chunk, force, !fin.empty(), &end);
+    // a forced chunk may be longer than the query's share, up to which its level
+    // is measured: it ends where it does in a level measured whole
+    while (forced >= 0) {
+      const uint32_t qi = cand_owner[(size_t)forced];
+      SLevel<Buf> &top = qs[qi]->stack.back();
+      ChunkCand &f = cand[(size_t)forced];
+      if (top.measured_to >= top.nunits() || end[(size_t)forced] < f.nunits) break;
+      if (top.bound(top.cursor, top.measured_to) * f.row_bytes > std::min(cfg.max_chunk, force)) break;
+      measure({{qi, 4 * std::max(cfg.measure_units, top.measured_to - top.cursor)}});
+      f.cursor = top.cursor - top.unit_base;
+      f.nunits = top.measured_to - top.unit_base;
+      forced = plan_chunks(cand, left, cfg.max_chunk, force, !fin.empty(), &end);
+    }
     uint64_t charged = live;
     for (size_t c = 0; c < cand.size(); ++c) {
       const uint32_t qi = cand_owner[c];
