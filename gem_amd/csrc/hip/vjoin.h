@@ -6,6 +6,7 @@
 
 #include "../host/heavy_pieces.h"
 #include "../host/vsched.h"
+#include "../host/walk_runs.h"
 #include "ctx.h"
 
 namespace gemd {

@@ -121,12 +121,14 @@ __global__ void __launch_bounds__(VB) k_vlen(const VItem *__restrict__ items, ui
 // ns whatever asks: 8,192 waves finding an empty queue took 95 us, and a queue
 // of 64-row tasks bounded every large launch.  Runs are as long as leaves a
 // wave about CLAIMS of them, so uneven tasks still even out.
-constexpr uint32_t CLAIMS = 4, MAX_RUN = 32;
+using gemh::CLAIMS;
+using gemh::MAX_RUN;
 struct Runs {
   uint32_t ntask, nrun, run;
   uint32_t per, nq, sub, given;
   unsigned int *q;
-  // n tasks (rows / 64: below 2^32); w, nw: this wave and the waves of the grid
+  // n tasks, below gemh::RUN_LIMIT: 64-row units of the rows in memory, or runs
+  // that gemh::plan_runs made; w, nw: this wave and the waves of the grid
   __device__ __forceinline__ Runs(uint64_t n, uint32_t w, uint32_t nw, uint32_t max_run, unsigned int *queue)
       : ntask((uint32_t)n), run(w) {
     const uint32_t p = ntask / (nw * CLAIMS);
@@ -160,9 +162,8 @@ __device__ __forceinline__ uint64_t list_addr(CLevel &L, uint32_t j, uint32_t p,
 }
 
 // ------------------------------------------------------ extend (walk) pass
-// Cost of a 64-row unit besides the entries it walks, in entries: its rows'
-// setup.  A run of a write walk has at most RUN_COST of it.
-constexpr uint32_t UNIT_COST = 256, RUN_COST = UNIT_COST * MAX_RUN;
+using gemh::RUN_COST;
+using gemh::UNIT_COST;
 
 // A unit that costs more than this part of a run is cut between its rows: row
 // i starts at the unit's cost plus UNIT_COST / 64 a row and the entries of the
@@ -1494,13 +1495,21 @@ struct HipSchedBackend {
     return old;
   }
 
-  // Item x to a launch whose waves take runs of about `cost` of it.
-  void add_by_cost(Launch &L, VItem it, const Item &x, uint64_t cost) {
+  // Runs of the walks over these items, CLAIMS per wave of the grid by cost (an
+  // entry of a level with other lists costs its searches too); false: too many
+  bool plan_runs(const std::vector<Item> &items, uint32_t grid, std::vector<uint32_t> *cost) const {
+    std::vector<gemh::WalkPiece> pieces;
+    for (const Item &x : items) pieces.push_back({x.out_rows, units_of(x), 4ull * qs[x.q]->max_nb[x.level] - 3});
+    return gemh::plan_runs(pieces, (uint64_t)grid * VW, cost);
+  }
+
+  // Item x to a launch whose waves take runs of `run_cost` of it.
+  void add_by_cost(Launch &L, VItem it, const Item &x, uint32_t run_cost) {
     it.units = x.rows->units.prefix->as<uint64_t>() + x.rows->units.unit0 + x.row_begin / gemh::SCHED_UNIT;
     it.nunits = (uint32_t)units_of(x);
-    it.run_cost = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(cost, 4 * UNIT_COST), RUN_COST);
+    it.run_cost = run_cost;
     L.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level],
-          (x.out_rows + UNIT_COST * units_of(x) - 1) / it.run_cost + 1);
+          gemh::WalkPiece{x.out_rows, units_of(x), 1}.runs(run_cost));
   }
 
   void extend(const std::vector<Item> &wr_items, const std::vector<Item> &fin_items, std::vector<uint64_t> *got_wr,
@@ -1513,40 +1522,32 @@ struct HipSchedBackend {
     size_t nctr = 0;
     // counters / work queues / walked-entry counts travel zeroed in the copy
     std::memset(slot.h_hdr + ExtSlot::HDR_HEAVYN, 0, slot.hdr_bytes - ExtSlot::HDR_HEAVYN);
-    // runs of the write walks (see unit_range): CLAIMS per wave of the grid by
-    // cost, an entry of a level with other lists costing its searches too
-    auto weight = [&](const Item &x) { return 4ull * qs[x.q]->max_nb[x.level] - 3; };
-    uint64_t run_cost = 0, fin_cost = 0;
+    // runs of the write walks (see unit_range), and of the final ones when all
+    // their pieces are measured (they are under a cap) and the runs few enough
+    std::vector<uint32_t> wr_cost, fin_cost;
     std::vector<std::pair<const LevelBuf *, LevelBuf::Units>> replaced;
-    // final walks: when all their pieces are measured (they are under a cap)
-    std::vector<Item> walked;
-    bool measured = !tc;
-    for (const Item &x : fin_items)
-      if (qs[x.q]->max_nb[x.level] > 1) {
-        walked.push_back(x);
-        measured = measured && x.out_rows;
-      }
-    if (measured && !walked.empty()) {
-      uint64_t cost = 0;
-      for (const Item &x : walked) cost += (x.out_rows + UNIT_COST * units_of(x)) * weight(x);
-      fin_cost = cost / ((uint64_t)slot.grid[1] * VW * CLAIMS) + 1;
-    } else {
-      walked.clear();
-    }
     if (!tc) {
-      uint64_t cost = 0;
-      for (const Item &x : wr_items) cost += (x.out_rows + UNIT_COST * units_of(x)) * weight(x);
-      run_cost = cost / ((uint64_t)slot.grid[0] * VW * CLAIMS) + 1;
+      std::vector<Item> walked;
+      bool measured = true;
+      for (const Item &x : fin_items)
+        if (qs[x.q]->max_nb[x.level] > 1) {
+          walked.push_back(x);
+          measured = measured && x.out_rows;
+        }
+      if (!measured || !plan_runs(walked, slot.grid[1], &fin_cost)) walked.clear();
+      if (!plan_runs(wr_items, slot.grid[0], &wr_cost))
+        throw Error{GEM_E_LIMIT, "too many runs in one write walk"};
       walked.insert(walked.end(), wr_items.begin(), wr_items.end());
       replaced = remeasure(walked);
     }
+    size_t nwr = 0, nfin = 0;
     for (const Item &x : wr_items) {
       VItem it = vitem(x);
       it.out = x.out->as<uint32_t>();
       it.out_cap = x.out_rows;
       it.counter = slot.dev_counter(nctr++);
-      if (run_cost)
-        add_by_cost(wr, it, x, run_cost / weight(x));
+      if (!tc)
+        add_by_cost(wr, it, x, wr_cost[nwr++]);
       else
         wr.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level]);
     }
@@ -1558,8 +1559,8 @@ struct HipSchedBackend {
       it.counter = slot.dev_counter(nctr++);
       if (qs[x.q]->max_nb[x.level] == 1)
         fin1.add(it, 1, qs[x.q]->max_ndup[x.level]);
-      else if (fin_cost)
-        add_by_cost(fin, it, x, fin_cost / weight(x));
+      else if (!fin_cost.empty())
+        add_by_cost(fin, it, x, fin_cost[nfin++]);
       else
         fin.add(it, qs[x.q]->max_nb[x.level], qs[x.q]->max_ndup[x.level]);
     }
