@@ -98,6 +98,7 @@ SIGNATURES = [
     ("gem_hip_set_heavy_split", C.c_int, [C.c_void_p, C.c_uint32, C.c_uint32]),
     ("gem_hip_set_graph", C.c_int, [C.c_void_p, C.c_int]),
     ("gem_hip_set_graph_residency", C.c_int, [C.c_void_p, C.c_int]),
+    ("gem_hip_set_slot_labels", C.c_int, [C.c_void_p, C.c_uint64]),
     ("gem_hip_set_relaxed_sharing", C.c_int, [C.c_void_p, C.c_int]),
     ("gem_hip_set_racing", C.c_int, [C.c_void_p, C.c_int]),
     ("gem_hip_set_prep_overlap", C.c_int, [C.c_void_p, C.c_int]),

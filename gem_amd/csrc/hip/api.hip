@@ -174,6 +174,12 @@ int gem_hip_set_graph_residency(gem_ctx *c, int host) {
   return GEM_OK;
 }
 
+int gem_hip_set_slot_labels(gem_ctx *c, uint64_t max_bytes) {
+  if (!c) return GEM_E_INVALID;
+  c->slot_label_bytes = max_bytes;
+  return GEM_OK;
+}
+
 int gem_hip_set_graph(gem_ctx *c, int on) {
   if (!c) return GEM_E_INVALID;
   c->use_graph = on != 0;
@@ -260,8 +266,8 @@ int gem_hip_load_data_csr(gem_ctx *c, const gem_csr_view *g) {
     }
     GEM_HIP_CHECK(hipMemcpyAsync(G.off.p, g->offsets, ((uint64_t)G.n + 1) * 8, hipMemcpyHostToDevice, s));
     if (c->graph_host) {
-      // Host-resident graph: the neighbour array (all but 12 B per vertex of
-      // the CSR) stays in host memory, pinned and mapped; the filter and table
+      // Host-resident graph: the neighbour array stays in host memory, pinned and
+      // mapped (offsets, labels and the slots' label bytes do not); the filter and table
       // kernels read it over PCIe, non-coherent so that L2 may cache it.
       G.nbr_host.alloc(std::max<uint64_t>(G.slots, 1) * 4, hipHostMallocMapped | hipHostMallocNonCoherent);
       parallel_copy(G.nbr_host.p, g->neighbors, G.slots * 4);

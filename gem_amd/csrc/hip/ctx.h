@@ -165,7 +165,9 @@ struct GraphDev {
   PinnedBuf nbr_host;  // u32[slots] in mapped pinned host memory (host-resident graph)
   const uint32_t *nbr_mapped = nullptr;  // device address of nbr_host
   DevBuf lab;     // u8[n] or u32[n] dense label ids
-  DevBuf nbr_lab; // u8[slots + 16] label of each adjacency slot's neighbour (byte labels; none if it does not fit)
+  // u8[slots + 16] label of each adjacency slot's neighbour, in HBM also when
+  // the neighbours are not (byte labels; none past gem_ctx::slot_label_bytes)
+  DevBuf nbr_lab;
   bool lab8 = true;
   std::unordered_map<uint32_t, uint32_t> label_id;  // original -> dense
   std::vector<uint64_t> label_freq;                 // dense id -> #vertices
@@ -286,6 +288,7 @@ struct gem_ctx {
   uint32_t heavy_t = 1024, heavy_chunk = 1024;  // batched walks: long driving lists split over waves
   uint32_t max_active = 64;                 // batched path: queries running at once (0 = all)
   int graph_host = 0;                       // next data graph: neighbours stay in pinned host memory
+  uint64_t slot_label_bytes = ~0ull;        // next data graph: largest slot label array (~0: by the free memory)
   bool relaxed_share = true;                // relaxed queries share one filter and one table build
   bool racing = true;                       // batched learned path: twins race stragglers
   bool prep_overlap = true;                 // batched learned path: later queries prepared during the join
@@ -416,7 +419,8 @@ inline void settle_times(gem_ctx *c) {
 // The data graph a context's filter and table kernels read.
 inline const GraphDev &graph(const gem_ctx *c) { return c->gsrc ? *c->gsrc : c->g; }
 
-// Labels of the adjacency slots of a loaded graph (when they fit).
+// Labels of the adjacency slots of a graph whose other arrays are loaded (when
+// they fit).
 void make_slot_labels(gem_ctx *c, GraphDev &G);
 void run_filter(gem_ctx *c, const gem_query_view *qv, uint32_t T);
 void run_tables(gem_ctx *c);

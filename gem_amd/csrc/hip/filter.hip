@@ -316,14 +316,26 @@ __global__ void k_slot_labels(const uint32_t *__restrict__ nbr, uint64_t slots, 
 
 void make_slot_labels(gem_ctx *c, GraphDev &G) {
   if (!G.lab8 || !G.slots) return;
-  // a quarter of the free memory at most (asked for when it could matter): a
-  // larger graph keeps the gathers
-  if (G.slots > (1ull << 28)) {
-    size_t free_b = 0, total_b = 0;
-    GEM_HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
-    if (G.slots > (free_b + pool_reusable_bytes()) / 4) return;
+  // A graph works without them (with gathers), so they are left out rather than
+  // failing a load: past the context's limit, by default a quarter of the free
+  // memory (asked for past 16 MiB: the answer takes 0.7 ms), or when refused.
+  const uint64_t bytes = G.slots + 16;
+  uint64_t most = c->slot_label_bytes;
+  if (most == ~0ull) {
+    most = 16ull << 20;
+    if (bytes > most) {
+      size_t free_b = 0, total_b = 0;
+      GEM_HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+      most = std::max<uint64_t>(most, (free_b + pool_reusable_bytes()) / 4);
+    }
   }
-  G.nbr_lab.alloc(G.slots + 16, c->stream);
+  if (bytes > most) return;
+  try {
+    G.nbr_lab.alloc(bytes, c->stream);
+  } catch (const Error &e) {
+    if (e.code != GEM_E_NOMEM) throw;
+    return;
+  }
   k_slot_labels<<<(uint32_t)std::min<uint64_t>((G.slots + 255) / 256, 16384), 256, 0, c->stream>>>(
       G.nbr_dev(), G.slots, G.lab.as<uint8_t>(), G.n, G.nbr_lab.as<uint8_t>());
   GEM_LAUNCH_CHECK("k_slot_labels");

@@ -193,6 +193,13 @@ class GemContext:
         host memory (read over PCIe by the filter and table kernels)."""
         self._check(self._lib.gem_hip_set_graph_residency(self._h, int(bool(host))), "gem_hip_set_graph_residency")
 
+    def set_slot_labels(self, max_bytes=None):
+        """Largest array of adjacency-slot labels (one byte a slot, in HBM) that
+        the next load_data may make: 0 leaves it out, None goes by the device
+        memory free then."""
+        limit = 2 ** 64 - 1 if max_bytes is None else int(max_bytes)
+        self._check(self._lib.gem_hip_set_slot_labels(self._h, limit), "gem_hip_set_slot_labels")
+
     def set_max_active(self, queries):
         """Queries of a batched run holding join levels at once (0 = all)."""
         self._check(self._lib.gem_hip_set_max_active(self._h, int(queries)), "gem_hip_set_max_active")

@@ -191,8 +191,20 @@ int gem_hip_load_data_csr(gem_ctx *ctx, const gem_csr_view *g);
  * out-of-core/lib/structure/src/unifiedTrie.cu:1224-1427): host = 0, in HBM
  * (default); host = 1, in pinned, mapped host memory that the filter and
  * table kernels read over PCIe, for graphs larger than HBM.  Offsets and
- * labels (12 B per vertex) stay in HBM.  Results do not depend on it. */
+ * labels (9 B per vertex with at most 255 labels, else 12), the ids of the
+ * vertices of degree above 64 (4 B each) and, by default, the slot labels below
+ * (1 B per adjacency slot) stay in HBM.  Results do not depend on it. */
 int gem_hip_set_graph_residency(gem_ctx *ctx, int host);
+/* Labels of the adjacency slots (no reference counterpart): when the next
+ * gem_hip_load_data_csr's graph has at most 255 labels, it also makes an array in
+ * HBM with the label of each adjacency slot's neighbour, num_slots + 16 bytes,
+ * wherever the neighbours are.  The filter then reads that instead of neighbours
+ * and their labels.  max_bytes: largest such array; 0 leaves it out; UINT64_MAX
+ * (default): up to a quarter of the device memory free then, or 16 MiB.  It is
+ * also left out when the device refuses the allocation.  It counts as used where
+ * a default level budget is taken from the free memory.  Results do not depend
+ * on it. */
+int gem_hip_set_slot_labels(gem_ctx *ctx, uint64_t max_bytes);
 
 /* Candidate filter for a new query (replaces filterSSM,
  * in-core/lib/filter/src/filter.cu:34-167 and the CPU form
