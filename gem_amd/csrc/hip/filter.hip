@@ -510,7 +510,7 @@ void run_filters(gem_ctx *c, QueryDev *Qds, const gem_query_view *const *qv, uin
     Qd.W = W;
     filter_prepare(G, Qd.Q, T, W, &P);
     Qd.can_off = P.can_off;
-    GEM_HIP_CHECK(hipEventRecord(c->ev[0], s));
+    if (!i) GEM_HIP_CHECK(hipEventRecord(c->ev[0], s));
     FilterBufs B;
     DevBuf &slot_of = runs[i].slot_of, &sums = runs[i].sums;
     if (!G.lab8) {
@@ -533,8 +533,8 @@ void run_filters(gem_ctx *c, QueryDev *Qds, const gem_query_view *const *qv, uin
     // adjacency slot of a label-matching vertex (neighbour id + its label; 1 B
     // with slot labels), the candidate bitmaps written
     prof_bytes(c, K_FILTER, 16.0 * G.n + (G.nbr_lab.p ? 1.0 : 8.0) * P.adj + nv * (double)W * 8);
-    GEM_HIP_CHECK(hipEventRecord(c->ev[1], s));
   }
+  GEM_HIP_CHECK(hipEventRecord(c->ev[1], s));
   GEM_HIP_CHECK(hipStreamSynchronize(s));
   hq = h;
   for (uint32_t i = 0; i < n; ++i) {
@@ -548,7 +548,8 @@ void run_filters(gem_ctx *c, QueryDev *Qds, const gem_query_view *const *qv, uin
     Qd.filtered = true;
   }
   prof_flush(c);
-  float ms = 0;  // the last query's
+  if (!n) return;
+  float ms = 0;  // of all n
   GEM_HIP_CHECK(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
   c->times.filter_ms = ms;
   c->times.index_ms = 0;  // the index (bitmap + rank) is a by-product of the filter

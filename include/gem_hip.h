@@ -295,7 +295,11 @@ int gem_hip_join(gem_ctx *ctx, const uint32_t *edge_order, uint64_t cap,
 
 /* Phase timings (milliseconds, HIP events on the context stream) of the
  * last filter / table build / join, mirroring the reference's printed phases
- * (in-core/src/main.cu:147-227). */
+ * (in-core/src/main.cu:147-227).  A batched run filters, and tables, up to 32
+ * queries together (one at a time with streamed tables): filter_ms and tables_ms
+ * are then those of the last such group.  The batched learned path gives the sums
+ * over its run, by the host's clock (a group's last table pass may still run on
+ * the device when its time is taken). */
 typedef struct gem_phase_times {
   float filter_ms;
   float index_ms;
