@@ -556,11 +556,10 @@ void run_filters(gem_ctx *c, QueryDev *Qds, const gem_query_view *const *qv, uin
 }
 
 // ------------------------------------------------ no-allocation variant
-// Scratch of gem_hip_filter_noalloc: the query description, the label map,
-// candidate-list offsets, bitmaps, tile counts, ranks and the heavy/hub lists
-// of one call, carved from one fixed device array (each device holds its own
-// copy until the process ends).  Calls that overlap on one device share it and
-// race.
+// Scratch of gem_hip_filter_noalloc: the label map, bitmaps, rank chunk sums and
+// ranks of one call, carved from one fixed device array (each device holds its
+// own copy until the process ends).  Calls that overlap on one device share it
+// and race.
 constexpr uint64_t FILTER_SCRATCH_BYTES = 64ull << 20;
 constexpr int SCRATCH_MAX_DEVICES = 64;
 static __device__ __align__(256) unsigned char scratch[FILTER_SCRATCH_BYTES];
@@ -578,6 +577,9 @@ void filter_scratch_init(int device) {
   g_scratch_ptr[device] = static_cast<unsigned char *>(p);
 }
 
+// What a call is accepted by: the documented bound, which does not move with the
+// kernels.  They take less than it (its terms: a query description, the label
+// map, list offsets, bitmaps, a count per tile, ranks, and vertex lists).
 uint64_t filter_scratch_bytes(const GraphDev &G, uint32_t nv) {
   const uint64_t W = (G.n + 63) / 64;
   const uint64_t hub_cap = std::max<uint32_t>(G.n_hub, 1);

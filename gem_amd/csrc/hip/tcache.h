@@ -71,8 +71,8 @@ class TableCache {
   bool plan(uint64_t total_tasks);
   const std::vector<Group> &groups() const { return groups_; }
   // Device counters for the group launches, zeroed: per group (GROUP_WORDS
-  // words) 3 work queues,
-  // 2 heavy-row queues and the heavy rows and pieces of both walks.
+  // words) 3 work queues, 2 heavy-row queues and the heavy rows and pieces of
+  // both walks.
   unsigned int *queues();
   // Copy stream: group g's block loads and map updates; the context stream
   // waits for them.

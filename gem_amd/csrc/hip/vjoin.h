@@ -41,9 +41,12 @@ struct VItem {
   const uint32_t *rows;
   uint64_t row_begin, row_end;
   uint32_t k;
-  uint32_t nunits;        // write walks: 64-row units of the range,
-  uint32_t run_cost, pad; // the cost of a wave's run of them
-  const uint64_t *units;  // and the prefix of their output bounds (nunits + 1)
+  // walks in runs of equal cost (write walks, measured final ones; run_cost 0:
+  // whole units): 64-row units of the range, the cost of a wave's run of them,
+  // and the prefix of their output bounds (nunits + 1)
+  uint32_t nunits;
+  uint32_t run_cost, pad;
+  const uint64_t *units;
   uint32_t *out;
   uint64_t out_cap;
   unsigned long long *counter;

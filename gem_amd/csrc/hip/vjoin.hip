@@ -31,9 +31,12 @@
 // out their places (one address serves one per 9-11 ns).  Hence rows hold only
 // the columns that are read again (VLevel::src; 2.1x fewer bytes written on 16
 // queries of up to 24 vertices, 2^20 R-MAT), and places are reserved once per
-// run of a one-list level and once per full stage of the others.  k_vext<write>
-// of one pass: 190 -> 107 ms on those queries, 13.3 -> 2.5 ms on 24 exact
-// queries of 4-9 vertices on 2^18.
+// run of a one-list level and once per full stage of the others.  With runs of
+// equal cost, units cut between rows and the searches below, k_vext<write> of
+// one pass went from 190 to 63 ms on those queries, from 13.3 to 2.1 ms on 24
+// exact queries of 4-9 vertices on 2^18.  While it runs now (63 ms pass), the L1
+// serves an access in three of four cycles, the vector units issue in two of
+// five, and rows go to HBM at 1.8 TB/s.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -1251,9 +1254,10 @@ struct ExtSlot {
     return HeavyOut{heavy[i].as<HeavyRow>(), pieces[i].as<uint32_t>(), hn + i, heavy_t, heavy_chunk};
   }
 
-  // (At most `most` blocks each.)  The three kernels over task ranges [b_i, e_i) of launch i (queues
-  // dq, WQ_WORDS words each), then the heavy rows the two walking launches set
-  // aside (queues hq, rows and pieces hn[0..1]; everything starts at zero).
+  // The three kernels over task ranges [b_i, e_i) of launch i (queues dq,
+  // WQ_WORDS words each), then the heavy rows the two walking launches set
+  // aside (queues hq, rows and pieces hn[0..1]; everything starts at zero), in
+  // at most `most` blocks each.
   template <bool OOC>
   void launch_kernels(gem_ctx *c, uint32_t most, const uint32_t *dn, unsigned int *dq, unsigned int *hq,
                       gemh::HeavyCounters *hn, bool prof_kernels, bool count_items, uint64_t b0, uint64_t e0, uint64_t b1,

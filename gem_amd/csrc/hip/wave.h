@@ -29,7 +29,6 @@ __device__ __forceinline__ u64x2 ld_pair(const uint64_t *p) {
   return *(const __attribute__((address_space(1))) u64x2 *)p;
 }
 
-// task g (global block index of the launch) -> item t, row block within item
 // Up to four consecutive words in one store.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x3 __attribute__((ext_vector_type(3), aligned(4)));

@@ -114,12 +114,12 @@ struct VertexPlan {
 // Vertex order of first appearance along a connected edge order, starting at
 // the non-leaf endpoint of the first edge (as the reference's first table).
 int vertex_order_from_edges(const QueryInfo &q, const uint32_t *edge_order, std::vector<uint32_t> *vorder);
-// Requires vorder[0] to be a non-leaf and every later vertex to have an
-// earlier neighbour.
 // live[i] (i >= 1): the vertex-order positions below i that level i or a later
 // one reads, as the key of a backward list or as an equal-label column,
 // ascending.  Level i's input rows hold these columns only.
 void live_columns(const VertexPlan &plan, std::vector<std::vector<uint32_t>> *live);
+// Requires vorder[0] to be a non-leaf and every later vertex to have an
+// earlier neighbour.
 int make_vertex_plan(const QueryInfo &q, const std::vector<uint32_t> &vorder, VertexPlan *plan);
 
 // ------------------------------------------------------- learned ordering

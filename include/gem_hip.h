@@ -312,6 +312,10 @@ int gem_hip_phase_times(const gem_ctx *ctx, gem_phase_times *out);
  * phases on the host only, in-core/src/main.cu:147-227).  While on, every
  * launch of the library's kernels is bracketed by HIP events on the context
  * stream and its algorithmic bytes (compulsory traffic) are accumulated.
+ * It changes what some calls launch: a counting join (gem_hip_match, gem_hip_join
+ * without embeddings) then runs step by step, as with a step log, in place of its
+ * chained and fused steps (k_chain, k_expand_select, which have no statistics
+ * here), and the batched paths run eagerly and prepare no query beside the join.
  * gem_hip_set_profiling(ctx, 1) also clears the statistics. */
 typedef struct gem_kernel_stat {
   char name[40];
